@@ -111,6 +111,61 @@ def test_full_58300_pair_sweep(cx):
     _check((st[sel], pnl[sel]), (rst, rpnl), "58,300 sample")
 
 
+_ONE = dict(offset=(0.85, 0.85, 0.0), sigma=(6.0, 6.0, 0.0))
+
+
+@pytest.mark.parametrize("bars,lead,fast,slow", [
+    (40, 0, (2, 9, 1), (3, 30, 1)),            # shorter than two words, warm-ups to its end
+    (1_055, 7, (3, 3, 0), (17, 17, 0)),        # one pair, one segment, a part word at each end
+    (2_049, 0, (5, 21, 1), (8, 24, 1)),        # 17 x 17: tiles of one row; equal rows inside
+    (9_001, 130, (2, 34, 2), (2, 34, 2)),      # every pair mirrored, the diagonal flat
+    (70_003, 0, (5, 60, 11), (200, 294, 47)),  # many segments, the longest periods
+])
+def test_word_and_tile_edges_bit_exact(cx, bars, lead, fast, slow):
+    """Series and grids that are no multiple of the walk's 32-bar words,
+    segments or 16 x 16 tiles."""
+    x = datagen.gbm_close(bars, 0.015, seed=bars)
+    x[:lead] = np.nan
+    f, s = vta.AlmaBatchRange(period=fast, **_ONE), vta.AlmaBatchRange(period=slow, **_ONE)
+    got = cx.run(x, f, s)
+    *_, ref = _oracle(x, f, s)
+    _check(got, ref, f"{bars} bars")
+
+
+def test_ties_and_undefined_rows_bit_exact(cx):
+    """Words that are all ties (a constant stretch longer than every window,
+    entered and left), and a row whose weights underflow to a zero sum (its
+    values are NaN, its pairs never hold a position)."""
+    rng = np.random.Generator(np.random.PCG64(75))
+    x = datagen.gbm_close(6_000, 0.015, seed=76)
+    x[1_000:2_500] = np.float32(64.0)
+    x[4_000:4_500] = np.repeat(x[4_000:4_500:50], 50)
+    x[5_000:] = rng.choice(np.array([1.0, 2.0], dtype=np.float32), size=1_000)
+    f = vta.AlmaBatchRange(period=(4, 32, 4), offset=(0.85, 0.85, 0.0), sigma=(6.0, 1e6, 999_994.0))
+    s = vta.AlmaBatchRange(period=(8, 40, 8), offset=(0.5, 0.85, 0.35), sigma=(6.0, 6.0, 0.0))
+    got = cx.run(x, f, s)
+    rows, idx, fc, sc, ref = _oracle(x, f, s)
+    assert np.isnan(rows[:, 500]).any()
+    _check(got, ref, "ties")
+    assert (ref[0][:, 1] + ref[0][:, 2] < 5_000).any()
+
+
+def test_rows_past_4_gib(cx):
+    """290 rows x 1.9M bars of f64 (4.4 GB): the walk's 64-bit row offsets.
+    Sampled pairs against the oracle; the pairs' own rows are the last ones."""
+    x = datagen.gbm_close(1_900_000, 0.0005, seed=77)
+    f = vta.AlmaBatchRange(period=(5, 294, 1), **_ONE)
+    s = vta.AlmaBatchRange(period=(40, 290, 250), **_ONE)
+    st, pnl = cx.run(x, f, s)
+    sel = [0, 35, 200, 289]
+    fp = [5 + i for i in sel]
+    rows = O.alma_batch(x.astype(np.float64), [(p, 0.85, 6.0) for p in fp + [40, 290]], nthreads=0)
+    rst, rpnl = O.cross_pairs(rows, x.astype(np.float64), [0, 0, 1, 1, 2, 2, 3, 3],
+                              [4, 5] * 4)
+    at = [2 * i + j for i in sel for j in (0, 1)]
+    _check((st[at], pnl[at]), (rst, rpnl), "rows past 4 GiB")
+
+
 def test_errors(cx):
     x = datagen.gbm_close(5_000, 0.015, seed=74)
     x[3_000] = np.nan

@@ -22,7 +22,8 @@ struct cross_args_host {
     const int32_t *row_period;
     const int32_t *fast_row;
     const int32_t *slow_row;
-    long long *part_i;
+    int32_t *part_n;
+    long long *part_ck;
     double *part_pnl;
     long long *out_i;
     double *out_pnl;
@@ -34,19 +35,26 @@ struct cross_args_host {
     int seg_len;
     int pmax;
     int ntiles_s;
-    int row_tile;
+    int ntiles;
+    int ldr;
+    uint32_t rows_bytes;
     int pad_;
 };
-static_assert(sizeof(cross_args_host) == 128, "cross_args layout");
+static_assert(sizeof(cross_args_host) == 144, "cross_args layout");
 
 constexpr size_t kMaxPeriod = 294;   // LDS staging of the f64 row kernel
 constexpr int kRowTile = 2048;       // bars per cross_rows_f64 workgroup (RW_T)
-// Workgroups of the pair walk (16 x 16 pairs x one time segment each).
-// Tiles of short periods trade more often and walk longer, so small units
-// balance the device: 58,300 pairs x 200k bars took 6.73 / 5.76 / 5.28 /
-// 5.18 / 5.12 / 5.11 ms at 2,048 / 4,046 / 8,100 / 12,000 / 16,000 / 23,000
-// workgroups (at most one segment per 2,048 bars).
-constexpr size_t kCrossWorkgroups = 16384;
+constexpr int kTileF = 16, kTileS = 16;   // pairs per wave of the walk (CR_F, CR_S)
+constexpr size_t kWord = 32;              // bars per word of the walk (CR_CH)
+// Waves of the pair walk (16 x 16 pairs x one time segment each).  Tiles of
+// short periods trade more often and walk longer, so small units balance the
+// device: 58,300 pairs x 200k bars took 2.46 / 2.31 / 2.21 / 2.20 ms (the
+// whole call) at 4,096 / 8,192 / 16,384 / 32,768 waves.  Segments are at least
+// 1,024 bars (the partials of a segment are read again) and a multiple of 8
+// in number (one XCD takes every 8th).
+constexpr size_t kCrossWaves = 16384;
+constexpr size_t kSegMin = 1024;
+constexpr size_t kSegMax = (size_t)1 << 18;   // CrossRun::s2
 
 // f64 batch weights in the oracle's order (alma.rs:1426-1436), not normalised.
 double weights_batch_raw(size_t period, double offset, double sigma, double *w) {
@@ -68,9 +76,9 @@ double weights_batch_raw(size_t period, double offset, double sigma, double *w) 
 struct vta_double_alma_plan {
     vta_ctx *ctx = nullptr;
     size_t T = 0, fv = 0;
-    int nfast = 0, nslow = 0, nrows = 0, pmax = 0, nseg = 0, seg_len = 0;
-    DevBuf prices, rows, w64, inv64, row_period, fast_row, slow_row, part_i, part_pnl, out_i,
-        out_pnl;
+    int nfast = 0, nslow = 0, nrows = 0, pmax = 0, nseg = 0, seg_len = 0, ntiles = 0, ldr = 0;
+    DevBuf prices, rows, w64, inv64, row_period, fast_row, slow_row, part_n, part_ck,
+        part_pnl, out_i, out_pnl;
 };
 
 namespace {
@@ -115,22 +123,26 @@ vta_status plan_build(vta_ctx *ctx, const float *prices, size_t len,
         return fail(VTA_ERR_INVALID_INPUT, "crossover supports periods <= %zu (got %zu)",
                     kMaxPeriod, pmax);
     const size_t nrows = rows.size();
+    const size_t ldr = (len + 63) & ~(size_t)63;   // whole words, 16-byte loads
     size_t npairs, rows_bytes;
     if (!mul_ok(fast.size(), slow.size(), &npairs) || npairs > (size_t)INT32_MAX ||
-        !mul_ok(nrows, len * sizeof(double), &rows_bytes))
+        !mul_ok(nrows, ldr * sizeof(double), &rows_bytes))
         return fail(VTA_ERR_INVALID_INPUT, "grid too large");
-    // time segments: about kCrossWorkgroups workgroups (VTA_CROSS_WGS overrides)
-    const size_t ntiles = ((fast.size() + 15) / 16) * ((slow.size() + 15) / 16);
-    size_t wgs = kCrossWorkgroups;
+    // time segments: about kCrossWaves waves (VTA_CROSS_WGS overrides)
+    const size_t ntiles =
+        ((fast.size() + kTileF - 1) / kTileF) * ((slow.size() + kTileS - 1) / kTileS);
+    size_t waves = kCrossWaves;
     if (const char *e = getenv("VTA_CROSS_WGS")) {
         const long v = atol(e);
-        if (v >= 1) wgs = (size_t)v;
+        if (v >= 1) waves = (size_t)v;
     }
-    size_t nseg = std::max<size_t>(1, (wgs + ntiles - 1) / ntiles);
-    nseg = std::min(nseg, std::max<size_t>(1, len / 2048));
-    const size_t seg_len = (len + nseg - 1) / nseg;
+    size_t nseg = (waves + ntiles - 1) / ntiles;
+    nseg = std::min((nseg + 7) & ~(size_t)7, std::max<size_t>(1, len / kSegMin));
+    nseg = std::max(nseg, (len + kSegMax - 1) / kSegMax);
+    size_t seg_len = (len + nseg - 1) / nseg;
+    seg_len = (seg_len + kWord - 1) / kWord * kWord;
     nseg = (len + seg_len - 1) / seg_len;
-    VTA_TRY(check_fits(rows_bytes + nseg * npairs * 40 + npairs * 40 + len * 4));
+    VTA_TRY(check_fits(rows_bytes + nseg * npairs * 28 + npairs * 40 + len * 4));
 
     auto *plan = new vta_double_alma_plan();
     plan->ctx = ctx;
@@ -142,6 +154,8 @@ vta_status plan_build(vta_ctx *ctx, const float *prices, size_t len,
     plan->pmax = (int)pmax;
     plan->nseg = (int)nseg;
     plan->seg_len = (int)seg_len;
+    plan->ntiles = (int)ntiles;
+    plan->ldr = (int)ldr;
     std::vector<double> w64(nrows * pmax, 0.0), inv(nrows);
     std::vector<int32_t> per(nrows);
     for (size_t r = 0; r < nrows; ++r) {
@@ -163,7 +177,8 @@ vta_status plan_build(vta_ctx *ctx, const float *prices, size_t len,
     if (st == VTA_OK) st = upload(ctx, plan->row_period, per.data(), per.size() * 4);
     if (st == VTA_OK) st = upload(ctx, plan->fast_row, frow.data(), frow.size() * 4);
     if (st == VTA_OK) st = upload(ctx, plan->slow_row, srow.data(), srow.size() * 4);
-    if (st == VTA_OK) st = plan->part_i.alloc(nseg * npairs * 4 * sizeof(long long));
+    if (st == VTA_OK) st = plan->part_n.alloc(nseg * npairs * 3 * sizeof(int32_t));
+    if (st == VTA_OK) st = plan->part_ck.alloc(nseg * npairs * sizeof(long long));
     if (st == VTA_OK) st = plan->part_pnl.alloc(nseg * npairs * sizeof(double));
     if (st == VTA_OK) st = plan->out_i.alloc(npairs * 4 * sizeof(long long));
     if (st == VTA_OK) st = plan->out_pnl.alloc(npairs * sizeof(double));
@@ -185,7 +200,8 @@ vta_status plan_enqueue(vta_double_alma_plan *p) {
     a.row_period = p->row_period.as<int32_t>();
     a.fast_row = p->fast_row.as<int32_t>();
     a.slow_row = p->slow_row.as<int32_t>();
-    a.part_i = p->part_i.as<long long>();
+    a.part_n = p->part_n.as<int32_t>();
+    a.part_ck = p->part_ck.as<long long>();
     a.part_pnl = p->part_pnl.as<double>();
     a.out_i = p->out_i.as<long long>();
     a.out_pnl = p->out_pnl.as<double>();
@@ -196,18 +212,22 @@ vta_status plan_enqueue(vta_double_alma_plan *p) {
     a.nseg = p->nseg;
     a.seg_len = p->seg_len;
     a.pmax = p->pmax;
-    a.ntiles_s = (p->nslow + 15) / 16;
-    a.row_tile = kRowTile;
-    const unsigned ntiles = (unsigned)(((p->nfast + 15) / 16) * a.ntiles_s);
+    a.ntiles_s = (p->nslow + kTileS - 1) / kTileS;
+    a.ntiles = p->ntiles;
+    a.ldr = p->ldr;
+    const size_t rows_bytes = (size_t)p->nrows * p->ldr * sizeof(double);
+    const bool wide = rows_bytes > UINT32_MAX;
+    a.rows_bytes = wide ? 0 : (uint32_t)rows_bytes;
     hipFunction_t f;
     VTA_TRY(get_function(ctx, "cross", "cross_rows_f64", &f));
     VTA_TRY(launch(ctx, f, dim3((unsigned)((p->T + kRowTile - 1) / kRowTile), (unsigned)p->nrows, 1),
                    dim3(256), 0, a));
-    VTA_TRY(get_function(ctx, "cross", "cross_pairs_f64", &f));
-    VTA_TRY(launch(ctx, f, dim3(ntiles, (unsigned)p->nseg, 1), dim3(256), 0, a));
+    VTA_TRY(get_function(ctx, "cross", wide ? "cross_pairs_f64_wide" : "cross_pairs_f64", &f));
+    VTA_TRY(launch(ctx, f, dim3(8u * (unsigned)((p->nseg + 7) / 8 * p->ntiles), 1, 1), dim3(64), 0,
+                   a));
     const size_t npairs = (size_t)p->nfast * p->nslow;
     VTA_TRY(get_function(ctx, "cross", "cross_reduce", &f));
-    return launch(ctx, f, dim3((unsigned)((npairs + 255) / 256), 1, 1), dim3(256), 0, a);
+    return launch(ctx, f, dim3((unsigned)((npairs + 63) / 64), 1, 1), dim3(256), 0, a);
 }
 
 vta_status plan_copy(vta_double_alma_plan *p, int64_t *stats4, double *pnl, size_t cap) {

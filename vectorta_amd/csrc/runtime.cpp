@@ -416,6 +416,7 @@ vta_status vta_ctx_preload(vta_ctx *ctx) {
         {"rolling", "mad_batch_f32"},
         {"cross", "cross_rows_f64"},
         {"cross", "cross_pairs_f64"},
+        {"cross", "cross_pairs_f64_wide"},
         {"cross", "cross_reduce"},
         {"rolling", "mad_ms1p_f32"},
         {"rolling", "mad_ms1p_reg16"},
