@@ -114,6 +114,60 @@ def test_scan_short_chunks_long_lead(ctxs, monkeypatch, name):
     assert err <= 1e-5, (name, err)
 
 
+def _scan_case(ctxs, name, n, period, flat=False, wild=False):
+    """One batch of `name` on n bars against the oracle.  flat: stretches whose
+    bars repeat one price (no change, no range, no movement).  wild: bars
+    whose close lies outside low..high, so a directional movement exceeds the
+    true range (also a movement over a zero true range)."""
+    h, lo, c = _hlc(n, 700 + n, lead=2)
+    if flat:
+        for t0 in range(40, n, 1_000):
+            for a in (h, lo, c):
+                a[t0:t0 + 150] = np.float32(100.0)
+    if wild:
+        c[5::7] *= np.float32(1.25)
+        h[6::7] = lo[6::7] = c[5::7][:h[6::7].size]
+    op = ctxs[name]
+    ps = op.expand_grid(period)
+    if name in ("atr", "adx"):
+        g = getattr(op, f"{name}_batch_dev")(h, lo, c, period).to_host()
+        ref = getattr(O, f"{name}_batch")(*[a.astype(np.float64) for a in (h, lo, c)], ps)
+    else:
+        g = getattr(op, f"{name}_batch_dev")(c, period).to_host()
+        ref = getattr(O, f"{name}_batch")(c.astype(np.float64), ps)
+    _check(g, ref, name)
+
+
+@pytest.mark.parametrize("n,combos", [
+    (65, 1),          # one 64-bar chunk and one bar
+    (257, 64),        # five chunks of one group: a block's four share a fold
+    (2_111, 193),     # 33 chunks of four groups, the last of one combo: span maps begin
+    (1_985, 257),     # five groups, 32 chunks: one level of folding
+    (16_321, 65),     # 256 chunks of two groups: the most of one level there
+    (16_447, 130),    # 257 chunks of three groups: nine spans, the last of one chunk
+    (20_001, 700)])   # eleven groups
+@pytest.mark.parametrize("name", ["ema", "rsi", "atr", "adx"])
+def test_scan_chunk_group_and_span_edges(ctxs, name, n, combos):
+    """The default chunking at the edges of its blocks, groups of 64 combos
+    and spans; periods from 2 up put many warm-ups across chunk ends (as many
+    as the series has bars for)."""
+    combos = min(combos, (n - 3) // 2 - 2)
+    _scan_case(ctxs, name, n, (2, 1 + combos, 1))
+
+
+@pytest.mark.parametrize("flat,wild", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("name,combos", [("rsi", 30), ("rsi", 300), ("adx", 30), ("adx", 300)])
+def test_scan_zero_denominators_and_odd_bars(ctxs, name, combos, flat, wild):
+    _scan_case(ctxs, name, 6_011, (2, 1 + combos, 1), flat, wild)
+
+
+@pytest.mark.parametrize("name,n", [("ema", 8_388_609), ("rsi", 4_194_400), ("adx", 2_796_301)])
+def test_scan_series_past_the_term_buffer(ctxs, name, n):
+    """64 MiB of terms hold 8,388,608 EMA bars (RSI half, ADX a third of that);
+    the rest run as a second segment from the handed-on states."""
+    _scan_case(ctxs, name, n, (14, 64, 50))
+
+
 def test_wilders_seeded_matches_replay(monkeypatch):
     """Wilders batches of up to 4,096 combos start each exact lane from a
     per-combo seed at its last warm-up bar; larger ones replay the warm-up

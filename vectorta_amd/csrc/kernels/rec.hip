@@ -25,19 +25,9 @@
 // poison ATR forever), so each stream carries a "clean" flag; an unclean
 // stream always starts exactly at first_valid.
 //
-// One-series batches (EMA, RSI, ATR, ADX, SMMA, Wilders) use an exact chunked
-// scan instead when the series is clean: every step after first_valid, the
-// warm-up included, is affine in the state, s_t = a_t s_{t-1} + f_t (a seed
-// sum has a_t = 1, the step that takes its mean 1/p, the smoothing beta), so
-// a chunk maps its start state s to g s + B, where g is the product of its
-// a_t and B is the chunk run from a zero state.  Pass 1 (phase 1) computes B
-// for every (chunk, combo) -- the chunk holding first_valid runs exactly from
-// there --, a per-combo pass (*_scan_combine) folds the chunks in order into
-// the exact state at every chunk end, and pass 3 (phase 3) runs every chunk
-// again from its exact start state and writes the outputs.  No lane replays
-// bars outside its chunk, so the chunk length is chosen for waves in flight
-// alone (Wilders, whose seed is summed in groups of four, starts carried
-// chunks only past its warm-up).
+// One-series batches use an exact chunked scan instead when the series is
+// clean (see "chunked scan" below): no lane replays bars outside its chunk, so
+// the chunk length is chosen for waves in flight alone.
 #include "vta_common.h"
 
 struct rec_args {
@@ -45,24 +35,32 @@ struct rec_args {
     const float *h;          // high (ATR, ADX)
     const float *l;          // low  (ATR, ADX)
     const int32_t *periods;  // batch: per combo; many-series: [0] only
-    const int32_t *fvs;      // many-series: per series; batch: [0] only
-    const int32_t *clean;    // many-series: per series; batch: [0] only
+    const int32_t *fvs;      // many-series: per series
+    const int32_t *clean;    // many-series: per series; batch: [0] a non-finite bar was
+                             // met, [1] an odd one (the word equals clean_epoch); NULL:
+                             // not clean
     const int32_t *fvs2;     // fused kernel: per-series first_valid of (high, low, close)
     float *out0;
     float *out1;
     float *out2;
-    double *carry;           // batch scan: [combo][chunk][states] chunk-end states
+    double *carry;           // batch scan: [chunk][state][64 x groups] chunk-end states, then
+                             // [span][state][64 x groups] the spans'
+    const double *terms;     // batch scan: per-bar terms from bar t0 on (scan_term_at)
+    const double *state_in;  // batch scan: [state][64 x groups] before bar t0, or NULL
+    double *state_out;       // batch scan: the same after bar t1 - 1, or NULL
     const float *alphas;     // EMA / Wilders: caller's smoothing factor (batch: per combo,
                              // many-series: [0]); NULL derives it from the period
-    double *seeds;           // Wilders batch: per-combo value at bar first_valid + period - 1
-                             // (wilders_seed), or NULL (exact lanes replay the warm-up)
     int T;                   // bars
     int nlanes;              // combos (batch) or series (many-series)
     int chunk;               // bars per chunk
     int p1, p2, p3;          // fused kernel periods (EMA, RSI, ATR)
-    int phase;               // batch: 0 burn-in/exact, 1 scan pass, 3 output pass of the scan
-    int clean_epoch;         // batch: 0, or clean = (clean[0] != clean_epoch), the word
-                             // batch_prepare stores the call's epoch in on a non-finite bar
+    int fv;                  // batch: first_valid
+    int nch, groups;         // batch: chunks, groups of 64 combos
+    int span;                // batch scan: chunks per span, 0 without spans
+    int t0, t1;              // batch scan: the bars of this launch
+    int tstride;
+    int scan;                // batch: 0 burn-in / exact lanes, else the scan (ADX: stage 1 or 2)
+    int clean_epoch;         // batch: the word scan_prepare stores in clean[0], [1]
 };
 
 #define REC_NAN __builtin_bit_cast(double, 0x7ff8000000000000ull)
@@ -88,15 +86,6 @@ __device__ __forceinline__ int bars_from(int c0, int c1, int from) {
 }
 
 // ---------------------------------------------------------------- engines
-//
-// Chunked-scan interface (one-series batches): gain(c0, c1) is the product of
-// the per-bar multipliers of the state over bars [c0, c1) (every step, warm-up
-// included, is affine in the state: s_t = a_t s_{t-1} + f_t), begin_carry(t0,
-// ...) restarts the engine after bar t0 from a carried state and
-// get_state(t1, ...) reads it after bar t1; the state is whichever quantity
-// the step carries at that bar (a seed sum during the warm-up, the average
-// after).  kWarmScan engines accept a carried start anywhere after
-// first_valid; the others only past the warm-up.
 
 struct EmaEng {
     static constexpr bool kSeedScan = false;
@@ -127,12 +116,7 @@ struct EmaEng {
         return prev;
     }
     __device__ double out_before_start(int t) const { return REC_NAN; }
-    static constexpr int kScan = 1;                  // states carried by the chunked scan
-    static constexpr bool kTwoStage = false;
-    static constexpr bool kAdvance = false;
     static constexpr int kPre = 0;
-    static constexpr int kStageW = 64;
-    static constexpr bool kSeeded = false;
     // steps t < seed_end() after the start are the warm-up accumulation only
     __device__ int seed_end() const { return fv + p; }
     __device__ double seed_step(int t, double x) {
@@ -148,20 +132,6 @@ struct EmaEng {
         if (fin(x)) prev = fma(beta, prev, alpha * x);
         return prev;
     }
-    // running mean: (v-1)/v per bar with v = t - fv + 1 (the product
-    // telescopes), then beta
-    static constexpr bool kWarmScan = true;
-    __device__ double gain(int c0, int c1) const {
-        const int m = min(c1, fv + p);
-        const double g = c0 < m ? (double)(c0 - fv) / (double)(m - fv) : 1.0;
-        const int n = bars_from(c0, c1, fv + p);
-        return n > 0 ? g * pow(beta, (double)n) : g;
-    }
-    __device__ void begin_carry(int t0, double x, const double *st) {
-        prev = st[0];
-        vc = t0 - fv + 1;
-    }
-    __device__ void get_state(int t1, double *st) const { st[0] = prev; }
 };
 
 // num / den for den > 0: an f32 reciprocal estimate refined by one f64 Newton
@@ -247,14 +217,7 @@ struct RsiEng {
         if (poisoned) return REC_NAN;
         return (double)rsi_ratio_f32(ag, al);
     }
-    static constexpr int kScan = 2;
-    static constexpr bool kTwoStage = false;
-    static constexpr bool kAdvance = true;
-    // the gain and loss of a bar are two ops: reading them from LDS
-    // (see drive_batch) measured slower (0.55 vs 0.47 ms, 1,250 x 200k)
     static constexpr int kPre = 0;
-    static constexpr int kStageW = 32;
-    static constexpr bool kSeeded = false;
     __device__ int seed_end() const { return fv + p; }
     __device__ double seed_step(int t, double x) {
         double d = x - px;
@@ -266,16 +229,6 @@ struct RsiEng {
         }
         return REC_NAN;
     }
-    __device__ int advance_from() const { return burn_ok_from(); }
-    // pass 1 of the chunked scan: the state update without the output ratio
-    __device__ void advance(double x) {
-        double d = x - px;
-        px = x;
-        double g = d > 0.0 ? d : 0.0;
-        double lo = d < 0.0 ? -d : 0.0;
-        ag = fma(ag, beta, inv_p * g);
-        al = fma(al, beta, inv_p * lo);
-    }
     __device__ double steady(double x) {
         double d = x - px;
         px = x;
@@ -286,20 +239,6 @@ struct RsiEng {
         if (poisoned) return REC_NAN;
         return (double)rsi_ratio_f32(ag, al);
     }
-    // seed sums (multiplier 1), times 1/p at fv+p, then beta
-    static constexpr bool kWarmScan = true;
-    __device__ double gain(int c0, int c1) const {
-        const int ws = fv + p;
-        const double g = (c0 <= ws && ws < c1) ? inv_p : 1.0;
-        const int n = bars_from(c0, c1, ws + 1);
-        return n > 0 ? g * pow(beta, (double)n) : g;
-    }
-    __device__ void begin_carry(int t0, double x, const double *st) {
-        px = x;
-        ag = st[0];
-        al = st[1];
-    }
-    __device__ void get_state(int t1, double *st) const { st[0] = ag; st[1] = al; }
 };
 
 __device__ __forceinline__ double true_range(double hi, double lo, double pc) {
@@ -337,12 +276,7 @@ struct AtrEng {
         rma = fma(-alpha, rma, rma) + alpha * tr;  // atr.rs:393
         return rma;
     }
-    static constexpr int kScan = 1;
-    static constexpr bool kTwoStage = false;
-    static constexpr bool kAdvance = false;
     static constexpr int kPre = 1;
-    static constexpr int kStageW = 64;
-    static constexpr bool kSeeded = false;
     __device__ int seed_end() const { return fv + p - 1; }
     __device__ double seed_step(int t, double h, double l, double c) {
         sum += true_range(h, l, pc);
@@ -360,25 +294,10 @@ struct AtrEng {
         o[0] = true_range(h, l, pc);
     }
     __device__ void set_prev(double, double, double c) { pc = c; }
-    __device__ void advance_pre(const double *) {}
     __device__ double steady_pre(const double *o) {
         rma = fma(-alpha, rma, rma) + alpha * o[0];
         return rma;
     }
-    // seed sum up to fv+p-1, where the mean is taken (1/p), then 1 - alpha
-    static constexpr bool kWarmScan = true;
-    __device__ double gain(int c0, int c1) const {
-        const int ws = fv + p - 1;
-        const double g = (c0 <= ws && ws < c1) ? 1.0 / (double)p : 1.0;
-        const int n = bars_from(c0, c1, ws + 1);
-        return n > 0 ? g * pow(1.0 - alpha, (double)n) : g;
-    }
-    __device__ void begin_carry(int t0, double h, double l, double c, const double *st) {
-        if (t0 < fv + p - 1) sum = st[0];
-        else rma = st[0];
-        pc = c;
-    }
-    __device__ void get_state(int t1, double *st) const { st[0] = t1 < fv + p - 1 ? sum : rma; }
 };
 
 // ATR fed by a precomputed true-range series (atr_wrapper.rs:626-700,
@@ -408,12 +327,7 @@ struct AtrTrEng {
         return rma;
     }
     __device__ double out_before_start(int t) const { return REC_NAN; }
-    static constexpr int kScan = 1;
-    static constexpr bool kTwoStage = false;
-    static constexpr bool kAdvance = false;
     static constexpr int kPre = 0;
-    static constexpr int kStageW = 64;
-    static constexpr bool kSeeded = false;
     __device__ int seed_end() const { return fv + p - 1; }
     __device__ double seed_step(int t, double tr) {
         sum += tr;
@@ -423,18 +337,6 @@ struct AtrTrEng {
         rma = fma(-alpha, rma, rma) + alpha * tr;
         return rma;
     }
-    static constexpr bool kWarmScan = true;
-    __device__ double gain(int c0, int c1) const {
-        const int ws = fv + p - 1;
-        const double g = (c0 <= ws && ws < c1) ? 1.0 / (double)p : 1.0;
-        const int n = bars_from(c0, c1, ws + 1);
-        return n > 0 ? g * pow(1.0 - alpha, (double)n) : g;
-    }
-    __device__ void begin_carry(int t0, double tr, const double *st) {
-        if (t0 < fv + p - 1) sum = st[0];
-        else rma = st[0];
-    }
-    __device__ void get_state(int t1, double *st) const { st[0] = t1 < fv + p - 1 ? sum : rma; }
 };
 
 struct AdxEng {
@@ -500,14 +402,7 @@ struct AdxEng {
         adx = (adx * pm1 + dx) * rp;
         return adx;
     }
-    // two stages: (atr, +DM, -DM) decay by omr; adx decays by pm1 * rp once
-    // the DX sequence is known, which needs the first stage's exact states
-    static constexpr int kScan = 4;
-    static constexpr bool kTwoStage = true;
-    static constexpr bool kAdvance = true;
     static constexpr int kPre = 3;
-    static constexpr int kStageW = 32;
-    static constexpr bool kSeeded = false;
     __device__ int seed_end() const { return fv + p; }
     __device__ double seed_step(int t, double ch, double cl, double cc) {
         double hl = ch - cl;
@@ -521,79 +416,6 @@ struct AdxEng {
         if (down > up && down > 0.0) mds += down;
         atr += tr;
         return REC_NAN;
-    }
-    // pass 1 needs the first stage only, which is a plain smoothing from
-    // i = p + 1 on
-    __device__ int advance_from() const { return fv + p + 1; }
-    // DX seed (adx.rs:369-409): bars fv+p < t < fv+2p-1 smooth the first
-    // stage and add DX to the seed sum; the ADX itself is not yet defined
-    __device__ int dx_seed_end() const { return fv + 2 * p - 1; }
-    __device__ void dx_seed_step(double ch, double cl, double cc) {
-        double hl = ch - cl;
-        double hpc = fabs(ch - pc);
-        double lpc = fabs(cl - pc);
-        double tr = fmax(fmax(hl, hpc), lpc);
-        double up = ch - ph;
-        double down = pl - cl;
-        ph = ch; pl = cl; pc = cc;
-        double pdm = (up > down && up > 0.0) ? up : 0.0;
-        double mdm = (down > up && down > 0.0) ? down : 0.0;
-        atr = atr * omr + tr;
-        pds = pds * omr + pdm;
-        mds = mds * omr + mdm;
-        const double sdm = pds + mds;
-        double dx = (atr != 0.0 && sdm != 0.0) ? dx_ratio(100.0 * fabs(pds - mds), sdm) : 0.0;
-        dx_sum += dx;
-    }
-    // first stage: seed sums (multiplier 1) up to i = p, then omr; second
-    // stage: restarted at i = p (first DX), DX summed (1) up to i = 2p-2,
-    // the mean at i = 2p-1 (rp), then pm1 * rp
-    static constexpr bool kWarmScan = true;
-    __device__ double gain(int c0, int c1) const {
-        const int n = bars_from(c0, c1, fv + p + 1);
-        return n > 0 ? pow(omr, (double)n) : 1.0;
-    }
-    __device__ double gain2(int c0, int c1) const {
-        if (c0 <= fv + p) return 0.0;
-        const int w = fv + 2 * p - 1;
-        const double g = (c0 <= w && w < c1) ? rp : 1.0;
-        const int n = bars_from(c0, c1, w + 1);
-        return n > 0 ? g * pow(pm1 * rp, (double)n) : g;
-    }
-    // second-stage state after bar t: undefined before i = p, the DX sum up
-    // to i = 2p-2, the ADX from i = 2p-1 on
-    __device__ void begin_carry(int t0, double h, double l, double c, const double *st) {
-        atr = st[0]; pds = st[1]; mds = st[2];
-        const int i0 = t0 - fv;
-        if (i0 < p) {
-            dx_sum = 0.0; adx = 0.0; dx_count = 0;
-        } else if (i0 < 2 * p - 1) {
-            dx_sum = st[3]; adx = 0.0; dx_count = i0 - p + 1;
-        } else {
-            dx_sum = 0.0; adx = st[3]; dx_count = p;
-        }
-        ph = h; pl = l; pc = c;
-    }
-    __device__ void get_state(int t1, double *st) const {
-        st[0] = atr; st[1] = pds; st[2] = mds;
-        const int i1 = t1 - fv;
-        st[3] = i1 < p ? 0.0 : (i1 < 2 * p - 1 ? dx_sum : adx);
-    }
-    // pass 1 of the chunked scan: the first stage only (the ADX stage is
-    // folded after pass 2)
-    __device__ void advance(double ch, double cl, double cc) {
-        double hl = ch - cl;
-        double hpc = fabs(ch - pc);
-        double lpc = fabs(cl - pc);
-        double tr = fmax(fmax(hl, hpc), lpc);
-        double up = ch - ph;
-        double down = pl - cl;
-        ph = ch; pl = cl; pc = cc;
-        double pdm = (up > down && up > 0.0) ? up : 0.0;
-        double mdm = (down > up && down > 0.0) ? down : 0.0;
-        atr = atr * omr + tr;
-        pds = pds * omr + pdm;
-        mds = mds * omr + mdm;
     }
     __device__ double steady(double ch, double cl, double cc) {
         double hl = ch - cl;
@@ -626,11 +448,6 @@ struct AdxEng {
         o[2] = (down > up && down > 0.0) ? down : 0.0;
     }
     __device__ void set_prev(double h, double l, double c) { ph = h; pl = l; pc = c; }
-    __device__ void advance_pre(const double *o) {
-        atr = atr * omr + o[0];
-        pds = pds * omr + o[1];
-        mds = mds * omr + o[2];
-    }
     __device__ double steady_pre(const double *o) {
         atr = atr * omr + o[0];
         pds = pds * omr + o[1];
@@ -672,12 +489,7 @@ struct SmmaEng {
         return prev;
     }
     __device__ double out_before_start(int t) const { return REC_NAN; }
-    static constexpr int kScan = 1;
-    static constexpr bool kTwoStage = false;
-    static constexpr bool kAdvance = false;
     static constexpr int kPre = 0;
-    static constexpr int kStageW = 64;
-    static constexpr bool kSeeded = false;
     __device__ int seed_end() const { return p == 1 ? fv : fv + p - 1; }
     __device__ double seed_step(int t, double x) {
         sum += x;
@@ -687,22 +499,6 @@ struct SmmaEng {
         if (p == 1) { prev = x; return x; }
         prev = (prev * pm1 + x) * rp;
         return prev;
-    }
-    // seed sum up to fv+p-1 (mean: 1/p), then pm1 * rp; p = 1 copies (0)
-    static constexpr bool kWarmScan = true;
-    __device__ double gain(int c0, int c1) const {
-        if (p == 1) return 0.0;
-        const int ws = fv + p - 1;
-        const double g = (c0 <= ws && ws < c1) ? 1.0 / (double)p : 1.0;
-        const int n = bars_from(c0, c1, ws + 1);
-        return n > 0 ? g * pow(pm1 * rp, (double)n) : g;
-    }
-    __device__ void begin_carry(int t0, double x, const double *st) {
-        if (p > 1 && t0 < fv + p - 1) sum = st[0];
-        else prev = st[0];
-    }
-    __device__ void get_state(int t1, double *st) const {
-        st[0] = (p > 1 && t1 < fv + p - 1) ? sum : prev;
     }
 };
 
@@ -737,15 +533,7 @@ struct WildersEng {
         return y;
     }
     __device__ double out_before_start(int t) const { return REC_NAN; }
-    static constexpr int kScan = 1;
-    static constexpr bool kTwoStage = false;
-    static constexpr bool kAdvance = false;
     static constexpr int kPre = 0;
-    static constexpr int kStageW = 64;
-    // a scan lane that would replay its warm-up from first_valid starts at
-    // its last warm-up bar from the precomputed seed instead (wilders_seed)
-    static constexpr bool kSeeded = true;
-    __device__ double begin_seeded(double seed) { y = seed; return y; }
     __device__ int seed_end() const { return fv + p - 1; }
     __device__ double seed_step(int t, double x) { return seed_bar(t - fv, x); }
     __device__ double steady(double x) {
@@ -753,12 +541,6 @@ struct WildersEng {
         y = fma(x - y, al, y);
         return y;
     }
-    // the seed is summed in groups of four (a two-word state), so a carried
-    // start is taken only past the warm-up: fma(x - y, al, y), i.e. 1 - al
-    static constexpr bool kWarmScan = false;
-    __device__ double gain(int c0, int c1) const { return pow(1.0 - al, (double)(c1 - c0)); }
-    __device__ void begin_carry(int t0, double x, const double *st) { y = st[0]; }
-    __device__ void get_state(int t1, double *st) const { st[0] = y; }
 };
 
 // ---------------------------------------------------------------- chunk planning
@@ -1063,101 +845,118 @@ extern "C" __global__ __launch_bounds__(64) void ms_ema_rsi_atr_f32(rec_args a) 
 
 // ---------------------------------------------------------------- one series, many params
 //
-// grid.x: groups of 64 combos, grid.y: chunks.  Lane = combo.  The wave
-// stages 64 bars of the series in LDS (one coalesced load, then broadcast
-// reads), and buffers 64 bars x 64 combos of output in LDS so each output row
-// segment is written as one coalesced 256-byte store.
-// What one block of a one-series batch pass (or one wave of a fold) works
-// on: the series, the combos' periods and outputs, the chunking, and which
-// combo group and chunk this block is (for a fold: `group` = the combo).
+// Lane = combo.  What one block of a one-series batch works on: the series,
+// the combos' periods and outputs, the chunking, and which combo group and
+// chunk this block is.
 struct batch_view {
     const float *x, *h, *l;
     const int32_t *periods;
-    double *carry;           // [combo][chunk][states]
     const float *alphas;     // per combo, or NULL (see apply_alpha)
-    const double *seeds;     // Wilders: per-combo seed, or NULL
-    int T, nlanes, chunk, nch, phase, fv, group, k;
-    bool clean;
+    double *carry;           // see rec_args
+    const double *terms, *state_in;
+    double *state_out;
+    int T, nlanes, chunk, nch, groups, span, fv, t0, t1, tstride, scan, group;
+    int kb, k;               // the block's first chunk, this wave's
+    bool clean, odd, coop;
 };
 
-// The view of a block of a direct launch: grid.x = combo groups (a fold: the
-// combo), grid.y = chunks.
+// A block is REC_WPB waves: with that many combo groups, one chunk of as many
+// groups, whose waves then read the same terms (one miss of the scalar cache
+// for four); else consecutive chunks of one group, which share the work of
+// folding the chunks before them (`coop`).
+#define REC_WPB 4
+__device__ __forceinline__ int block_wave() {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+__device__ __forceinline__ void block_chunk(batch_view &v, int flat) {
+    v.coop = v.groups < REC_WPB;
+    if (v.coop) {
+        const int per = (v.nch + REC_WPB - 1) / REC_WPB;
+        v.group = flat / per;
+        v.kb = flat % per * REC_WPB;
+        v.k = v.kb + block_wave();
+    } else {
+        v.group = flat / v.nch * REC_WPB + block_wave();
+        v.kb = v.k = flat % v.nch;
+    }
+}
+// Whether the wave has a chunk at all.
+__device__ __forceinline__ bool wave_idle(const batch_view &v) {
+    return v.k >= v.nch || v.group >= v.groups;
+}
+
+// The view of a wave of a direct launch: the blocks of a group in order.
 __device__ __forceinline__ batch_view view_of(const rec_args &a) {
     batch_view v;
     v.x = a.x; v.h = a.h; v.l = a.l;
     v.periods = a.periods;
-    v.carry = a.carry;
     v.alphas = a.alphas;
-    v.seeds = a.seeds;
+    v.carry = a.carry;
+    v.terms = a.terms;
+    v.state_in = a.state_in;
+    v.state_out = a.state_out;
     v.T = a.T;
     v.nlanes = a.nlanes;
     v.chunk = a.chunk;
-    v.nch = (a.T + a.chunk - 1) / a.chunk;
-    v.phase = a.phase;
-    v.fv = a.fvs[0];
-    v.group = blockIdx.x;
-    v.k = blockIdx.y;
-    v.clean = a.clean != nullptr &&
-              (a.clean_epoch != 0 ? a.clean[0] != a.clean_epoch : a.clean[0] != 0);
+    v.nch = a.nch;
+    v.groups = a.groups;
+    v.span = a.span;
+    v.fv = a.fv;
+    v.t0 = a.t0;
+    v.t1 = a.t1;
+    v.tstride = a.tstride;
+    v.scan = a.scan;
+    block_chunk(v, blockIdx.x);
+    v.clean = a.clean != nullptr && a.clean[0] != a.clean_epoch;
+    v.odd = a.clean != nullptr && a.clean[1] == a.clean_epoch;
     return v;
 }
 
+// LDS of a wave, dynamic (batch_lds_bytes, rec.cpp): the bars or the per-bar
+// terms formed from them, and the 64-row output staging of drive_batch; the
+// scan's output pass has its own staging in the same bytes (at most 10 KiB, so
+// that four blocks of four waves fit a CU).
+#define REC_STAGE 33         // floats per staged row of drive_batch (32 bars + 1)
+#define REC_ROW 36           // floats per row staged by scan_output (16-byte rows)
+template <class E>
+__device__ __forceinline__ double *wave_lds() {
+    constexpr int drive = (E::kPre > 1 ? E::kPre * 512 : 3 * 256) + 64 * REC_STAGE * 4;
+    constexpr int scan = 64 * REC_ROW * 4;
+    extern __shared__ __align__(16) double rec_lds[];
+    return rec_lds + block_wave() * ((drive > scan ? drive : scan) / 8);
+}
+
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Exact and burn-in lanes: the wave stages 64 bars of the series in LDS (one
+// coalesced load, then broadcast reads) and 64 rows x 32 bars of output.  An
+// unclean series runs exactly from first_valid.
 template <class E, int NIN>
 __device__ __forceinline__ void drive_batch(const batch_view &a, float *out) {
-    __shared__ __align__(16) float xs[3][64];
     // per-bar terms every combo shares (E::kPre of them, f64): lane j computes
-    // them for bar tb + j, so the steady and pass-1 loops read them instead of
+    // them for bar tb + j, so the steady loop reads them instead of
     // recomputing them in every lane
     constexpr int NPRE = E::kPre;
-    __shared__ __align__(16) double pv[NPRE > 0 ? NPRE : 1][64];
-    // 64 x 65 output staging in dynamic LDS, launched only with the passes
-    // that write rows (a pass without stores keeps more waves per CU)
-    // 64 rows x SW bars (+1 pad), flushed every SW bars: engines whose steps
-    // are long (RSI, ADX) flush every 32 bars, which leaves LDS for ~3 waves
-    // per SIMD where 64-bar staging allows 2; the others keep 64-bar row
-    // segments
-    constexpr int SW = E::kStageW;    // the host launches 64 x (SW + 1) floats
-                                      // of dynamic LDS (batch_stage_bytes, rec.cpp)
-    extern __shared__ float ob_dyn[];
-    float (*ob)[SW + 1] = reinterpret_cast<float (*)[SW + 1]>(ob_dyn);
+    double *pv = wave_lds<E>();                                    // [NPRE][64], or
+    float *xs = reinterpret_cast<float *>(pv);                     // [3][64]
+    float *ob = xs + (NPRE > 1 ? NPRE * 128 : 3 * 64);             // [64][REC_STAGE]
     const int lane = threadIdx.x & 63;
     const int c = a.group * 64 + lane;
     const bool active = c < a.nlanes;
     const int T = a.T;
-    const int k = a.k;
-    const bool clean = a.clean;
-    // a scan pass over an unclean series: its lanes run exactly from
-    // first_valid, so the output pass runs the whole series in chunk 0 and
-    // every other block of the scan has nothing to do
-    if (a.phase != 0 && !clean && (a.phase != 3 || k != 0)) return;
-    const int c0 = (a.phase != 0 && !clean) ? 0 : k * a.chunk;
-    const int c1 = (a.phase != 0 && !clean) ? T : min(c0 + a.chunk, T);
+    const int c0 = a.k * a.chunk;
+    const int c1 = min(c0 + a.chunk, T);
     const int fv = a.fv;
     const int p = active ? a.periods[c] : 1;
     E e;
     e.setup(p, fv);
     if (active) apply_alpha(e, a.alphas, c);
-    bool burn = false, carried = false, seeded = false;
-    int start;
-    if (a.phase != 0) {
-        // chunked scan: chunks after first_valid (past the warm-up for engines
-        // without kWarmScan) start from a carried state at c0 - 1; an unclean
-        // series runs every chunk exactly from first_valid
-        carried = active && clean &&
-                  (E::kWarmScan ? c0 > e.exact_start() : c0 >= e.burn_ok_from());
-        start = active ? (carried ? c0 - 1 : e.exact_start()) : T;
-    } else {
-        start = active ? lane_start(e, c0, clean, &burn) : T;
-    }
-    double seedv = 0.0;
-    if constexpr (E::kSeeded) {
-        // an exact start whose seed is known begins at the last warm-up bar
-        if (active && !carried && !burn && a.seeds) {
-            seeded = true;
-            start = e.fv + e.p - 1;
-            seedv = a.seeds[c];
-        }
-    }
+    bool burn = false;
+    const int start = active ? lane_start(e, c0, a.clean, &burn) : T;
     if constexpr (E::kSeedScan) {
         // RSI burn-in: the seed window's NaN rule still has to be seen
         if (burn) {
@@ -1165,48 +964,28 @@ __device__ __forceinline__ void drive_batch(const batch_view &a, float *out) {
             for (int t = fv + 1; t <= min(fv + p, T - 1); ++t) e.seed_scan(t, (double)a.x[t]);
         }
     }
-    // carried start state: zeros (pass 1), the exact first-stage states with a
-    // zero second stage (pass 2 of a two-stage engine), or all exact (pass 3)
-    constexpr int S = E::kScan > 0 ? E::kScan : 1;
-    double st0[S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) st0[i] = 0.0;
-    if (carried && a.phase >= 2) {
-        const double *cs = a.carry + ((size_t)c * a.nch + (k - 1)) * S;
-        const int n = (E::kTwoStage && a.phase == 2) ? S - 1 : S;
-#pragma unroll
-        for (int i = 0; i < S; ++i)
-            if (i < n) st0[i] = cs[i];
-    }
-    const bool emit = a.phase == 0 || a.phase == 3;
-    // 32-bar staging: rows of bars tb + 32 hh .. + 31, each store two rows x
-    // 32 consecutive bars (lane & 31 = bar, lane >> 5 = row parity)
+    // rows of bars tb + 32 hh .. + 31, each store two rows x 32 consecutive
+    // bars (lane & 31 = bar, lane >> 5 = row parity)
     const int nrow = min(64, a.nlanes - a.group * 64);
     auto flush_half = [&](int tb, int hh) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
         const int t = tb + 32 * hh + (lane & 31);
         if (tb + 32 * hh + 32 > c0) {
             const bool ok = t >= c0 && t < c1;
 #pragma unroll 4
             for (int i = 0; i < 32; ++i) {
                 const int r = 2 * i + (lane >> 5);
-                if (ok && r < nrow) out[(size_t)(a.group * 64 + r) * T + t] = ob[r][lane & (SW - 1)];
+                if (ok && r < nrow)
+                    out[(size_t)(a.group * 64 + r) * T + t] = ob[r * REC_STAGE + (lane & 31)];
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_sync();
     };
-    // a carried lane restarts after bar c0 - 1 here, from that one bar read
-    // directly, so the wave need not run the 64-bar block holding it
-    if (carried) {
-        const int tp = c0 - 1;
-        if constexpr (NIN == 1) e.begin_carry(tp, (double)a.x[tp], st0);
-        else e.begin_carry(tp, (double)a.h[tp], (double)a.l[tp], (double)a.x[tp], st0);
-    }
-    const int t_begin = wave_min(carried ? c0 : min(start, c0)) & ~63;
+    auto emit = [&](int tb, int j, double y) {
+        ob[lane * REC_STAGE + (j & 31)] = (float)y;
+        if ((j & 31) == 31) flush_half(tb, j >> 5);
+    };
+    const int t_begin = wave_min(min(start, c0)) & ~63;
     // bars of the next block are loaded into registers while the current one
     // is processed (with the bar before each, for the per-bar terms)
     float nx0, nx1 = 0.0f, nx2 = 0.0f, np0 = 0.0f, np1 = 0.0f, np2 = 0.0f;
@@ -1226,190 +1005,65 @@ __device__ __forceinline__ void drive_batch(const batch_view &a, float *out) {
             }
         }
     };
-    // a whole block that seeded lanes can run without the per-bar start logic
-    auto seeded_block = [&](int tb) {
-        if constexpr (E::kSeeded && NIN == 1)
-            return tb + 64 <= c1 &&
-                   __all(!active || seeded || (start < tb && tb >= e.burn_ok_from()));
-        else
-            return false;
-    };
     load_next(t_begin);
     for (int tb = t_begin; tb < c1; tb += 64) {
-        xs[0][lane] = nx0;
-        if (NIN == 3) {
-            xs[1][lane] = nx1;
-            xs[2][lane] = nx2;
-        }
-        if constexpr (NPRE > 0) {
-            double o[NPRE];
-            E::pre((double)nx1, (double)nx2, (double)nx0, (double)np1, (double)np2, (double)np0, o);
-#pragma unroll
-            for (int i = 0; i < NPRE; ++i) pv[i][lane] = o[i];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        load_next(tb + 64);
         // lean path: a full block in which every lane is past its start and
-        // its warm-up -- only the engine's steady update, bars read four at a
-        // time
+        // its warm-up -- only the engine's steady update
         const bool lean = tb + 64 <= c1 && __all(!active || (start < tb && tb >= e.burn_ok_from()));
-        bool advanced = false;
-        if constexpr (E::kAdvance) {
-            if (a.phase == 1 && tb + 64 <= c1 &&
-                __all(!active || (start < tb && tb >= e.advance_from()))) {
-                // pass 1: the state update only, no outputs
-                if constexpr (NPRE > 0) {
-#pragma unroll 4
-                    for (int j = 0; j < 64; ++j) {
-                        double o[NPRE];
+        const float lx0 = __shfl(nx0, 63), lx1 = __shfl(nx1, 63), lx2 = __shfl(nx2, 63);
+        if (NPRE > 0 && lean) {
+            double o[NPRE > 0 ? NPRE : 1];
+            if constexpr (NPRE > 0)
+                E::pre((double)nx1, (double)nx2, (double)nx0, (double)np1, (double)np2,
+                       (double)np0, o);
 #pragma unroll
-                        for (int i = 0; i < NPRE; ++i) o[i] = pv[i][j];
-                        e.advance_pre(o);
-                    }
-                    e.set_prev(xs[1][63], xs[2][63], xs[0][63]);
-                } else
-#pragma unroll 2
-                for (int j = 0; j < 64; j += 4) {
-                    const float4 x4 = *reinterpret_cast<const float4 *>(&xs[0][j]);
-                    if constexpr (NIN == 1) {
-                        e.advance(x4.x);
-                        e.advance(x4.y);
-                        e.advance(x4.z);
-                        e.advance(x4.w);
-                    } else {
-                        const float4 h4 = *reinterpret_cast<const float4 *>(&xs[1][j]);
-                        const float4 l4 = *reinterpret_cast<const float4 *>(&xs[2][j]);
-                        e.advance(h4.x, l4.x, x4.x);
-                        e.advance(h4.y, l4.y, x4.y);
-                        e.advance(h4.z, l4.z, x4.z);
-                        e.advance(h4.w, l4.w, x4.w);
-                    }
-                }
-                advanced = true;
+            for (int i = 0; i < NPRE; ++i) pv[i * 64 + lane] = o[i];
+        } else {
+            xs[lane] = nx0;
+            if (NIN == 3) {
+                xs[64 + lane] = nx1;
+                xs[128 + lane] = nx2;
             }
         }
-        if constexpr (E::kTwoStage) {
-            // ADX's DX seed: every lane between its first-stage seed and its
-            // first ADX for the whole block (outputs NaN)
-            if (!advanced && tb + 64 <= c1 &&
-                __all(!active || (start < tb && tb > e.fv + e.p && tb + 64 <= e.dx_seed_end()))) {
-#pragma unroll 2
-                for (int j = 0; j < 64; j += 4) {
-                    const float4 x4 = *reinterpret_cast<const float4 *>(&xs[0][j]);
-                    const float4 h4 = *reinterpret_cast<const float4 *>(&xs[1][j]);
-                    const float4 l4 = *reinterpret_cast<const float4 *>(&xs[2][j]);
-                    e.dx_seed_step(h4.x, l4.x, x4.x);
-                    e.dx_seed_step(h4.y, l4.y, x4.y);
-                    e.dx_seed_step(h4.z, l4.z, x4.z);
-                    e.dx_seed_step(h4.w, l4.w, x4.w);
-                    if (emit) {
-                        ob[lane][j & (SW - 1)] = (float)REC_NAN;
-                        ob[lane][(j + 1) & (SW - 1)] = (float)REC_NAN;
-                        ob[lane][(j + 2) & (SW - 1)] = (float)REC_NAN;
-                        ob[lane][(j + 3) & (SW - 1)] = (float)REC_NAN;
-                        if (SW == 32 && ((j + 4) & 31) == 0) flush_half(tb, j >> 5);
-                    }
-                }
-                e.dx_count += 64;
-                advanced = true;
-            }
-        }
-        if (advanced) {
-            // block done
-        } else if (lean) {
+        wave_lds_sync();
+        load_next(tb + 64);
+        if (lean) {
           if constexpr (NPRE > 0) {
 #pragma unroll 4
             for (int j = 0; j < 64; ++j) {
                 double o[NPRE];
 #pragma unroll
-                for (int i = 0; i < NPRE; ++i) o[i] = pv[i][j];
-                const double y = e.steady_pre(o);
-                if (emit) {
-                    ob[lane][j & (SW - 1)] = (float)y;
-                    if (SW == 32 && (j & 31) == 31) flush_half(tb, j >> 5);
-                }
+                for (int i = 0; i < NPRE; ++i) o[i] = pv[i * 64 + j];
+                emit(tb, j, e.steady_pre(o));
             }
-            e.set_prev(xs[1][63], xs[2][63], xs[0][63]);
+            e.set_prev((double)lx1, (double)lx2, (double)lx0);
           } else {
 #pragma unroll 2
             for (int j = 0; j < 64; j += 4) {
-                const float4 x4 = *reinterpret_cast<const float4 *>(&xs[0][j]);
-                double y0, y1, y2, y3;
-                if constexpr (NIN == 1) {
-                    y0 = e.steady(x4.x);
-                    y1 = e.steady(x4.y);
-                    y2 = e.steady(x4.z);
-                    y3 = e.steady(x4.w);
-                } else {
-                    const float4 h4 = *reinterpret_cast<const float4 *>(&xs[1][j]);
-                    const float4 l4 = *reinterpret_cast<const float4 *>(&xs[2][j]);
-                    y0 = e.steady(h4.x, l4.x, x4.x);
-                    y1 = e.steady(h4.y, l4.y, x4.y);
-                    y2 = e.steady(h4.z, l4.z, x4.z);
-                    y3 = e.steady(h4.w, l4.w, x4.w);
-                }
-                if (emit) {
-                    ob[lane][j & (SW - 1)] = (float)y0;
-                    ob[lane][(j + 1) & (SW - 1)] = (float)y1;
-                    ob[lane][(j + 2) & (SW - 1)] = (float)y2;
-                    ob[lane][(j + 3) & (SW - 1)] = (float)y3;
-                    if (SW == 32 && ((j + 4) & 31) == 0) flush_half(tb, j >> 5);
-                }
+                const float4 x4 = *reinterpret_cast<const float4 *>(&xs[j]);
+                emit(tb, j, e.steady(x4.x));
+                emit(tb, j + 1, e.steady(x4.y));
+                emit(tb, j + 2, e.steady(x4.z));
+                emit(tb, j + 3, e.steady(x4.w));
             }
           }
-        } else if (seeded_block(tb)) {
-            // lanes that start from a seed in this block or a later one run the
-            // steady update on every bar, take the seed at their start bar and
-            // write NaN before it; the others are past their warm-ups
-            if constexpr (E::kSeeded) {
-                auto sbar = [&](int t, float x) {
-                    double y = e.steady(x);
-                    if (t == start) y = e.begin_seeded(seedv);
-                    return t < start ? REC_NAN : y;
-                };
-#pragma unroll 2
-                for (int j = 0; j < 64; j += 4) {
-                    const float4 x4 = *reinterpret_cast<const float4 *>(&xs[0][j]);
-                    const double y0 = sbar(tb + j, x4.x);
-                    const double y1 = sbar(tb + j + 1, x4.y);
-                    const double y2 = sbar(tb + j + 2, x4.z);
-                    const double y3 = sbar(tb + j + 3, x4.w);
-                    if (emit) {
-                        ob[lane][j & (SW - 1)] = (float)y0;
-                        ob[lane][(j + 1) & (SW - 1)] = (float)y1;
-                        ob[lane][(j + 2) & (SW - 1)] = (float)y2;
-                        ob[lane][(j + 3) & (SW - 1)] = (float)y3;
-                        if (SW == 32 && ((j + 4) & 31) == 0) flush_half(tb, j >> 5);
-                    }
-                }
-            }
         } else if (tb + 64 <= c1 && __all(!active || (start < tb && tb + 64 <= e.seed_end()))) {
             // every lane still accumulating its warm-up seed for the whole block
 #pragma unroll 2
             for (int j = 0; j < 64; j += 4) {
-                const float4 x4 = *reinterpret_cast<const float4 *>(&xs[0][j]);
-                double y0, y1, y2, y3;
+                const float4 x4 = *reinterpret_cast<const float4 *>(&xs[j]);
                 if constexpr (NIN == 1) {
-                    y0 = e.seed_step(tb + j, x4.x);
-                    y1 = e.seed_step(tb + j + 1, x4.y);
-                    y2 = e.seed_step(tb + j + 2, x4.z);
-                    y3 = e.seed_step(tb + j + 3, x4.w);
+                    emit(tb, j, e.seed_step(tb + j, x4.x));
+                    emit(tb, j + 1, e.seed_step(tb + j + 1, x4.y));
+                    emit(tb, j + 2, e.seed_step(tb + j + 2, x4.z));
+                    emit(tb, j + 3, e.seed_step(tb + j + 3, x4.w));
                 } else {
-                    const float4 h4 = *reinterpret_cast<const float4 *>(&xs[1][j]);
-                    const float4 l4 = *reinterpret_cast<const float4 *>(&xs[2][j]);
-                    y0 = e.seed_step(tb + j, h4.x, l4.x, x4.x);
-                    y1 = e.seed_step(tb + j + 1, h4.y, l4.y, x4.y);
-                    y2 = e.seed_step(tb + j + 2, h4.z, l4.z, x4.z);
-                    y3 = e.seed_step(tb + j + 3, h4.w, l4.w, x4.w);
-                }
-                if (emit) {
-                    ob[lane][j & (SW - 1)] = (float)y0;
-                    ob[lane][(j + 1) & (SW - 1)] = (float)y1;
-                    ob[lane][(j + 2) & (SW - 1)] = (float)y2;
-                    ob[lane][(j + 3) & (SW - 1)] = (float)y3;
-                    if (SW == 32 && ((j + 4) & 31) == 0) flush_half(tb, j >> 5);
+                    const float4 h4 = *reinterpret_cast<const float4 *>(&xs[64 + j]);
+                    const float4 l4 = *reinterpret_cast<const float4 *>(&xs[128 + j]);
+                    emit(tb, j, e.seed_step(tb + j, h4.x, l4.x, x4.x));
+                    emit(tb, j + 1, e.seed_step(tb + j + 1, h4.y, l4.y, x4.y));
+                    emit(tb, j + 2, e.seed_step(tb + j + 2, h4.z, l4.z, x4.z));
+                    emit(tb, j + 3, e.seed_step(tb + j + 3, h4.w, l4.w, x4.w));
                 }
             }
         } else
@@ -1417,199 +1071,685 @@ __device__ __forceinline__ void drive_batch(const batch_view &a, float *out) {
             const int t = tb + j;
             double y = REC_NAN;
             if (active && t < c1) {
-                const double x = xs[0][j];
+                const double x = xs[j];
                 if (t == start) {
-                    // (a carried lane began before the loop)
                     if constexpr (NIN == 1) {
-                        if (carried) {
-                        } else if (seeded) {
-                            if constexpr (E::kSeeded) y = e.begin_seeded(seedv);
-                        } else if (burn) e.begin_burn(x);
-                        else y = e.begin_exact(x);
+                        if (burn) e.begin_burn(x); else y = e.begin_exact(x);
                     } else {
-                        if (carried) {
-                        } else if (burn) e.begin_burn(xs[1][j], xs[2][j], x);
-                        else y = e.begin_exact(xs[1][j], xs[2][j], x);
+                        if (burn) e.begin_burn(xs[64 + j], xs[128 + j], x);
+                        else y = e.begin_exact(xs[64 + j], xs[128 + j], x);
                     }
                 } else if (t > start) {
                     if constexpr (NIN == 1) y = e.step(t, x);
-                    else y = e.step(t, xs[1][j], xs[2][j], x);
+                    else y = e.step(t, xs[64 + j], xs[128 + j], x);
                 }
             }
-            if (emit) {
-                ob[lane][j & (SW - 1)] = (float)y;
-                if (SW == 32 && (j & 31) == 31) flush_half(tb, j >> 5);
-            }
+            emit(tb, j, y);
         }
-        // 64-bar staging: one flush per block, after whichever path ran; each
-        // store writes one row x 64 bars (lane = bar)
-        if (SW == 64 && emit) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (tb + 64 > c0) {
-                const int t = tb + lane;
-                const bool ok = t >= c0 && t < c1;
-                for (int r = 0; r < nrow; ++r)
-                    if (ok) out[(size_t)(a.group * 64 + r) * T + t] = ob[r][lane & (SW - 1)];
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    if constexpr (E::kScan > 0) {
-        // chunk-end states: all of them after pass 1; after pass 2 (two-stage
-        // engines) only the second stage's, next to the folded first stage
-        if ((a.phase == 1 || a.phase == 2) && active && k + 1 < a.nch) {
-            double st[S];
-            e.get_state(c1 - 1, st);
-            double *cs = a.carry + ((size_t)c * a.nch + k) * S;
-            const int lo = a.phase == 2 ? S - 1 : 0;
-#pragma unroll
-            for (int i = 0; i < S; ++i)
-                if (i >= lo) cs[i] = st[i];
-        }
+        wave_lds_sync();
     }
 }
 
-// Folds the chunk-end states of pass 1 in chunk order, in place: a carried
-// chunk k maps the state at its start to s_k = g_k s_{k-1} + b_k, with b_k its
-// zero-start run and g_k = gain(c0, c1); a chunk that ran exactly from
-// first_valid has g_k = 0.  One wave per combo; the carry holds [combo]
-// [chunk][state].  64 chunks at a time: an inclusive scan of the affine maps
-// across the lanes, (g, b) o (g', b') = (g g', g b' + b), then the previous
-// row's last state applied.  Two-stage engines fold their first-stage states
-// after pass 1 (a.phase = 1) and their second-stage state after pass 2.
-// A chunk that ends before first_valid stores an undefined state; the chunk
-// after it always has g = 0, so a g = 0 step selects b instead of forming
-// 0 * s (which is NaN for an undefined s).
+// ---------------------------------------------------------------- chunked scan
+//
+// A clean series (every bar from first_valid on finite) in chunks of whole
+// 64-bar blocks.  Up to a per-combo bar sw the state is the plain sum of the
+// bars' terms, after it s = beta s + w f: with the averages kept as sums
+// (p times Wilder's average; RSI's and DX's ratios cancel the factor) every
+// indicator is s = (t > sw ? beta : 1) s + f, an affine map of the state, and
+// the terms f are the same for every combo.  So
+//   scan_prepare   forms the terms once per bar in f64 (EMA, SMMA, Wilders the
+//                  close, RSI 100 x the gain and the absolute change, ATR the true
+//                  range, ADX +DM + -DM, +DM - -DM and the true range: the
+//                  ratios' own numerators and denominators), zero before
+//                  first_valid,
+//   scan_states    runs each chunk from a zero state: one fma per state, bar
+//                  and combo, the term a scalar operand,
+//   scan_output    folds the chunks before its own in order, s_k = g_k s_{k-1}
+//                  + b_k with g_k the product of the chunk's multipliers,
+//                  runs its chunk from that exact state and writes it;
+//   scan_spans     between them (long scans) folds every `span` chunks into
+//                  one map first, so that a wave folds at most the spans and
+//                  one span's chunks.
+// ADX's second stage (the sum, then the smoothing of DX) is a scan of its own
+// over DX: scan_output without stores (scan = 2) gives its chunk states.
+// The terms come through the scalar cache: the combos of a wave share them, so
+// the vector unit only does the combos' own work, no block stages bars in LDS
+// and a warm-up bar costs two selects more than another.  Terms of more
+// than the context's buffer holds run in segments [t0, t1), the states passed
+// on in state_in / state_out.
+//
+// Whole calls before (bars staged in LDS and widened in every lane, a launch
+// with one wave per combo folding the chunks) and now:
+//   1,250 EMA / RSI / ADX x 200k bars (1.0 GB)   282 / 366 / 709 -> 239 / 266 / 448 us
+//   33 RSI x 10,007 bars                         59 -> 18 us
+//   40 RSI series of up to 50k bars, 74 MB       124 -> 71 us
+// The first two are near the rate such rows are written at (~5.2 TB/s, 193
+// us); ADX is bound by its two divisions and two f64 rounds per output.
+
+typedef const __attribute__((address_space(4))) double scan_term;
+
+// Per-combo constants of the scan.
+struct scan_lane {
+    double beta;             // multiplier past sw
+    double w;                // weight of a term past sw (EMA alpha, else 1)
+    double kap;              // factor on the state at sw (EMA 1 / p, else 1)
+    double scale, scale0;    // output = scale s past sw, scale0 s at sw
+    int sw;                  // last bar of the plain sum
+    int first;               // first bar with an output
+    int sw2;                 // ADX: last bar of the DX sum
+};
+
 template <class E>
-__device__ __forceinline__ void scan_combine(const batch_view &a) {
-    const int c = a.group;                  // the combo
-    const int lane = threadIdx.x & 63;
-    if (c >= a.nlanes || !a.clean) return;
-    E e;
-    e.setup(a.periods[c], a.fv);
-    apply_alpha(e, a.alphas, c);
-    constexpr int S = E::kScan > 0 ? E::kScan : 1;
-    int lo = 0, hi = S;
-    bool second = false;
-    if constexpr (E::kTwoStage) {
-        if (a.phase == 2) {
-            lo = S - 1;
-            second = true;
-        } else {
-            hi = S - 1;
+__device__ __forceinline__ scan_lane scan_params(const batch_view &a, int c, bool active) {
+    scan_lane q;
+    const int p = active ? a.periods[c] : 1;
+    const double pf = (double)p;
+    q.w = q.kap = q.scale = q.scale0 = 1.0;
+    q.sw = a.fv + p - 1;
+    q.first = q.sw;
+    q.sw2 = 0;
+    if constexpr (__is_same(E, EmaEng)) {
+        q.w = active && a.alphas ? (double)a.alphas[c] : 2.0 / (pf + 1.0);
+        q.beta = 1.0 - q.w;
+        q.kap = 1.0 / pf;
+        q.first = a.fv;
+    } else if constexpr (__is_same(E, WildersEng)) {
+        const double al = active && a.alphas ? (double)a.alphas[c] : 1.0 / pf;
+        q.beta = p == 1 ? 0.0 : 1.0 - al;        // p = 1 copies after its first bar
+        q.scale = p == 1 ? 1.0 : al;
+        q.scale0 = al;
+    } else if constexpr (__is_same(E, SmmaEng)) {
+        q.scale = q.scale0 = 1.0 / pf;
+        q.beta = (pf - 1.0) * q.scale;
+    } else {
+        const double rp = 1.0 / pf;
+        q.beta = 1.0 - rp;
+        q.scale = q.scale0 = rp;
+        if constexpr (__is_same(E, RsiEng)) {
+            q.sw = q.first = a.fv + p;
+        } else if constexpr (__is_same(E, AdxEng)) {
+            q.sw = a.fv + p;
+            q.sw2 = a.fv + 2 * p - 1;
+            q.first = p == 1 ? a.fv + 2 : q.sw2;
+            q.scale = 100.0 * rp;
         }
     }
-    const int nch = (a.T + a.chunk - 1) / a.chunk;
-    const int nst = nch - 1;                 // chunk-end states read by later chunks
-    double *base = a.carry + (size_t)c * nch * S;
-    double cin[S];
+    return q;
+}
+
+template <class E> struct scan_dims {                // terms and first-stage states
+    static constexpr int N = __is_same(E, AdxEng) ? 3 : (__is_same(E, RsiEng) ? 2 : 1);
+    static constexpr int S = __is_same(E, AdxEng) ? 4 : N;
+};
+
+// Wave-wide maximum, as a scalar.
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
+
+// Where term i of an indicator with n of them is for bar r of the buffer:
+// [tstride][2] pairs for two or three terms, then the third's [tstride].
+__host__ __device__ __forceinline__ size_t scan_term_at(int n, int i, int tstride, long r) {
+    return n == 1 ? (size_t)r : i < 2 ? 2 * (size_t)r + i : 2 * (size_t)tstride + r;
+}
+
+// Terms i of bars t, t + 1, ... (every second value for i < 2 of a pair).
+template <class E>
+__device__ __forceinline__ scan_term *scan_at(const batch_view &a, int i, int t) {
+    return (scan_term *)(a.terms + scan_term_at(scan_dims<E>::N, i, a.tstride, t - a.t0));
+}
+
+// The N terms of U bars from bar t on.
+template <class E, int N, int U>
+__device__ __forceinline__ void scan_fetch(const batch_view &a, int t, double (&f)[U][N]) {
+    constexpr int step = scan_dims<E>::N == 1 ? 1 : 2;
+    scan_term *p = scan_at<E>(a, 0, t);
 #pragma unroll
-    for (int i = 0; i < S; ++i) cin[i] = 0.0;
-    for (int r0 = 0; r0 < nst; r0 += 64) {
-        const int k = r0 + lane;
-        const bool ok = k < nst;
-        const int c0 = k * a.chunk;
-        const int c1 = min(c0 + a.chunk, a.T);
-        const bool carried =
-            ok && (E::kWarmScan ? c0 > e.exact_start() : c0 >= e.burn_ok_from());
-        double g = 0.0;
-        if (carried) {
-            if constexpr (E::kTwoStage) g = second ? e.gain2(c0, c1) : e.gain(c0, c1);
-            else g = e.gain(c0, c1);
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < (N < 2 ? N : 2); ++i) f[u][i] = p[u * step + i];
+    if constexpr (N > 2) {
+        scan_term *q = scan_at<E>(a, 2, t);
+#pragma unroll
+        for (int u = 0; u < U; ++u) f[u][2] = q[u];
+    }
+}
+
+// Brings the lines of the terms of bars [c0, c1) into the L2, all at once:
+// scalar loads run one or two lines ahead of their use only, and the terms,
+// written by another kernel, are in no L2 yet (the passes waited ~1,500 cycles
+// on every eight bars).  `keep` takes the values, so that the loads are made.
+template <class E>
+__device__ __forceinline__ void scan_touch(const batch_view &a, int c0, int c1, double &keep) {
+    // (the third term, of odd series only, is left to the scalar loads)
+    constexpr int step = scan_dims<E>::N == 1 ? 1 : 2;
+    const double *p = a.terms + (size_t)step * (c0 - a.t0);
+    for (int r = 16 * (int)(threadIdx.x & 63); r < step * (c1 - c0); r += 64 * 16) {
+        const double v = p[r];
+        asm volatile("" : "+v"(keep) : "v"(v));
+    }
+}
+
+// s = beta s + f with the term as a scalar operand (the compiler would move it
+// to vector registers first, two more instructions per term).
+__device__ __forceinline__ void scan_step(double &s, double beta, double f) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(beta), "v"(s), "s"(f));
+    s = r;
+}
+
+// beta^n, n >= 0.
+__device__ __forceinline__ double scan_pow(double beta, int n) {
+    double r = 1.0;
+    for (; __any(n > 0); n >>= 1) {
+        if (n & 1) r *= beta;
+        beta *= beta;
+    }
+    return r;
+}
+
+// One scan of a wave's combos: plain sums up to bar sw (at most `last` over
+// the wave), times kap there, then beta.
+struct scan_sum {
+    double beta, kap;
+    int sw, last;
+};
+
+// Folds chunks [j, j1) of `chunk` bars onto M states, their loads eight at a
+// time ahead of the chain; gg (may be NULL): times their multipliers.  Past the
+// chunk that holds the wave's last sum every multiplier is beta^chunk; up
+// to it a chunk's is 1, that of its sum's last bar, or beta^chunk by combo.
+// `zero`: the states are zero, so the first multiplier does not matter.
+template <int M>
+__device__ __forceinline__ void scan_chain(const batch_view &a, const scan_sum &q, int chunk,
+                                           const double *b, size_t step, size_t cp, int j, int j1,
+                                           bool zero, double *s, double *gg) {
+    if (j >= j1) return;
+    const double gl = scan_pow(q.beta, chunk);
+    const int jl = q.last < a.t0 ? -1 : (q.last - a.t0) / chunk;
+    double v[M][8];
+    auto fetch = [&](int at) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int i = 0; i < M; ++i) v[i][u] = b[(size_t)min(at + u, j1 - 1) * step + i * cp];
+    };
+    if (j <= jl && !(zero && !gg && j == jl)) {
+        const int r = q.sw - a.t0;                   // < 0: before this segment
+        const int jm = r < 0 ? -1 : r / chunk;
+        const double gm = q.kap * scan_pow(q.beta, r < 0 ? 0 : chunk - 1 - r % chunk);
+        for (const int m = min(j1, jl + 1); j < m; ++j) {
+            const double g = j > jm ? gl : (j == jm ? gm : 1.0);
+            if (gg) *gg *= g;
+#pragma unroll
+            for (int i = 0; i < M; ++i) s[i] = fma(g, s[i], b[(size_t)j * step + i * cp]);
         }
-        double b[S];
+    }
+    for (; j < j1; j += 8) {
+        fetch(j);
 #pragma unroll
-        for (int i = 0; i < S; ++i) b[i] = (ok && i >= lo && i < hi) ? base[(size_t)k * S + i] : 0.0;
+        for (int u = 0; u < 8; ++u)
+            if (j + u < j1) {
+                if (gg) *gg *= gl;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const double gu = __shfl_up(g, o);
-            double bu[S];
+                for (int i = 0; i < M; ++i) s[i] = fma(gl, s[i], v[i][u]);
+            }
+    }
+}
+
+// The exact states [i0, i0 + M) of combo c at the start of the wave's chunk
+// (sum up to bar sw, then beta): the segment's incoming state, the spans, then
+// the chunks, in a cooperative block each wave a share of the chunks before
+// the block as one affine map (lds: 64 (M + 1) doubles per wave; every wave of
+// the block calls it).
+template <int M>
+__device__ __forceinline__ void scan_start(const batch_view &a, const scan_sum &q, int S, int i0,
+                                           int c, double *s, double *lds) {
+    const size_t cp = (size_t)a.groups * 64, step = (size_t)S * cp;
+    const double *b = a.carry + (size_t)i0 * cp + c;
+    const bool idle = wave_idle(a), zero = a.state_in == nullptr;
 #pragma unroll
-            for (int i = 0; i < S; ++i) bu[i] = __shfl_up(b[i], o);
-            if (lane >= o) {
+    for (int i = 0; i < M; ++i)
+        s[i] = !zero && !idle ? a.state_in[(size_t)(i0 + i) * cp + c] : 0.0;
+    int j = 0;
+    if (a.span && !idle) {
+        const int n = a.k / a.span;
+        scan_chain<M>(a, q, a.chunk * a.span, b + (size_t)a.nch * step, step, cp, 0, n, zero, s,
+                      nullptr);
+        j = n * a.span;
+    }
+    if (!a.coop) {
+        if (!idle)
+            scan_chain<M>(a, q, a.chunk, b, step, cp, j, a.k, zero && j == 0, s, nullptr);
+        return;
+    }
+    const int lane = threadIdx.x & 63, w = a.k - a.kb;
+    double m[M], gg = 1.0;
 #pragma unroll
-                for (int i = 0; i < S; ++i) b[i] = g != 0.0 ? fma(g, bu[i], b[i]) : b[i];
-                g *= gu;
+    for (int i = 0; i < M; ++i) m[i] = 0.0;
+    // (an idle wave's share counts too; a span holds whole blocks)
+    const int j0 = a.span ? a.kb / a.span * a.span : 0, all = a.kb - j0;
+    scan_chain<M>(a, q, a.chunk, b, step, cp, j0 + all * w / REC_WPB,
+                  j0 + all * (w + 1) / REC_WPB, false, m, &gg);
+    double v[M][REC_WPB - 1];                        // the chunks of the block before this one
+#pragma unroll
+    for (int u = 0; u < REC_WPB - 1; ++u)
+#pragma unroll
+        for (int i = 0; i < M; ++i)
+            v[i][u] = b[(size_t)min(a.kb + u, a.nch - 1) * step + i * cp];
+    double *to = lds + w * 64 * (M + 1) + lane;
+    to[0] = gg;
+#pragma unroll
+    for (int i = 0; i < M; ++i) to[64 * (i + 1)] = m[i];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < REC_WPB; ++q) {
+        const double *from = lds + q * 64 * (M + 1) + lane;
+#pragma unroll
+        for (int i = 0; i < M; ++i) s[i] = fma(from[0], s[i], from[64 * (i + 1)]);
+    }
+    const int r = q.sw - a.t0, jm = r < 0 ? -1 : r / a.chunk;
+    const double gl = scan_pow(q.beta, a.chunk);
+    const double gm = q.kap * scan_pow(q.beta, r < 0 ? 0 : a.chunk - 1 - r % a.chunk);
+#pragma unroll
+    for (int u = 0; u < REC_WPB - 1; ++u)
+        if (u < w) {
+            const double g = a.kb + u > jm ? gl : (a.kb + u == jm ? gm : 1.0);
+#pragma unroll
+            for (int i = 0; i < M; ++i) s[i] = fma(g, s[i], v[i][u]);
+        }
+    __syncthreads();
+}
+
+// Pass 1: the chunk's states from zero, for G groups [a.group, a.group + G) per
+// wave: each term read then feeds G lanes' combos (the scalar cache hands out
+// a line every ~16 cycles, more than one group's fma of it takes: 1,250 EMAs x
+// 200k bars took 36 us at one group per wave, 27 at four).  ODD (ADX only):
+// the true range is summed too (see scan_prepare).
+template <class E, bool ODD, int G>
+__device__ __forceinline__ void scan_states(const batch_view &a) {
+    constexpr int N = __is_same(E, AdxEng) && !ODD ? 2 : scan_dims<E>::N;
+    constexpr int S = scan_dims<E>::S;
+    constexpr bool EMA = __is_same(E, EmaEng);
+    const int lane = threadIdx.x & 63;
+    const int c0 = a.t0 + a.k * a.chunk, c1 = c0 + a.chunk;
+    double keep = 0.0;
+    scan_touch<E>(a, c0, c1, keep);
+    scan_lane q[G];
+    double s[G][N];
+    int smax = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int c = (a.group + g) * 64 + lane;
+        q[g] = scan_params<E>(a, c, c < a.nlanes);
+        smax = max(smax, q[g].sw);
+#pragma unroll
+        for (int i = 0; i < N; ++i) s[g][i] = 0.0;
+    }
+    smax = wave_max(smax);
+    int t = c0;
+    const bool mixed = t <= smax;                    // a sum in this chunk
+    // eight bars' terms at a time, the next eight on their way (a scalar load
+    // per bar would be waited for per bar)
+    double f[8][N];
+    if (mixed) {
+        scan_fetch<E, N, 8>(a, t, f);
+        for (const int m = EMA ? c1 : min(c1, (smax + 8) & ~7); t < m; t += 8) {
+            double n[8][N];
+            scan_fetch<E, N, 8>(a, min(t + 8, c1 - 8), n);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const bool past = t + u > q[g].sw;
+                    const double b = past ? q[g].beta : 1.0;
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        s[g][i] = fma(b, s[g][i], EMA && past ? q[g].w * f[u][i] : f[u][i]);
+                        if (EMA && t + u == q[g].sw) s[g][i] *= q[g].kap;
+                    }
+                }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int i = 0; i < N; ++i) f[u][i] = n[u][i];
+        }
+    }
+    auto steps = [&](const double (&from)[8][N]) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int i = 0; i < N; ++i) scan_step(s[g][i], q[g].beta, from[u][i]);
+    };
+    if (t < c1) scan_fetch<E, N, 8>(a, t, f);
+    for (; t + 8 < c1; t += 8) {
+        double n[8][N];
+        scan_fetch<E, N, 8>(a, t + 8, n);
+        steps(f);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int i = 0; i < N; ++i) f[u][i] = n[u][i];
+    }
+    if (t < c1) steps(f);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if (a.group + g >= a.groups) continue;
+        double *o = a.carry + (size_t)a.k * S * a.groups * 64 + (a.group + g) * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            o[(size_t)i * a.groups * 64] = EMA && !mixed ? s[g][i] * q[g].w : s[g][i];
+    }
+}
+
+// State i of one group's whole span q from zero: one wave per group, span and
+// state (block.y).
+template <class E>
+__device__ __forceinline__ void scan_spans(const batch_view &a, int q, int i) {
+    constexpr int S = scan_dims<E>::S;
+    const int c = a.group * 64 + (threadIdx.x & 63);
+    const size_t cp = (size_t)a.groups * 64, step = (size_t)S * cp;
+    const scan_lane p = scan_params<E>(a, c, c < a.nlanes);
+    const int sw = a.scan == 2 ? p.sw2 : p.sw;
+    const scan_sum sum{p.beta, p.kap, sw, wave_max(sw)};
+    double *b = a.carry + (size_t)i * cp + c;
+    double s[1] = {0.0};
+    scan_chain<1>(a, sum, a.chunk, b, step, cp, q * a.span, (q + 1) * a.span, true, s, nullptr);
+    b[(size_t)(a.nch + q) * step] = s[0];
+}
+
+// RSI from the sums of 100 times the gain and of the absolute change, DX / 100 from the DM difference
+// and sum, in f32 as rsi_ratio_f32 and dx_ratio form them (50 and 0 for a zero
+// denominator).
+__device__ __forceinline__ float scan_rsi(double gain, double all) {
+    const float den = (float)all;
+    if (!(den > 1e-30f && den < 1e30f))
+        return all == 0.0 ? 50.0f : (float)(gain / all);
+    float r = __builtin_amdgcn_rcpf(den);
+    r = fmaf(fmaf(-den, r, 1.0f), r, r);
+    return (float)gain * r;
+}
+__device__ __forceinline__ float scan_dx(double diff, double all) {
+    return all != 0.0 ? (float)dx_ratio(fabs(diff), all) : 0.0f;
+}
+
+// A chunk from its exact start state: the outputs (EMIT), or ADX's second
+// stage from zero for its scan.  Blocks of 32 bars past every sum run the
+// plain updates, eight terms at a time; the others select per bar.
+template <class E, bool ODD, bool EMIT>
+__device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
+    constexpr bool EMA = __is_same(E, EmaEng), RSI = __is_same(E, RsiEng),
+                   ADX = __is_same(E, AdxEng);
+    constexpr int N = ADX && !ODD ? 2 : scan_dims<E>::N;
+    constexpr int S = scan_dims<E>::S;
+    extern __shared__ __align__(16) double rec_lds[];
+    float *ob = EMIT ? reinterpret_cast<float *>(wave_lds<E>()) : nullptr;   // [64][REC_ROW]
+    const int lane = threadIdx.x & 63;
+    const int c = a.group * 64 + lane;
+    const size_t cp = (size_t)a.groups * 64;
+    const int c0 = a.t0 + a.k * a.chunk, c1 = min(c0 + a.chunk, a.t1);
+    double keep = 0.0;
+    if (!wave_idle(a)) scan_touch<E>(a, c0, c1, keep);
+    const scan_lane q = scan_params<E>(a, c, c < a.nlanes);
+    double s[N], dxs = 0.0;                          // dxs: ADX's second stage
+    scan_start<N>(a, scan_sum{q.beta, q.kap, q.sw, wave_max(q.sw)}, S, 0, c, s, rec_lds);
+    const int last = wave_max(ADX ? max(q.sw2, q.first) : q.sw);
+    if (ADX && EMIT)
+        scan_start<1>(a, scan_sum{q.beta, 1.0, q.sw2, last}, S, S - 1, c, &dxs, rec_lds);
+    if (wave_idle(a) || (!EMIT && a.k + 1 >= a.nch)) return;
+    const int nrow = min(64, a.nlanes - a.group * 64);
+    float *row0 = out + (size_t)(a.group * 64 + (lane >> 3)) * a.T + 4 * (lane & 7);
+    const float *src = ob + (lane >> 3) * REC_ROW + 4 * (lane & 7);
+    for (int tb = c0; tb < c1; tb += 32) {
+        float *dst = ob + lane * REC_ROW;
+        if (tb > last) {
+#pragma unroll
+            for (int b = 0; b < 32; b += 4) {
+                double f[4][N];
+                scan_fetch<E, N, 4>(a, tb + b, f);
+                {
+                    float y[4];
+                    if constexpr (RSI || ADX) {
+                        // four bars' denominators are checked together against
+                        // the f32 reciprocal's range; outside it, the f64 forms
+                        double u0[4], u1[4];         // denominators and numerators
+                        bool some = true;            // no zero range sum (ODD)
+                        float num[4], den[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                            for (int i = 0; i < N; ++i) scan_step(s[i], q.beta, f[u][i]);
+                            u0[u] = RSI ? s[1] : s[0];
+                            u1[u] = RSI ? s[0] : s[1];
+                            // a zero range sum makes DX zero
+                            if (ODD) u0[u] = s[N - 1] != 0.0 ? u0[u] : 0.0;
+                            if (ODD) some = some && s[N - 1] != 0.0;
+                            num[u] = fabsf((float)u1[u]);
+                            den[u] = (float)u0[u];
+                        }
+                        // (as integers: none is negative, and a NaN is above all)
+                        uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const uint32_t d = __builtin_bit_cast(uint32_t, den[u]);
+                            lo = min(lo, d);
+                            hi = max(hi, d);
+                        }
+                        const bool fast = lo > __builtin_bit_cast(uint32_t, 1e-30f) &&
+                                          hi < __builtin_bit_cast(uint32_t, 1e30f) && some;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            float r = __builtin_amdgcn_rcpf(den[u]);
+                            r = fmaf(fmaf(-den[u], r, 1.0f), r, r);
+                            y[u] = num[u] * r;
+                        }
+                        if (!fast) {
+#pragma unroll
+                            for (int u = 0; u < 4; ++u)
+                                y[u] = RSI ? scan_rsi(u1[u], u0[u]) : scan_dx(u1[u], u0[u]);
+                        }
+                        if constexpr (ADX) {
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) {
+                                dxs = fma(q.beta, dxs, (double)y[u]);
+                                y[u] = (float)(dxs * q.scale);
+                            }
+                        }
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            if (EMA) s[0] = fma(q.beta, s[0], q.w * f[u][0]);
+                            else scan_step(s[0], q.beta, f[u][0]);
+                            y[u] = (float)(EMA ? s[0] : s[0] * q.scale);
+                        }
+                    }
+                    if (EMIT)
+                        *reinterpret_cast<float4 *>(dst + b) = make_float4(y[0], y[1], y[2], y[3]);
+                }
+            }
+        } else {
+            // EMA's running mean divides by the bars so far, the same for
+            // every combo: lane j forms the reciprocal for bar tb + j
+            double inv = 0.0;
+            if (EMA) inv = 1.0 / (double)(tb + (lane & 31) - a.fv + 1);
+            double f[4][N];
+            scan_fetch<E, N, 4>(a, tb, f);
+            for (int b = 0; b < 32; b += 4) {
+                double n[4][N];                      // the next four bars' terms
+                scan_fetch<E, N, 4>(a, tb + min(b + 4, 28), n);
+                float y[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int t = tb + b + u;
+                    const bool past = t > q.sw;
+                    const double g = past ? q.beta : 1.0;
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        s[i] = fma(g, s[i], EMA && past ? q.w * f[u][i] : f[u][i]);
+                        if (EMA && t == q.sw) s[i] *= q.kap;
+                    }
+                    double v;
+                    if constexpr (EMA) {
+                        const double iv = __shfl(inv, b + u);   // every lane takes part
+                        v = t < q.sw ? s[0] * iv : s[0];
+                    } else if constexpr (RSI) {
+                        v = (double)scan_rsi(s[0], s[1]);
+                    } else if constexpr (ADX) {
+                        const bool some = !ODD || s[N - 1] != 0.0;
+                        const double dx = (double)scan_dx(s[1], some ? s[0] : 0.0);
+                        dxs = fma(t > q.sw2 ? q.beta : 1.0, dxs, t >= q.sw ? dx : 0.0);
+                        v = dxs * q.scale;
+                    } else {
+                        v = s[0] * (t == q.sw ? q.scale0 : q.scale);
+                    }
+                    y[u] = t >= q.first ? (float)v : VTA_QNAN_F32;
+                }
+                if (EMIT)
+                    *reinterpret_cast<float4 *>(dst + b) = make_float4(y[0], y[1], y[2], y[3]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int i = 0; i < N; ++i) f[u][i] = n[u][i];
             }
         }
+        if (EMIT) {
+            // eight rows x 128 bytes per store
+            wave_lds_sync();
+            typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));
+            if (tb + 32 <= c1) {
 #pragma unroll
-        for (int i = 0; i < S; ++i) {
-            const double y = g != 0.0 ? fma(g, cin[i], b[i]) : b[i];
-            if (ok && i >= lo && i < hi) base[(size_t)k * S + i] = y;
-            cin[i] = __shfl(y, 63);
+                for (int i = 0; i < 8; ++i)
+                    if (8 * i + (lane >> 3) < nrow)
+                        *reinterpret_cast<row4 *>(row0 + (size_t)(8 * i) * a.T + tb) =
+                            *reinterpret_cast<const row4 *>(src + 8 * i * REC_ROW);
+            } else {
+                for (int i = 0; i < 8; ++i)
+                    for (int u = 0; u < 4; ++u)
+                        if (8 * i + (lane >> 3) < nrow && tb + 4 * (lane & 7) + u < c1)
+                            row0[(size_t)(8 * i) * a.T + tb + u] = src[8 * i * REC_ROW + u];
+            }
+            wave_lds_sync();
         }
+    }
+    if (EMIT) {
+        if (a.state_out && a.k == a.nch - 1) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) a.state_out[(size_t)i * cp + c] = s[i];
+            if (ADX) a.state_out[(size_t)(S - 1) * cp + c] = dxs;
+        }
+    } else {
+        a.carry[((size_t)a.k * S + S - 1) * cp + c] = dxs;
     }
 }
 
-extern "C" __global__ __launch_bounds__(64) void ema_batch_f32(rec_args a) {
-    drive_batch<EmaEng, 1>(view_of(a), a.out0);
+// The passes of a block: scan_states (all chunks but the last), ADX's second
+// stage, the output pass (an unclean series: one exact chunk in the first
+// block of each group).
+template <class E>
+__device__ __forceinline__ void scan_pass1(batch_view a) {
+    if (!a.clean) return;
+    const bool odd = __is_same(E, AdxEng) && a.odd;
+    if (a.coop) {
+        if (a.k + 1 >= a.nch) return;
+        if (odd) scan_states<E, true, 1>(a);
+        else scan_states<E, false, 1>(a);
+    } else {
+        // four groups per wave: the first quarter of the blocks take all chunks
+        // (a whole run of them, so that every XCD has its share) but those
+        // with a sum in them, whose steps are long: the next blocks take
+        // these, one group per wave
+        const int w = a.group % REC_WPB, quarter = (a.nch + REC_WPB - 1) / REC_WPB;
+        a.group -= w;
+        int sw = 0;
+        for (int g = 0; g < REC_WPB; ++g) {
+            const int c = (a.group + g) * 64 + (int)(threadIdx.x & 63);
+            sw = max(sw, scan_params<E>(a, c, c < a.nlanes).sw);
+        }
+        sw = wave_max(sw);
+        int sums = sw < a.t0 ? 0 : (sw - a.t0) / a.chunk + 1;
+        if (quarter + sums > a.nch) sums = 0;        // (too few blocks for that)
+        if (a.k >= quarter) {
+            a.k -= quarter;
+            a.group += w;
+            if (a.k >= sums || a.k + 1 >= a.nch || a.group >= a.groups) return;
+            if (odd) scan_states<E, true, 1>(a);
+            else scan_states<E, false, 1>(a);
+            return;
+        }
+        a.k = REC_WPB * a.k + w;
+        if (a.k < sums || a.k + 1 >= a.nch) return;
+        if (odd) scan_states<E, true, REC_WPB>(a);
+        else scan_states<E, false, REC_WPB>(a);
+    }
 }
-extern "C" __global__ __launch_bounds__(64) void rsi_batch_f32(rec_args a) {
-    drive_batch<RsiEng, 1>(view_of(a), a.out0);
+__device__ __forceinline__ void scan_pass2(const batch_view &a) {
+    if (!a.clean || a.nch < 2) return;               // (a one-chunk job has no carry)
+    if (a.odd) scan_output<AdxEng, true, false>(a, nullptr);
+    else scan_output<AdxEng, false, false>(a, nullptr);
 }
-extern "C" __global__ __launch_bounds__(64) void atr_batch_f32(rec_args a) {
-    drive_batch<AtrEng, 3>(view_of(a), a.out0);
+template <class E, int NIN>
+__device__ __forceinline__ void batch_pass(batch_view a, float *out) {
+    if (a.scan == 0) {
+        if (!wave_idle(a)) drive_batch<E, NIN>(a, out);
+    } else if (!a.clean) {
+        if (wave_idle(a) || a.k != 0 || a.t0 != 0) return;
+        a.chunk = a.T;
+        drive_batch<E, NIN>(a, out);
+    } else if (__is_same(E, AdxEng) && a.odd) {
+        scan_output<E, true, true>(a, out);
+    } else {
+        scan_output<E, false, true>(a, out);
+    }
 }
-extern "C" __global__ __launch_bounds__(64) void smma_batch_f32(rec_args a) {
-    drive_batch<SmmaEng, 1>(view_of(a), a.out0);
-}
-extern "C" __global__ __launch_bounds__(64) void wilders_batch_f32(rec_args a) {
-    drive_batch<WildersEng, 1>(view_of(a), a.out0);
-}
-extern "C" __global__ __launch_bounds__(64) void adx_batch_f32(rec_args a) {
-    drive_batch<AdxEng, 3>(view_of(a), a.out0);
-}
-extern "C" __global__ __launch_bounds__(64) void adx_scan_combine(rec_args a) {
-    scan_combine<AdxEng>(view_of(a));
-}
-extern "C" __global__ __launch_bounds__(64) void atr_tr_batch_f32(rec_args a) {
-    drive_batch<AtrTrEng, 1>(view_of(a), a.out0);
-}
-extern "C" __global__ __launch_bounds__(64) void atr_tr_scan_combine(rec_args a) {
-    scan_combine<AtrTrEng>(view_of(a));
+template <class E>
+__device__ __forceinline__ void span_pass(batch_view &a, int flat) {
+    if (!a.clean) return;
+    const int per = (a.nch - 1) / a.span;            // spans read by later chunks
+    const int i = a.scan == 2 ? scan_dims<E>::S - 1 : (int)blockIdx.y;
+    if (__is_same(E, AdxEng) && i == 2 && !a.odd) return;
+    a.group = flat / per;
+    scan_spans<E>(a, flat % per, i);
 }
 
-// True range of one series (tr_from_hlc_f32 in the reference): 0 before
-// first_valid, high - low at first_valid, then max(h - l, |h - c[t-1]|,
-// |l - c[t-1]|), evaluated in f64 (exact for f32 inputs) and rounded once.
 // ---------------------------------------------------------------- packed batches
 //
 // Many one-series batches of one indicator in one launch per scan pass: job j
 // is a series (its own length, first_valid and output) with its own period
-// table.  A pass is a 1-D grid over every job's (combo group, chunk) blocks,
-// job j owning blocks [block0, block0 + groups * nch); a fold is a 1-D grid
-// over every job's combos, job j owning [combo0, combo0 + nlanes).  A block
-// finds its job by binary search over block0 (combo0), then runs exactly the
-// block of that job's direct launch, so a job's outputs are bit-identical
+// table.  A pass is a 1-D grid over every job's blocks (a combo group and
+// REC_WPB chunks, or the other way round), job j owning those from block0 on;
+// the span folds are a 1-D grid likewise, from span0 on.  A block finds its
+// job by binary search over block0 (span0), then runs exactly
+// the block of that job's direct launch, so a job's outputs are bit-identical
 // alone and packed.
 struct rec_job {
     const float *x, *h, *l;
     const int32_t *periods;
     float *out;
-    double *carry;           // this job's [combo][chunk][states]
-    int T, nlanes, fv, chunk, nch, groups, block0, combo0;
+    double *carry;           // this job's [chunk][state][64 x groups] and spans
+    double *terms;           // this job's [term][tstride]
+    int T, nlanes, fv, chunk, nch, groups, block0, span0, tstride, span;
 };
 
 struct rec_pack_args {
     const rec_job *jobs;
-    const int32_t *flags;    // per job: 1 if a bar at or after first_valid is non-finite
+    const int32_t *flags;    // per job: [2 j] a non-finite bar, [2 j + 1] an odd one was met
+                             // (the word equals epoch)
     int n_jobs;
-    int phase;
+    int scan;
+    int epoch;
+    int pad_;
 };
 
-// The last job whose first block (combo) is <= flat; jobs are in order.
-__device__ __forceinline__ int pack_find(const rec_pack_args &p, int flat, bool combos) {
+// The last job whose first block (span) is <= flat; jobs are in order.
+__device__ __forceinline__ int pack_find(const rec_pack_args &p, int flat, bool spans) {
     int lo = 0, hi = p.n_jobs - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        const int first = combos ? p.jobs[mid].combo0 : p.jobs[mid].block0;
+        const int first = spans ? p.jobs[mid].span0 : p.jobs[mid].block0;
         if (first <= flat) lo = mid; else hi = mid - 1;
     }
-    return lo;
+    return __builtin_amdgcn_readfirstlane(lo);
 }
 
 __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
@@ -1617,72 +1757,178 @@ __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     batch_view v;
     v.x = jb.x; v.h = jb.h; v.l = jb.l;
     v.periods = jb.periods;
-    v.carry = jb.carry;
     v.alphas = nullptr;
-    v.seeds = nullptr;
+    v.carry = jb.carry;
+    v.terms = jb.terms;
+    v.state_in = nullptr;
+    v.state_out = nullptr;
     v.T = jb.T;
     v.nlanes = jb.nlanes;
-    v.chunk = jb.chunk;
-    v.nch = jb.nch;
-    v.phase = p.phase;
+    v.chunk = __builtin_amdgcn_readfirstlane(jb.chunk);
+    v.nch = __builtin_amdgcn_readfirstlane(jb.nch);
+    v.groups = __builtin_amdgcn_readfirstlane(jb.groups);
+    v.span = __builtin_amdgcn_readfirstlane(jb.span);
     v.fv = jb.fv;
-    v.clean = p.flags[j] == 0;
-    v.group = 0;
-    v.k = 0;
+    v.t0 = 0;
+    v.t1 = __builtin_amdgcn_readfirstlane(jb.T);
+    v.tstride = jb.tstride;
+    v.scan = v.nch > 1 ? p.scan : 0;                 // one chunk: exact lanes
+    v.clean = p.flags[2 * j] != p.epoch;
+    v.odd = p.flags[2 * j + 1] == p.epoch;
+    v.group = v.kb = v.k = 0;
+    v.coop = false;
     return v;
 }
 
-template <class E, int NIN>
-__device__ __forceinline__ void packed_pass(const rec_pack_args &p) {
+__device__ __forceinline__ batch_view pack_block(const rec_pack_args &p, float **out) {
     const int flat = blockIdx.x;
     const int j = pack_find(p, flat, false);
     batch_view v = pack_view(p, j);
-    const int local = flat - p.jobs[j].block0;
-    const int groups = p.jobs[j].groups;
-    v.group = local % groups;
-    v.k = local / groups;
-    drive_batch<E, NIN>(v, p.jobs[j].out);
+    block_chunk(v, flat - __builtin_amdgcn_readfirstlane(p.jobs[j].block0));
+    *out = p.jobs[j].out;
+    return v;
 }
 
+// (a job without spans owns no block here: the next job starts at its span0)
 template <class E>
-__device__ __forceinline__ void packed_fold(const rec_pack_args &p) {
+__device__ __forceinline__ void packed_spans(const rec_pack_args &p) {
     const int flat = blockIdx.x;
     const int j = pack_find(p, flat, true);
     batch_view v = pack_view(p, j);
-    v.group = flat - p.jobs[j].combo0;
-    scan_combine<E>(v);
+    span_pass<E>(v, flat - __builtin_amdgcn_readfirstlane(p.jobs[j].span0));
 }
 
-#define REC_PACKED(NAME, ENG, NIN)                                                           \
-    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_f32(rec_pack_args p) {    \
-        packed_pass<ENG, NIN>(p);                                                            \
+#define REC_BATCH(NAME, ENG, NIN)                                                            \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_scan_states(rec_args a) {       \
+        scan_pass1<ENG>(view_of(a));                                                         \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_fold(rec_pack_args p) {   \
-        packed_fold<ENG>(p);                                                                 \
+    extern "C" __global__ __launch_bounds__(64) void NAME##_scan_spans(rec_args a) {         \
+        batch_view v = view_of(a);                                                           \
+        span_pass<ENG>(v, blockIdx.x);                                                       \
+    }                                                                                        \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_batch_f32(rec_args a) {         \
+        batch_pass<ENG, NIN>(view_of(a), a.out0);                                            \
     }
+#define REC_PACKED(NAME, ENG, NIN)                                                           \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_states(rec_pack_args p) { \
+        float *out;                                                                          \
+        scan_pass1<ENG>(pack_block(p, &out));                                                \
+    }                                                                                        \
+    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_spans(rec_pack_args p) {  \
+        packed_spans<ENG>(p);                                                                \
+    }                                                                                        \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32(rec_pack_args p) {    \
+        float *out;                                                                          \
+        const batch_view v = pack_block(p, &out);                                            \
+        batch_pass<ENG, NIN>(v, out);                                                        \
+    }
+REC_BATCH(ema, EmaEng, 1)
+REC_BATCH(rsi, RsiEng, 1)
+REC_BATCH(atr, AtrEng, 3)
+REC_BATCH(adx, AdxEng, 3)
+REC_BATCH(smma, SmmaEng, 1)
+REC_BATCH(wilders, WildersEng, 1)
+REC_BATCH(atr_tr, AtrTrEng, 1)
 REC_PACKED(ema, EmaEng, 1)
 REC_PACKED(rsi, RsiEng, 1)
 REC_PACKED(atr, AtrEng, 3)
 REC_PACKED(adx, AdxEng, 3)
 REC_PACKED(smma, SmmaEng, 1)
 REC_PACKED(wilders, WildersEng, 1)
-
-// Per-job non-finite flags: grid (blocks, jobs); block (b, j) checks bars
-// first_valid + b*256 + tid, stepping by gridDim.x * 256.  flags[j] must be 0
-// on entry; every failing lane stores 1.
-extern "C" __global__ __launch_bounds__(256) void packed_nonfinite_flag(const rec_job *jobs,
-                                                                        int32_t *flags,
-                                                                        int hlc) {
-    const rec_job &jb = jobs[blockIdx.y];
-    bool bad = false;
-    for (long t = (long)jb.fv + (long)blockIdx.x * 256 + threadIdx.x; t < jb.T;
-         t += (long)gridDim.x * 256) {
-        bad = bad || !vta_isfinite(jb.x[t]);
-        if (hlc) bad = bad || !vta_isfinite(jb.h[t]) || !vta_isfinite(jb.l[t]);
-    }
-    if (bad) flags[blockIdx.y] = 1;
+extern "C" __global__ __launch_bounds__(256) void adx_scan_stage2(rec_args a) {
+    scan_pass2(view_of(a));
+}
+extern "C" __global__ __launch_bounds__(256) void adx_packed_stage2(rec_pack_args p) {
+    float *out;
+    scan_pass2(pack_block(p, &out));
 }
 
+// The per-bar terms of one series at bar t (kind: 0 the close, 1 RSI, 2 ATR,
+// 3 ADX), zero outside (RSI, ADX: the first delta is at first_valid + 1)
+// [first_valid, T), and whether its inputs are not finite, or odd: a
+// directional move above the true range (a previous close outside its
+// high..low).  Without an odd bar +DM and -DM never exceed the true range
+// they are summed beside, so a zero range sum has a zero DM sum and the
+// DX rule for it (adx.rs:370-390) needs no range sum; with one the range is
+// summed too.
+struct scan_bar { bool bad, odd; };
+__device__ __forceinline__ scan_bar scan_bar_terms(const float *x, const float *h, const float *l,
+                                                   int T, int fv, int kind, long t, double *f) {
+    f[0] = f[1] = f[2] = 0.0;
+    scan_bar r{false, false};
+    if (t < fv || t >= T) return r;
+    const double c = x[t], hi = h ? (double)h[t] : 0.0, lo = l ? (double)l[t] : 0.0;
+    r.bad = !fin(c) || !fin(hi) || !fin(lo);
+    if (kind == 0) {
+        f[0] = c;
+    } else if (t == fv) {
+        if (kind == 2) f[0] = hi - lo;
+    } else if (kind == 1) {
+        const double d = c - (double)x[t - 1];
+        f[0] = d > 0.0 ? 100.0 * d : 0.0;
+        f[1] = fabs(d);
+    } else if (kind == 2) {
+        f[0] = true_range(hi, lo, (double)x[t - 1]);
+    } else {
+        double o[3];
+        AdxEng::pre(hi, lo, c, (double)h[t - 1], (double)l[t - 1], (double)x[t - 1], o);
+        f[0] = o[1] + o[2];      // (one of them is zero)
+        f[1] = o[1] - o[2];
+        f[2] = o[0];
+        r.odd = o[1] > o[0] || o[2] > o[0];
+    }
+    return r;
+}
+
+// The one launch before a device-resident one-series batch: the terms of bars
+// [t0, t1) (t1 up to a whole 64-bar block past the series; none when terms is
+// NULL), meta[2] = epoch when a bar at or after first_valid is not finite and
+// meta[3] = epoch when one is odd, so the batch reads its flags as meta ==
+// epoch and the words need no clearing (each call brings a new epoch); and,
+// with warms, vta_check_warms' check of the reference's warm indices against
+// first_valid + period - 1 (a mismatch stores 1 in *err).  Grid: enough threads
+// for the bars checked or formed from bar `from` on, and for n.
+extern "C" __global__ __launch_bounds__(256) void scan_prepare(
+    const float *__restrict__ x, const float *__restrict__ h, const float *__restrict__ l, int T,
+    int first_valid, int kind, int nterms, int from, int t0, int t1, int tstride,
+    double *__restrict__ terms, int epoch, int32_t *__restrict__ meta,
+    const int32_t *__restrict__ periods, const int32_t *__restrict__ warms, int n,
+    int32_t *__restrict__ err) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const long t = (long)from + i;
+    double f[3];
+    const scan_bar r = scan_bar_terms(x, h, l, T, first_valid, kind, t, f);
+    if (terms && t >= t0 && t < t1)
+        for (int q = 0; q < nterms; ++q) terms[scan_term_at(nterms, q, tstride, t - t0)] = f[q];
+    if (r.bad) meta[2] = epoch;
+    if (r.odd) meta[3] = epoch;
+    if (warms && i < n && (long long)warms[i] != (long long)first_valid + periods[i] - 1)
+        err[0] = 1;
+}
+
+// The same for every job of a pack: grid (blocks, jobs).
+extern "C" __global__ __launch_bounds__(256) void packed_prepare(const rec_job *jobs,
+                                                                 int32_t *flags, int kind,
+                                                                 int nterms, int epoch) {
+    const rec_job &jb = jobs[blockIdx.y];
+    const int end = jb.nch > 1 ? jb.tstride : jb.T;  // a one-chunk job has no terms
+    bool bad = false, odd = false;
+    for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < end; t += (long)gridDim.x * 256) {
+        double f[3];
+        const scan_bar r = scan_bar_terms(jb.x, jb.h, jb.l, jb.T, jb.fv, kind, t, f);
+        if (jb.nch > 1)
+            for (int q = 0; q < nterms; ++q)
+                jb.terms[scan_term_at(nterms, q, jb.tstride, t)] = f[q];
+        bad = bad || r.bad;
+        odd = odd || r.odd;
+    }
+    if (bad) flags[2 * blockIdx.y] = epoch;
+    if (odd) flags[2 * blockIdx.y + 1] = epoch;
+}
+
+// True range of one series (tr_from_hlc_f32 in the reference): 0 before
+// first_valid, high - low at first_valid, then max(h - l, |h - c[t-1]|,
+// |l - c[t-1]|), evaluated in f64 (exact for f32 inputs) and rounded once.
 extern "C" __global__ __launch_bounds__(256) void tr_from_hlc_f32(
     const float *__restrict__ h, const float *__restrict__ l, const float *__restrict__ c, int T,
     int first_valid, float *__restrict__ tr) {
@@ -1692,71 +1938,6 @@ extern "C" __global__ __launch_bounds__(256) void tr_from_hlc_f32(
     if (t == first_valid) v = (float)((double)h[t] - (double)l[t]);
     else if (t > first_valid) v = (float)true_range(h[t], l[t], c[t - 1]);
     tr[t] = v;
-}
-
-extern "C" __global__ __launch_bounds__(64) void ema_scan_combine(rec_args a) {
-    scan_combine<EmaEng>(view_of(a));
-}
-extern "C" __global__ __launch_bounds__(64) void rsi_scan_combine(rec_args a) {
-    scan_combine<RsiEng>(view_of(a));
-}
-extern "C" __global__ __launch_bounds__(64) void atr_scan_combine(rec_args a) {
-    scan_combine<AtrEng>(view_of(a));
-}
-extern "C" __global__ __launch_bounds__(64) void smma_scan_combine(rec_args a) {
-    scan_combine<SmmaEng>(view_of(a));
-}
-extern "C" __global__ __launch_bounds__(64) void wilders_scan_combine(rec_args a) {
-    scan_combine<WildersEng>(view_of(a));
-}
-
-// Per-combo Wilders seed of a one-series batch (wave = combo): the value the
-// lane reaches at bar fv + p - 1 by replaying its warm-up (seed_bar): groups
-// of four bars g = ((x0 + x1) + x2) + x3, each group's own bars added in
-// order, summed from 0.0 one group after another, times the smoothing
-// factor.  Lanes form 64 groups (256 bars) at a time from one coalesced
-// read; the wave then adds them in group order (each read out of its lane),
-// so the sum is the same sequence of f64 operations as the replay.  Combos
-// whose warm-up passes the series end get no seed (their lanes have no
-// output).
-extern "C" __global__ __launch_bounds__(256) void wilders_seed(rec_args a) {
-    const int lane = threadIdx.x & 63;
-    const int c = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (c >= a.nlanes) return;
-    const int fv = a.fvs[0];
-    WildersEng e;
-    e.setup(__builtin_amdgcn_readfirstlane(a.periods[c]), fv);
-    apply_alpha(e, a.alphas, c);
-    const int p = e.p;
-    if (p < 1 || (long)fv + p - 1 >= a.T) return;
-    const float *x = a.x + fv;
-    auto group = [&](int b) {
-        const int k0 = b + 4 * lane;
-        double g = 0.0;
-        if (k0 < p) {
-            g = (double)x[k0];
-            if (k0 + 1 < p) g += (double)x[k0 + 1];
-            if (k0 + 2 < p) g += (double)x[k0 + 2];
-            if (k0 + 3 < p) g += (double)x[k0 + 3];
-        }
-        return g;
-    };
-    double sum = 0.0;
-    double g = group(0);
-    for (int b = 0; b < p; b += 256) {
-        const double gn = b + 256 < p ? group(b + 256) : 0.0;   // next 256 bars in flight
-        const int ng = min(64, (p - b + 3) >> 2);
-        const unsigned long long gb = __builtin_bit_cast(unsigned long long, g);
-        const int lo = (int)(unsigned)gb, hi = (int)(unsigned)(gb >> 32);
-        for (int j = 0; j < ng; ++j) {
-            const unsigned long long v =
-                ((unsigned long long)(unsigned)__builtin_amdgcn_readlane(hi, j) << 32) |
-                (unsigned)__builtin_amdgcn_readlane(lo, j);
-            sum += __builtin_bit_cast(double, v);
-        }
-        g = gn;
-    }
-    if (lane == 0) a.seeds[c] = sum * e.al;
 }
 
 // ---------------------------------------------------------------- preparation
@@ -1834,50 +2015,6 @@ extern "C" __global__ __launch_bounds__(64) void ms_first_nonfinite_from_first_v
     const float *__restrict__ x, int T, int N, const int32_t *__restrict__ fvs,
     int32_t *__restrict__ z) {
     ms_scan_from_fv(x, T, N, fvs, z, true);
-}
-
-// Single series: clean flag = no non-finite input in [first_valid, T).
-// The one launch before a device-resident one-series batch: meta[0] =
-// first_valid (the batch kernels' fvs[0]); meta[2] = epoch when a bar of x
-// (and h, l) at or after first_valid is not finite, so the batch reads its
-// clean flag as meta[2] != epoch and the word needs no clearing (each call
-// brings a new epoch); and, with warms, vta_check_warms' check of the
-// reference's warm indices against first_valid + period - 1 (a mismatch
-// stores 1 in *err).  Grid: enough threads for max(T - first_valid, n).
-extern "C" __global__ __launch_bounds__(256) void batch_prepare(
-    const float *__restrict__ x, const float *__restrict__ h, const float *__restrict__ l,
-    int T, int first_valid, int epoch, int32_t *__restrict__ meta,
-    const int32_t *__restrict__ periods, const int32_t *__restrict__ warms, int n,
-    int32_t *__restrict__ err) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i == 0) meta[0] = first_valid;
-    const int t = i + first_valid;
-    if (t < T) {
-        bool bad = !vta_isfinite(x[t]);
-        if (h) bad = bad || !vta_isfinite(h[t]);
-        if (l) bad = bad || !vta_isfinite(l[t]);
-        if (bad) meta[2] = epoch;
-    }
-    if (warms && i < n && (long long)warms[i] != (long long)first_valid + periods[i] - 1)
-        err[0] = 1;
-}
-
-// flag[0] must be 0 on entry (see vta_fill_i32); every failing lane stores 1.
-extern "C" __global__ __launch_bounds__(256) void series_nonfinite_flag(
-    const float *__restrict__ x, const float *__restrict__ h, const float *__restrict__ l,
-    int T, int first_valid, int32_t *__restrict__ flag) {
-    const int t = blockIdx.x * 256 + threadIdx.x + first_valid;
-    if (t >= T) return;
-    bool bad = !vta_isfinite(x[t]);
-    if (h) bad = bad || !vta_isfinite(h[t]);
-    if (l) bad = bad || !vta_isfinite(l[t]);
-    if (bad) flag[0] = 1;
-}
-
-// clean[0] = (flag[0] == 0): turns the non-finite flag into the engines' clean word.
-extern "C" __global__ __launch_bounds__(64) void flag_to_clean(const int32_t *__restrict__ flag,
-                                                               int32_t *__restrict__ clean) {
-    if (threadIdx.x == 0) clean[0] = flag[0] == 0 ? 1 : 0;
 }
 
 // The reference's device forms of SMMA, SWMA and Wilders take per-combo warm

@@ -3,6 +3,7 @@
 // CudaAtr (src/cuda/atr_wrapper.rs), CudaAdx (src/cuda/adx_wrapper.rs), plus the
 // fused EMA + RSI + ATR many-series launch.  Kernels: kernels/rec.hip.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -28,16 +29,23 @@ struct rec_args_host {
     float *out1;
     float *out2;
     double *carry;
+    const double *terms;
+    const double *state_in;
+    double *state_out;
     const float *alphas;
-    double *seeds;
     int T;
     int nlanes;
     int chunk;
     int p1, p2, p3;
-    int phase;
+    int fv;
+    int nch, groups;
+    int span;
+    int t0, t1;
+    int tstride;
+    int scan;
     int clean_epoch;
 };
-static_assert(sizeof(rec_args_host) == 136, "rec_args layout");
+static_assert(sizeof(rec_args_host) == 184, "rec_args layout");
 
 enum Ind {
     IND_EMA = 0,
@@ -159,20 +167,32 @@ bool host_clean(const float *x, const float *h, const float *l, size_t n, size_t
     return true;
 }
 
-// Output staging of the one-series batch kernels, needed by the passes that
-// write rows (phase 0 and 3): 64 rows x (W + 1) floats of dynamic LDS, W the
-// bars staged between flushes (32 for RSI and ADX, whose longer steps gain
-// from the extra resident waves; 64 for the others; kStageW in kernels/rec.hip).
-unsigned batch_stage_bytes(Ind k) {
-    const unsigned w = (k == IND_RSI || k == IND_ADX) ? 32u : 64u;
-    return 64u * (w + 1u) * (unsigned)sizeof(float);
+// Blocks of the one-series kernels: kWpb waves (REC_WPB), one chunk of as many
+// groups of 64 combos, or consecutive chunks of one group (block_chunk).
+constexpr unsigned kWpb = 4;
+size_t batch_blocks(size_t groups, size_t nch) {
+    return groups < kWpb ? groups * ((nch + kWpb - 1) / kWpb) : (groups + kWpb - 1) / kWpb * nch;
 }
 
-// Wilders seeds: doubles from byte 32,768 of the context scratch, one per
-// combo, for batches of up to 4,096 combos (larger ones replay the warm-ups).
-constexpr size_t kSeedOffset = 32 * 1024;
-constexpr size_t kSeedCombos = (vta_ctx::kScratchBytes - kSeedOffset) / sizeof(double);
-static_assert(kSeedOffset >= (kArgErrorWord + 1) * sizeof(int32_t), "seeds after the error word");
+// Chunks per span of the scan (a whole number of blocks), 0 for none.  A
+// wave folds the chunks before its own, four waves of a block sharing it when
+// they take one group's (groups < kWpb): one level up to 256 chunks there and
+// kSpan elsewhere; beyond that the span maps first (7 us for 782 chunks of
+// 1,250 combos) and a wave folds the spans and its own span's chunks.
+constexpr size_t kSpan = 32;
+size_t scan_span(size_t groups, size_t nch) {
+    return nch > (groups < kWpb ? 256u : kSpan) ? kSpan : 0;
+}
+
+// Dynamic LDS of the one-series output kernels, per wave 64 rows x 36 floats
+// of the scan, or (in the same bytes) drive_batch's bars or shared per-bar
+// terms and 64 x 33 floats (wave_lds).
+unsigned batch_lds_bytes(Ind k) {
+    const unsigned bars = k == IND_ADX ? 3u * 512u : 3u * 256u;
+    return kWpb * std::max(64u * 36u * 4u, bars + 64u * 33u * 4u);
+}
+// ADX's second stage folds (64 x 4 doubles per wave) without staging rows.
+constexpr unsigned kFoldLds = kWpb * 64 * 4 * sizeof(double);
 
 vta_status launch_rec(vta_ctx *ctx, const char *kname, rec_args_host &a, unsigned groups,
                       unsigned chunks, unsigned block = 64, unsigned smem = 0) {
@@ -181,87 +201,146 @@ vta_status launch_rec(vta_ctx *ctx, const char *kname, rec_args_host &a, unsigne
     return launch(ctx, f, dim3(groups, chunks, 1), dim3(block), smem, a);
 }
 
-// Chunked-scan launch: chunks sized for ~kScanWaves waves, at least 64 bars
-// and at most 1,024 chunks (the fold walks them 64 at a time; a Wilders lane
-// whose warm-up spans several chunks starts from its seed at the last
-// warm-up bar, or, past kSeedCombos, replays the warm-up exactly from
-// first_valid in each), and as many as the
-// context's carry buffer holds for C
-// combos; pass 1, the per-combo fold (one wave per combo; two rounds for
-// ADX), pass 3.  Small requests are latency-bound, so their chunk is short:
-// 16 one-series requests of 10,000 bars x 32 periods (EMA, RSI, ADX, SMA,
-// BB) took 2.69 / 1.96 / 1.34 ms with 256- / 128- / 64-bar chunks.  Sets
-// *done = false (nothing launched) when one chunk would cover the series.
-// Measured on 1,250 periods x 200k bars: EMA 0.395 / 0.365 / 0.336 ms and ADX
-// 1.14 / 1.24 / 1.09 ms at 2,048 / 4,096 / 8,192 waves (an earlier build);
-// later EMA 0.298 / 0.285 and RSI 0.442 / 0.398 ms at 8,192 / 16,384 waves
-// (256-bar chunks, the 1,024-chunk cap); flat on small shapes, whose chunks
-// sit at the 64-bar floor either way.
-constexpr size_t kScanWaves = 16384;
+// Chunk length of the scan, by the bars of all 64-combo groups together: a
+// wave's chunk is a serial chain, so a short call takes 64 bars, the shortest;
+// a long one has waves to spare and folds and restarts fewer, longer chunks.
+// Whole calls in us at 64 / 128 / 256 / 384 bars per chunk:
+//   33 RSI x 10,007 bars       18.4 / 22.1 / 30.9 / 40.7
+//   300 RSI x 10,007           28.6 / 32.9 / 46.5 / 51.4
+//   60 ADX x 50,000            50.0 / 60.6 / 72.2 / 90.1
+//   640 ADX x 50,000            137 /  119 /  119 /  159
+//   640 EMA x 50,000           54.0 / 52.1 / 59.2 / 75.5
+//   700 EMA x 180,001           284 /  268 /  275 /  285
+//   1,250 EMA x 200,000         375 /  249 /  239 /  246
+//   1,250 ADX x 200,000         580 /  580 /  447 /  446
+// So 128 bars from kWaves128 such chunks on, 256 from kWaves256 on; at most
+// 4,096 chunks, and as many as the context's carry buffer holds.
+constexpr size_t kWaves128 = 2048, kWaves256 = 8192;
 
 size_t scan_states(Ind k) { return k == IND_RSI ? 2 : k == IND_ADX ? 4 : 1; }
+size_t scan_terms(Ind k) { return k == IND_RSI ? 2 : k == IND_ADX ? 3 : 1; }
+int scan_kind(Ind k) { return k == IND_RSI ? 1 : k == IND_ATR ? 2 : k == IND_ADX ? 3 : 0; }
 
-const char *combine_kernel(Ind k) {
-    static const char *n[] = {"ema_scan_combine",  "rsi_scan_combine",     "atr_scan_combine",
-                              "adx_scan_combine",  "smma_scan_combine",    "wilders_scan_combine",
-                              "atr_tr_scan_combine"};
+const char *states_kernel(Ind k) {
+    static const char *n[] = {"ema_scan_states",  "rsi_scan_states",  "atr_scan_states",
+                              "adx_scan_states",  "smma_scan_states", "wilders_scan_states",
+                              "atr_tr_scan_states"};
     return n[k];
+}
+const char *spans_kernel(Ind k) {
+    static const char *n[] = {"ema_scan_spans",  "rsi_scan_spans",  "atr_scan_spans",
+                              "adx_scan_spans",  "smma_scan_spans", "wilders_scan_spans",
+                              "atr_tr_scan_spans"};
+    return n[k];
+}
+
+// Bars of one segment of a T-bar scan: all of them, or what the term buffer
+// holds (whole 64-bar blocks).
+size_t scan_segment(Ind k, size_t T) {
+    const size_t fit = vta_ctx::kTermBytes / (scan_terms(k) * sizeof(double)) & ~(size_t)63;
+    return std::min(T, fit);
 }
 
 // The chunked scan's chunk length for T bars x C combos of indicator k (the
 // rule above), or 0 when the series is not scanned (one chunk would cover
 // it, or the carry buffer holds fewer than two chunk-end states per combo).
-size_t scan_chunk(const vta_ctx *ctx, Ind k, size_t T, size_t C, size_t max_p) {
+size_t scan_chunk(const vta_ctx *ctx, Ind k, size_t T, size_t C) {
     if (getenv("VTA_REC_NO_SCAN")) return 0;
     // states per (chunk, combo): RSI 2; ADX 4 (three first-stage states and
     // the ADX itself, folded in two rounds); the others 1
     const size_t S = scan_states(k);
     const size_t groups = (C + 63) / 64;
-    size_t waves = kScanWaves;
+    const bool whole = scan_segment(k, T) == T;
+    T = scan_segment(k, T);
+    size_t waves = 0;
     if (ctx->tune[VTA_TUNE_SCAN_WAVES] > 0) {
         waves = (size_t)ctx->tune[VTA_TUNE_SCAN_WAVES];
     } else if (const char *e = getenv("VTA_SCAN_WAVES")) {
         long v = atol(e);
         if (v >= 64) waves = (size_t)v;
     }
-    const size_t want = std::max<size_t>(1, waves / groups);
-    size_t chunk = std::max<size_t>({64, (T + want - 1) / want, (T + 1023) / 1024});
+    size_t chunk = std::max<size_t>(64, (T + 4095) / 4096);
+    if (waves)
+        chunk = std::max(chunk, T / std::max<size_t>(1, waves / groups));
+    else
+        chunk = std::max({chunk, std::min<size_t>(128, T * groups / kWaves128),
+                          std::min<size_t>(256, T * groups / kWaves256)});
     if (const char *e = getenv("VTA_SCAN_CHUNK")) {
         long v = atol(e);
         if (v >= 64) chunk = (size_t)v;
     }
-    const size_t max_chunks = vta_ctx::kCarryBytes / (C * S * sizeof(double));
+    // (a row of states per chunk and per span; two more are handed from
+    // segment to segment)
+    size_t max_chunks = vta_ctx::kCarryBytes / (groups * 64 * S * sizeof(double));
+    if (!whole) max_chunks -= std::min<size_t>(max_chunks, 2);
+    max_chunks = max_chunks * kSpan / (kSpan + 1);
     if (max_chunks < 2) return 0;
     if ((T + chunk - 1) / chunk > max_chunks) chunk = (T + max_chunks - 1) / max_chunks;
     chunk = (chunk + 63) & ~(size_t)63;
     return (T + chunk - 1) / chunk < 2 ? 0 : chunk;
 }
 
-vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t T, size_t C, size_t max_p,
-                       bool *done) {
-    *done = false;
-    const size_t chunk = scan_chunk(ctx, k, T, C, max_p);
-    if (chunk == 0) return VTA_OK;
-    const size_t groups = (C + 63) / 64;
-    const size_t nch = (T + chunk - 1) / chunk;
-    a.chunk = (int)chunk;
-    a.carry = static_cast<double *>(ctx->carry);
-    hipFunction_t fb, fc;
+// The flags and terms launch before a batch (kernels/rec.hip, scan_prepare):
+// terms of bars [t0, t1), all bars checked with the first segment.
+vta_status prepare_launch(vta_ctx *ctx, Ind k, const rec_args_host &a, size_t t0, size_t t1,
+                          bool terms, const int32_t *d_warms) {
+    hipFunction_t prep;
+    VTA_TRY(get_function(ctx, "rec", "scan_prepare", &prep));
+    int32_t *meta = static_cast<int32_t *>(ctx->scratch);
+    const size_t from = t0;
+    size_t end = terms ? t1 : 0;
+    if (t0 == 0) end = std::max({end, (size_t)a.T, d_warms ? (size_t)a.nlanes : 0});
+    return launch(ctx, prep, dim3((unsigned)((end - from + 255) / 256)), dim3(256), 0, a.x, a.h,
+                  a.l, a.T, a.fv, scan_kind(k), (int)scan_terms(k), (int)from, (int)t0, (int)t1,
+                  a.tstride, terms ? ctx->terms : static_cast<double *>(nullptr), a.clean_epoch,
+                  meta, a.periods, d_warms, a.nlanes, meta + kArgErrorWord);
+}
+
+// `a` holds the inputs, outputs, flags and sizes; chunk from scan_chunk.
+vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
+                       const int32_t *d_warms) {
+    const size_t T = (size_t)a.T, seg = scan_segment(k, T), S = scan_states(k);
+    hipFunction_t fs, ff, fb, f2 = nullptr;
+    VTA_TRY(get_function(ctx, "rec", states_kernel(k), &fs));
+    VTA_TRY(get_function(ctx, "rec", spans_kernel(k), &ff));
     VTA_TRY(get_function(ctx, "rec", batch_kernel(k), &fb));
-    VTA_TRY(get_function(ctx, "rec", combine_kernel(k), &fc));
-    a.phase = 1;
-    VTA_TRY(launch(ctx, fb, dim3((unsigned)groups, (unsigned)nch, 1), dim3(64), 0, a));
-    VTA_TRY(launch(ctx, fc, dim3((unsigned)C), dim3(64), 0, a));
-    if (k == IND_ADX) {
-        // second stage: DX from the exact first-stage states, ADX from zero
-        a.phase = 2;
-        VTA_TRY(launch(ctx, fb, dim3((unsigned)groups, (unsigned)nch, 1), dim3(64), 0, a));
-        VTA_TRY(launch(ctx, fc, dim3((unsigned)C), dim3(64), 0, a));
+    if (k == IND_ADX) VTA_TRY(get_function(ctx, "rec", "adx_scan_stage2", &f2));
+    const size_t row = S * a.groups * 64;
+    double *handed[2] = {static_cast<double *>(ctx->carry), nullptr};
+    handed[1] = handed[0] + row;
+    a.carry = seg < T ? handed[1] + row : handed[0];
+    a.terms = ctx->terms;
+    a.chunk = (int)chunk;
+    for (size_t t0 = 0, n = 0; t0 < T; t0 += seg, ++n) {
+        const size_t t1 = std::min(T, t0 + seg);
+        const size_t nch = (t1 - t0 + chunk - 1) / chunk;
+        a.t0 = (int)t0;
+        a.t1 = (int)t1;
+        a.nch = (int)nch;
+        const size_t bars = (t1 - t0 + 63) & ~(size_t)63;
+        a.tstride = (int)bars;
+        a.state_in = n > 0 ? handed[(n - 1) & 1] : nullptr;
+        a.state_out = t1 < T ? handed[n & 1] : nullptr;
+        VTA_TRY(prepare_launch(ctx, k, a, t0, std::min(t0 + bars, (size_t)INT32_MAX), true,
+                               n == 0 ? d_warms : nullptr));
+        const dim3 grid((unsigned)batch_blocks(a.groups, nch)), block(64 * kWpb);
+        a.span = (int)scan_span(a.groups, nch);
+        const unsigned spans = a.span ? (unsigned)((nch - 1) / a.span * a.groups) : 0;
+        if (nch > 1) {
+            a.scan = 1;
+            VTA_TRY(launch(ctx, fs, grid, block, 0, a));
+            if (spans)
+                VTA_TRY(launch(ctx, ff, dim3(spans, (unsigned)scan_terms(k)), dim3(64), 0, a));
+            if (k == IND_ADX) {
+                // second stage: DX from the exact first-stage states, its sums from zero
+                VTA_TRY(launch(ctx, f2, grid, block, kFoldLds, a));
+                a.scan = 2;
+                if (spans) VTA_TRY(launch(ctx, ff, dim3(spans), dim3(64), 0, a));
+            }
+        }
+        a.scan = 1;
+        VTA_TRY(launch(ctx, fb, grid, block, batch_lds_bytes(k), a));
     }
-    a.phase = 3;
-    VTA_TRY(launch(ctx, fb, dim3((unsigned)groups, (unsigned)nch, 1), dim3(64),
-                   batch_stage_bytes(k), a));
-    *done = true;
     return VTA_OK;
 }
 
@@ -284,54 +363,56 @@ void record_batch(vta_ctx *ctx, Ind k, bool chunked) {
     if (s >= 0) ctx->sel_batch[s] = {chunked ? VTA_SELECTED_CHUNKED : VTA_SELECTED_PLAIN, 64};
 }
 
-// One series x many periods, device input and output, fv and clean known.
-// max_p = 0: the longest period is not known on the host (the reference's
-// device forms pass none), so no burn-in is planned from it: the series runs
-// as a chunked scan (Wilders chunks then are not stretched to the longest
-// warm-up), or else exactly from first_valid in one chunk.  d_alphas
-// (per combo, may be NULL) overrides the EMA / Wilders smoothing factor.
+// One series x many periods, device input and output.  `clean`: false when
+// the host has met a non-finite bar after first_valid (the series then runs
+// exactly from there, as it does when scan_prepare meets one).  max_p = 0: the
+// longest period is not known on the host (the reference's device forms pass
+// none), so no burn-in is planned from it: the series runs as a chunked scan,
+// or else exactly from first_valid in one chunk.  d_alphas (per combo, may
+// be NULL) overrides the EMA / Wilders smoothing factor; d_warms (may be NULL)
+// are checked against first_valid + period - 1.
 vta_status batch_launch(vta_ctx *ctx, Ind k, const float *d_x, const float *d_h,
                         const float *d_l, const int32_t *d_periods, size_t max_p, size_t T,
-                        size_t C, const int32_t *d_fv1, const int32_t *d_clean1, bool clean,
-                        float *d_out, const float *d_alphas = nullptr, int clean_epoch = 0) {
+                        size_t C, size_t fv, bool clean, float *d_out,
+                        const float *d_alphas = nullptr, const int32_t *d_warms = nullptr) {
     rec_args_host a{};
     a.x = d_x;
     a.h = d_h;
     a.l = d_l;
     a.periods = d_periods;
-    a.fvs = d_fv1;
-    a.clean = d_clean1;
-    a.clean_epoch = clean_epoch;
     a.out0 = d_out;
     a.alphas = d_alphas;
     a.T = (int)T;
     a.nlanes = (int)C;
+    a.fv = (int)fv;
+    a.groups = (int)((C + 63) / 64);
     const bool plain = plain_batch(ctx, k);
-    if (k == IND_WILDERS && C <= kSeedCombos) {
-        // per-combo seeds (the second half of the context scratch): an exact
-        // lane then starts at its last warm-up bar instead of replaying the
-        // warm-up from first_valid in every chunk the warm-up spans
-        a.seeds = reinterpret_cast<double *>(static_cast<char *>(ctx->scratch) + kSeedOffset);
-        VTA_TRY(launch_rec(ctx, "wilders_seed", a, (unsigned)((C + 3) / 4), 1, 256));
+    const size_t chunk = clean && !plain ? scan_chunk(ctx, k, T, C) : 0;
+    if (clean) {
+        // context scratch words [2] and [3]: the flags of this call, which
+        // hold its epoch where a bar is not finite (odd); an epoch repeated
+        // after 2^31 calls can only read a clean series as unclean, which
+        // runs exactly (and correctly) from first_valid
+        if (++ctx->prep_epoch > INT32_MAX || ctx->prep_epoch == 0) ctx->prep_epoch = 1;
+        a.clean_epoch = (int)ctx->prep_epoch;
+        a.clean = static_cast<int32_t *>(ctx->scratch) + 2;
+        if (d_warms) ctx->arg_check_pending = true;
     }
-    // (a Wilders warm-up longer than a chunk without seeds is still exact:
-    // its lanes replay it from first_valid, see test_scan_short_chunks_long_lead)
-    if (clean && !plain) {
-        bool done;
-        VTA_TRY(scan_launch(ctx, k, a, T, C, max_p, &done));
-        if (done) {
-            record_batch(ctx, k, true);
-            return VTA_OK;
-        }
+    if (chunk) {
+        record_batch(ctx, k, true);
+        return scan_launch(ctx, k, a, chunk, d_warms);
     }
-    unsigned groups = (unsigned)((C + 63) / 64);
+    if (clean) VTA_TRY(prepare_launch(ctx, k, a, 0, 0, false, d_warms));
     // a caller-supplied smoothing factor is not the one the burn-in length
     // would be planned from, so those batches also run in one chunk
-    a.chunk = (plain || max_p == 0 || d_alphas) ? (int)T
-                                                : pick_chunk_batch(k, max_p, T, groups, clean);
-    unsigned chunks = (unsigned)((T + a.chunk - 1) / a.chunk);
-    record_batch(ctx, k, chunks > 1);
-    return launch_rec(ctx, batch_kernel(k), a, groups, chunks, 64, batch_stage_bytes(k));
+    a.chunk = (plain || max_p == 0 || d_alphas)
+                  ? (int)T
+                  : pick_chunk_batch(k, max_p, T, (size_t)a.groups, clean);
+    a.nch = (int)((T + a.chunk - 1) / a.chunk);
+    a.t1 = (int)T;
+    record_batch(ctx, k, a.nch > 1);
+    return launch_rec(ctx, batch_kernel(k), a, (unsigned)batch_blocks(a.groups, a.nch), 1, 64 * kWpb,
+                      batch_lds_bytes(k));
 }
 
 vta_status batch_dev(vta_ctx *ctx, Ind k, const float *x, const float *h, const float *l,
@@ -363,19 +444,16 @@ vta_status batch_dev(vta_ctx *ctx, Ind k, const float *x, const float *h, const 
     size_t nin = hlc(k) ? 3 : 1;
     VTA_TRY(check_fits(n_out + nin * len * sizeof(float)));
     std::vector<int32_t> per(ps.begin(), ps.end());
-    int32_t meta[2] = {(int32_t)fv, clean ? 1 : 0};
-    DevBuf dx, dh, dl, dp, dm, dout;
+    DevBuf dx, dh, dl, dp, dout;
     VTA_TRY(upload(ctx, dx, x, len * sizeof(float)));
     if (nin == 3) {
         VTA_TRY(upload(ctx, dh, h, len * sizeof(float)));
         VTA_TRY(upload(ctx, dl, l, len * sizeof(float)));
     }
     VTA_TRY(upload(ctx, dp, per.data(), per.size() * sizeof(int32_t)));
-    VTA_TRY(upload(ctx, dm, meta, sizeof(meta)));
     VTA_TRY(dout.alloc(n_out));
     VTA_TRY(batch_launch(ctx, k, dx.as<float>(), dh.as<float>(), dl.as<float>(),
-                         dp.as<int32_t>(), max_p, len, C, dm.as<int32_t>(),
-                         dm.as<int32_t>() + 1, clean, dout.as<float>()));
+                         dp.as<int32_t>(), max_p, len, C, fv, clean, dout.as<float>()));
     VTA_HIP(hipStreamSynchronize(ctx->stream));
     out->ptr = static_cast<float *>(dout.release());
     out->rows = C;
@@ -402,27 +480,11 @@ vta_status batch_device(vta_ctx *ctx, Ind k, const float *d_x, const float *d_h,
                                            "and first_valid < series_len");
     if (series_len > INT32_MAX || n_combos > INT32_MAX || max_period > series_len)
         return fail(VTA_ERR_INVALID_INPUT, "series_len, n_combos or max_period out of range");
-    // context scratch: [0] first_valid, [2] the non-finite word; one launch
-    // (batch_prepare) stores both and checks the warm indices.  The word
-    // holds this call's epoch if a bar is not finite, so it is never
-    // cleared; an epoch repeated after 2^31 calls can only read a clean
-    // series as unclean, which runs exactly (and correctly) from first_valid.
-    int32_t *meta = static_cast<int32_t *>(ctx->scratch);
-    if (++ctx->prep_epoch > INT32_MAX || ctx->prep_epoch == 0) ctx->prep_epoch = 1;
-    const int epoch = (int)ctx->prep_epoch;
-    hipFunction_t prep;
-    VTA_TRY(get_function(ctx, "rec", "batch_prepare", &prep));
-    int32_t *err = static_cast<int32_t *>(ctx->scratch) + kArgErrorWord;
-    if (d_warms) ctx->arg_check_pending = true;
-    const int64_t span = std::max<int64_t>(series_len - first_valid, d_warms ? n_combos : 0);
-    VTA_TRY(launch(ctx, prep, dim3((unsigned)((span + 255) / 256)), dim3(256), 0, d_x,
-                   hlc(k) ? d_h : nullptr, hlc(k) ? d_l : nullptr, (int)series_len,
-                   (int)first_valid, epoch, meta, d_periods, d_warms, (int)n_combos, err));
-    // Chunked with burn-in: a series found unclean still runs correctly, since
-    // every lane of an unclean stream starts exactly at first_valid.
-    return batch_launch(ctx, k, d_x, d_h, d_l, d_periods, (size_t)max_period,
-                        (size_t)series_len, (size_t)n_combos, meta, meta + 2, true, d_out,
-                        d_alphas, epoch);
+    // (scan_prepare finds whether every bar is finite: a series found unclean
+    // runs exactly from first_valid)
+    return batch_launch(ctx, k, d_x, hlc(k) ? d_h : nullptr, hlc(k) ? d_l : nullptr, d_periods,
+                        (size_t)max_period, (size_t)series_len, (size_t)n_combos,
+                        (size_t)first_valid, true, d_out, d_alphas, d_warms);
 }
 
 vta_status ms_launch(vta_ctx *ctx, Ind k, const float *d_x, const float *d_h, const float *d_l,
@@ -1007,7 +1069,7 @@ vta_status vta_ema_rsi_atr_many_series_dev(vta_ctx *ctx, const float *close_tm,
 
 // ---------------------------------------------------------------- packed batches
 
-static_assert(sizeof(PackJob) == 80, "rec_job layout");
+static_assert(sizeof(PackJob) == 96, "rec_job layout");
 
 namespace {
 
@@ -1015,16 +1077,21 @@ struct rec_pack_args_host {
     const void *jobs;
     const int32_t *flags;
     int n_jobs;
-    int phase;
+    int scan;
+    int epoch;
+    int pad_;
 };
-static_assert(sizeof(rec_pack_args_host) == 24, "rec_pack_args layout");
+static_assert(sizeof(rec_pack_args_host) == 32, "rec_pack_args layout");
 
-const char *packed_kernel(Ind k, bool fold) {
-    static const char *p[] = {"ema_packed_f32", "rsi_packed_f32", "atr_packed_f32",
-                              "adx_packed_f32", "smma_packed_f32", "wilders_packed_f32"};
-    static const char *f[] = {"ema_packed_fold", "rsi_packed_fold", "atr_packed_fold",
-                              "adx_packed_fold", "smma_packed_fold", "wilders_packed_fold"};
-    return fold ? f[k] : p[k];
+const char *packed_kernel(Ind k, int pass) {   // 0 states, 1 spans, 2 output
+    static const char *n[][3] = {
+        {"ema_packed_states", "ema_packed_spans", "ema_packed_f32"},
+        {"rsi_packed_states", "rsi_packed_spans", "rsi_packed_f32"},
+        {"atr_packed_states", "atr_packed_spans", "atr_packed_f32"},
+        {"adx_packed_states", "adx_packed_spans", "adx_packed_f32"},
+        {"smma_packed_states", "smma_packed_spans", "smma_packed_f32"},
+        {"wilders_packed_states", "wilders_packed_spans", "wilders_packed_f32"}};
+    return n[k][pass];
 }
 
 }  // namespace
@@ -1032,9 +1099,8 @@ const char *packed_kernel(Ind k, bool fold) {
 namespace vta {
 
 vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, size_t n_jobs,
-                       std::vector<PackJob> &tab, std::vector<size_t> &carry_off,
-                       size_t *carry_elems, PackDims *dims) {
-    if (!ctx || !jobs || !dims || !carry_elems)
+                       std::vector<PackJob> &tab, size_t *work_elems, PackDims *dims) {
+    if (!ctx || !jobs || !dims || !work_elems)
         return fail(VTA_ERR_INVALID_INPUT, "null argument");
     if (kind < (int)VTA_REC_EMA || kind > (int)VTA_REC_WILDERS)
         return fail(VTA_ERR_INVALID_INPUT, "unknown indicator kind %d", kind);
@@ -1043,8 +1109,7 @@ vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, si
     const Ind k = (Ind)kind;
     const size_t S = scan_states(k);
     tab.assign(n_jobs, PackJob{});
-    carry_off.assign(n_jobs, 0);
-    size_t blocks = 0, combos = 0, elems = 0, span = 1;
+    size_t blocks = 0, spans = 0, elems = 0, bars = 1;
     for (size_t j = 0; j < n_jobs; ++j) {
         const vta_rec_job &q = jobs[j];
         if (!q.d_close || !q.d_periods || !q.d_out || (hlc(k) && (!q.d_high || !q.d_low)))
@@ -1056,8 +1121,8 @@ vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, si
                         "first_valid < series_len", j);
         const size_t T = (size_t)q.series_len, C = (size_t)q.n_combos;
         // the chunking of the job's own _device call (one exact chunk where
-        // that call would not scan)
-        size_t chunk = scan_chunk(ctx, k, T, C, (size_t)q.max_period);
+        // that call would not scan, or would in segments)
+        size_t chunk = scan_segment(k, T) == T ? scan_chunk(ctx, k, T, C) : 0;
         if (chunk == 0) chunk = T;
         const size_t nch = (T + chunk - 1) / chunk;
         const size_t groups = (C + 63) / 64;
@@ -1074,47 +1139,71 @@ vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, si
         e.chunk = (int)chunk;
         e.nch = (int)nch;
         e.groups = (int)groups;
+        e.terms = nullptr;
+        e.tstride = (int)((T + 63) & ~(size_t)63);
         e.block0 = (int)blocks;
-        e.combo0 = (int)combos;
-        carry_off[j] = elems;
-        blocks += groups * nch;
-        combos += C;
-        elems += C * nch * S;
-        span = std::max(span, T - (size_t)q.first_valid);
-        if (blocks > (size_t)INT32_MAX || combos > (size_t)INT32_MAX)
+        e.span = nch > 1 ? (int)scan_span(groups, nch) : 0;
+        e.span0 = (int)spans;
+        blocks += batch_blocks(groups, nch);
+        const size_t nsp = e.span ? (nch - 1) / e.span : 0;
+        spans += groups * nsp;
+        if (nch > 1) elems += groups * 64 * (nch + nsp) * S + scan_terms(k) * (size_t)e.tstride;
+        bars = std::max(bars, T + 63);
+        if (blocks > (size_t)INT32_MAX || spans > (size_t)INT32_MAX)
             return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "packed grid exceeds 2^31 blocks");
     }
     dims->kind = kind;
     dims->n_jobs = (int)n_jobs;
     dims->total_blocks = (unsigned)blocks;
-    dims->total_combos = (unsigned)combos;
-    dims->flag_blocks = (unsigned)std::min<size_t>((span + 255) / 256, 1024);
-    *carry_elems = elems;
+    dims->total_spans = (unsigned)spans;
+    dims->flag_blocks = (unsigned)std::min<size_t>((bars + 255) / 256, 1024);
+    *work_elems = elems;
     return VTA_OK;
 }
 
-vta_status pack_launch(vta_ctx *ctx, const PackDims &d, const void *d_jobs, int32_t *d_flags) {
+void pack_bind(const PackDims &d, std::vector<PackJob> &tab, double *work) {
     const Ind k = (Ind)d.kind;
-    hipFunction_t fill, flag, fp, ff;
-    VTA_TRY(get_function(ctx, "rec", "vta_fill_i32", &fill));
-    VTA_TRY(get_function(ctx, "rec", "packed_nonfinite_flag", &flag));
-    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, false), &fp));
-    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, true), &ff));
-    VTA_TRY(launch(ctx, fill, dim3((unsigned)((d.n_jobs + 255) / 256)), dim3(256), 0, d_flags,
-                   d.n_jobs, 0));
-    VTA_TRY(launch(ctx, flag, dim3(d.flag_blocks, (unsigned)d.n_jobs), dim3(256), 0, d_jobs,
-                   d_flags, hlc(k) ? 1 : 0));
-    rec_pack_args_host a{d_jobs, d_flags, d.n_jobs, 1};
-    VTA_TRY(launch(ctx, fp, dim3(d.total_blocks), dim3(64), 0, a));
-    VTA_TRY(launch(ctx, ff, dim3(d.total_combos), dim3(64), 0, a));
-    if (k == IND_ADX) {
-        a.phase = 2;
-        VTA_TRY(launch(ctx, fp, dim3(d.total_blocks), dim3(64), 0, a));
-        VTA_TRY(launch(ctx, ff, dim3(d.total_combos), dim3(64), 0, a));
+    for (PackJob &e : tab) {
+        if (e.nch < 2) continue;
+        e.carry = work;
+        const size_t nsp = e.span ? (e.nch - 1) / e.span : 0;
+        work += (size_t)e.groups * 64 * (e.nch + nsp) * scan_states(k);
+        e.terms = work;
+        work += scan_terms(k) * (size_t)e.tstride;
     }
-    a.phase = 3;
-    VTA_TRY(launch(ctx, fp, dim3(d.total_blocks), dim3(64), batch_stage_bytes(k), a));
-    return VTA_OK;
+}
+
+std::vector<unsigned char> pack_image(const std::vector<PackJob> &tab) {
+    std::vector<unsigned char> v(pack_flags_off(tab.size()) + tab.size() * 2 * sizeof(int32_t), 0);
+    if (!tab.empty()) memcpy(v.data(), tab.data(), pack_flags_off(tab.size()));
+    return v;
+}
+
+vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch) {
+    const Ind k = (Ind)d.kind;
+    hipFunction_t prep, fs, ff, fb, f2 = nullptr;
+    VTA_TRY(get_function(ctx, "rec", "packed_prepare", &prep));
+    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 0), &fs));
+    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 1), &ff));
+    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 2), &fb));
+    if (k == IND_ADX) VTA_TRY(get_function(ctx, "rec", "adx_packed_stage2", &f2));
+    int32_t *flags = reinterpret_cast<int32_t *>(static_cast<char *>(d_image) +
+                                                 pack_flags_off((size_t)d.n_jobs));
+    VTA_TRY(launch(ctx, prep, dim3(d.flag_blocks, (unsigned)d.n_jobs), dim3(256), 0,
+                   static_cast<const void *>(d_image), flags, scan_kind(k), (int)scan_terms(k),
+                   epoch));
+    rec_pack_args_host a{d_image, flags, d.n_jobs, 1, epoch, 0};
+    const dim3 block(64 * kWpb);
+    VTA_TRY(launch(ctx, fs, dim3(d.total_blocks), block, 0, a));
+    if (d.total_spans)
+        VTA_TRY(launch(ctx, ff, dim3(d.total_spans, (unsigned)scan_terms(k)), dim3(64), 0, a));
+    if (k == IND_ADX) {
+        VTA_TRY(launch(ctx, f2, dim3(d.total_blocks), block, kFoldLds, a));
+        a.scan = 2;
+        if (d.total_spans) VTA_TRY(launch(ctx, ff, dim3(d.total_spans), dim3(64), 0, a));
+        a.scan = 1;
+    }
+    return launch(ctx, fb, dim3(d.total_blocks), block, batch_lds_bytes(k), a);
 }
 
 }  // namespace vta
@@ -1122,7 +1211,8 @@ vta_status pack_launch(vta_ctx *ctx, const PackDims &d, const void *d_jobs, int3
 struct vta_rec_pack {
     int device = 0;
     PackDims dims{};
-    DevBuf jobs, flags, carry;
+    DevBuf image, work;
+    mutable std::atomic<uint32_t> epoch{0};   // launches so far
 };
 
 extern "C" {
@@ -1133,16 +1223,15 @@ vta_status vta_rec_pack_create(vta_ctx *ctx, vta_rec_kind kind, const vta_rec_jo
     if (!ctx || !jobs || !out) return fail(VTA_ERR_INVALID_INPUT, "null argument");
     *out = nullptr;
     std::vector<PackJob> tab;
-    std::vector<size_t> off;
     size_t elems = 0;
     auto pk = std::make_unique<vta_rec_pack>();
-    VTA_TRY(pack_layout(ctx, (int)kind, jobs, n_jobs, tab, off, &elems, &pk->dims));
+    VTA_TRY(pack_layout(ctx, (int)kind, jobs, n_jobs, tab, &elems, &pk->dims));
     pk->device = ctx->device;
     VTA_HIP(hipSetDevice(ctx->device));
-    VTA_TRY(pk->carry.alloc(std::max<size_t>(elems, 1) * sizeof(double)));
-    VTA_TRY(pk->flags.alloc(n_jobs * sizeof(int32_t)));
-    for (size_t j = 0; j < n_jobs; ++j) tab[j].carry = pk->carry.as<double>() + off[j];
-    VTA_TRY(upload(ctx, pk->jobs, tab.data(), n_jobs * sizeof(PackJob)));
+    VTA_TRY(pk->work.alloc(std::max<size_t>(elems, 1) * sizeof(double)));
+    pack_bind(pk->dims, tab, pk->work.as<double>());
+    const std::vector<unsigned char> image = pack_image(tab);
+    VTA_TRY(upload(ctx, pk->image, image.data(), image.size()));
     *out = pk.release();
     return VTA_OK;
 }
@@ -1153,7 +1242,7 @@ vta_status vta_rec_pack_launch(vta_ctx *ctx, const vta_rec_pack *pk) {
     if (pk->device != ctx->device)
         return fail(VTA_ERR_DEVICE_MISMATCH, "pack built on device %d, context on %d", pk->device,
                     ctx->device);
-    return pack_launch(ctx, pk->dims, pk->jobs.p, pk->flags.as<int32_t>());
+    return pack_launch(ctx, pk->dims, pk->image.p, (int)(pk->epoch++ % INT32_MAX) + 1);
 }
 
 vta_status vta_rec_pack_destroy(vta_rec_pack *pk) {

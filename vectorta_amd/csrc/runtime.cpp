@@ -294,12 +294,13 @@ vta_status vta_ctx_create(int device_id, vta_ctx **out) {
         delete ctx;
         return fail(VTA_ERR_HIP, "clearing the context scratch failed");
     }
-    if (hipMalloc(&ctx->carry, vta_ctx::kCarryBytes) != hipSuccess) {
+    if (hipMalloc(&ctx->carry, vta_ctx::kCarryBytes + vta_ctx::kTermBytes) != hipSuccess) {
         (void)hipFree(ctx->scratch);
         (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return fail(VTA_ERR_OUT_OF_MEMORY, "hipMalloc of the context carry buffer failed");
     }
+    ctx->terms = reinterpret_cast<double *>(static_cast<char *>(ctx->carry) + vta_ctx::kCarryBytes);
     const char *kd = getenv("VTA_KERNEL_DIR");
     ctx->kernel_dir = (kd && *kd) ? std::string(kd) : library_dir();
     noalloc_setup(device_id);   // device address of the allocation-free scratch
@@ -382,14 +383,24 @@ vta_status vta_ctx_preload(vta_ctx *ctx) {
         {"rec", "rsi_ms1p_f32"},
         {"rec", "atr_ms1p_f32"},
         {"rec", "adx_ms1p_f32"},
-        {"rec", "ema_scan_combine"},
-        {"rec", "rsi_scan_combine"},
-        {"rec", "atr_scan_combine"},
-        {"rec", "smma_scan_combine"},
-        {"rec", "wilders_scan_combine"},
-        {"rec", "adx_scan_combine"},
+        {"rec", "scan_prepare"},
+        {"rec", "packed_prepare"},
+        {"rec", "ema_scan_states"},
+        {"rec", "rsi_scan_states"},
+        {"rec", "atr_scan_states"},
+        {"rec", "adx_scan_states"},
+        {"rec", "adx_scan_stage2"},
+        {"rec", "smma_scan_states"},
+        {"rec", "wilders_scan_states"},
+        {"rec", "atr_tr_scan_states"},
+        {"rec", "ema_scan_spans"},
+        {"rec", "rsi_scan_spans"},
+        {"rec", "atr_scan_spans"},
+        {"rec", "adx_scan_spans"},
+        {"rec", "smma_scan_spans"},
+        {"rec", "wilders_scan_spans"},
+        {"rec", "atr_tr_scan_spans"},
         {"rec", "atr_tr_batch_f32"},
-        {"rec", "atr_tr_scan_combine"},
         {"rec", "tr_from_hlc_f32"},
         {"rec", "smma_batch_f32"},
         {"rec", "wilders_batch_f32"},
@@ -403,8 +414,6 @@ vta_status vta_ctx_preload(vta_ctx *ctx) {
         {"fir", "series_first_nonfinite_dfv"},
         {"rec", "ms_ema_rsi_atr_f32"},
         {"rec", "ms_prepare_meta"},
-        {"rec", "series_nonfinite_flag"},
-        {"rec", "flag_to_clean"},
         {"rec", "vta_fill_i32"},
         {"rec", "vta_check_warms"},
         {"rec", "ms_clean_from_first_valids"},

@@ -25,11 +25,15 @@ struct vta_ctx {
     // of the enqueue-only entry points; reused in stream order)
     void *scratch = nullptr;
     static constexpr size_t kScratchBytes = 64 * 1024;
-    // chunk-end states of the recurrences' chunked scan ([combo][chunk][state]
+    // chunk-end states of the recurrences' chunked scan ([chunk][state][combo]
     // f64), reused in stream order by every batch launch of the context;
-    // 64 MiB holds 1,250 ADX combos (four states) at 1,024 chunks
+    // 64 MiB holds 1,280 ADX combos (four states) at 1,024 chunks
     void *carry = nullptr;
     static constexpr size_t kCarryBytes = 64u << 20;
+    // the scan's per-bar terms, in the same allocation: 8.4M bars of one term,
+    // 2.8M of ADX's three (longer series run in segments)
+    double *terms = nullptr;
+    static constexpr size_t kTermBytes = 64u << 20;
     // launch-shape knobs (vta_tune_knob); 0 = built-in heuristic
     int64_t tune[VTA_TUNE_KNOB_COUNT] = {};
     // EMA / RSI / ADX / PNR kernel policies and the forms their last batch and
@@ -40,7 +44,7 @@ struct vta_ctx {
     // an enqueue-only call with device-side argument checks (warm indices) has
     // run since the last vta_ctx_synchronize, which then reads the error word
     bool arg_check_pending = false;
-    // epoch of the last device-resident one-series batch (batch_prepare)
+    // epoch of the last device-resident one-series batch (scan_prepare)
     uint32_t prep_epoch = 0;
 };
 
@@ -253,19 +257,27 @@ struct PackJob {
     const int32_t *periods;
     float *out;
     double *carry;
-    int T, nlanes, fv, chunk, nch, groups, block0, combo0;
+    double *terms;
+    int T, nlanes, fv, chunk, nch, groups, block0, span0, tstride, span;
 };
 struct PackDims {
     int kind = 0, n_jobs = 0;
-    unsigned total_blocks = 0, total_combos = 0, flag_blocks = 1;
+    unsigned total_blocks = 0, total_spans = 0, flag_blocks = 1;
 };
-// Validates the jobs like the _device forms and lays out the table; each
-// job's carry pointer is left null, its offset (in doubles) in carry_off.
+// Validates the jobs like the _device forms and lays out the table; the
+// chunk states and terms of all jobs take work_elems doubles, which
+// pack_bind hands out from `work`.
 vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, size_t n_jobs,
-                       std::vector<PackJob> &tab, std::vector<size_t> &carry_off,
-                       size_t *carry_elems, PackDims *dims);
-// d_flags: n_jobs int32 words (cleared by the launch itself).
-vta_status pack_launch(vta_ctx *ctx, const PackDims &d, const void *d_jobs, int32_t *d_flags);
+                       std::vector<PackJob> &tab, size_t *work_elems, PackDims *dims);
+void pack_bind(const PackDims &d, std::vector<PackJob> &tab, double *work);
+// The device image of a pack: the table, then its flags (pack_flags_off bytes
+// in), which start as zeros.
+std::vector<unsigned char> pack_image(const std::vector<PackJob> &tab);
+inline size_t pack_flags_off(size_t n_jobs) { return n_jobs * sizeof(PackJob); }
+// d_image: pack_image on the device.  epoch: positive, another one for every
+// launch over the same flags (a repeated one can only read a clean job as
+// unclean, which runs exactly from first_valid).
+vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch);
 
 // Packed one-series BB batches (rolling.cpp): bb_job of rolling.hip.
 struct BbPackJob {

@@ -880,17 +880,16 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
     }
     if (jobs.empty()) return true;
     std::vector<PackJob> tab;
-    std::vector<size_t> off;
+    std::vector<unsigned char> image;
     size_t elems = 0;
     PackDims dims;
-    vta_status v = pack_layout(ctx, rk, jobs.data(), jobs.size(), tab, off, &elems, &dims);
-    void *d_tab = nullptr, *d_flags = nullptr, *d_carry = nullptr;
+    vta_status v = pack_layout(ctx, rk, jobs.data(), jobs.size(), tab, &elems, &dims);
+    void *d_tab = nullptr, *d_work = nullptr;
     if (v == VTA_OK) {
-        d_tab = s->arena.alloc(tab.size() * sizeof(PackJob));
-        d_flags = s->arena.alloc(tab.size() * sizeof(int32_t));
-        d_carry = s->arena.alloc(std::max<size_t>(elems, 1) * sizeof(double));
-        if (!d_tab || !d_flags || !d_carry) {
-            for (void *p : {d_tab, d_flags, d_carry})
+        d_tab = s->arena.alloc(pack_image(tab).size());
+        d_work = s->arena.alloc(std::max<size_t>(elems, 1) * sizeof(double));
+        if (!d_tab || !d_work) {
+            for (void *p : {d_tab, d_work})
                 if (p) s->arena.release(p);
             (void)hipStreamSynchronize(ctx->stream);   // the period tables' copies
             for (auto &q : g)
@@ -900,18 +899,18 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
                 }
             return false;
         }
-        for (size_t j = 0; j < tab.size(); ++j)
-            tab[j].carry = static_cast<double *>(d_carry) + off[j];
-        hipError_t e = hipMemcpyAsync(d_tab, tab.data(), tab.size() * sizeof(PackJob),
-                                      hipMemcpyHostToDevice, ctx->stream);
+        pack_bind(dims, tab, static_cast<double *>(d_work));
+        image = pack_image(tab);
+        hipError_t e = hipMemcpyAsync(d_tab, image.data(), image.size(), hipMemcpyHostToDevice,
+                                      ctx->stream);
         if (e != hipSuccess) v = fail(VTA_ERR_HIP, "hipMemcpyAsync: %s", hipGetErrorString(e));
     }
-    if (v == VTA_OK) v = pack_launch(ctx, dims, d_tab, static_cast<int32_t *>(d_flags));
+    if (v == VTA_OK) v = pack_launch(ctx, dims, d_tab, 1);
     const double t_launch = now_s() - s->t0;
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (v == VTA_OK && e != hipSuccess)
         v = fail(VTA_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
-    for (void *p : {d_tab, d_flags, d_carry})
+    for (void *p : {d_tab, d_work})
         if (p) s->arena.release(p);
     for (size_t i : member) {
         st[i] = v;
