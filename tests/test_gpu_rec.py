@@ -161,10 +161,10 @@ def test_scan_zero_denominators_and_odd_bars(ctxs, name, combos, flat, wild):
     _scan_case(ctxs, name, 6_011, (2, 1 + combos, 1), flat, wild)
 
 
-@pytest.mark.parametrize("name,n", [("ema", 8_388_609), ("rsi", 4_194_400), ("adx", 2_796_301)])
+@pytest.mark.parametrize("name,n", [("ema", 1_048_577), ("rsi", 1_048_700), ("adx", 1_050_000)])
 def test_scan_series_past_the_term_buffer(ctxs, name, n):
-    """64 MiB of terms hold 8,388,608 EMA bars (RSI half, ADX a third of that);
-    the rest run as a second segment from the handed-on states."""
+    """8 MiB of terms hold 1,048,576 EMA bars (RSI half, ADX a third of that);
+    the rest run as further segments from the handed-on states."""
     _scan_case(ctxs, name, n, (14, 64, 50))
 
 

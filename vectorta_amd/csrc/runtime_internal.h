@@ -27,13 +27,13 @@ struct vta_ctx {
     static constexpr size_t kScratchBytes = 64 * 1024;
     // chunk-end states of the recurrences' chunked scan ([chunk][state][combo]
     // f64), reused in stream order by every batch launch of the context;
-    // 64 MiB holds 1,280 ADX combos (four states) at 1,024 chunks
+    // 56 MiB holds 1,280 ADX combos (four states) at 860 chunks and their spans
     void *carry = nullptr;
-    static constexpr size_t kCarryBytes = 64u << 20;
-    // the scan's per-bar terms, in the same allocation: 8.4M bars of one term,
-    // 2.8M of ADX's three (longer series run in segments)
+    static constexpr size_t kCarryBytes = 56u << 20;
+    // the scan's per-bar terms, in the same allocation: 1.05M bars of one term,
+    // 0.35M of ADX's three (longer series run in segments)
     double *terms = nullptr;
-    static constexpr size_t kTermBytes = 64u << 20;
+    static constexpr size_t kTermBytes = 8u << 20;
     // launch-shape knobs (vta_tune_knob); 0 = built-in heuristic
     int64_t tune[VTA_TUNE_KNOB_COUNT] = {};
     // EMA / RSI / ADX / PNR kernel policies and the forms their last batch and
