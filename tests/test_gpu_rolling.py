@@ -3,22 +3,26 @@
 Bar: NaN warm-up prefixes and poison rules bit-exact everywhere.  PNR selects
 an input value, and MAD's median/deviation arithmetic is the oracle's f64
 sequence on the same f32 inputs, so both must equal f32(oracle) bit for bit.
-BB re-anchors its f64 window sums at every chunk start: values within 1e-6
-relative of the f64 oracle (bands of prices ~100; f32 output rounding is 6e-8),
+BB sums each window in f64 (many series: running sums re-anchored at every chunk
+start): values within 1e-6 relative of the f64 oracle (bands of prices ~100; f32 output rounding is 6e-8),
 +-Inf positions identical.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle as O
 import vectorta_amd as vta
-from vectorta_amd import datagen
+from vectorta_amd import datagen, lib
+from vectorta_amd._lib import check
 from tests.conftest import require_gpu
 from tests.helpers import max_rel_err, nan_mask_equal
 
 pytestmark = pytest.mark.gpu
 
 BB_TOL = 1e-6
+P = ctypes.c_void_p
 
 
 @pytest.fixture(scope="module")
@@ -107,6 +111,75 @@ def test_bb_batch_poison_rules(ops):
         refs = [O.bollinger_bands(xd, p, a, b) for p, a, b in combos]
         _bb_check(out, [np.stack([r[i] for r in refs]) for i in range(3)], f"poison {bad}")
         assert np.isnan(out[1][:, 21_050:]).all()
+
+
+def _bb_device(ops, jobs, pack):
+    """Upper / middle / lower of (x, periods, devup, devdn, largest period)
+    jobs, one device call each or one packed launch."""
+    ctx = ops["bb"].ctx
+    specs, keep = [], []
+    for x, per, up, dn, mx in jobs:
+        fv = int(np.argmax(~np.isnan(x)))
+        bad = np.flatnonzero(~np.isfinite(x[fv:]))
+        d = [ctx.to_device(np.ascontiguousarray(a)) for a in
+             (x, np.asarray(per, np.int32), np.asarray(up, np.float64), np.asarray(dn, np.float64))]
+        o = [ctx.alloc(len(per) * x.size * 4) for _ in range(3)]
+        specs.append({"prices": d[0], "periods": d[1], "devup": d[2], "devdn": d[3],
+                      "upper": o[0], "middle": o[1], "lower": o[2], "series_len": x.size,
+                      "first_valid": fv, "first_nonfinite": fv + int(bad[0]) if bad.size else x.size,
+                      "n_combos": len(per), "max_period": mx})
+        keep.append((d, o))
+    if pack:
+        pk = vta.BbPack(ctx, specs)
+        pk.launch()
+    else:
+        for q in specs:
+            check(lib().vta_bollinger_bands_batch_device(
+                ctx.handle, P(q["prices"].ptr), q["series_len"], q["first_valid"],
+                q["first_nonfinite"], P(q["periods"].ptr), P(q["devup"].ptr), P(q["devdn"].ptr),
+                q["n_combos"], q["max_period"], *(P(q[k].ptr) for k in ("upper", "middle", "lower"))))
+    ctx.synchronize()
+    out = [[b.copy_to_host(np.float32).reshape(q["n_combos"], -1) for b in o]
+           for q, (_, o) in zip(specs, keep)]
+    if pack:
+        pk.close()
+    for d, o in keep:
+        for b in d + o:
+            b.free()
+    return out
+
+
+def test_bb_batch_tile_edges(ops):
+    """Bars either side of a 1,024-bar tile and of a wave's 256; periods either
+    side of the 16-bar sums, rising, falling, in no order and repeated; more
+    combos than a block takes; a period above the stated largest; the longest
+    period of the tile form and one more (the long form); non-finite bars in
+    the warm-up, at a tile's edges and in the last bar.  Alone and packed give
+    the same bits, both the oracle's values (sums of at most 2,049 positive
+    f64 terms: far inside the 1e-6 of the other tests)."""
+    def job(n, per, lead=0, bad=(), val=np.nan, mx=None):
+        x = datagen.gbm_close(n, 0.01, seed=n + len(per))
+        x[:lead] = np.nan
+        for b in bad:
+            x[b] = val
+        per = list(per)
+        return (x, per, np.linspace(1.0, 3.0, len(per)), np.linspace(2.5, 0.5, len(per)),
+                mx or max(per))
+    jobs = [job(1, [1]), job(17, range(1, 18)), job(255, [16, 15, 17, 1, 33, 33, 32]),
+            job(1_023, range(48, 1, -1), lead=3), job(1_024, [1, 5, 5, 5, 2, 1_000], lead=24),
+            job(1_025, [31, 64], lead=1_024 - 63), job(2_049, range(2, 202), lead=5),
+            job(5_000, [7, 20, 90], mx=20), job(4_100, [2_048, 3, 2_047]),
+            job(4_100, [2_049, 3]), job(120_000, range(2, 68), lead=1),
+            job(3_000, [2, 40, 300], lead=2, bad=(100,)),
+            job(3_000, [2, 40, 300], lead=2, bad=(1_023, 1_030), val=np.inf),
+            job(3_000, [2, 40, 300], lead=2, bad=(2_048,), val=-np.inf),
+            job(3_000, [2, 40, 2_100], bad=(1_024,)), job(3_000, [1, 4], bad=(2_999,))]
+    alone, packed = _bb_device(ops, jobs, False), _bb_device(ops, jobs, True)
+    for i, ((x, per, up, dn, _), a3, p3) in enumerate(zip(jobs, alone, packed)):
+        for a, p in zip(a3, p3):
+            assert np.array_equal(a.view(np.uint32), p.view(np.uint32)), i
+        refs = [O.bollinger_bands(x.astype(np.float64), p, u, d) for p, u, d in zip(per, up, dn)]
+        _bb_check(a3, [np.stack([r[k] for r in refs]) for k in range(3)], f"tile edges job {i}")
 
 
 def test_bb_many_series_jumps_shape(ops):

@@ -11,8 +11,9 @@
 //
 // Time is cut into chunks; every chunk rebuilds its window state exactly from
 // the W bars before it (windowed indicators need no burn-in approximation).
-// BB re-anchors its f64 sums at every chunk start; its "poison forever" rule
-// is reproduced from the series' first non-finite bar (see bb_run).
+// BB re-anchors its f64 sums at every chunk start (one-series batches sum each
+// window by itself, see the tile form); its "poison forever" rule is reproduced
+// from the series' first non-finite bar (see bb_run).
 //
 // PNR and MAD keep each lane's window sorted in LDS (column layout, stride 64
 // lanes, so every lane hits its own bank): one binary search for the outgoing
@@ -33,11 +34,11 @@
 struct roll_args {
     const float *x;
     const int32_t *p_len;    // batch: per combo
-    const double *p_a;       // batch: BB devup / PNR percentage per combo
-    const double *p_b;       // batch: BB devdn per combo
+    const double *p_a;       // batch: PNR percentage per combo
+    const double *p_b;
     const int32_t *fvs;      // many-series: per series; batch: [0]
-    const int32_t *poison;   // BB: first non-finite bar >= first_valid, per series (ms)
-                             // or [0] (batch); null means none known (one chunk)
+    const int32_t *poison;   // BB: first non-finite bar >= first_valid, per series;
+                             // null means none known (one chunk)
     float *out0;
     float *out1;
     float *out2;
@@ -241,28 +242,198 @@ extern "C" __global__ __launch_bounds__(64) void bb_ms1p_f32(roll_args a) {
     else bb_run<false>(e, c0, c1, z, active, ld, st, nullptr);
 }
 
-// one series x many (period, devup, devdn): grid.x = combos / 64, grid.y = chunks.
-// Lane = combo; all lanes step through the chunk's bars together (the same
-// output rule as bb_run: re-anchor at the first output bar of the chunk,
-// replaying at most p bars after the first non-finite bar z, NaN from z + p).
-// What one block of a one-series BB batch works on: the series, the combos'
-// periods / deviations and outputs, the chunking, first_valid, the first
-// non-finite bar z (T if none), and which combo group and chunk it is.
-struct bb_view {
+// ---------------------------------------------------------------- BB batches
+//
+// One series x many (period, devup, devdn): what a launch, or one job of a
+// packed launch, works on.  z: the first non-finite bar at or after
+// first_valid (T if none).  hist > 0: the tile form, `chunk` combos per block
+// and `groups` such combo blocks; hist 0: the long form (below), chunks of
+// `chunk` bars of `groups` groups of 64 combos.  Of a packed launch job j owns
+// the blocks from block0 up to the next job's.
+struct bb_job {
     const float *x;
     const int32_t *p_len;
     const double *p_a, *p_b;
     float *out0, *out1, *out2;
-    int T, nlanes, chunk, fv, z, group, k;
+    int T, nlanes, fv, z, chunk, groups, block0, hist;
 };
 
-__device__ __forceinline__ void bb_batch_body(const bb_view &a) {
+// Tile form (periods up to 2,048): a block takes BT bars and up to BB_COMBOS
+// combos, lane = bar, so every store is 256 consecutive bytes of a row and
+// the combos' parameters are wave-uniform.  The block holds its bars and the
+// `hist` before them in LDS, with the f64 sum and sum of squares of the 16
+// bars ending at each of them.  A lane keeps its bars' window sums in
+// registers and grows them from combo to combo, by 16-bar sums, then by
+// single bars; a shorter period starts over, and the next width of the same
+// period reuses the mean and deviation.  Sums are only ever added to: no bar
+// leaves a window again, so their rounding error is that of p additions.
+// Every output class of bb_run holds by itself: a window up to z + p - 1 sums
+// the non-finite bars it holds.
+//
+// Stores bound it: 100 periods x 5 widths x 60,000 bars (360 MB) take 72 us,
+// 5.0 TB/s.  Lane = combo with running sums and the rows put together in LDS
+// (the long form) took 273 there: 1,160 waves, 25.6 KB of LDS each, a serial
+// chain of a whole chunk.  One combo of 1,000 bars: 42.7 -> 4.4 us.
+#define BB_BT 1024
+#define BB_COMBOS 64
+
+typedef double bb_pair __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void bb_tile_body(const bb_job &a, int local) {
+    extern __shared__ __align__(16) double bb_lds[];
+    __shared__ double up_s[BB_COMBOS], dn_s[BB_COMBOS];
+    __shared__ int p_s[BB_COMBOS];
+    const int tid = threadIdx.x;
+    const int T = a.T, hist = a.hist, n = hist + BB_BT;
+    const int tiles = (T + BB_BT - 1) / BB_BT;
+    const int t0 = local % tiles * BB_BT, cg = local / tiles * a.chunk;
+    const int nc = min(a.chunk, a.nlanes - cg);
+    bb_pair *w16 = reinterpret_cast<bb_pair *>(bb_lds);     // [n]: bars j - 15 .. j
+    float *xs = reinterpret_cast<float *>(w16 + n);         // [n]: bars t0 - hist ..
+    for (int j = tid; j < n; j += 256) {
+        const int u = t0 - hist + j;
+        xs[j] = u >= 0 && u < T ? a.x[u] : 0.0f;
+    }
+    for (int j = tid; j < nc; j += 256) {
+        p_s[j] = a.p_len[cg + j];
+        up_s[j] = a.p_a[cg + j];
+        dn_s[j] = a.p_b[cg + j];
+    }
+    __syncthreads();
+    for (int j = tid; j < n; j += 256) {
+        if (j < 15) continue;
+        bb_pair w = {0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const double v = (double)xs[j - i];
+            w.x += v;
+            w.y += v * v;
+        }
+        w16[j] = w;
+    }
+    __syncthreads();
+
+    // the wave's 256 bars, lane's bars 64 apart
+    const int lane = tid & 63, tb = t0 + (tid >> 6) * 256;
+    const int nb = min(256, T - tb);
+    if (nb <= 0) return;
+    const int at = hist + tb - t0 + lane;                   // slot of bar tb + lane
+    double s[4], q[4], m[4], sd[4];
+    int have = 0, last = INT_MIN;                           // bars in s, q; period of m, sd
+#pragma unroll
+    for (int b = 0; b < 4; ++b) s[b] = q[b] = m[b] = sd[b] = 0.0;
+    const bool down = p_s[0] > p_s[nc - 1];                 // a falling grid runs backwards
+    for (int i = 0; i < nc; ++i) {
+        const int c = down ? nc - 1 - i : i;
+        const int p = __builtin_amdgcn_readfirstlane(p_s[c]);
+        const long warm = (long)a.fv + p - 1, zp = (long)a.z + p;
+        const size_t row = (size_t)(cg + c) * T + tb + lane;
+        if (warm >= tb + nb || zp <= tb) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                if (64 * b + lane < nb) {
+                    a.out0[row + 64 * b] = VTA_QNAN_F32;
+                    a.out1[row + 64 * b] = VTA_QNAN_F32;
+                    a.out2[row + 64 * b] = VTA_QNAN_F32;
+                }
+            }
+            continue;
+        }
+        if (p != last) {
+            if (p < have) {
+                have = 0;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) s[b] = q[b] = 0.0;
+            }
+            const int in = min(p, hist);                    // (bars held in LDS)
+            for (; have + 16 <= in; have += 16) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const bb_pair w = w16[at + 64 * b - have];
+                    s[b] += w.x;
+                    q[b] += w.y;
+                }
+            }
+            for (; have < in; ++have) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const double v = (double)xs[at + 64 * b - have];
+                    s[b] += v;
+                    q[b] += v * v;
+                }
+            }
+            // (a period above the stated largest: its bars from memory)
+            for (; have < p; ++have) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const double v = (double)a.x[min(max(tb + lane + 64 * b - have, 0), T - 1)];
+                    s[b] += v;
+                    q[b] += v * v;
+                }
+            }
+            const double inv_n = 1.0 / (double)p;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                m[b] = s[b] * inv_n;
+                const double var = (q[b] * inv_n) - (m[b] * m[b]);
+                sd[b] = sqrt(fmax(var, 0.0));
+            }
+            last = p;
+        }
+        const double up = up_s[c], dn = dn_s[c];
+        if (nb == 256 && warm <= tb && zp >= tb + 256) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                a.out0[row + 64 * b] = (float)(m[b] + up * sd[b]);
+                a.out1[row + 64 * b] = (float)m[b];
+                a.out2[row + 64 * b] = (float)(m[b] - dn * sd[b]);
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int t = tb + lane + 64 * b;
+                const bool ok = t >= warm && t < zp;
+                if (64 * b + lane < nb) {
+                    a.out0[row + 64 * b] = ok ? (float)(m[b] + up * sd[b]) : VTA_QNAN_F32;
+                    a.out1[row + 64 * b] = ok ? (float)m[b] : VTA_QNAN_F32;
+                    a.out2[row + 64 * b] = ok ? (float)(m[b] - dn * sd[b]) : VTA_QNAN_F32;
+                }
+            }
+        }
+    }
+}
+
+extern "C" __global__ __launch_bounds__(256) void bb_batch_f32(bb_job j) {
+    bb_tile_body(j, blockIdx.x);
+}
+
+// The job of block `flat` in a packed launch.
+__device__ __forceinline__ const bb_job &bb_find(const bb_job *jobs, int n_jobs, int flat) {
+    int lo = 0, hi = n_jobs - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (jobs[mid].block0 <= flat) lo = mid; else hi = mid - 1;
+    }
+    return jobs[lo];
+}
+
+extern "C" __global__ __launch_bounds__(256) void bb_packed_f32(const bb_job *jobs, int n_jobs) {
+    const bb_job j = bb_find(jobs, n_jobs, blockIdx.x);
+    bb_tile_body(j, (int)blockIdx.x - j.block0);
+}
+
+// Long form (periods past the tile form's LDS): lane = combo; all lanes step
+// through the chunk's bars together (the same output rule as bb_run: re-anchor
+// at the first output bar of the chunk, replaying at most p bars after the
+// first non-finite bar z, NaN from z + p).
+__device__ __forceinline__ void bb_long_body(const bb_job &a, int local) {
     __shared__ float ob[3][64 * RB_LD];
     const int lane = threadIdx.x & 63;
-    const int c = a.group * 64 + lane;
+    const int group = local % a.groups;
+    const int c = group * 64 + lane;
     const bool active = c < a.nlanes;
     const int T = a.T;
-    const int c0 = a.k * a.chunk;
+    const int c0 = local / a.groups * a.chunk;
     const int c1 = min(c0 + a.chunk, T);
     const int cc = min(c, a.nlanes - 1);
     BbEng e;
@@ -310,69 +481,20 @@ __device__ __forceinline__ void bb_batch_body(const bb_view &a) {
             }
         }
         rb_sync();
-        rb_flush(ob[0], a.out0, a.group * 64, a.nlanes, T, t0, nb);
-        rb_flush(ob[1], a.out1, a.group * 64, a.nlanes, T, t0, nb);
-        rb_flush(ob[2], a.out2, a.group * 64, a.nlanes, T, t0, nb);
+        rb_flush(ob[0], a.out0, group * 64, a.nlanes, T, t0, nb);
+        rb_flush(ob[1], a.out1, group * 64, a.nlanes, T, t0, nb);
+        rb_flush(ob[2], a.out2, group * 64, a.nlanes, T, t0, nb);
         rb_sync();
     }
 }
 
-extern "C" __global__ __launch_bounds__(64) void bb_batch_f32(roll_args a) {
-    bb_view v;
-    v.x = a.x;
-    v.p_len = a.p_len;
-    v.p_a = a.p_a;
-    v.p_b = a.p_b;
-    v.out0 = a.out0;
-    v.out1 = a.out1;
-    v.out2 = a.out2;
-    v.T = a.T;
-    v.nlanes = a.nlanes;
-    v.chunk = a.chunk;
-    v.fv = a.fvs[0];
-    v.z = a.poison ? a.poison[0] : a.T;
-    v.group = blockIdx.x;
-    v.k = blockIdx.y;
-    bb_batch_body(v);
+extern "C" __global__ __launch_bounds__(64) void bb_long_batch_f32(bb_job j) {
+    bb_long_body(j, blockIdx.x);
 }
 
-// Packed one-series BB batches: job j = one series with its own combos;
-// a 1-D grid over every job's (combo group, chunk) blocks, job j owning
-// [block0, block0 + groups * ceil(T / chunk)); each block finds its job by
-// binary search and runs exactly the block of the job's direct launch.
-struct bb_job {
-    const float *x;
-    const int32_t *p_len;
-    const double *p_a, *p_b;
-    float *out0, *out1, *out2;
-    int T, nlanes, fv, z, chunk, groups, block0, pad_;
-};
-
-extern "C" __global__ __launch_bounds__(64) void bb_packed_f32(const bb_job *jobs, int n_jobs) {
-    const int flat = blockIdx.x;
-    int lo = 0, hi = n_jobs - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (jobs[mid].block0 <= flat) lo = mid; else hi = mid - 1;
-    }
-    const bb_job &j = jobs[lo];
-    const int local = flat - j.block0;
-    bb_view v;
-    v.x = j.x;
-    v.p_len = j.p_len;
-    v.p_a = j.p_a;
-    v.p_b = j.p_b;
-    v.out0 = j.out0;
-    v.out1 = j.out1;
-    v.out2 = j.out2;
-    v.T = j.T;
-    v.nlanes = j.nlanes;
-    v.chunk = j.chunk;
-    v.fv = j.fv;
-    v.z = j.z;
-    v.group = local % j.groups;
-    v.k = local / j.groups;
-    bb_batch_body(v);
+extern "C" __global__ __launch_bounds__(64) void bb_long_packed_f32(const bb_job *jobs, int n_jobs) {
+    const bb_job j = bb_find(jobs, n_jobs, blockIdx.x);
+    bb_long_body(j, (int)blockIdx.x - j.block0);
 }
 
 // ---------------------------------------------------------------- sorted window

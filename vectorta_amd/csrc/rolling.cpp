@@ -78,7 +78,7 @@ int roll_chunk(const vta_ctx *ctx, size_t T, size_t lanes, size_t max_w, bool ch
 }
 
 const char *kname(RInd k, bool batch) {
-    static const char *b[] = {"bb_batch_f32", "pnr_batch_f32", "mad_batch_f32"};
+    static const char *b[] = {nullptr, "pnr_batch_f32", "mad_batch_f32"};   // (BB: bb_batch_launch)
     static const char *m[] = {"bb_ms1p_f32", "pnr_ms1p_f32", "mad_ms1p_f32"};
     return batch ? b[k] : m[k];
 }
@@ -262,6 +262,8 @@ vta_status validate(RInd k, const std::vector<Combo> &cs, size_t len, size_t fv,
     return VTA_OK;
 }
 
+vta_status bb_batch_launch(vta_ctx *ctx, const vta_bb_job &q);
+
 vta_status batch_dev(vta_ctx *ctx, RInd k, const float *x, size_t len,
                      const std::vector<Combo> &cs, int nout, vta_device_array_f32 *out) {
     if (!ctx || !out || !x) return fail(VTA_ERR_INVALID_INPUT, "null argument");
@@ -289,6 +291,22 @@ vta_status batch_dev(vta_ctx *ctx, RInd k, const float *x, size_t len,
     VTA_TRY(upload(ctx, db, pb.data(), C * sizeof(double)));
     VTA_TRY(upload(ctx, dm, meta, sizeof(meta)));
     for (int i = 0; i < nout; ++i) VTA_TRY(o[i].alloc(n_out));
+    if (k == R_BB) {
+        vta_bb_job q{};
+        q.d_prices = dx.as<float>();
+        q.d_periods = dl.as<int32_t>();
+        q.d_devup = da.as<double>();
+        q.d_devdn = db.as<double>();
+        q.d_upper = o[0].as<float>();
+        q.d_middle = o[1].as<float>();
+        q.d_lower = o[2].as<float>();
+        q.series_len = (int32_t)len;
+        q.first_valid = meta[0];
+        q.first_nonfinite = meta[1];
+        q.n_combos = (int32_t)C;
+        q.max_period = (int32_t)mx;
+        VTA_TRY(bb_batch_launch(ctx, q));
+    }
     roll_args_host a{};
     a.x = dx.as<float>();
     a.p_len = dl.as<int32_t>();
@@ -301,7 +319,7 @@ vta_status batch_dev(vta_ctx *ctx, RInd k, const float *x, size_t len,
     a.out2 = o[2].as<float>();
     a.T = (int)len;
     a.nlanes = (int)C;
-    VTA_TRY(roll_launch(ctx, k, true, a, mx, true));
+    if (k != R_BB) VTA_TRY(roll_launch(ctx, k, true, a, mx, true));
     VTA_HIP(hipStreamSynchronize(ctx->stream));
     for (int i = 0; i < nout; ++i) {
         out[i].ptr = static_cast<float *>(o[i].release());
@@ -377,6 +395,126 @@ vta_status ms_device(vta_ctx *ctx, RInd k, const float *d_x, const int32_t *d_fv
 
 }  // namespace
 
+// ---------------------------------------------------------------- BB batches
+
+static_assert(sizeof(BbPackJob) == 88, "bb_job layout");
+
+namespace {
+
+// Bars per block and longest period of the tile form (BB_BT), the most combos
+// of one of its blocks (BB_COMBOS).  Longer periods need more than 64 KB of LDS
+// per block and take the long form; at 1,900..2,000 x 5 widths x 60,000 bars
+// the tile form takes 104 us, the long form 3,289.
+// A block takes as many combos as leave kBbBlocks blocks (kBbBlocksTall where
+// growing the first window takes longer): 500 combos of 5..104 x 60,000 bars
+// in 2,048 / 1,024 blocks 72.6 / 76.0 us, 148 of 1,900.. 87.2 / 62.9.
+constexpr size_t kBbTile = 1024, kBbHist = 2048, kBbCombos = 64;
+constexpr size_t kBbBlocks = 2048, kBbBlocksTall = 1024;
+
+// The launch of one batch: its table entry and blocks.
+BbPackJob bb_job_of(const vta_ctx *ctx, const vta_bb_job &q, size_t *blocks) {
+    const size_t T = (size_t)q.series_len, C = (size_t)q.n_combos, mx = (size_t)q.max_period;
+    BbPackJob e{};
+    e.x = q.d_prices;
+    e.p_len = q.d_periods;
+    e.p_a = q.d_devup;
+    e.p_b = q.d_devdn;
+    e.out0 = q.d_upper;
+    e.out1 = q.d_middle;
+    e.out2 = q.d_lower;
+    e.T = (int)T;
+    e.nlanes = (int)C;
+    e.fv = q.first_valid;
+    e.z = q.first_nonfinite;
+    if (mx <= kBbHist) {
+        const size_t tiles = (T + kBbTile - 1) / kBbTile;
+        const size_t want = mx <= 256 ? kBbBlocks : kBbBlocksTall;
+        const size_t per = std::min(kBbCombos, std::max<size_t>(1, C * tiles / want));
+        e.hist = (int)((mx + 15) & ~(size_t)15);
+        e.chunk = (int)per;
+        e.groups = (int)((C + per - 1) / per);
+        *blocks = tiles * (size_t)e.groups;
+    } else {
+        e.chunk = roll_chunk(ctx, T, C, mx, true, 0);
+        e.groups = (int)((C + 63) / 64);
+        *blocks = (size_t)e.groups * ((T + (size_t)e.chunk - 1) / (size_t)e.chunk);
+    }
+    return e;
+}
+
+unsigned bb_tile_lds(int hist) { return 20u * ((unsigned)hist + (unsigned)kBbTile); }
+
+vta_status bb_batch_launch(vta_ctx *ctx, const vta_bb_job &q) {
+    size_t blocks;
+    const BbPackJob e = bb_job_of(ctx, q, &blocks);
+    if (blocks > (size_t)INT32_MAX)
+        return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "grid exceeds 2^31 blocks");
+    hipFunction_t f;
+    VTA_TRY(get_function(ctx, "rolling", e.hist ? "bb_batch_f32" : "bb_long_batch_f32", &f));
+    return launch(ctx, f, dim3((unsigned)blocks), dim3(e.hist ? 256 : 64),
+                  e.hist ? bb_tile_lds(e.hist) : 0, e);
+}
+
+}  // namespace
+
+namespace vta {
+
+vta_status bb_pack_layout(const vta_ctx *ctx, const vta_bb_job *jobs, size_t n_jobs,
+                          std::vector<BbPackJob> &tab, BbPackDims *dims) {
+    if (!ctx || !jobs || !dims) return fail(VTA_ERR_INVALID_INPUT, "null argument");
+    if (n_jobs == 0 || n_jobs > 65535)
+        return fail(VTA_ERR_INVALID_INPUT, "n_jobs must be in 1..65535 (got %zu)", n_jobs);
+    std::vector<BbPackJob> tail;
+    size_t tile_blocks = 0, long_blocks = 0;
+    tab.clear();
+    *dims = BbPackDims{};
+    for (size_t j = 0; j < n_jobs; ++j) {
+        const vta_bb_job &q = jobs[j];
+        // the checks of vta_bollinger_bands_batch_device
+        if (!q.d_prices || !q.d_periods || !q.d_devup || !q.d_devdn || !q.d_upper ||
+            !q.d_middle || !q.d_lower)
+            return fail(VTA_ERR_INVALID_INPUT, "job %zu: null pointer", j);
+        if (q.series_len <= 0 || q.n_combos <= 0 || q.max_period <= 0 || q.first_valid < 0 ||
+            q.first_valid >= q.series_len || q.first_nonfinite < q.first_valid ||
+            q.first_nonfinite > q.series_len || q.series_len - q.first_valid < q.max_period)
+            return fail(VTA_ERR_INVALID_INPUT, "job %zu: invalid sizes", j);
+        size_t blocks;
+        BbPackJob e = bb_job_of(ctx, q, &blocks);
+        size_t &total = e.hist ? tile_blocks : long_blocks;
+        e.block0 = (int)total;
+        total += blocks;
+        if (total > (size_t)INT32_MAX)
+            return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "packed grid exceeds 2^31 blocks");
+        (e.hist ? tab : tail).push_back(e);
+        if (e.hist) dims->tile_lds = std::max(dims->tile_lds, bb_tile_lds(e.hist));
+    }
+    dims->n_tile = (int)tab.size();
+    dims->n_long = (int)tail.size();
+    dims->tile_blocks = (unsigned)tile_blocks;
+    dims->long_blocks = (unsigned)long_blocks;
+    tab.insert(tab.end(), tail.begin(), tail.end());
+    return VTA_OK;
+}
+
+vta_status bb_pack_launch(vta_ctx *ctx, const void *d_jobs, const BbPackDims &dims) {
+    hipFunction_t f;
+    if (dims.n_tile) {
+        VTA_TRY(get_function(ctx, "rolling", "bb_packed_f32", &f));
+        VTA_TRY(launch(ctx, f, dim3(dims.tile_blocks), dim3(256), dims.tile_lds, d_jobs,
+                       dims.n_tile));
+    }
+    if (dims.n_long) {
+        VTA_TRY(get_function(ctx, "rolling", "bb_long_packed_f32", &f));
+        VTA_TRY(launch(ctx, f, dim3(dims.long_blocks), dim3(64), 0,
+                       static_cast<const void *>(static_cast<const BbPackJob *>(d_jobs) +
+                                                 dims.n_tile),
+                       dims.n_long));
+    }
+    return VTA_OK;
+}
+
+}  // namespace vta
+
 extern "C" {
 
 // ------------------------------------------------------------------ Bollinger Bands
@@ -415,26 +553,20 @@ vta_status vta_bollinger_bands_batch_device(vta_ctx *ctx, const float *d_prices,
         first_valid >= series_len || first_nonfinite < first_valid ||
         first_nonfinite > series_len || series_len - first_valid < max_period)
         return fail(VTA_ERR_INVALID_INPUT, "invalid sizes");
-    // per-call metadata {first_valid, first_nonfinite} in the context scratch,
-    // written by a fill kernel in stream order
-    int32_t *meta = static_cast<int32_t *>(ctx->scratch) + 128;
-    hipFunction_t fill;
-    VTA_TRY(get_function(ctx, "rec", "vta_fill_i32", &fill));
-    VTA_TRY(launch(ctx, fill, dim3(1), dim3(256), 0, meta, 1, (int)first_valid));
-    VTA_TRY(launch(ctx, fill, dim3(1), dim3(256), 0, meta + 1, 1, (int)first_nonfinite));
-    roll_args_host a{};
-    a.x = d_prices;
-    a.p_len = d_periods;
-    a.p_a = d_devup;
-    a.p_b = d_devdn;
-    a.fvs = meta;
-    a.poison = meta + 1;
-    a.out0 = d_upper;
-    a.out1 = d_middle;
-    a.out2 = d_lower;
-    a.T = series_len;
-    a.nlanes = n_combos;
-    return roll_launch(ctx, R_BB, true, a, (size_t)max_period, true);
+    vta_bb_job q{};
+    q.d_prices = d_prices;
+    q.d_periods = d_periods;
+    q.d_devup = d_devup;
+    q.d_devdn = d_devdn;
+    q.d_upper = d_upper;
+    q.d_middle = d_middle;
+    q.d_lower = d_lower;
+    q.series_len = series_len;
+    q.first_valid = first_valid;
+    q.first_nonfinite = first_nonfinite;
+    q.n_combos = n_combos;
+    q.max_period = max_period;
+    return bb_batch_launch(ctx, q);
 }
 
 vta_status vta_bollinger_bands_many_series_one_param_time_major_dev(
@@ -547,66 +679,9 @@ vta_status vta_medium_ad_many_series_one_param_device(vta_ctx *ctx, const float 
 
 // ---------------------------------------------------------------- packed BB batches
 
-static_assert(sizeof(BbPackJob) == 88, "bb_job layout");
-
-namespace vta {
-
-vta_status bb_pack_layout(const vta_ctx *ctx, const vta_bb_job *jobs, size_t n_jobs,
-                          std::vector<BbPackJob> &tab, unsigned *total_blocks) {
-    if (!ctx || !jobs || !total_blocks) return fail(VTA_ERR_INVALID_INPUT, "null argument");
-    if (n_jobs == 0 || n_jobs > 65535)
-        return fail(VTA_ERR_INVALID_INPUT, "n_jobs must be in 1..65535 (got %zu)", n_jobs);
-    tab.assign(n_jobs, BbPackJob{});
-    size_t blocks = 0;
-    for (size_t j = 0; j < n_jobs; ++j) {
-        const vta_bb_job &q = jobs[j];
-        // the checks of vta_bollinger_bands_batch_device
-        if (!q.d_prices || !q.d_periods || !q.d_devup || !q.d_devdn || !q.d_upper ||
-            !q.d_middle || !q.d_lower)
-            return fail(VTA_ERR_INVALID_INPUT, "job %zu: null pointer", j);
-        if (q.series_len <= 0 || q.n_combos <= 0 || q.max_period <= 0 || q.first_valid < 0 ||
-            q.first_valid >= q.series_len || q.first_nonfinite < q.first_valid ||
-            q.first_nonfinite > q.series_len || q.series_len - q.first_valid < q.max_period)
-            return fail(VTA_ERR_INVALID_INPUT, "job %zu: invalid sizes", j);
-        const size_t T = (size_t)q.series_len, C = (size_t)q.n_combos;
-        const size_t chunk = (size_t)roll_chunk(ctx, T, C, (size_t)q.max_period, true, 0);
-        const size_t nch = (T + chunk - 1) / chunk;
-        const size_t groups = (C + 63) / 64;
-        BbPackJob &e = tab[j];
-        e.x = q.d_prices;
-        e.p_len = q.d_periods;
-        e.p_a = q.d_devup;
-        e.p_b = q.d_devdn;
-        e.out0 = q.d_upper;
-        e.out1 = q.d_middle;
-        e.out2 = q.d_lower;
-        e.T = (int)T;
-        e.nlanes = (int)C;
-        e.fv = q.first_valid;
-        e.z = q.first_nonfinite;
-        e.chunk = (int)chunk;
-        e.groups = (int)groups;
-        e.block0 = (int)blocks;
-        blocks += groups * nch;
-        if (blocks > (size_t)INT32_MAX)
-            return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "packed grid exceeds 2^31 blocks");
-    }
-    *total_blocks = (unsigned)blocks;
-    return VTA_OK;
-}
-
-vta_status bb_pack_launch(vta_ctx *ctx, const void *d_jobs, int n_jobs, unsigned total_blocks) {
-    hipFunction_t f;
-    VTA_TRY(get_function(ctx, "rolling", "bb_packed_f32", &f));
-    return launch(ctx, f, dim3(total_blocks), dim3(64), 0, d_jobs, n_jobs);
-}
-
-}  // namespace vta
-
 struct vta_bb_pack {
     int device = 0;
-    int n_jobs = 0;
-    unsigned total_blocks = 0;
+    BbPackDims dims;
     DevBuf jobs;
 };
 
@@ -619,9 +694,8 @@ vta_status vta_bb_pack_create(vta_ctx *ctx, const vta_bb_job *jobs, size_t n_job
     *out = nullptr;
     std::vector<BbPackJob> tab;
     auto pk = std::make_unique<vta_bb_pack>();
-    VTA_TRY(bb_pack_layout(ctx, jobs, n_jobs, tab, &pk->total_blocks));
+    VTA_TRY(bb_pack_layout(ctx, jobs, n_jobs, tab, &pk->dims));
     pk->device = ctx->device;
-    pk->n_jobs = (int)n_jobs;
     VTA_HIP(hipSetDevice(ctx->device));
     VTA_TRY(upload(ctx, pk->jobs, tab.data(), n_jobs * sizeof(BbPackJob)));
     *out = pk.release();
@@ -634,7 +708,7 @@ vta_status vta_bb_pack_launch(vta_ctx *ctx, const vta_bb_pack *pk) {
     if (pk->device != ctx->device)
         return fail(VTA_ERR_DEVICE_MISMATCH, "pack built on device %d, context on %d", pk->device,
                     ctx->device);
-    return bb_pack_launch(ctx, pk->jobs.p, pk->n_jobs, pk->total_blocks);
+    return bb_pack_launch(ctx, pk->jobs.p, pk->dims);
 }
 
 vta_status vta_bb_pack_destroy(vta_bb_pack *pk) {

@@ -279,17 +279,22 @@ inline size_t pack_flags_off(size_t n_jobs) { return n_jobs * sizeof(PackJob); }
 // unclean, which runs exactly from first_valid).
 vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch);
 
-// Packed one-series BB batches (rolling.cpp): bb_job of rolling.hip.
+// One-series BB batches (rolling.cpp): bb_job of rolling.hip, and a packed
+// table's launches (the tile-form jobs come first in it).
 struct BbPackJob {
     const float *x;
     const int32_t *p_len;
     const double *p_a, *p_b;
     float *out0, *out1, *out2;
-    int T, nlanes, fv, z, chunk, groups, block0, pad_;
+    int T, nlanes, fv, z, chunk, groups, block0, hist;
+};
+struct BbPackDims {
+    int n_tile = 0, n_long = 0;
+    unsigned tile_blocks = 0, long_blocks = 0, tile_lds = 0;
 };
 vta_status bb_pack_layout(const vta_ctx *ctx, const vta_bb_job *jobs, size_t n_jobs,
-                          std::vector<BbPackJob> &tab, unsigned *total_blocks);
-vta_status bb_pack_launch(vta_ctx *ctx, const void *d_jobs, int n_jobs, unsigned total_blocks);
+                          std::vector<BbPackJob> &tab, BbPackDims *dims);
+vta_status bb_pack_launch(vta_ctx *ctx, const void *d_jobs, const BbPackDims &dims);
 
 // bf16 round-to-nearest-even of an f32 (bit pattern).
 uint16_t bf16_rne(float f);

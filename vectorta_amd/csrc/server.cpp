@@ -684,8 +684,8 @@ bool run_packed_bb(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>
     }
     if (jobs.empty()) return true;
     std::vector<BbPackJob> tab;
-    unsigned blocks = 0;
-    vta_status v = bb_pack_layout(ctx, jobs.data(), jobs.size(), tab, &blocks);
+    BbPackDims dims;
+    vta_status v = bb_pack_layout(ctx, jobs.data(), jobs.size(), tab, &dims);
     void *d_tab = nullptr;
     if (v == VTA_OK) {
         d_tab = s->arena.alloc(tab.size() * sizeof(BbPackJob));
@@ -703,7 +703,7 @@ bool run_packed_bb(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>
                                       hipMemcpyHostToDevice, ctx->stream);
         if (e != hipSuccess) v = fail(VTA_ERR_HIP, "hipMemcpyAsync: %s", hipGetErrorString(e));
     }
-    if (v == VTA_OK) v = bb_pack_launch(ctx, d_tab, (int)tab.size(), blocks);
+    if (v == VTA_OK) v = bb_pack_launch(ctx, d_tab, dims);
     const double t_launch = now_s() - s->t0;
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (v == VTA_OK && e != hipSuccess)
