@@ -314,3 +314,44 @@ def test_auto_selects_checked_split_on_price_series(alma):
     err = max_rel_err(g, ref)
     print(f"alma auto (split-F16) max rel err {err:.3e}")
     assert err <= 1e-5
+
+
+@pytest.mark.parametrize("kernel", ["fp32", "mfma", "mfma_f16x3"])
+@pytest.mark.parametrize("n", [45, 63, 129, 511, 1_026, 4_099, 20_001])
+def test_sweep_ragged_rows_and_short_runs(alma, kernel, n):
+    """Rows whose starts are not 16-byte aligned, and workgroup runs of 2 to 16
+    tiles: a launch that shortens its runs gives the bits of a packed launch,
+    which does not.  Bars a hundred times higher sit where runs of 2, 4 and 8
+    tiles end, so an anchor that saw another window would change the outputs."""
+    from vectorta_amd import autotune as at
+    x = datagen.gbm_close(n, 0.015, seed=n)
+    x[63::128] *= np.float32(100.0)
+    x[:2] = np.nan
+    sw = vta.AlmaBatchRange(period=(3, 40, 1), offset=(0.85, 0.85, 0.0), sigma=(6.0, 6.0, 0.0))
+    C = len(_combos(sw))
+    ctx = alma.ctx
+    dx, out, own = ctx.to_device(x), ctx.alloc(C * n * 4), ctx.alloc(C * n * 4)
+    pack = vta.AlmaPack(ctx, [{"prices": dx, "out": out, "sweep": sw, "series_len": n,
+                               "first_valid": 2}], kernel=kernel)
+    at.set_tuning(ctx, at.ALMA_MFMA_VARIANT, 9)
+    plan = alma.sweep_plan(sw, n, kernel=kernel)
+    pack.launch()
+    plan.launch(dx.ptr, 2, own.ptr)
+    ctx.synchronize()
+    at.set_tuning(ctx, at.ALMA_MFMA_VARIANT, 0)
+    g, r = (b.copy_to_host().reshape(C, n) for b in (own, out))
+    assert np.array_equal(g.view(np.uint32), r.view(np.uint32))
+    ref = O.alma_batch(x.astype(np.float64), _combos(sw))
+    plan.launch(dx.ptr, 2, own.ptr)              # the built-in form for this size
+    ctx.synchronize()
+    for got in (g, own.copy_to_host().reshape(C, n)):
+        nan_mask_equal(got, ref)
+        # weights sum to 1 and the split sees |x - anchor| <= half the range, so
+        # the dropped lo * lo and the two residuals are at most 3 * 2^-16 of that
+        # (bf16; half precision and FP32 stay below it)
+        assert_close(got, ref, rtol=5e-6, atol=3 * 2.0 ** -16 * float(np.nanmax(x)) / 2,
+                     what=f"{kernel} {n}")
+    plan.close()
+    pack.close()
+    for b in (dx, out, own):
+        b.free()

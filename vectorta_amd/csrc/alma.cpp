@@ -221,8 +221,10 @@ struct alma_sw_args_host {
     int n_tiles;
     int kmax;
     int group_base;
+    int run;
+    int pad_;
 };
-static_assert(sizeof(alma_sw_args_host) == 96, "alma_sw_args layout");
+static_assert(sizeof(alma_sw_args_host) == 104, "alma_sw_args layout");
 
 struct vta_alma_sweep_plan {
     size_t series_len = 0;
@@ -242,11 +244,28 @@ bool mf_shared_staging() {
 }
 constexpr size_t kMfMaxPeriod = 256;
 
-// Diagonal-form sweep kernels (alma_sweep_*): tiles per workgroup run, and the
+// Diagonal-form sweep kernels (alma_sweep_*): most tiles per workgroup run, and the
 // variant the F16 form runs by default (direct stores: 299 us against 311 us
 // for the transposed stores on the 200,000 x 1,250 sweep at sustained clocks).
 constexpr int kSweepRunTiles = 16;
 constexpr int kSweepDefaultVariant = 9;
+
+// Tiles per workgroup of a diagonal-form launch.  A run is serial (its weights
+// are read once for all its tiles), and two workgroups fit a CU: a launch
+// halves its runs until it has kSweepBlocks workgroups.  Whole calls in us at
+// runs of 16 / 8 / 4 tiles (workgroups at 16), F16 form:
+//   10,000 bars x 380 (60)        36.5 / 27.1 / 16.6 (12.3 at 2)
+//   41,117 bars x 380 (243)       36.9 / 31.2 / 26.1
+//   20,001 bars x 1,140 (360)     40.6 / 34.4 / 35.6
+//   100,001 bars x 380 (588)      53.8 / 52.9 / 61.0
+//   200,003 bars x 1,050 (3,519)   279 /  292 /  357
+constexpr size_t kSweepBlocks = 640;
+int sweep_run(int n_tiles, int n_groups, int rs) {
+    int run = kSweepRunTiles;
+    while (run > rs && (size_t)((n_tiles + run - 1) / run) * (size_t)n_groups < kSweepBlocks)
+        run /= 2;
+    return run;
+}
 
 int mfg_stride_host(int npair) { return ((npair + 15) >> 5) * 32 + 16; }
 
@@ -546,7 +565,8 @@ vta_status tables_launch(vta_ctx *ctx, const AlmaTables &t, const unsigned char 
         hipFunction_t fn;
         VTA_TRY(get_function(ctx, "alma", kNames[f16 ? 1 : 0][variant - 8], &fn));
         ctx->alma_selected = t.kernel;
-        const unsigned gx = (unsigned)((a.n_tiles + kSweepRunTiles - 1) / kSweepRunTiles);
+        a.run = sweep_run(a.n_tiles, t.n_groups, rs);
+        const unsigned gx = (unsigned)((a.n_tiles + a.run - 1) / a.run);
         return launch(ctx, fn, dim3(gx, (unsigned)t.n_groups, 1), dim3(256), (unsigned)smem, a);
     }
     const bool shared = variant == 0 ? mf_shared_staging() : variant <= 4;
@@ -858,6 +878,7 @@ vta_status alma_pack_build(vta_ctx *ctx, vta_alma_batch_kernel kernel,
             a.n_tiles = (int)((T + 31) / 32);
             a.kmax = t.kmax;
             a.group_base = 0;
+            a.run = kSweepRunTiles;
             memcpy(img.records.data() + j * rec, &a, sizeof a);
             const int32_t *grp =
                 reinterpret_cast<const int32_t *>(t.blob.data() + t.off[AlmaTables::GROUPS]);

@@ -72,7 +72,7 @@ __device__ __forceinline__ void alma_f32_tile(const float *__restrict__ prices,
     const int block_bad = __syncthreads_or(bad);
 
     const int tl = tid * 4;
-    const bool vec_ok = ((series_len & 3) == 0) && (t0 + tl + 3 < series_len);
+    const bool vec_ok = t0 + tl + 3 < series_len;
     for (int cc = 0; cc < ALMA_CB; ++cc) {
         const int c = c0 + cc;
         if (c >= n_combos) break;
@@ -117,7 +117,7 @@ __device__ __forceinline__ void alma_f32_tile(const float *__restrict__ prices,
         float r3 = (t + 3 >= warm) ? a3 : VTA_QNAN_F32;
         float *row = out + (size_t)c * series_len;
         if (vec_ok) {
-            *reinterpret_cast<float4 *>(row + t) = make_float4(r0, r1, r2, r3);
+            *reinterpret_cast<vta_row4 *>(row + t) = vta_row4{r0, r1, r2, r3};
         } else {
             if (t + 0 < series_len) row[t + 0] = r0;
             if (t + 1 < series_len) row[t + 1] = r1;
@@ -485,8 +485,8 @@ __device__ __forceinline__ void alma_mf_wave(const alma_mf_args &a, int nb, int 
                     }
                     v[i] = (t >= my_warm) ? val : VTA_QNAN_F32;
                 }
-                if (((T & 3) == 0) && tb + 3 < T) {
-                    *reinterpret_cast<float4 *>(row + tb) = make_float4(v[0], v[1], v[2], v[3]);
+                if (tb + 3 < T) {
+                    *reinterpret_cast<vta_row4 *>(row + tb) = vta_row4{v[0], v[1], v[2], v[3]};
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -629,7 +629,7 @@ __device__ __forceinline__ void alma_mfg_wave(const alma_mfg_args &a, int nb, in
         if (j + 1 < nt) load_a(j + 1, 0, ah_n, al_n);
         const float anchor = anch[j];
         const int t_tile = (tile_begin + j) * 32;
-        if (badf[j] == 0 && t_tile >= warm_max && t_tile + 32 <= T && (T & 3) == 0) {
+        if (badf[j] == 0 && t_tile >= warm_max && t_tile + 32 <= T) {
             // steady state (wave-uniform): every bar of the tile is a finite
             // output; transpose through LDS, then whole-line stores
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -648,8 +648,8 @@ __device__ __forceinline__ void alma_mfg_wave(const alma_mfg_args &a, int nb, in
                 const float4 v =
                     *reinterpret_cast<const float4 *>(tbuf + ((lane >> 3) + 8 * s) * 36 + tcol);
                 if (trow[s] >= 0)
-                    *reinterpret_cast<float4 *>(a.out + (size_t)trow[s] * (size_t)T + t_tile +
-                                                tcol) = v;
+                    *reinterpret_cast<vta_row4 *>(a.out + (size_t)trow[s] * (size_t)T + t_tile +
+                                                  tcol) = vta_row4{v.x, v.y, v.z, v.w};
             }
             continue;
         }
@@ -673,8 +673,8 @@ __device__ __forceinline__ void alma_mfg_wave(const alma_mfg_args &a, int nb, in
                 }
                 v[i] = (t >= my_warm) ? val : VTA_QNAN_F32;
             }
-            if (((T & 3) == 0) && tb + 3 < T) {
-                *reinterpret_cast<float4 *>(row + tb) = make_float4(v[0], v[1], v[2], v[3]);
+            if (tb + 3 < T) {
+                *reinterpret_cast<vta_row4 *>(row + tb) = vta_row4{v[0], v[1], v[2], v[3]};
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -728,13 +728,13 @@ __device__ __forceinline__ void alma_mfg_wave2(const alma_mfg_args &a, int nb, i
     auto epilogue = [&](const vta_f32x16 &acc, int j) {
         const float anchor = anch[j];
         const int t_tile = (tile_begin + j) * 32;
-        if (badf[j] == 0 && t_tile >= warm_max && t_tile + 32 <= T && (T & 3) == 0) {
+        if (badf[j] == 0 && t_tile >= warm_max && t_tile + 32 <= T) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int tb = t_tile + 8 * q + 4 * g;
-                *reinterpret_cast<float4 *>(row + tb) =
-                    make_float4(acc[4 * q + 0] + anchor, acc[4 * q + 1] + anchor,
-                                acc[4 * q + 2] + anchor, acc[4 * q + 3] + anchor);
+                *reinterpret_cast<vta_row4 *>(row + tb) =
+                    vta_row4{acc[4 * q + 0] + anchor, acc[4 * q + 1] + anchor,
+                             acc[4 * q + 2] + anchor, acc[4 * q + 3] + anchor};
             }
             return;
         }
@@ -756,8 +756,8 @@ __device__ __forceinline__ void alma_mfg_wave2(const alma_mfg_args &a, int nb, i
                 }
                 v[i] = (t >= my_warm) ? val : VTA_QNAN_F32;
             }
-            if (((T & 3) == 0) && tb + 3 < T) {
-                *reinterpret_cast<float4 *>(row + tb) = make_float4(v[0], v[1], v[2], v[3]);
+            if (tb + 3 < T) {
+                *reinterpret_cast<vta_row4 *>(row + tb) = vta_row4{v[0], v[1], v[2], v[3]};
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -1004,6 +1004,8 @@ struct alma_sw_args {
     int n_tiles;
     int kmax;
     int group_base;
+    int run;                     // tiles per workgroup: 16, 8, 4 or 2 (a multiple of RS)
+    int pad_;
 };
 
 // dwords per staged array of a sub-run of RS tiles: kg/2 + 16 RS pairs, padded
@@ -1087,7 +1089,7 @@ __device__ __forceinline__ void sw_epilogue(const alma_sw_args &a, const vta_f32
     bool redo = tile_bad;
     if (F16 && !redo) redo = sw_guard_violated(y, cguard * unscale, t_tile, g, my_row, my_warm,
                                                warm_max, T);
-    const bool steady = !redo && t_tile >= warm_max && t_tile + 32 <= T && (T & 3) == 0;
+    const bool steady = !redo && t_tile >= warm_max && t_tile + 32 <= T;
     if (steady && XPOSE) {
         // transpose through the wave's LDS tile: each store instruction then
         // writes 8 combos x 128 contiguous bytes
@@ -1107,8 +1109,8 @@ __device__ __forceinline__ void sw_epilogue(const alma_sw_args &a, const vta_f32
             const float4 v =
                 *reinterpret_cast<const float4 *>(tbuf + ((lane >> 3) + 8 * s) * 36 + tcol);
             if (trow[s] >= 0)
-                *reinterpret_cast<float4 *>(a.out + (size_t)trow[s] * (size_t)T + t_tile + tcol) =
-                    v;
+                *reinterpret_cast<vta_row4 *>(a.out + (size_t)trow[s] * (size_t)T + t_tile + tcol) =
+                    vta_row4{v.x, v.y, v.z, v.w};
         }
         return;
     }
@@ -1117,8 +1119,8 @@ __device__ __forceinline__ void sw_epilogue(const alma_sw_args &a, const vta_f32
     if (steady) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<float4 *>(row + t_tile + 8 * q + 4 * g) =
-                make_float4(y[4 * q + 0], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]);
+            *reinterpret_cast<vta_row4 *>(row + t_tile + 8 * q + 4 * g) =
+                vta_row4{y[4 * q + 0], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
         return;
     }
 #pragma unroll
@@ -1139,8 +1141,8 @@ __device__ __forceinline__ void sw_epilogue(const alma_sw_args &a, const vta_f32
             }
             v[i] = (t >= my_warm) ? val : VTA_QNAN_F32;
         }
-        if (((T & 3) == 0) && tb + 3 < T) {
-            *reinterpret_cast<float4 *>(row + tb) = make_float4(v[0], v[1], v[2], v[3]);
+        if (tb + 3 < T) {
+            *reinterpret_cast<vta_row4 *>(row + tb) = vta_row4{v[0], v[1], v[2], v[3]};
         } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -1389,7 +1391,7 @@ __device__ __forceinline__ void sw_wave(const alma_sw_args &a, int nb, int tile_
     }
 }
 
-// grid.x = runs of SW_R tiles, grid.y = N-block groups (heaviest first);
+// grid.x = runs of a.run <= SW_R tiles, grid.y = N-block groups (heaviest first);
 // block = 256 (4 waves).  Dynamic LDS, in floats: xs (32 SW_R + kmax + 33
 // prices), 3 per sub-run (anchor, scale, unscale), SW_R tile flags, 3 x 32
 // block statistics, then SW_NSUB x 4 x sw_stride(kmax) staged dwords (16-byte
@@ -1417,10 +1419,14 @@ __device__ __forceinline__ void alma_sw_entry(const alma_sw_args &a, int run, in
                   wave * (DEFER ? RS : 1) * 32 * 36;
     const int T = a.series_len;
     const int fv = a.first_valid;
-    const int tile_begin = run * SW_R;
-    const int nt = min(SW_R, a.n_tiles - tile_begin);
+    const int tile_begin = run * a.run;
+    const int nt = min(a.run, a.n_tiles - tile_begin);
     const int t_lo = tile_begin * 32 - kg + 1;      // xs index 0
-    const int nx = nt * 32 + kg + 1;
+    // the last window's bars; a run that ends inside a span of SW_R tiles takes
+    // the rest of their 32-bar statistics block too, as a longer run has it,
+    // so the anchors (and every output) are the same for each run length
+    const bool inside = (tile_begin + nt) % SW_R != 0 && tile_begin + nt < a.n_tiles;
+    const int nx = nt * 32 + kg + (inside ? 32 : 1);
     for (int i = tid; i < nx; i += 256) {
         const int idx = t_lo + i;
         const float x = vta_ld_clamped(a.prices, idx, fv, T);

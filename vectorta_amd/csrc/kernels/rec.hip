@@ -1616,13 +1616,12 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
         if (EMIT) {
             // eight rows x 128 bytes per store
             wave_lds_sync();
-            typedef float row4 __attribute__((ext_vector_type(4), aligned(4)));
             if (tb + 32 <= c1) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
                     if (8 * i + (lane >> 3) < nrow)
-                        *reinterpret_cast<row4 *>(row0 + (size_t)(8 * i) * a.T + tb) =
-                            *reinterpret_cast<const row4 *>(src + 8 * i * REC_ROW);
+                        *reinterpret_cast<vta_row4 *>(row0 + (size_t)(8 * i) * a.T + tb) =
+                            *reinterpret_cast<const vta_row4 *>(src + 8 * i * REC_ROW);
             } else {
                 for (int i = 0; i < 8; ++i)
                     for (int u = 0; u < 4; ++u)
