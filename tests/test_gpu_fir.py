@@ -123,6 +123,48 @@ def test_many_series(ops, name):
         _check(g, ref, f"{name} many-series p={p}")
 
 
+@pytest.mark.parametrize("n,longest", [(1_025, 255), (3_001, 1_023), (9_000, 1_700),
+                                       (70_001, 90)])
+def test_device_batch_prefix_runs_and_replays(ops, n, longest):
+    """A thread's run of staged bars from one to past the eight it keeps in
+    registers, one to all of the 64 searchers for the first non-finite bar, and
+    a captured call replayed over other data in the same buffer: a bar that is
+    not finite, none, and one elsewhere, each against the oracle."""
+    lead = 3
+    for name, p0 in (("sma", 1), ("wma", 2), ("swma", 1)):
+        op = ops[name]
+        ps = np.unique(np.linspace(p0, longest, 9).astype(np.int32))
+        base = datagen.gbm_close(n, 0.01, seed=n)
+        base[:lead] = np.nan
+        d_x, d_p = op.ctx.to_device(base), op.ctx.to_device(ps)
+        d_w = op.ctx.to_device((lead + ps - 1).astype(np.int32))
+        d_o = op.ctx.alloc(ps.size * n * 4)
+
+        def call():
+            if name == "swma":
+                op.swma_batch_device(d_x, d_p, d_w, n, ps.size, int(ps.max()), d_o)
+            else:
+                getattr(op, f"{name}_batch_device")(d_x, d_p, n, ps.size, lead, int(ps.max()), d_o)
+        call()
+        op.synchronize()
+        op.ctx.begin_capture()
+        call()
+        graph = op.ctx.end_capture()
+        for bad in (None, n - 1, None, n // 2, lead + 1):
+            x = base.copy()
+            if bad is not None:
+                x[bad] = np.nan
+            check(vta.lib().vta_memcpy_htod(op.ctx.handle, ctypes.c_void_p(d_x.ptr),
+                                            x.ctypes.data_as(ctypes.c_void_p), x.nbytes))
+            graph.launch()
+            op.synchronize()
+            got = d_o.copy_to_host(np.float32).reshape(ps.size, n)
+            _check(got, _batch_oracle(name, x, ps), f"{name} n={n} bad={bad}")
+        graph.destroy()
+        for b in (d_x, d_p, d_w, d_o):
+            b.free()
+
+
 def test_device_entry_points(ops):
     """Enqueue-only forms on device-resident inputs, with the reference
     wrappers' argument lists, equal the host-input forms."""

@@ -17,7 +17,8 @@ namespace {
 struct fir_args_host {
     const float *x;
     const int32_t *periods;
-    const int32_t *meta;
+    const int32_t *fvp;
+    const int32_t *zparts;
     const int32_t *fvs;
     const int32_t *zs;
     float *out;
@@ -30,25 +31,40 @@ struct fir_args_host {
     int period;
     int group;
     int ring;
+    int fv;
+    int nparts;
     int pad_;
 };
-static_assert(sizeof(fir_args_host) == 88, "fir_args layout");
+static_assert(sizeof(fir_args_host) == 104, "fir_args layout");
+
+// Blocks that look for the first non-finite bar (one wave reads their finds).
+constexpr int64_t kZParts = 64;
 
 enum Fir { FIR_SMA = 0, FIR_WMA = 1, FIR_SWMA = 2 };
 
 // Combos per workgroup of the batch kernel (the context's VTA_TUNE_FIR_GROUP
 // knob, else VTA_FIR_GROUP, 1..256).
-// Measured on 1,250 periods x 200k bars: 64 per workgroup amortise the tile's
-// prefix scan best (SMA 0.24 ms vs 0.30 ms at 16).  Lane groups of four bars
-// with 16-byte stores were 5-15% slower than one 4-byte store per lane (their
-// strided LDS reads conflict) and were dropped.
-unsigned fir_group(const vta_ctx *ctx) {
+// The tile's prefixes are formed once per workgroup: 64 combos share them where
+// there are two arrays, 16 where there is one (SMA; the shorter groups' rows
+// then lie closer together), and a launch of few tiles takes fewer, down to
+// one, for at least kBatchBlocks workgroups.  Whole calls in us at 16 / 32 / 64:
+//   1,250 WMA x 200,000 bars     261 / 218 / 212
+//   1,250 SWMA x 200,000         313 / 260 / 238
+//   1,250 SMA x 200,000          198 / 208 / 209
+//   1,000 SMA x 150,001          156 / 163 / 175
+//   300 SWMA x 50,001           27.0 / 31.7 / 46.4   (14 by the rule: 27.5)
+//   33 WMA x 10,007             13.9 / 20.6 / 21.0   (1: 8.1)
+// Lane groups of four bars with 16-byte stores were 5-15% slower than one
+// 4-byte store per lane (their strided LDS reads conflict).
+constexpr size_t kBatchBlocks = 1024;
+unsigned fir_group(const vta_ctx *ctx, Fir k, size_t tiles, size_t C) {
     if (ctx->tune[VTA_TUNE_FIR_GROUP] > 0) return (unsigned)ctx->tune[VTA_TUNE_FIR_GROUP];
     if (const char *e = getenv("VTA_FIR_GROUP")) {
         long v = atol(e);
         if (v >= 1 && v <= 256) return (unsigned)v;
     }
-    return 64;
+    return (unsigned)std::min<size_t>(k == FIR_SMA ? 16 : 64,
+                                      std::max<size_t>(1, C * tiles / kBatchBlocks));
 }
 
 // Grids: SMA sma.rs:705-755 (expand_grid_sma), WMA wma_wrapper.rs:324-350
@@ -81,7 +97,7 @@ vta_status check_period(Fir k, size_t p, size_t len, size_t fv) {
 // the longest period would leave fewer than two workgroups per CU (then 512,
 // 256); the LDS holds (tile + max_p + 2) doubles per prefix array.
 vta_status batch_launch(vta_ctx *ctx, Fir k, const float *d_x, const int32_t *d_periods,
-                        const int32_t *d_meta, size_t T, size_t C, size_t max_p, float *d_out) {
+                        const int32_t *d_fv, int fv, const int32_t *d_zparts, int nparts, size_t T, size_t C, size_t max_p, float *d_out) {
     const size_t narr = k == FIR_SMA ? 1 : 2;
     const size_t limit = ctx->props.sharedMemPerBlock;
     size_t tile = 1024, smem = 0;
@@ -98,14 +114,17 @@ vta_status batch_launch(vta_ctx *ctx, Fir k, const float *d_x, const int32_t *d_
     fir_args_host a{};
     a.x = d_x;
     a.periods = d_periods;
-    a.meta = d_meta;
+    a.fvp = d_fv;
+    a.fv = fv;
+    a.zparts = d_zparts;
+    a.nparts = nparts;
     a.out = d_out;
     a.T = (int)T;
     a.nlanes = (int)C;
     a.kind = (int)k;
     a.tile = (int)tile;
     a.span_cap = (int)(tile + max_p + 1);
-    const unsigned group = fir_group(ctx);
+    const unsigned group = fir_group(ctx, k, (T + tile - 1) / tile, C);
     a.group = (int)group;
     unsigned gx = (unsigned)((T + tile - 1) / tile);
     unsigned gy = (unsigned)((C + group - 1) / group);
@@ -200,8 +219,8 @@ vta_status batch_dev(vta_ctx *ctx, Fir k, const float *x, size_t len,
     VTA_TRY(upload(ctx, dp, per.data(), C * sizeof(int32_t)));
     VTA_TRY(upload(ctx, dm, meta, sizeof(meta)));
     VTA_TRY(dout.alloc(n_out));
-    VTA_TRY(batch_launch(ctx, k, dx.as<float>(), dp.as<int32_t>(), dm.as<int32_t>(), len, C,
-                         max_p, dout.as<float>()));
+    VTA_TRY(batch_launch(ctx, k, dx.as<float>(), dp.as<int32_t>(), nullptr, meta[0],
+                         dm.as<int32_t>() + 1, 1, len, C, max_p, dout.as<float>()));
     VTA_HIP(hipStreamSynchronize(ctx->stream));
     out->ptr = static_cast<float *>(dout.release());
     out->rows = C;
@@ -227,26 +246,18 @@ vta_status batch_device(vta_ctx *ctx, Fir k, const float *d_x, const int32_t *d_
                     "series_len, n_combos must be positive, first_valid < series_len and "
                     "%zu <= max_period <= series_len - first_valid", min_period(k));
     int32_t *meta = static_cast<int32_t *>(ctx->scratch) + 192;
-    hipFunction_t fill;
-    VTA_TRY(get_function(ctx, "rec", "vta_fill_i32", &fill));
-    VTA_TRY(launch(ctx, fill, dim3(1), dim3(256), 0, meta + 1, 1, (int)series_len));
-    if (d_warms) {
+    int32_t *parts = meta + 16;
+    if (d_warms)
         VTA_TRY(check_warms_device(ctx, d_periods, d_warms, (int)n_combos, (int)series_len, -1,
                                    (int)max_period, meta));
-        hipFunction_t fnf;
-        VTA_TRY(get_function(ctx, "fir", "series_first_nonfinite_dfv", &fnf));
-        VTA_TRY(launch(ctx, fnf, dim3((unsigned)((series_len + 255) / 256)), dim3(256), 0, d_x,
-                       (int)series_len, (const int32_t *)meta, meta + 1));
-    } else {
-        hipFunction_t fnf;
-        VTA_TRY(get_function(ctx, "fir", "series_first_nonfinite", &fnf));
-        VTA_TRY(launch(ctx, fill, dim3(1), dim3(256), 0, meta, 1, (int)first_valid));
-        unsigned nb = (unsigned)((series_len - first_valid + 255) / 256);
-        VTA_TRY(launch(ctx, fnf, dim3(nb), dim3(256), 0, d_x, (int)series_len, (int)first_valid,
-                       meta + 1));
-    }
-    return batch_launch(ctx, k, d_x, d_periods, meta, (size_t)series_len, (size_t)n_combos,
-                        (size_t)max_period, d_out);
+    const int32_t *d_fv = d_warms ? meta : nullptr;
+    const unsigned nparts = (unsigned)std::min<int64_t>(kZParts, (series_len + 1023) / 1024);
+    hipFunction_t fnf;
+    VTA_TRY(get_function(ctx, "fir", "series_nonfinite_parts", &fnf));
+    VTA_TRY(launch(ctx, fnf, dim3(nparts), dim3(256), 0, d_x, (int)series_len, d_fv,
+                   (int)first_valid, parts));
+    return batch_launch(ctx, k, d_x, d_periods, d_fv, (int)first_valid, parts, (int)nparts,
+                        (size_t)series_len, (size_t)n_combos, (size_t)max_period, d_out);
 }
 
 // sma_batch_dev_from_device (sma_wrapper.rs:830-860): device prices, host

@@ -3,8 +3,8 @@
 // One series x many periods (fir_batch_f32).  A workgroup owns a tile of
 // consecutive bars [t0, t0 + tile) and a group of consecutive combos.  It stages
 // the tile plus the group's look-back once and turns it into two local f64
-// prefix sums in LDS (block scan: wave scan by shuffles, wave totals through
-// LDS), with the local index i of bar s0 + i:
+// prefix sums in LDS (each thread a run of bars, the runs' totals scanned by
+// shuffles and wave totals through LDS), with the local index i of bar s0 + i:
 //   A[i+1] = sum_{i' <= i} x[s0 + i'],   B[i+1] = sum_{i' <= i} i' * x[s0 + i']
 // (bars before first_valid count as 0, like the reference's batch prefixes).
 // Every output is then O(1) differences of prefixes (Lt = A index of bar t):
@@ -16,7 +16,10 @@
 //            C[k] = k A[k] - B[k] (the prefix of the prefix), times 1/(a b).
 // Local prefixes keep the magnitudes at (tile + period) bars instead of the
 // whole series, so the differences lose ~eps * (tile + p)^k / p^k, far below
-// f32 rounding; the kernel is bound by the coalesced row stores.
+// f32 rounding; the kernel is bound by the coalesced row stores: 1,250 WMA x
+// 200k bars (1.0 GB) take 206 us (4.9 TB/s); 231 with a block scan and two
+// barriers per 256 staged bars, which every workgroup waits out before its
+// first store, and the periods read one after another.
 //
 // Many series x one period, time-major (fir_ms1p_{sma,wma,swma}_f32): one lane per series,
 // one wave per (64 series, time chunk).  Each chunk replays the reference's
@@ -39,7 +42,9 @@
 struct fir_args {
     const float *x;           // batch: [T]; many-series: [T][N] time-major
     const int32_t *periods;   // batch: per combo
-    const int32_t *meta;      // batch: [0] first_valid, [1] first non-finite bar (T if none)
+    const int32_t *fvp;       // batch: first_valid on the device, or null (fv)
+    const int32_t *zparts;    // batch: nparts (<= 64) candidates, the least of which is the
+                              // first non-finite bar (T if none)
     const int32_t *fvs;       // many-series: per series first_valid
     const int32_t *zs;        // many-series: per series first non-finite bar, or null
     float *out;
@@ -52,6 +57,8 @@ struct fir_args {
     int period;               // many-series
     int group;                // batch: combos per workgroup (<= FIR_GMAX)
     int ring;                 // many-series: rows of the LDS ring (>= longest lag + 8), 0 = none
+    int fv;                   // batch
+    int nparts;               // batch
     int pad_;
 };
 
@@ -80,15 +87,22 @@ extern "C" __global__ __launch_bounds__(256) void fir_batch_f32(fir_args a) {
     const int t0 = blockIdx.x * a.tile;
     const int c0 = blockIdx.y * a.group;
     const int nc = min(a.group, a.nlanes - c0);
-    const int fv = a.meta[0];
-    const int z = a.meta[1];
-    int pg = 1;
-    bool bad = false;
-    for (int j = 0; j < nc; ++j) {
+    const int fv = a.fvp ? a.fvp[0] : a.fv;
+    int z = lane < a.nparts ? a.zparts[lane] : T;
+    for (int o = 32; o > 0; o >>= 1) z = min(z, __shfl_xor(z, o));
+    z = __builtin_amdgcn_readfirstlane(z);
+    int pg = 1, pmin = 1;                        // (each wave looks at all of them)
+    for (int j = lane; j < nc; j += 64) {
         const int p = a.periods[c0 + j];
         pg = max(pg, p);
-        bad = bad || p < 1;
+        pmin = min(pmin, p);
     }
+    for (int o = 32; o > 0; o >>= 1) {
+        pg = max(pg, __shfl_xor(pg, o));
+        pmin = min(pmin, __shfl_xor(pmin, o));
+    }
+    pg = __builtin_amdgcn_readfirstlane(pg);
+    const bool bad = __builtin_amdgcn_readfirstlane(pmin) < 1;
     const int tend = min(t0 + a.tile, T);
     if (bad || pg > a.span_cap - a.tile - 1) {
         // a period outside [1, max_period] (device-side input of the enqueue
@@ -117,48 +131,71 @@ extern "C" __global__ __launch_bounds__(256) void fir_batch_f32(fir_args a) {
     double *B = lds + a.span_cap + 1;
     const bool wantB = a.kind != 0;
 
-    // ---- local prefix sums A, B over the staged bars
-    double carA = 0.0, carB = 0.0;
+    // ---- local prefix sums A, B over the staged bars: a thread sums its own
+    // run of bars, the threads' totals are scanned, and the thread walks its
+    // run again from its start value (one barrier for the whole tile)
+    const int per = (span + 255) / 256;
+    const int i0 = min(tid * per, span), i1 = min(i0 + per, span);
+    auto bar = [&](int i) -> double {
+        const int t = s0 + i;
+        return t >= fv && t < T ? (double)a.x[t] : 0.0;
+    };
+    double first[8];                             // (all at once)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) first[k] = i0 + k < i1 ? bar(i0 + k) : 0.0;
+    double sa = 0.0, sb = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        sa += first[k];
+        sb += (double)(i0 + k) * first[k];
+    }
+    for (int i = i0 + 8; i < i1; ++i) {
+        const double v = bar(i);
+        sa += v;
+        sb += (double)i * v;
+    }
+    double pa = sa, pb = sb;                     // inclusive over the wave's threads
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const double ya = __shfl_up(pa, o);
+        const double yb = __shfl_up(pb, o);
+        if (lane >= o) {
+            pa += ya;
+            pb += yb;
+        }
+    }
+    if (lane == 63) {
+        wtot[0][w] = pa;
+        wtot[1][w] = pb;
+    }
     if (tid == 0) {
         A[0] = 0.0;
         if (wantB) B[0] = 0.0;
     }
-    for (int base = 0; base < span; base += 256) {
-        const int i = base + tid;
-        const int t = s0 + i;
-        double xv = 0.0;
-        if (i < span && t >= fv && t < T) xv = (double)a.x[t];
-        double sa = xv;
-        double sb = (double)i * xv;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const double ya = __shfl_up(sa, o);
-            const double yb = __shfl_up(sb, o);
-            if (lane >= o) {
-                sa += ya;
-                sb += yb;
-            }
-        }
-        if (lane == 63) {
-            wtot[0][w] = sa;
-            wtot[1][w] = sb;
-        }
-        __syncthreads();
-        double oa = carA, ob = carB;
-        for (int k = 0; k < w; ++k) {
-            oa += wtot[0][k];
-            ob += wtot[1][k];
-        }
-        if (i < span) {
-            A[i + 1] = oa + sa;
-            if (wantB) B[i + 1] = ob + sb;
-        }
-        for (int k = 0; k < 4; ++k) {
-            carA += wtot[0][k];
-            carB += wtot[1][k];
-        }
-        __syncthreads();
+    double ea = __shfl_up(pa, 1), eb = __shfl_up(pb, 1);
+    if (lane == 0) ea = eb = 0.0;
+    __syncthreads();
+    for (int k = 0; k < w; ++k) {
+        ea += wtot[0][k];
+        eb += wtot[1][k];
     }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        ea += first[k];
+        eb += (double)(i0 + k) * first[k];
+        if (i0 + k < i1) {
+            A[i0 + k + 1] = ea;
+            if (wantB) B[i0 + k + 1] = eb;
+        }
+    }
+    for (int i = i0 + 8; i < i1; ++i) {
+        const double v = bar(i);
+        ea += v;
+        eb += (double)i * v;
+        A[i + 1] = ea;
+        if (wantB) B[i + 1] = eb;
+    }
+    __syncthreads();
 
     // SWMA reads only C[k] = k A[k] - B[k] (the prefix of the prefix) and A:
     // fold C into the B array once per tile
@@ -428,21 +465,20 @@ extern "C" __global__ __launch_bounds__(64) void fir_ms1p_sma_f32(fir_args a) { 
 extern "C" __global__ __launch_bounds__(64) void fir_ms1p_wma_f32(fir_args a) { fir_ms1p<1, 8>(a); }
 extern "C" __global__ __launch_bounds__(64) void fir_ms1p_swma_f32(fir_args a) { fir_ms1p<2, 16>(a); }
 
-// Single series: the first bar at or after first_valid whose value is not
-// finite.  z[0] must hold T on entry (vta_fill_i32).
-// The same with first_valid read from the device (*fvp, in [0, T]): grid over
-// the whole series.
-extern "C" __global__ __launch_bounds__(256) void series_first_nonfinite_dfv(
-    const float *__restrict__ x, int T, const int32_t *__restrict__ fvp,
-    int32_t *__restrict__ z) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= T || t < fvp[0]) return;
-    if (!vta_isfinite(x[t])) atomicMin(z, t);
-}
-
-extern "C" __global__ __launch_bounds__(256) void series_first_nonfinite(
-    const float *__restrict__ x, int T, int first_valid, int32_t *__restrict__ z) {
-    const int t = blockIdx.x * 256 + threadIdx.x + first_valid;
-    if (t >= T) return;
-    if (!vta_isfinite(x[t])) atomicMin(z, t);
+// Single series: every block's first bar at or after first_valid (*fvp, or fv)
+// whose value is not finite, T if it sees none; the batch kernel takes the
+// least of the up to 64 of them, so no word has to be set beforehand.
+extern "C" __global__ __launch_bounds__(256) void series_nonfinite_parts(
+    const float *__restrict__ x, int T, const int32_t *__restrict__ fvp, int fv,
+    int32_t *__restrict__ parts) {
+    __shared__ int least[4];
+    const int from = fvp ? fvp[0] : fv;
+    int z = T;
+    for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < T; t += (long)gridDim.x * 256)
+        if (t >= from && !vta_isfinite(x[t])) z = min(z, (int)t);
+    for (int o = 32; o > 0; o >>= 1) z = min(z, __shfl_xor(z, o));
+    if ((threadIdx.x & 63) == 0) least[threadIdx.x >> 6] = z;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        parts[blockIdx.x] = min(min(least[0], least[1]), min(least[2], least[3]));
 }

@@ -410,8 +410,7 @@ vta_status vta_ctx_preload(vta_ctx *ctx) {
         {"fir", "fir_ms1p_sma_f32"},
         {"fir", "fir_ms1p_wma_f32"},
         {"fir", "fir_ms1p_swma_f32"},
-        {"fir", "series_first_nonfinite"},
-        {"fir", "series_first_nonfinite_dfv"},
+        {"fir", "series_nonfinite_parts"},
         {"rec", "ms_ema_rsi_atr_f32"},
         {"rec", "ms_prepare_meta"},
         {"rec", "vta_fill_i32"},
