@@ -168,6 +168,28 @@ def test_scan_series_past_the_term_buffer(ctxs, name, n):
     _scan_case(ctxs, name, n, (14, 64, 50))
 
 
+@pytest.mark.parametrize("n,combos", [(120_001, 560), (120_031, 565), (61_042, 1_100), (900_019, 75)])
+@pytest.mark.parametrize("name", ["ema", "rsi", "atr", "adx"])
+def test_scan_rows_off_the_lines(ctxs, name, n, combos):
+    """Outputs of 256 MiB and more whose rows start anywhere in a 128-byte line:
+    chunks store whole lines and run into the next chunk for the last one.  The
+    first and last rows equal the oracle's; the first also those of a shorter
+    sweep, which stores tile by tile (in other chunks, so within two f32 ulps of
+    100).  900,019 bars take several segments for RSI and ADX."""
+    h, lo, c = _hlc(n, 90 + combos, lead=2)
+    op, a = ctxs[name], (h, lo, c) if name in ("atr", "adx") else (c,)
+    run = getattr(op, f"{name}_batch_dev")
+    g = run(*a, (2, 1 + combos, 1)).to_host()
+    assert g.nbytes >= 256 << 20 and n % 32
+    some = 12
+    part = run(*a, (2, 1 + some, 1)).to_host()
+    f = [v.astype(np.float64) for v in a]
+    _check(g[:some], getattr(O, f"{name}_batch")(*f, list(range(2, 2 + some))), name)
+    _check(g[-2:], getattr(O, f"{name}_batch")(*f, [combos, combos + 1]), name)
+    nan_mask_equal(g[:some], part)
+    assert max_rel_err(g[:some], part.astype(np.float64), floor=1e-3) <= 2e-6
+
+
 def test_wilders_seeded_matches_replay(monkeypatch):
     """Wilders batches of up to 4,096 combos start each exact lane from a
     per-combo seed at its last warm-up bar; larger ones replay the warm-up

@@ -61,6 +61,8 @@ struct rec_args {
     int tstride;
     int scan;                // batch: 0 burn-in / exact lanes, else the scan (ADX: stage 1 or 2)
     int clean_epoch;         // batch: the word scan_prepare stores in clean[0], [1]
+    int rag;                 // batch scan: whole lines of rows that start anywhere (scan_output)
+    int pad_;
 };
 
 #define REC_NAN __builtin_bit_cast(double, 0x7ff8000000000000ull)
@@ -857,7 +859,7 @@ struct batch_view {
     double *state_out;
     int T, nlanes, chunk, nch, groups, span, fv, t0, t1, tstride, scan, group;
     int kb, k;               // the block's first chunk, this wave's
-    bool clean, odd, coop;
+    bool clean, odd, coop, rag;
 };
 
 // A block is REC_WPB waves: with that many combo groups, one chunk of as many
@@ -909,6 +911,7 @@ __device__ __forceinline__ batch_view view_of(const rec_args &a) {
     block_chunk(v, blockIdx.x);
     v.clean = a.clean != nullptr && a.clean[0] != a.clean_epoch;
     v.odd = a.clean != nullptr && a.clean[1] == a.clean_epoch;
+    v.rag = a.rag != 0;
     return v;
 }
 
@@ -1477,14 +1480,23 @@ __device__ __forceinline__ float scan_dx(double diff, double all) {
 // A chunk from its exact start state: the outputs (EMIT), or ADX's second
 // stage from zero for its scan.  Blocks of 32 bars past every sum run the
 // plain updates, eight terms at a time; the others select per bar.
-template <class E, bool ODD, bool EMIT>
+//
+// RAG (rows that do not all start on a 128-byte line): a wave keeps its last
+// two tiles of 32 bars and stores whole lines only, those that start in its
+// chunk; for the last of them it runs one tile into the next chunk.  Stored
+// tile by tile, each line of such rows is written in two parts some
+// microseconds apart, more of them open at once than the L2 holds: 1,250 EMA x
+// 180,001 bars 466 us, 266 with whole lines (180,000 bars: 220).
+template <class E, bool ODD, bool EMIT, bool RAG = false>
 __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
     constexpr bool EMA = __is_same(E, EmaEng), RSI = __is_same(E, RsiEng),
                    ADX = __is_same(E, AdxEng);
     constexpr int N = ADX && !ODD ? 2 : scan_dims<E>::N;
     constexpr int S = scan_dims<E>::S;
     extern __shared__ __align__(16) double rec_lds[];
-    float *ob = EMIT ? reinterpret_cast<float *>(wave_lds<E>()) : nullptr;   // [64][REC_ROW]
+    float *ob = nullptr;                             // [64][REC_ROW], RAG [64][64]
+    if (RAG) ob = reinterpret_cast<float *>(rec_lds) + block_wave() * 64 * 64;
+    else if (EMIT) ob = reinterpret_cast<float *>(wave_lds<E>());
     const int lane = threadIdx.x & 63;
     const int c = a.group * 64 + lane;
     const size_t cp = (size_t)a.groups * 64;
@@ -1501,8 +1513,43 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
     const int nrow = min(64, a.nlanes - a.group * 64);
     float *row0 = out + (size_t)(a.group * 64 + (lane >> 3)) * a.T + 4 * (lane & 7);
     const float *src = ob + (lane >> 3) * REC_ROW + 4 * (lane & 7);
-    for (int tb = c0; tb < c1; tb += 32) {
-        float *dst = ob + lane * REC_ROW;
+    const bool end = c1 == a.t1;
+    // RAG: bars 4 j of row r sit at columns 4 j ^ 4 (r mod 16) of its two tiles
+    // (a wave's float4 writes then fall on all banks)
+    auto place = [&](int tb, int b) -> float4 * {
+        return reinterpret_cast<float4 *>(
+            RAG ? ob + lane * 64 + (((tb & 32) + b) ^ (4 * (lane & 15))) : ob + lane * REC_ROW + b);
+    };
+    // ... and stores, of each row, the line that bar tb lies in: the tile
+    // before tb and the one at tb hold it
+    auto lines = [&](int tb) {
+        const int lim = min(end ? c1 : c1 + 32, a.t1);
+        const uint32_t base = (uint32_t)(reinterpret_cast<uintptr_t>(out) >> 2);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = 8 * i + (lane >> 3);
+            const uint32_t at = base + (uint32_t)(a.group * 64 + r) * (uint32_t)a.T + (uint32_t)tb;
+            const int line = tb - (int)(at & 31);
+            const int t = line + 4 * (lane & 7), x = 4 * (r & 15);
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = ob[r * 64 + (((t + u) & 63) ^ x)];
+            // the line is this chunk's if it starts in it; a first chunk also
+            // takes the part of the one before that lies in it
+            const bool own = line >= c0 ? line < c1 : c0 == a.t0;
+            if (r >= nrow || !own) continue;
+            float *o = out + (size_t)(a.group * 64 + r) * a.T;
+            if (line >= c0 && line + 32 <= lim) {
+                *reinterpret_cast<vta_row4 *>(o + t) = vta_row4{v[0], v[1], v[2], v[3]};
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (t + u >= c0 && t + u < lim) o[t + u] = v[u];
+            }
+        }
+    };
+    int tb = c0;
+    for (; tb < (RAG && !end ? c1 + 32 : c1); tb += 32) {
         if (tb > last) {
 #pragma unroll
             for (int b = 0; b < 32; b += 4) {
@@ -1565,7 +1612,7 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
                         }
                     }
                     if (EMIT)
-                        *reinterpret_cast<float4 *>(dst + b) = make_float4(y[0], y[1], y[2], y[3]);
+                        *place(tb, b) = make_float4(y[0], y[1], y[2], y[3]);
                 }
             }
         } else {
@@ -1606,7 +1653,7 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
                     y[u] = t >= q.first ? (float)v : VTA_QNAN_F32;
                 }
                 if (EMIT)
-                    *reinterpret_cast<float4 *>(dst + b) = make_float4(y[0], y[1], y[2], y[3]);
+                    *place(tb, b) = make_float4(y[0], y[1], y[2], y[3]);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -1616,7 +1663,9 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
         if (EMIT) {
             // eight rows x 128 bytes per store
             wave_lds_sync();
-            if (tb + 32 <= c1) {
+            if (RAG) {
+                lines(tb);
+            } else if (tb + 32 <= c1) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
                     if (8 * i + (lane >> 3) < nrow)
@@ -1631,6 +1680,7 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
             wave_lds_sync();
         }
     }
+    if (RAG && end) lines(tb);
     if (EMIT) {
         if (a.state_out && a.k == a.nch - 1) {
 #pragma unroll
@@ -1696,7 +1746,10 @@ __device__ __forceinline__ void batch_pass(batch_view a, float *out) {
         a.chunk = a.T;
         drive_batch<E, NIN>(a, out);
     } else if (__is_same(E, AdxEng) && a.odd) {
-        scan_output<E, true, true>(a, out);
+        if (a.rag) scan_output<E, true, true, true>(a, out);
+        else scan_output<E, true, true>(a, out);
+    } else if (a.rag) {
+        scan_output<E, false, true, true>(a, out);
     } else {
         scan_output<E, false, true>(a, out);
     }
@@ -1774,6 +1827,7 @@ __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     v.scan = v.nch > 1 ? p.scan : 0;                 // one chunk: exact lanes
     v.clean = p.flags[2 * j] != p.epoch;
     v.odd = p.flags[2 * j + 1] == p.epoch;
+    v.rag = false;
     v.group = v.kb = v.k = 0;
     v.coop = false;
     return v;

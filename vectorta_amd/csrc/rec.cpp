@@ -44,8 +44,10 @@ struct rec_args_host {
     int tstride;
     int scan;
     int clean_epoch;
+    int rag;
+    int pad_;
 };
-static_assert(sizeof(rec_args_host) == 184, "rec_args layout");
+static_assert(sizeof(rec_args_host) == 192, "rec_args layout");
 
 enum Ind {
     IND_EMA = 0,
@@ -296,6 +298,24 @@ vta_status prepare_launch(vta_ctx *ctx, Ind k, const rec_args_host &a, size_t t0
                   meta, a.periods, d_warms, a.nlanes, meta + kArgErrorWord);
 }
 
+// Rows that do not all start on a 128-byte line: from kRagBytes of rows on,
+// what the memory-side cache holds, the output pass stores whole lines
+// (scan_output's RAG form).  Below that the cache puts half lines together and
+// the extra tile per chunk costs more.  Whole calls in us, tiles / lines:
+//   300 EMA x 50,001 bars (60 MB)      39.9 / 49.2
+//   600 EMA x 50,001 (120 MB)          58.1 / 64.2
+//   1,200 ADX x 30,001 (144 MB)         136 /  157
+//   400 RSI x 180,001 (288 MB)          194 /  156
+//   400 ADX x 180,001 (288 MB)          267 /  258
+//   700 EMA x 180,004 (504 MB)          257 /  167
+//   1,250 EMA x 180,001 (900 MB)        466 /  266
+constexpr unsigned kRagLds = 64 * 64 * sizeof(float);
+constexpr size_t kRagBytes = 256u << 20;
+bool ragged_rows(const rec_args_host &a) {
+    return (a.T % 32 != 0 || reinterpret_cast<uintptr_t>(a.out0) % 128 != 0) &&
+           (size_t)a.T * (size_t)a.nlanes * sizeof(float) >= kRagBytes;
+}
+
 // `a` holds the inputs, outputs, flags and sizes; chunk from scan_chunk.
 vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
                        const int32_t *d_warms) {
@@ -311,6 +331,7 @@ vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
     a.carry = seg < T ? handed[1] + row : handed[0];
     a.terms = ctx->terms;
     a.chunk = (int)chunk;
+    a.rag = ragged_rows(a);
     for (size_t t0 = 0, n = 0; t0 < T; t0 += seg, ++n) {
         const size_t t1 = std::min(T, t0 + seg);
         const size_t nch = (t1 - t0 + chunk - 1) / chunk;
@@ -339,7 +360,7 @@ vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
             }
         }
         a.scan = 1;
-        VTA_TRY(launch(ctx, fb, grid, block, batch_lds_bytes(k), a));
+        VTA_TRY(launch(ctx, fb, grid, block, a.rag ? kWpb * kRagLds : batch_lds_bytes(k), a));
     }
     return VTA_OK;
 }
