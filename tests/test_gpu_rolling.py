@@ -460,6 +460,18 @@ def test_pnr_window_forms_many_series(ops, monkeypatch, chunk):
         _same_bits(outs[1], outs[2], f"pnr forms len {length}")
 
 
+def test_pnr_every_register_capacity(ops):
+    """The register kernels of every four slots, with full and part-filled last
+    slots: the same bits as the LDS form (which other tests hold to the oracle)."""
+    rows, cols = 700, 70
+    x = _ragged_panel(rows, cols, seed=94, quant=0.05)
+    pnr = ops["pnr"]
+    for length in [n for cap in range(4, 129, 4) for n in (cap - 3, cap)]:
+        g = [_with_form(pnr.ctx, form, lambda: pnr.pnr_many_series_one_param_time_major_dev(
+            x, cols, rows, length, 70.0).to_host()) for form in (1, 2)]
+        _same_bits(g[0], g[1], f"pnr forms len {length}")
+
+
 @pytest.mark.parametrize("chunk", [None, "160"])
 def test_mad_window_forms_many_series(ops, monkeypatch, chunk):
     """Many-series MAD in the register form (capacities 16..64, even and odd

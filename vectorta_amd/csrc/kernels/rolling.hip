@@ -929,7 +929,7 @@ template <int N> struct RwVecD { typedef double v __attribute__((ext_vector_type
 // over every slot.
 template <int CAP>
 struct RegWin {
-    static_assert(CAP % 16 == 0, "register window capacity");
+    static_assert(CAP % 2 == 0, "register window capacity");
     typename RwVecF<CAP / 2>::v e, o;
     __device__ __forceinline__ float get(int p) const {
         return p >= CAP ? INFINITY : (p & 1) ? o[p >> 1] : e[p >> 1];
@@ -1276,7 +1276,7 @@ __device__ __forceinline__ float rw_mad(const RegWin<CAP> &w, int len) {
 // selection as rw_mad.
 template <int LEN>
 struct MadLen {
-    static constexpr int CAP = (LEN + 15) / 16 * 16;
+    static constexpr int CAP = (LEN + 1) / 2 * 2;
     static constexpr int NP = rw_pow2(LEN);
     static constexpr int MID = LEN >> 1;
     static constexpr bool ODD = (LEN & 1) != 0;
@@ -1363,7 +1363,12 @@ __device__ __forceinline__ void mad_reg_body(const roll_args &a) {
     extern "C" __global__ __launch_bounds__(64, 2) void mad_ms1p_reg##CAP(roll_args a) {   \
         mad_reg_body<CAP>(a);                                                              \
     }
-RW_PNR(16) RW_PNR(32) RW_PNR(48) RW_PNR(64) RW_PNR(80) RW_PNR(96) RW_PNR(112) RW_PNR(128)
+// One kernel per four slots, a step's cost being its slots: BB + PNR 100 + MAD 64
+// on 1,024 x 50,000 take 1,539 us, 1,598 with PNR's 100 keys in 112 slots.
+RW_PNR(4) RW_PNR(8) RW_PNR(12) RW_PNR(16) RW_PNR(20) RW_PNR(24) RW_PNR(28) RW_PNR(32)
+RW_PNR(36) RW_PNR(40) RW_PNR(44) RW_PNR(48) RW_PNR(52) RW_PNR(56) RW_PNR(60) RW_PNR(64)
+RW_PNR(68) RW_PNR(72) RW_PNR(76) RW_PNR(80) RW_PNR(84) RW_PNR(88) RW_PNR(92) RW_PNR(96)
+RW_PNR(100) RW_PNR(104) RW_PNR(108) RW_PNR(112) RW_PNR(116) RW_PNR(120) RW_PNR(124) RW_PNR(128)
 // periods 1-3 (the length-templated kernels below start at 4)
 RW_MAD(16)
 #define RW_MAD_LEN(L)                                                                      \

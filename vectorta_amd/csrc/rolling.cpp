@@ -83,14 +83,15 @@ const char *kname(RInd k, bool batch) {
     return batch ? b[k] : m[k];
 }
 
-// Register-window capacity (the window length rounded up to 16 slots) of the
+// Register-window capacity (the window length rounded up to 4 slots, PNR) of the
 // many-series PNR / MAD kernels, 0 when the LDS form runs: the knob's choice,
 // else the register form wherever a kernel exists (PNR up to 128 slots, MAD
 // up to 64: a longer MAD window's f64 deviation paths no longer fit the
 // VGPRs beside the window).
 int reg_window_cap(const vta_ctx *ctx, RInd k, size_t len) {
     if (k == R_BB || ctx->tune[VTA_TUNE_ROLL_FORM] == 1) return 0;
-    const size_t cap = (len + 15) / 16 * 16;
+    const size_t unit = k == R_PNR ? 4 : 16;
+    const size_t cap = (len + unit - 1) / unit * unit;
     if (cap == 0 || cap > (k == R_PNR ? 128u : 64u)) return 0;
     return (int)cap;
 }

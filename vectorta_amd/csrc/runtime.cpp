@@ -435,10 +435,10 @@ vta_status vta_ctx_preload(vta_ctx *ctx) {
         hipFunction_t f;
         VTA_TRY(get_function(ctx, s[0], s[1], &f));
     }
-    // register-window PNR kernels (16..128 slots) and MAD kernels per period
+    // register-window PNR kernels (4..128 slots) and MAD kernels per period
     // (4..64)
     char name[32];
-    for (int cap = 16; cap <= 128; cap += 16) {
+    for (int cap = 4; cap <= 128; cap += 4) {
         hipFunction_t f;
         snprintf(name, sizeof name, "pnr_ms1p_reg%d", cap);
         VTA_TRY(get_function(ctx, "rolling", name, &f));
