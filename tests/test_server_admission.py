@@ -1,0 +1,45 @@
+"""Admission of the request server under a full memory budget, on the CPU: the
+library's host sources are compiled with AddressSanitizer and linked with a
+device-less HIP runtime (tests/native), and each scenario runs in a process
+of its own."""
+import os
+import subprocess
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+from tests.conftest import ROOT
+
+NATIVE = os.path.join(ROOT, "tests", "native")
+CSRC = os.path.join(ROOT, "vectorta_amd", "csrc")
+ROCM = os.environ.get("ROCM", "/opt/rocm")
+SOURCES = ["runtime", "alma", "rec", "rolling", "cross", "fir", "server", "dlpack", "graph", "tune"]
+
+
+@pytest.fixture(scope="session")
+def program(tmp_path_factory):
+    out = tmp_path_factory.mktemp("native")
+    flags = ["-O1", "-g", "-std=c++17", "-pthread", "-fsanitize=address", "-D__HIP_PLATFORM_AMD__",
+             f"-I{ROCM}/include", f"-I{ROOT}/include", f"-I{CSRC}", f"-I{NATIVE}"]
+
+    def compile_one(src):
+        obj = str(out / (os.path.basename(src) + ".o"))
+        subprocess.run(["g++", *flags, "-c", src, "-o", obj], check=True)
+        return obj
+
+    srcs = [os.path.join(CSRC, s + ".cpp") for s in SOURCES]
+    srcs += [os.path.join(NATIVE, s) for s in ("fake_hip.cpp", "server_admission.cpp")]
+    with ThreadPoolExecutor(4) as pool:
+        objs = list(pool.map(compile_one, srcs))
+    exe = str(out / "server_admission")
+    subprocess.run(["g++", "-fsanitize=address", "-pthread", *objs, "-o", exe, "-ldl"], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("scenario", ["hit_evicts_another", "hit_never_fits", "hit_served_as_miss",
+                                      "hit_waits_for_release", "pack_of_hits"])
+def test_admission(program, scenario):
+    # (another preloaded library may come before the sanitizer's)
+    env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")
+    r = subprocess.run([program, scenario], env=env, capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr

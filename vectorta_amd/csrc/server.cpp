@@ -216,44 +216,58 @@ size_t grid_outputs(const vta_request &r, size_t *n_combos, int *n_out) {
     }
 }
 
+// Evicts the cached series `e` if no request uses it.
+bool evict_entry(vta_server *s, const std::shared_ptr<CacheEntry> &e) {
+    if (e->refs > 0 || !e->ready) return false;
+    s->pending_free.push_back(e->d_close);
+    if (e->d_high) s->pending_free.push_back(e->d_high);
+    if (e->d_low) s->pending_free.push_back(e->d_low);
+    s->in_use -= e->bytes;
+    s->lru.erase(e->lru);
+    s->cache.erase(e->key);
+    return true;
+}
+
 void evict_lru(vta_server *s, size_t need) {
-    auto it = s->lru.begin();
-    while (s->in_use + need > s->budget && it != s->lru.end()) {
-        auto e = s->cache.find(*it);
-        if (e == s->cache.end() || e->second->refs > 0 || !e->second->ready) {
-            ++it;
-            continue;
-        }
-        std::shared_ptr<CacheEntry> ent = e->second;
-        s->pending_free.push_back(ent->d_close);
-        if (ent->d_high) s->pending_free.push_back(ent->d_high);
-        if (ent->d_low) s->pending_free.push_back(ent->d_low);
-        s->in_use -= ent->bytes;
-        s->cache.erase(e);
-        it = s->lru.erase(it);
+    for (auto it = s->lru.begin(); s->in_use + need > s->budget && it != s->lru.end();) {
+        const std::shared_ptr<CacheEntry> e = s->cache.at(*it);
+        ++it;                               // (eviction removes e's place in the list)
+        evict_entry(s, e);
     }
 }
 
 // Called with s->mu held: admits the queued request at `it` if the HBM budget
 // holds its outputs (and its series, on a cache miss), evicting cached series
-// if needed.  Returns it (removed from the queue) or null.
+// if needed -- never the one it hits, which it holds meanwhile.  Outputs that
+// the budget cannot hold beside that series make it a miss, once nothing else
+// uses the series.  Returns the request (removed from the queue) or null.
 std::shared_ptr<Req> admit_at(vta_server *s, std::deque<std::shared_ptr<Req>>::iterator it) {
     std::shared_ptr<Req> q = *it;
-    auto hit = q->r.series_key ? s->cache.find(q->r.series_key) : s->cache.end();
-    const bool is_hit = hit != s->cache.end();
-    const size_t series = is_hit ? 0 : q->series_bytes;
+    std::shared_ptr<CacheEntry> hit;
+    if (q->r.series_key) {
+        auto f = s->cache.find(q->r.series_key);
+        if (f != s->cache.end()) hit = f->second;
+    }
+    if (hit && q->out_bytes + hit->bytes > s->budget) {
+        if (!evict_entry(s, hit)) return nullptr;
+        hit.reset();
+    }
+    const size_t series = hit ? 0 : q->series_bytes;
     const size_t need = q->out_bytes + series;
+    if (hit) hit->refs += 1;
     if (s->in_use + need > s->budget) evict_lru(s, need);
-    if (s->in_use + need > s->budget) return nullptr;
+    if (s->in_use + need > s->budget) {
+        if (hit) hit->refs -= 1;
+        return nullptr;
+    }
     s->queue.erase(it);
     s->in_use += need;
     s->peak_in_use = std::max(s->peak_in_use, s->in_use);
     q->series_reserved = series;
-    q->uploader = !is_hit;
-    if (is_hit) {
-        q->entry = hit->second;
-        q->entry->refs += 1;
-        s->lru.splice(s->lru.end(), s->lru, q->entry->lru);   // most recently used
+    q->uploader = !hit;
+    if (hit) {
+        q->entry = hit;
+        s->lru.splice(s->lru.end(), s->lru, hit->lru);   // most recently used
     } else {
         auto e = std::make_shared<CacheEntry>();
         e->key = q->r.series_key;
@@ -275,8 +289,10 @@ std::shared_ptr<Req> admit_at(vta_server *s, std::deque<std::shared_ptr<Req>>::i
 std::shared_ptr<Req> try_admit(vta_server *s) {
     while (!s->queue.empty()) {
         std::shared_ptr<Req> q = s->queue.front();
-        const bool is_hit = q->r.series_key && s->cache.count(q->r.series_key);
-        if (q->out_bytes + (is_hit ? 0 : q->series_bytes) > s->budget) {
+        auto f = q->r.series_key ? s->cache.find(q->r.series_key) : s->cache.end();
+        const size_t hit_bytes = f != s->cache.end() ? f->second->bytes : SIZE_MAX;
+        if (q->out_bytes > s->budget ||
+            std::min(q->series_bytes, hit_bytes) > s->budget - q->out_bytes) {
             // can never fit: fail it now (nothing was reserved for it)
             s->queue.pop_front();
             q->out_bytes = 0;
