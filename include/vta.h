@@ -849,8 +849,10 @@ vta_status vta_double_alma_plan_destroy(vta_double_alma_plan *plan);
  * worker threads, each with its own context and stream on device_id, take
  * one-series batch requests from a FIFO queue; a request is admitted when a
  * slot is free and hbm_budget bytes hold its outputs plus, on a series-cache
- * miss, its series.  Results stay on the device (counted against the budget)
- * until vta_server_release.  Series are cached under the client's key
+ * miss, its series, each in one piece (between results of other sizes a
+ * request that the budget holds may have to wait for neighbours' release).
+ * Results stay on the device (counted against the budget) until
+ * vta_server_release.  Series are cached under the client's key
  * (series_key != 0 and cache = 1), evicted least-recently-used when admission
  * needs room; a request always carries its host data, used on a miss.  Results
  * are the library's batch kernels on the same inputs: identical whether a

@@ -144,6 +144,27 @@ void pack_of_hits() {
     CHECK(v.stats().queued == 0);
 }
 
+// Free memory in pieces between results that the client holds: a request that
+// the budget holds, but no piece, waits for its neighbours' release.
+void fragmented_arena() {
+    constexpr size_t kSmall = 5, kN = 128;               // 2 MB results
+    constexpr size_t kLarge = 300;                       // (the arena's end holds 208 rows)
+    Server v(kN * kSmall + 1);
+    std::vector<uint64_t> ids;
+    for (size_t i = 0; i < kN; ++i) ids.push_back(v.submit(1, kSmall));
+    for (const uint64_t id : ids) CHECK(v.wait(id) == VTA_OK);
+    for (size_t i = 0; i < kN; i += 2) CHECK(vta_server_release(v.s, ids[i]) == VTA_OK);
+    CHECK(v.stats().in_use + kLarge * kRow <= v.stats().budget);
+    const uint64_t id = v.submit(1, kLarge);
+    vta_result res{};
+    CHECK(vta_server_wait(v.s, id, 300, &res) == VTA_ERR_TIMEOUT);
+    CHECK(v.stats().queued == 1);
+    for (size_t i = 1; i < kN; i += 2) CHECK(vta_server_release(v.s, ids[i]) == VTA_OK);
+    CHECK(v.wait(id) == VTA_OK);
+    CHECK(vta_server_release(v.s, id) == VTA_OK);
+    CHECK(v.stats().in_use <= kRow);
+}
+
 const struct {
     const char *name;
     void (*run)();
@@ -151,7 +172,8 @@ const struct {
                   {"hit_never_fits", hit_never_fits},
                   {"hit_served_as_miss", hit_served_as_miss},
                   {"hit_waits_for_release", hit_waits_for_release},
-                  {"pack_of_hits", pack_of_hits}};
+                  {"pack_of_hits", pack_of_hits},
+                  {"fragmented_arena", fragmented_arena}};
 
 }  // namespace
 

@@ -37,7 +37,8 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["hit_evicts_another", "hit_never_fits", "hit_served_as_miss",
-                                      "hit_waits_for_release", "pack_of_hits"])
+                                      "hit_waits_for_release", "pack_of_hits",
+                                      "fragmented_arena"])
 def test_admission(program, scenario):
     # (another preloaded library may come before the sanitizer's)
     env = dict(os.environ, ASAN_OPTIONS="verify_asan_link_order=0:detect_leaks=0")

@@ -8,7 +8,10 @@
 // outputs plus, on a cache miss, its series upload; outputs stay reserved
 // until the client releases them.  Series live in a device cache keyed by the
 // client's 64-bit key; unreferenced entries are evicted least-recently-used
-// when admission needs room.  The kernels are the library's public entry
+// when admission needs room.  A request's outputs and series are placed in the
+// device memory as it is admitted: the budget counts bytes, and with results
+// of all sizes between the free ones a request that it holds may still find no
+// block long enough, and then waits for one like for the budget.  The kernels are the library's public entry
 // points, so a result is bit-identical whether the request runs alone or in
 // a mix.
 #include <algorithm>
@@ -62,6 +65,8 @@ struct Req {
     vta_request r{};
     std::vector<float> close, high, low;   // host copies
     SeriesMeta meta;
+    size_t n_combos = 0;
+    int n_out = 0;
     size_t out_bytes = 0;                  // reserved for outputs
     size_t series_bytes = 0;               // device bytes of the series
     size_t series_reserved = 0;            // reserved at admission (misses only)
@@ -171,7 +176,6 @@ struct vta_server {
     std::vector<vta_ctx *> ctxs;
     std::vector<std::thread> workers;
     Arena arena;                        // all served-path device memory
-    std::vector<void *> pending_free;   // collected under mu, returned after unlocking
     std::vector<float *> pinned;        // per-slot pinned staging for series uploads
     std::vector<size_t> pinned_cap;
     double t0 = 0.0;
@@ -216,71 +220,115 @@ size_t grid_outputs(const vta_request &r, size_t *n_combos, int *n_out) {
     }
 }
 
+void release_series(vta_server *s, CacheEntry &e) {
+    for (float **p : {&e.d_close, &e.d_high, &e.d_low}) {
+        s->arena.release(*p);
+        *p = nullptr;
+    }
+}
+
+void release_outputs(vta_server *s, vta_result &res) {
+    for (vta_device_array_f32 &o : res.out) {
+        s->arena.release(o.ptr);
+        o.ptr = nullptr;
+    }
+}
+
 // Evicts the cached series `e` if no request uses it.
 bool evict_entry(vta_server *s, const std::shared_ptr<CacheEntry> &e) {
     if (e->refs > 0 || !e->ready) return false;
-    s->pending_free.push_back(e->d_close);
-    if (e->d_high) s->pending_free.push_back(e->d_high);
-    if (e->d_low) s->pending_free.push_back(e->d_low);
+    release_series(s, *e);
     s->in_use -= e->bytes;
     s->lru.erase(e->lru);
     s->cache.erase(e->key);
     return true;
 }
 
-void evict_lru(vta_server *s, size_t need) {
-    for (auto it = s->lru.begin(); s->in_use + need > s->budget && it != s->lru.end();) {
-        const std::shared_ptr<CacheEntry> e = s->cache.at(*it);
-        ++it;                               // (eviction removes e's place in the list)
-        evict_entry(s, e);
+// Evicts the least recently used series that no request uses, if there is one.
+bool evict_one(vta_server *s) {
+    for (const uint64_t key : s->lru)
+        if (evict_entry(s, s->cache.at(key))) return true;
+    return false;
+}
+
+// Arena blocks of request q's outputs (into q.res) and, for a miss, of its
+// series (into e); false, with none taken, when one of them finds no room.
+bool place(vta_server *s, Req &q, CacheEntry &e, bool miss) {
+    bool ok = true;
+    auto take = [&](float **p, size_t floats) {
+        *p = ok ? static_cast<float *>(s->arena.alloc(floats * sizeof(float))) : nullptr;
+        ok = *p != nullptr;
+    };
+    for (int i = 0; i < q.n_out; ++i) {
+        take(&q.res.out[i].ptr, q.n_combos * e.meta.len);
+        q.res.out[i].rows = q.n_combos;
+        q.res.out[i].cols = e.meta.len;
     }
+    if (miss) {
+        take(&e.d_close, e.meta.len);
+        if (e.meta.hlc) {
+            take(&e.d_high, e.meta.len);
+            take(&e.d_low, e.meta.len);
+        }
+    }
+    if (ok) return true;
+    release_outputs(s, q.res);
+    if (miss) release_series(s, e);
+    return false;
 }
 
 // Called with s->mu held: admits the queued request at `it` if the HBM budget
-// holds its outputs (and its series, on a cache miss), evicting cached series
-// if needed -- never the one it hits, which it holds meanwhile.  Outputs that
-// the budget cannot hold beside that series make it a miss, once nothing else
-// uses the series.  Returns the request (removed from the queue) or null.
+// holds its outputs (and its series, on a cache miss) and they find room,
+// evicting cached series if needed -- not the one it hits, which it holds
+// meanwhile.  Outputs that the budget cannot hold beside that series, or that
+// find no room beside it, make it a miss, once nothing else uses the series.
+// Returns the request (removed from the queue) or null.
 std::shared_ptr<Req> admit_at(vta_server *s, std::deque<std::shared_ptr<Req>>::iterator it) {
     std::shared_ptr<Req> q = *it;
-    std::shared_ptr<CacheEntry> hit;
+    std::shared_ptr<CacheEntry> e;
+    bool hit = false;
     if (q->r.series_key) {
         auto f = s->cache.find(q->r.series_key);
-        if (f != s->cache.end()) hit = f->second;
+        hit = f != s->cache.end();
+        if (hit) e = f->second;
     }
-    if (hit && q->out_bytes + hit->bytes > s->budget) {
-        if (!evict_entry(s, hit)) return nullptr;
-        hit.reset();
+    if (hit && q->out_bytes + e->bytes > s->budget) {
+        if (!evict_entry(s, e)) return nullptr;
+        hit = false;
     }
-    const size_t series = hit ? 0 : q->series_bytes;
-    const size_t need = q->out_bytes + series;
-    if (hit) hit->refs += 1;
-    if (s->in_use + need > s->budget) evict_lru(s, need);
-    if (s->in_use + need > s->budget) {
-        if (hit) hit->refs -= 1;
-        return nullptr;
+    size_t need;
+    for (;;) {
+        need = q->out_bytes + (hit ? 0 : q->series_bytes);
+        if (!hit) {
+            e = std::make_shared<CacheEntry>();
+            e->key = q->r.series_key;
+            e->meta = q->meta;
+            e->bytes = q->series_bytes;
+            e->cached = q->r.cache && q->r.series_key != 0;
+        }
+        e->refs += 1;
+        while (s->in_use + need > s->budget && evict_one(s)) {
+        }
+        const bool fits = s->in_use + need <= s->budget;
+        bool placed = fits && place(s, *q, *e, !hit);
+        while (fits && !placed && evict_one(s)) placed = place(s, *q, *e, !hit);
+        if (placed) break;
+        e->refs -= 1;
+        if (!hit || !fits || !evict_entry(s, e)) return nullptr;
+        hit = false;
     }
     s->queue.erase(it);
     s->in_use += need;
     s->peak_in_use = std::max(s->peak_in_use, s->in_use);
-    q->series_reserved = series;
+    q->series_reserved = hit ? 0 : q->series_bytes;
     q->uploader = !hit;
+    q->entry = e;
     if (hit) {
-        q->entry = hit;
-        s->lru.splice(s->lru.end(), s->lru, hit->lru);   // most recently used
-    } else {
-        auto e = std::make_shared<CacheEntry>();
-        e->key = q->r.series_key;
-        e->meta = q->meta;
-        e->bytes = q->series_bytes;
-        e->refs = 1;
-        e->cached = q->r.cache && q->r.series_key != 0;
-        if (e->cached) {
-            s->lru.push_back(e->key);
-            e->lru = std::prev(s->lru.end());
-            s->cache.emplace(e->key, e);
-        }
-        q->entry = e;
+        s->lru.splice(s->lru.end(), s->lru, e->lru);   // most recently used
+    } else if (e->cached) {
+        s->lru.push_back(e->key);
+        e->lru = std::prev(s->lru.end());
+        s->cache.emplace(e->key, e);
     }
     return q;
 }
@@ -356,16 +404,8 @@ vta_status upload_series(vta_server *s, int slot, vta_ctx *ctx, Req &q) {
         std::memcpy(stage + q.meta.len, q.high.data(), n);
         std::memcpy(stage + 2 * q.meta.len, q.low.data(), n);
     }
-    e.d_close = static_cast<float *>(s->arena.alloc(n));
-    if (!e.d_close) return fail(VTA_ERR_OUT_OF_MEMORY, "device arena exhausted");
     VTA_HIP(hipMemcpyAsync(e.d_close, stage, n, hipMemcpyHostToDevice, ctx->stream));
     if (q.meta.hlc) {
-        e.d_high = static_cast<float *>(s->arena.alloc(n));
-        e.d_low = static_cast<float *>(s->arena.alloc(n));
-        if (!e.d_high || !e.d_low) {
-            (void)hipStreamSynchronize(ctx->stream);
-            return fail(VTA_ERR_OUT_OF_MEMORY, "device arena exhausted");
-        }
         VTA_HIP(hipMemcpyAsync(e.d_high, stage + q.meta.len, n, hipMemcpyHostToDevice,
                                ctx->stream));
         VTA_HIP(hipMemcpyAsync(e.d_low, stage + 2 * q.meta.len, n, hipMemcpyHostToDevice,
@@ -404,15 +444,6 @@ struct ArenaTable {
         return static_cast<T *>(p);
     }
 };
-
-vta_status alloc_out(vta_server *s, vta_device_array_f32 &o, size_t rows, size_t cols) {
-    void *p = s->arena.alloc(rows * cols * sizeof(float));
-    if (!p) return fail(VTA_ERR_OUT_OF_MEMORY, "device arena exhausted");
-    o.ptr = static_cast<float *>(p);
-    o.rows = rows;
-    o.cols = cols;
-    return VTA_OK;
-}
 
 // The grid's sweep plan, built on a miss outside plan_mu (the host table build
 // of a large grid takes milliseconds and must not hold up the other slots);
@@ -463,7 +494,6 @@ vta_status run_request(vta_server *s, vta_ctx *ctx, Req &q) {
                 return fail(VTA_ERR_INVALID_INPUT, "not enough valid data (needed >= %zu)", mp);
             res.n_outputs = 1;
             res.n_combos = nc;
-            VTA_TRY(alloc_out(s, res.out[0], nc, T));
             VTA_TRY(alma_grid_plan_launch(ctx, plan, e.d_close, T, (size_t)m.fv_close,
                                           res.out[0].ptr));
             res.t_launch = now_s() - t0;
@@ -497,7 +527,6 @@ vta_status run_request(vta_server *s, vta_ctx *ctx, Req &q) {
             VTA_TRY(dp.put(s, ctx, per));
             res.n_outputs = 1;
             res.n_combos = n;
-            VTA_TRY(alloc_out(s, res.out[0], n, T));
             if (r.kind == VTA_REQ_EMA)
                 VTA_TRY(vta_ema_batch_device(ctx, e.d_close, dp.as<int32_t>(), nullptr, T,
                                              (size_t)fv, n, res.out[0].ptr));
@@ -538,7 +567,6 @@ vta_status run_request(vta_server *s, vta_ctx *ctx, Req &q) {
             VTA_TRY(dd.put(s, ctx, dn));
             res.n_outputs = 3;
             res.n_combos = n;
-            for (int i = 0; i < 3; ++i) VTA_TRY(alloc_out(s, res.out[i], n, T));
             VTA_TRY(vta_bollinger_bands_batch_device(
                 ctx, e.d_close, (int32_t)T, m.fv_close, m.z_close, dp.as<int32_t>(),
                 du.as<double>(), dd.as<double>(), (int32_t)n, (int32_t)maxp, res.out[0].ptr,
@@ -552,26 +580,6 @@ vta_status run_request(vta_server *s, vta_ctx *ctx, Req &q) {
     }
 }
 
-// Moves the result's device pointers to `out` (freed later, outside mu).
-void take_outputs(vta_result &res, std::vector<void *> &out) {
-    for (int i = 0; i < 3; ++i)
-        if (res.out[i].ptr) {
-            out.push_back(res.out[i].ptr);
-            res.out[i].ptr = nullptr;
-        }
-}
-
-// Called without mu held: stream-ordered frees of everything collected.
-void flush_frees(vta_server *s, std::vector<void *> &mine) {
-    {
-        std::lock_guard<std::mutex> lk(s->mu);
-        mine.insert(mine.end(), s->pending_free.begin(), s->pending_free.end());
-        s->pending_free.clear();
-    }
-    for (void *p : mine) s->arena.release(p);
-    mine.clear();
-}
-
 // Uploads the request's series (its uploader) or waits until another slot
 // has (a cache hit or a concurrent miss on the same key).
 vta_status prepare_series(vta_server *s, int slot, vta_ctx *ctx, Req &q) {
@@ -582,10 +590,7 @@ vta_status prepare_series(vta_server *s, int slot, vta_ctx *ctx, Req &q) {
         std::lock_guard<std::mutex> lk(s->mu);
         if (st != VTA_OK) {
             (void)hipStreamSynchronize(ctx->stream);
-            if (e.d_close) s->pending_free.push_back(e.d_close);
-            if (e.d_high) s->pending_free.push_back(e.d_high);
-            if (e.d_low) s->pending_free.push_back(e.d_low);
-            e.d_close = e.d_high = e.d_low = nullptr;
+            release_series(s, e);
             if (e.cached) {
                 // drop the broken entry; its bytes go back with this request
                 s->cache.erase(e.key);
@@ -612,19 +617,14 @@ void finish_request(vta_server *s, vta_ctx *ctx, Req &q, vta_status st) {
     q.res.t_done = now_s() - s->t0;
     if (st != VTA_OK) {
         (void)hipStreamSynchronize(ctx->stream);
-        take_outputs(q.res, s->pending_free);
+        release_outputs(s, q.res);
         s->in_use -= q.out_bytes;
         q.out_bytes = 0;
     }
     e.refs -= 1;
     if (!e.cached) {
         // a one-off series, or an entry dropped after a failed upload
-        if (e.refs == 0) {
-            if (e.d_close) s->pending_free.push_back(e.d_close);
-            if (e.d_high) s->pending_free.push_back(e.d_high);
-            if (e.d_low) s->pending_free.push_back(e.d_low);
-            e.d_close = e.d_high = e.d_low = nullptr;
-        }
+        if (e.refs == 0) release_series(s, e);
         s->in_use -= q.series_reserved;
         q.series_reserved = 0;
     }
@@ -674,7 +674,6 @@ bool run_packed_bb(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>
                            : tables.back()->put(s, ctx, t == 1 ? ups[i] : dns[i]);
             }
         }
-        for (int o = 0; o < 3 && v == VTA_OK; ++o) v = alloc_out(s, q.res.out[o], n, T);
         if (v != VTA_OK) {
             st[i] = v;
             continue;
@@ -707,12 +706,6 @@ bool run_packed_bb(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>
         d_tab = s->arena.alloc(tab.size() * sizeof(BbPackJob));
         if (!d_tab) {
             (void)hipStreamSynchronize(ctx->stream);   // the parameter tables' copies
-            for (auto &q : g)
-                for (int o = 0; o < 3; ++o)
-                    if (q->res.out[o].ptr) {
-                        s->arena.release(q->res.out[o].ptr);
-                        q->res.out[o].ptr = nullptr;
-                    }
             return false;
         }
         hipError_t e = hipMemcpyAsync(d_tab, tab.data(), tab.size() * sizeof(BbPackJob),
@@ -770,11 +763,6 @@ bool run_packed_alma(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Re
             alone.push_back(i);
             continue;
         }
-        v = alloc_out(s, q.res.out[0], nc, T);
-        if (v != VTA_OK) {
-            st[i] = v;
-            continue;
-        }
         q.res.n_outputs = 1;
         q.res.n_combos = nc;
         src.push_back({&t, alma_plan_device(plan), e.d_close, q.res.out[0].ptr, T,
@@ -796,11 +784,7 @@ bool run_packed_alma(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Re
             for (void *p : {d_rec, d_items})
                 if (p) s->arena.release(p);
             d_rec = d_items = nullptr;
-            for (size_t i : member) {
-                s->arena.release(g[i]->res.out[0].ptr);
-                g[i]->res.out[0].ptr = nullptr;
-                alone.push_back(i);
-            }
+            alone.insert(alone.end(), member.begin(), member.end());
             member.clear();
             v = VTA_OK;
         }
@@ -874,7 +858,6 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
             tables.push_back(std::make_unique<ArenaTable>());
             v = tables.back()->put(s, ctx, pers[i]);
         }
-        if (v == VTA_OK) v = alloc_out(s, q.res.out[0], n, T);
         if (v != VTA_OK) {
             st[i] = v;
             continue;
@@ -908,11 +891,6 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
             for (void *p : {d_tab, d_work})
                 if (p) s->arena.release(p);
             (void)hipStreamSynchronize(ctx->stream);   // the period tables' copies
-            for (auto &q : g)
-                if (q->res.out[0].ptr) {
-                    s->arena.release(q->res.out[0].ptr);
-                    q->res.out[0].ptr = nullptr;
-                }
             return false;
         }
         pack_bind(dims, tab, static_cast<double *>(d_work));
@@ -941,7 +919,6 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
 void worker(vta_server *s, int slot) {
     vta_ctx *ctx = s->ctxs[slot];
     (void)hipSetDevice(s->device);
-    std::vector<void *> local_frees;
     for (;;) {
         std::vector<std::shared_ptr<Req>> g;
         {
@@ -966,7 +943,6 @@ void worker(vta_server *s, int slot) {
             s->in_flight += (int)g.size();
             s->peak_in_flight = std::max(s->peak_in_flight, s->in_flight);
         }
-        flush_frees(s, local_frees);   // evictions made room for these requests
         std::vector<vta_status> st(g.size(), VTA_OK);
         for (size_t i = 0; i < g.size(); ++i) st[i] = prepare_series(s, slot, ctx, *g[i]);
         bool done = false;
@@ -993,7 +969,6 @@ void worker(vta_server *s, int slot) {
                     st[i] = run_request(s, ctx, *g[i]);
                 }
         for (size_t i = 0; i < g.size(); ++i) finish_request(s, ctx, *g[i], st[i]);
-        flush_frees(s, local_frees);
     }
 }
 
@@ -1050,16 +1025,7 @@ vta_status vta_server_destroy(vta_server *s) {
     }
     for (auto &t : s->workers) t.join();
     (void)hipSetDevice(s->device);
-    std::vector<void *> frees;
-    for (auto &kv : s->reqs)
-        if (kv.second->done) take_outputs(kv.second->res, frees);
-    for (auto &kv : s->cache) {
-        frees.push_back(kv.second->d_close);
-        if (kv.second->d_high) frees.push_back(kv.second->d_high);
-        if (kv.second->d_low) frees.push_back(kv.second->d_low);
-    }
-    flush_frees(s, frees);
-    (void)hipDeviceSynchronize();
+    (void)hipDeviceSynchronize();   // (the arena goes with the server)
     for (auto &kv : s->alma_plans) alma_grid_plan_destroy(kv.second);
     for (float *p : s->pinned)
         if (p) (void)hipHostFree(p);
@@ -1094,9 +1060,7 @@ vta_status vta_server_submit(vta_server *s, const vta_request *r, uint64_t *req_
         size_t a = first_nan_end(q->high.data(), n), b = first_nan_end(q->low.data(), n);
         q->meta.fv_adx = (int32_t)std::max({a, b, fvc});
     }
-    size_t n_combos = 0;
-    int n_out = 1;
-    const size_t cells = grid_outputs(*r, &n_combos, &n_out);
+    const size_t cells = grid_outputs(*r, &q->n_combos, &q->n_out);
     if (cells == 0) return fail(VTA_ERR_INVALID_INPUT, "invalid parameter grid");
     if (!mul_ok(cells, n, &q->out_bytes) || !mul_ok(q->out_bytes, sizeof(float), &q->out_bytes))
         return fail(VTA_ERR_INVALID_INPUT, "output size overflow");
@@ -1132,21 +1096,16 @@ vta_status vta_server_wait(vta_server *s, uint64_t req_id, int timeout_ms, vta_r
 vta_status vta_server_release(vta_server *s, uint64_t req_id) {
     clear_error();
     if (!s) return fail(VTA_ERR_INVALID_INPUT, "null argument");
-    std::vector<void *> frees;
-    {
-        std::lock_guard<std::mutex> lk(s->mu);
-        auto it = s->reqs.find(req_id);
-        if (it == s->reqs.end()) return fail(VTA_ERR_INVALID_INPUT, "unknown request");
-        std::shared_ptr<Req> q = it->second;
-        if (!q->done) return fail(VTA_ERR_INVALID_INPUT, "request still running");
-        take_outputs(q->res, frees);
-        s->in_use -= q->out_bytes;
-        q->out_bytes = 0;
-        s->reqs.erase(it);
-        s->cv_admit.notify_all();
-    }
-    (void)hipSetDevice(s->device);
-    flush_frees(s, frees);
+    std::lock_guard<std::mutex> lk(s->mu);
+    auto it = s->reqs.find(req_id);
+    if (it == s->reqs.end()) return fail(VTA_ERR_INVALID_INPUT, "unknown request");
+    std::shared_ptr<Req> q = it->second;
+    if (!q->done) return fail(VTA_ERR_INVALID_INPUT, "request still running");
+    release_outputs(s, q->res);   // (before the admissions that it makes room for)
+    s->in_use -= q->out_bytes;
+    q->out_bytes = 0;
+    s->reqs.erase(it);
+    s->cv_admit.notify_all();
     return VTA_OK;
 }
 
