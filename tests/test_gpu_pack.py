@@ -139,6 +139,78 @@ def test_pack_matches_direct_calls(kind):
             b.free()
 
 
+# Jobs that their own calls run in further segments (terms past 8 MiB: EMA,
+# ATR, SMMA, Wilders above 1,048,576 bars, RSI half, ADX a third of that) or
+# store by whole lines (256 MiB of rows off the 128-byte lines), in groups of
+# 64 combos by fours and below; beside short ones.
+# (series_len, leading NaN, first and last period, interior non-finite bar)
+LONG = {"ema": [(1_100_003, 2, 5, 8, None), (120_001, 0, 2, 561, None), (3_000, 0, 2, 60, None)],
+        "rsi": [(600_001, 0, 14, 16, None), (700, 0, 14, 14, None), (900_019, 7, 2, 76, None),
+                (1_200_000, 3, 9, 9, 700_000), (524_288, 0, 5, 6, None)],
+        "atr": [(1_048_640, 1, 2, 6, None), (50, 0, 2, 4, None)],
+        "adx": [(400_003, 2, 14, 80, None), (9_000, 0, 2, 30, None), (720_001, 3, 2, 101, None),
+                (170_003, 0, 2, 460, None), (1_100_000, 0, 30, 31, 1_000_000)],
+        "smma": [(1_048_641, 5, 7, 9, None), (2_097_153, 0, 2_000, 2_001, None)],
+        "wilders": [(900_001, 0, 1, 80, None), (1_500_000, 9, 1, 3, None)]}
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_pack_of_long_series_matches_direct_calls(kind):
+    require_gpu()
+    ctx = vta.HipContext(0)
+    rng = np.random.Generator(np.random.PCG64(190 + KINDS.index(kind)))
+    jobs, bufs, host = [], [], []
+    for i, (T, lead, p0, p1, bad) in enumerate(LONG[kind]):
+        c = datagen.gbm_close(T, 0.001, seed=520 + i)
+        _, hi, lo, c = datagen.ohlc_from_close(c, rng)
+        for a in (hi, lo, c):
+            a[:lead] = np.nan
+        if bad is not None:
+            c[bad] = np.nan
+        periods = np.arange(p0, p1 + 1, dtype=np.int32)
+        C = int(periods.size)
+        d = {"c": ctx.to_device(c), "h": ctx.to_device(hi), "l": ctx.to_device(lo),
+             "p": ctx.to_device(periods), "out": ctx.alloc(C * T * 4),
+             "direct": ctx.alloc(C * T * 4),
+             "w": ctx.to_device((lead + periods - 1).astype(np.int32))}
+        job = {"close": d["c"], "periods": d["p"], "out": d["out"], "series_len": T,
+               "first_valid": lead, "n_combos": C, "max_period": p1}
+        if kind in HLC:
+            job["high"], job["low"] = d["h"], d["l"]
+        jobs.append(job)
+        bufs.append(d)
+        host.append((c, hi, lo, [int(p) for p in periods]))
+    pack = vta.RecPack(ctx, kind, jobs)
+    ctx.begin_capture()
+    pack.launch()
+    graph = ctx.end_capture()
+    for job, d in zip(jobs, bufs):
+        _direct(kind, ctx, d, job)
+    for launch in (pack.launch, graph.launch):
+        for d in bufs:
+            check(lib().vta_memcpy_htod(ctx.handle, P(d["out"].ptr),
+                                        np.full(d["out"].nbytes // 4, -3.0,
+                                                np.float32).ctypes.data_as(P), d["out"].nbytes))
+        launch()
+        ctx.synchronize()
+        for i, (job, d) in enumerate(zip(jobs, bufs)):
+            C, T = job["n_combos"], job["series_len"]
+            g = d["out"].copy_to_host(np.float32).reshape(C, T)
+            r = d["direct"].copy_to_host(np.float32).reshape(C, T)
+            assert np.array_equal(g.view(np.uint32), r.view(np.uint32)), (kind, i, LONG[kind][i])
+            c, hi, lo, periods = host[i]
+            some = sorted({0, C - 1})
+            ref = _oracle(kind, c, hi, lo, [periods[k] for k in some])
+            nan_mask_equal(g[some], ref)
+            err = max_rel_err(g[some], ref, floor=1e-3 if kind in ("rsi", "adx") else 0.0)
+            assert err <= 1e-5, (kind, i, err)
+    graph.destroy()
+    pack.close()
+    for d in bufs:
+        for b in d.values():
+            b.free()
+
+
 def test_pack_rejects_bad_jobs():
     require_gpu()
     ctx = vta.HipContext(0)

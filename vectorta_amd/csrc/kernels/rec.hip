@@ -1773,7 +1773,8 @@ __device__ __forceinline__ void span_pass(batch_view &a, int flat) {
 // the span folds are a 1-D grid likewise, from span0 on.  A block finds its
 // job by binary search over block0 (span0), then runs exactly
 // the block of that job's direct launch, so a job's outputs are bit-identical
-// alone and packed.
+// alone and packed.  A job that its own call runs in segments has an entry for
+// each, and the passes run for all first segments, then for all second ones.
 struct rec_job {
     const float *x, *h, *l;
     const int32_t *periods;
@@ -1782,9 +1783,17 @@ struct rec_job {
     double *terms;           // this job's [term][tstride]
     int T, nlanes, fv, chunk, nch, groups, block0, span0, tstride, span;
 };
+// Beside the table's entry, in a pack with segments: the entry's bars and job
+// (whose flags are its), the states as in rec_args.
+struct rec_seg {
+    const double *state_in;
+    double *state_out;
+    int t0, t1, job, pad_;
+};
 
 struct rec_pack_args {
     const rec_job *jobs;
+    const rec_seg *segs;
     const int32_t *flags;    // per job: [2 j] a non-finite bar, [2 j + 1] an odd one was met
                              // (the word equals epoch)
     int n_jobs;
@@ -1804,6 +1813,9 @@ __device__ __forceinline__ int pack_find(const rec_pack_args &p, int flat, bool 
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// (SEG: a pack with segments.  In others entry j is all of job j: what segments
+// need beyond that took 2 of the 71 us of 40 RSI series)
+template <bool SEG>
 __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     const rec_job &jb = p.jobs[j];
     batch_view v;
@@ -1812,8 +1824,8 @@ __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     v.alphas = nullptr;
     v.carry = jb.carry;
     v.terms = jb.terms;
-    v.state_in = nullptr;
-    v.state_out = nullptr;
+    v.state_in = SEG ? p.segs[j].state_in : nullptr;
+    v.state_out = SEG ? p.segs[j].state_out : nullptr;
     v.T = jb.T;
     v.nlanes = jb.nlanes;
     v.chunk = __builtin_amdgcn_readfirstlane(jb.chunk);
@@ -1821,33 +1833,35 @@ __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     v.groups = __builtin_amdgcn_readfirstlane(jb.groups);
     v.span = __builtin_amdgcn_readfirstlane(jb.span);
     v.fv = jb.fv;
-    v.t0 = 0;
-    v.t1 = __builtin_amdgcn_readfirstlane(jb.T);
+    v.t0 = SEG ? __builtin_amdgcn_readfirstlane(p.segs[j].t0) : 0;
+    v.t1 = __builtin_amdgcn_readfirstlane(SEG ? p.segs[j].t1 : jb.T);
     v.tstride = jb.tstride;
-    v.scan = v.nch > 1 ? p.scan : 0;                 // one chunk: exact lanes
-    v.clean = p.flags[2 * j] != p.epoch;
-    v.odd = p.flags[2 * j + 1] == p.epoch;
+    v.scan = v.nch > 1 || v.t0 > 0 ? p.scan : 0;     // one chunk: exact lanes
+    const int f = SEG ? __builtin_amdgcn_readfirstlane(p.segs[j].job) : j;
+    v.clean = p.flags[2 * f] != p.epoch;
+    v.odd = p.flags[2 * f + 1] == p.epoch;
     v.rag = false;
     v.group = v.kb = v.k = 0;
     v.coop = false;
     return v;
 }
 
+template <bool SEG>
 __device__ __forceinline__ batch_view pack_block(const rec_pack_args &p, float **out) {
     const int flat = blockIdx.x;
     const int j = pack_find(p, flat, false);
-    batch_view v = pack_view(p, j);
+    batch_view v = pack_view<SEG>(p, j);
     block_chunk(v, flat - __builtin_amdgcn_readfirstlane(p.jobs[j].block0));
     *out = p.jobs[j].out;
     return v;
 }
 
 // (a job without spans owns no block here: the next job starts at its span0)
-template <class E>
+template <class E, bool SEG>
 __device__ __forceinline__ void packed_spans(const rec_pack_args &p) {
     const int flat = blockIdx.x;
     const int j = pack_find(p, flat, true);
-    batch_view v = pack_view(p, j);
+    batch_view v = pack_view<SEG>(p, j);
     span_pass<E>(v, flat - __builtin_amdgcn_readfirstlane(p.jobs[j].span0));
 }
 
@@ -1862,19 +1876,23 @@ __device__ __forceinline__ void packed_spans(const rec_pack_args &p) {
     extern "C" __global__ __launch_bounds__(256) void NAME##_batch_f32(rec_args a) {         \
         batch_pass<ENG, NIN>(view_of(a), a.out0);                                            \
     }
-#define REC_PACKED(NAME, ENG, NIN)                                                           \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_states(rec_pack_args p) { \
+#define REC_PACKED_(NAME, ENG, NIN, SEG, X)                                                  \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_states##X(               \
+        rec_pack_args p) {                                                                   \
         float *out;                                                                          \
-        scan_pass1<ENG>(pack_block(p, &out));                                                \
+        scan_pass1<ENG>(pack_block<SEG>(p, &out));                                          \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_spans(rec_pack_args p) {  \
-        packed_spans<ENG>(p);                                                                \
+    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_spans##X(rec_pack_args p) { \
+        packed_spans<ENG, SEG>(p);                                                           \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32(rec_pack_args p) {    \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32##X(rec_pack_args p) { \
         float *out;                                                                          \
-        const batch_view v = pack_block(p, &out);                                            \
+        const batch_view v = pack_block<SEG>(p, &out);                                      \
         batch_pass<ENG, NIN>(v, out);                                                        \
     }
+#define REC_PACKED(NAME, ENG, NIN)                                                           \
+    REC_PACKED_(NAME, ENG, NIN, false, )                                                     \
+    REC_PACKED_(NAME, ENG, NIN, true, _seg)
 REC_BATCH(ema, EmaEng, 1)
 REC_BATCH(rsi, RsiEng, 1)
 REC_BATCH(atr, AtrEng, 3)
@@ -1893,7 +1911,11 @@ extern "C" __global__ __launch_bounds__(256) void adx_scan_stage2(rec_args a) {
 }
 extern "C" __global__ __launch_bounds__(256) void adx_packed_stage2(rec_pack_args p) {
     float *out;
-    scan_pass2(pack_block(p, &out));
+    scan_pass2(pack_block<false>(p, &out));
+}
+extern "C" __global__ __launch_bounds__(256) void adx_packed_stage2_seg(rec_pack_args p) {
+    float *out;
+    scan_pass2(pack_block<true>(p, &out));
 }
 
 // The per-bar terms of one series at bar t (kind: 0 the close, 1 RSI, 2 ATR,
@@ -1977,6 +1999,30 @@ extern "C" __global__ __launch_bounds__(256) void packed_prepare(const rec_job *
     }
     if (bad) flags[2 * blockIdx.y] = epoch;
     if (odd) flags[2 * blockIdx.y + 1] = epoch;
+}
+
+// The same for the entries of a level of a pack with segments: grid (blocks,
+// entries).
+extern "C" __global__ __launch_bounds__(256) void packed_prepare_seg(const rec_job *jobs,
+                                                                     const rec_seg *segs,
+                                                                     int32_t *flags, int kind,
+                                                                     int nterms, int epoch) {
+    const rec_job &jb = jobs[blockIdx.y];
+    const int t0 = segs[blockIdx.y].t0, job = segs[blockIdx.y].job;
+    const bool scan = jb.nch > 1 || t0 > 0;
+    const int bars = scan ? jb.tstride : jb.T;
+    bool bad = false, odd = false;
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < bars; i += (long)gridDim.x * 256) {
+        double f[3];
+        const scan_bar r = scan_bar_terms(jb.x, jb.h, jb.l, jb.T, jb.fv, kind, t0 + i, f);
+        if (scan)
+            for (int q = 0; q < nterms; ++q)
+                jb.terms[scan_term_at(nterms, q, jb.tstride, i)] = f[q];
+        bad = bad || r.bad;
+        odd = odd || r.odd;
+    }
+    if (bad) flags[2 * job] = epoch;
+    if (odd) flags[2 * job + 1] = epoch;
 }
 
 // True range of one series (tr_from_hlc_f32 in the reference): 0 before

@@ -1090,29 +1090,29 @@ vta_status vta_ema_rsi_atr_many_series_dev(vta_ctx *ctx, const float *close_tm,
 
 // ---------------------------------------------------------------- packed batches
 
-static_assert(sizeof(PackJob) == 96, "rec_job layout");
+static_assert(sizeof(PackJob) == 96 && sizeof(PackSeg) == 32, "rec_job, rec_seg layout");
 
 namespace {
 
 struct rec_pack_args_host {
     const void *jobs;
+    const void *segs;
     const int32_t *flags;
     int n_jobs;
     int scan;
     int epoch;
     int pad_;
 };
-static_assert(sizeof(rec_pack_args_host) == 32, "rec_pack_args layout");
+static_assert(sizeof(rec_pack_args_host) == 40, "rec_pack_args layout");
 
-const char *packed_kernel(Ind k, int pass) {   // 0 states, 1 spans, 2 output
-    static const char *n[][3] = {
-        {"ema_packed_states", "ema_packed_spans", "ema_packed_f32"},
-        {"rsi_packed_states", "rsi_packed_spans", "rsi_packed_f32"},
-        {"atr_packed_states", "atr_packed_spans", "atr_packed_f32"},
-        {"adx_packed_states", "adx_packed_spans", "adx_packed_f32"},
-        {"smma_packed_states", "smma_packed_spans", "smma_packed_f32"},
-        {"wilders_packed_states", "wilders_packed_spans", "wilders_packed_f32"}};
-    return n[k][pass];
+const char *packed_kernel(Ind k, int pass, bool seg) {   // 0 states, 1 spans, 2 output
+#define VTA_PACKED(n)                                                                     \
+    {{n "_packed_states", n "_packed_states_seg"}, {n "_packed_spans", n "_packed_spans_seg"}, \
+     {n "_packed_f32", n "_packed_f32_seg"}}
+    static const char *n[][3][2] = {VTA_PACKED("ema"), VTA_PACKED("rsi"),  VTA_PACKED("atr"),
+                                    VTA_PACKED("adx"), VTA_PACKED("smma"), VTA_PACKED("wilders")};
+#undef VTA_PACKED
+    return n[k][pass][seg];
 }
 
 }  // namespace
@@ -1120,7 +1120,7 @@ const char *packed_kernel(Ind k, int pass) {   // 0 states, 1 spans, 2 output
 namespace vta {
 
 vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, size_t n_jobs,
-                       std::vector<PackJob> &tab, size_t *work_elems, PackDims *dims) {
+                       PackTable &tab, size_t *work_elems, PackDims *dims) {
     if (!ctx || !jobs || !dims || !work_elems)
         return fail(VTA_ERR_INVALID_INPUT, "null argument");
     if (kind < (int)VTA_REC_EMA || kind > (int)VTA_REC_WILDERS)
@@ -1129,8 +1129,10 @@ vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, si
         return fail(VTA_ERR_INVALID_INPUT, "n_jobs must be in 1..65535 (got %zu)", n_jobs);
     const Ind k = (Ind)kind;
     const size_t S = scan_states(k);
-    tab.assign(n_jobs, PackJob{});
-    size_t blocks = 0, spans = 0, elems = 0, bars = 1;
+    std::vector<PackTable> levels(1);
+    size_t elems = 0;
+    *dims = PackDims{};
+    dims->levels.resize(1);
     for (size_t j = 0; j < n_jobs; ++j) {
         const vta_rec_job &q = jobs[j];
         if (!q.d_close || !q.d_periods || !q.d_out || (hlc(k) && (!q.d_high || !q.d_low)))
@@ -1140,91 +1142,151 @@ vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, si
             return fail(VTA_ERR_INVALID_INPUT,
                         "job %zu: series_len, n_combos and max_period must be positive and "
                         "first_valid < series_len", j);
+        // the segments and chunks of the job's own _device call (one exact
+        // chunk where that call would not scan).  RSI of 600,000 x 6, 900,000
+        // x 4 and two short series: 180 us (268 as direct calls); 111 ms with
+        // the long ones as one exact chunk.
         const size_t T = (size_t)q.series_len, C = (size_t)q.n_combos;
-        // the chunking of the job's own _device call (one exact chunk where
-        // that call would not scan, or would in segments)
-        size_t chunk = scan_segment(k, T) == T ? scan_chunk(ctx, k, T, C) : 0;
-        if (chunk == 0) chunk = T;
-        const size_t nch = (T + chunk - 1) / chunk;
         const size_t groups = (C + 63) / 64;
-        PackJob &e = tab[j];
-        e.x = q.d_close;
-        e.h = hlc(k) ? q.d_high : nullptr;
-        e.l = hlc(k) ? q.d_low : nullptr;
-        e.periods = q.d_periods;
-        e.out = q.d_out;
-        e.carry = nullptr;                      // set once the buffer exists
-        e.T = (int)T;
-        e.nlanes = (int)C;
-        e.fv = q.first_valid;
-        e.chunk = (int)chunk;
-        e.nch = (int)nch;
-        e.groups = (int)groups;
-        e.terms = nullptr;
-        e.tstride = (int)((T + 63) & ~(size_t)63);
-        e.block0 = (int)blocks;
-        e.span = nch > 1 ? (int)scan_span(groups, nch) : 0;
-        e.span0 = (int)spans;
-        blocks += batch_blocks(groups, nch);
-        const size_t nsp = e.span ? (nch - 1) / e.span : 0;
-        spans += groups * nsp;
-        if (nch > 1) elems += groups * 64 * (nch + nsp) * S + scan_terms(k) * (size_t)e.tstride;
-        bars = std::max(bars, T + 63);
-        if (blocks > (size_t)INT32_MAX || spans > (size_t)INT32_MAX)
-            return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "packed grid exceeds 2^31 blocks");
+        const size_t chunk = scan_chunk(ctx, k, T, C);
+        const size_t seg = chunk ? scan_segment(k, T) : T;
+        for (size_t t0 = 0, level = 0; t0 < T; t0 += seg, ++level) {
+            if (level == levels.size()) {
+                levels.emplace_back();
+                dims->levels.emplace_back();
+            }
+            PackLevel &lv = dims->levels[level];
+            const size_t t1 = std::min(T, t0 + seg);
+            const size_t nch = chunk ? (t1 - t0 + chunk - 1) / chunk : 1;
+            PackSeg s{};                            // (the buffers once there are any)
+            PackJob e{};
+            e.x = q.d_close;
+            e.h = hlc(k) ? q.d_high : nullptr;
+            e.l = hlc(k) ? q.d_low : nullptr;
+            e.periods = q.d_periods;
+            e.out = q.d_out;
+            e.T = (int)T;
+            e.nlanes = (int)C;
+            e.fv = q.first_valid;
+            s.t0 = (int)t0;
+            s.t1 = (int)t1;
+            s.job = (int)j;
+            e.chunk = (int)(chunk ? chunk : T);
+            e.nch = (int)nch;
+            e.groups = (int)groups;
+            e.tstride = chunk ? (int)((t1 - t0 + 63) & ~(size_t)63) : 0;
+            e.span = nch > 1 ? (int)scan_span(groups, nch) : 0;
+            const size_t nsp = e.span ? (nch - 1) / e.span : 0;
+            const size_t blocks = lv.blocks + batch_blocks(groups, nch);
+            const size_t spans = lv.spans + groups * nsp;
+            if (blocks > (size_t)INT32_MAX || spans > (size_t)INT32_MAX)
+                return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "packed grid exceeds 2^31 blocks");
+            e.block0 = (int)lv.blocks;
+            e.span0 = (int)lv.spans;
+            lv.blocks = (unsigned)blocks;
+            lv.spans = (unsigned)spans;
+            lv.flag_blocks = std::max(
+                lv.flag_blocks, (unsigned)std::min<size_t>((t1 - t0 + 63 + 255) / 256, 1024));
+            elems += scan_terms(k) * (size_t)e.tstride;
+            if (t0 == 0 && chunk) elems += groups * 64 * (nch + nsp + (seg < T ? 2 : 0)) * S;
+            levels[level].jobs.push_back(e);
+            levels[level].segs.push_back(s);
+        }
     }
     dims->kind = kind;
     dims->n_jobs = (int)n_jobs;
-    dims->total_blocks = (unsigned)blocks;
-    dims->total_spans = (unsigned)spans;
-    dims->flag_blocks = (unsigned)std::min<size_t>((bars + 255) / 256, 1024);
+    tab = PackTable{};
+    for (size_t l = 0; l < levels.size(); ++l) {
+        dims->levels[l].first = (int)tab.jobs.size();
+        dims->levels[l].n = (int)levels[l].jobs.size();
+        tab.jobs.insert(tab.jobs.end(), levels[l].jobs.begin(), levels[l].jobs.end());
+        tab.segs.insert(tab.segs.end(), levels[l].segs.begin(), levels[l].segs.end());
+    }
+    if (tab.jobs.size() > (size_t)INT32_MAX)
+        return fail(VTA_ERR_LAUNCH_CONFIG_TOO_LARGE, "packed table exceeds 2^31 entries");
+    dims->n_entries = (int)tab.jobs.size();
     *work_elems = elems;
     return VTA_OK;
 }
 
-void pack_bind(const PackDims &d, std::vector<PackJob> &tab, double *work) {
+// (a job's segments follow one another: one carry, and two rows of states that
+// its segments hand on in turn)
+void pack_bind(const PackDims &d, PackTable &tab, double *work) {
     const Ind k = (Ind)d.kind;
-    for (PackJob &e : tab) {
-        if (e.nch < 2) continue;
-        e.carry = work;
-        const size_t nsp = e.span ? (e.nch - 1) / e.span : 0;
-        work += (size_t)e.groups * 64 * (e.nch + nsp) * scan_states(k);
-        e.terms = work;
-        work += scan_terms(k) * (size_t)e.tstride;
-    }
+    std::vector<double *> carry((size_t)d.n_jobs, nullptr), handed((size_t)d.n_jobs, nullptr);
+    for (size_t l = 0; l < d.levels.size(); ++l)
+        for (int i = d.levels[l].first; i < d.levels[l].first + d.levels[l].n; ++i) {
+            PackJob &e = tab.jobs[(size_t)i];
+            PackSeg &s = tab.segs[(size_t)i];
+            if (!e.tstride) continue;
+            const size_t row = (size_t)e.groups * 64 * scan_states(k);
+            if (l == 0) {
+                const size_t nsp = e.span ? (e.nch - 1) / e.span : 0;
+                carry[s.job] = work;
+                work += row * (e.nch + nsp);
+                handed[s.job] = work;
+                if (s.t1 < e.T) work += 2 * row;
+            }
+            e.carry = carry[s.job];
+            if (l > 0) s.state_in = handed[s.job] + ((l - 1) & 1) * row;
+            if (s.t1 < e.T) s.state_out = handed[s.job] + (l & 1) * row;
+            e.terms = work;
+            work += scan_terms(k) * (size_t)e.tstride;
+        }
 }
 
-std::vector<unsigned char> pack_image(const std::vector<PackJob> &tab) {
-    std::vector<unsigned char> v(pack_flags_off(tab.size()) + tab.size() * 2 * sizeof(int32_t), 0);
-    if (!tab.empty()) memcpy(v.data(), tab.data(), pack_flags_off(tab.size()));
+// Bytes before the segments of a pack's image, and before its flags.
+size_t pack_segs_off(const PackDims &d) { return (size_t)d.n_entries * sizeof(PackJob); }
+size_t pack_flags_off(const PackDims &d) {
+    return pack_segs_off(d) + (d.levels.size() > 1 ? (size_t)d.n_entries * sizeof(PackSeg) : 0);
+}
+
+std::vector<unsigned char> pack_image(const PackDims &d, const PackTable &tab) {
+    std::vector<unsigned char> v(pack_flags_off(d) + (size_t)d.n_jobs * 2 * sizeof(int32_t), 0);
+    memcpy(v.data(), tab.jobs.data(), pack_segs_off(d));
+    if (d.levels.size() > 1)
+        memcpy(v.data() + pack_segs_off(d), tab.segs.data(), pack_flags_off(d) - pack_segs_off(d));
     return v;
 }
 
 vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch) {
     const Ind k = (Ind)d.kind;
+    const bool seg = d.levels.size() > 1;
     hipFunction_t prep, fs, ff, fb, f2 = nullptr;
-    VTA_TRY(get_function(ctx, "rec", "packed_prepare", &prep));
-    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 0), &fs));
-    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 1), &ff));
-    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 2), &fb));
-    if (k == IND_ADX) VTA_TRY(get_function(ctx, "rec", "adx_packed_stage2", &f2));
-    int32_t *flags = reinterpret_cast<int32_t *>(static_cast<char *>(d_image) +
-                                                 pack_flags_off((size_t)d.n_jobs));
-    VTA_TRY(launch(ctx, prep, dim3(d.flag_blocks, (unsigned)d.n_jobs), dim3(256), 0,
-                   static_cast<const void *>(d_image), flags, scan_kind(k), (int)scan_terms(k),
-                   epoch));
-    rec_pack_args_host a{d_image, flags, d.n_jobs, 1, epoch, 0};
-    const dim3 block(64 * kWpb);
-    VTA_TRY(launch(ctx, fs, dim3(d.total_blocks), block, 0, a));
-    if (d.total_spans)
-        VTA_TRY(launch(ctx, ff, dim3(d.total_spans, (unsigned)scan_terms(k)), dim3(64), 0, a));
-    if (k == IND_ADX) {
-        VTA_TRY(launch(ctx, f2, dim3(d.total_blocks), block, kFoldLds, a));
-        a.scan = 2;
-        if (d.total_spans) VTA_TRY(launch(ctx, ff, dim3(d.total_spans), dim3(64), 0, a));
-        a.scan = 1;
+    VTA_TRY(get_function(ctx, "rec", seg ? "packed_prepare_seg" : "packed_prepare", &prep));
+    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 0, seg), &fs));
+    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 1, seg), &ff));
+    VTA_TRY(get_function(ctx, "rec", packed_kernel(k, 2, seg), &fb));
+    if (k == IND_ADX)
+        VTA_TRY(get_function(ctx, "rec", seg ? "adx_packed_stage2_seg" : "adx_packed_stage2", &f2));
+    const char *image = static_cast<const char *>(d_image);
+    const PackJob *jobs = reinterpret_cast<const PackJob *>(image);
+    const PackSeg *segs = reinterpret_cast<const PackSeg *>(image + pack_segs_off(d));
+    int32_t *flags = reinterpret_cast<int32_t *>(static_cast<char *>(d_image) + pack_flags_off(d));
+    // all terms first: a job's flags are of its whole series
+    for (const PackLevel &lv : d.levels) {
+        const dim3 grid(lv.flag_blocks, (unsigned)lv.n), block(256);
+        const void *j = jobs + lv.first, *s = segs + lv.first;
+        VTA_TRY(seg ? launch(ctx, prep, grid, block, 0, j, s, flags, scan_kind(k),
+                             (int)scan_terms(k), epoch)
+                    : launch(ctx, prep, grid, block, 0, j, flags, scan_kind(k),
+                             (int)scan_terms(k), epoch));
     }
-    return launch(ctx, fb, dim3(d.total_blocks), block, batch_lds_bytes(k), a);
+    const dim3 block(64 * kWpb);
+    for (const PackLevel &lv : d.levels) {
+        rec_pack_args_host a{jobs + lv.first, segs + lv.first, flags, lv.n, 1, epoch, 0};
+        VTA_TRY(launch(ctx, fs, dim3(lv.blocks), block, 0, a));
+        if (lv.spans)
+            VTA_TRY(launch(ctx, ff, dim3(lv.spans, (unsigned)scan_terms(k)), dim3(64), 0, a));
+        if (k == IND_ADX) {
+            VTA_TRY(launch(ctx, f2, dim3(lv.blocks), block, kFoldLds, a));
+            a.scan = 2;
+            if (lv.spans) VTA_TRY(launch(ctx, ff, dim3(lv.spans), dim3(64), 0, a));
+            a.scan = 1;
+        }
+        VTA_TRY(launch(ctx, fb, dim3(lv.blocks), block, batch_lds_bytes(k), a));
+    }
+    return VTA_OK;
 }
 
 }  // namespace vta
@@ -1243,7 +1305,7 @@ vta_status vta_rec_pack_create(vta_ctx *ctx, vta_rec_kind kind, const vta_rec_jo
     clear_error();
     if (!ctx || !jobs || !out) return fail(VTA_ERR_INVALID_INPUT, "null argument");
     *out = nullptr;
-    std::vector<PackJob> tab;
+    PackTable tab;
     size_t elems = 0;
     auto pk = std::make_unique<vta_rec_pack>();
     VTA_TRY(pack_layout(ctx, (int)kind, jobs, n_jobs, tab, &elems, &pk->dims));
@@ -1251,7 +1313,7 @@ vta_status vta_rec_pack_create(vta_ctx *ctx, vta_rec_kind kind, const vta_rec_jo
     VTA_HIP(hipSetDevice(ctx->device));
     VTA_TRY(pk->work.alloc(std::max<size_t>(elems, 1) * sizeof(double)));
     pack_bind(pk->dims, tab, pk->work.as<double>());
-    const std::vector<unsigned char> image = pack_image(tab);
+    const std::vector<unsigned char> image = pack_image(pk->dims, tab);
     VTA_TRY(upload(ctx, pk->image, image.data(), image.size()));
     *out = pk.release();
     return VTA_OK;

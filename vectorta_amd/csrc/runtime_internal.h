@@ -31,7 +31,8 @@ struct vta_ctx {
     void *carry = nullptr;
     static constexpr size_t kCarryBytes = 56u << 20;
     // the scan's per-bar terms, in the same allocation: 1.05M bars of one term,
-    // 0.35M of ADX's three (longer series run in segments)
+    // 0.35M of ADX's three (longer series run in segments, in packs too, whose
+    // terms are in the pack's own buffer: a job's outputs are its own call's)
     double *terms = nullptr;
     static constexpr size_t kTermBytes = 8u << 20;
     // launch-shape knobs (vta_tune_knob); 0 = built-in heuristic
@@ -260,20 +261,35 @@ struct PackJob {
     double *terms;
     int T, nlanes, fv, chunk, nch, groups, block0, span0, tstride, span;
 };
+struct PackSeg {
+    const double *state_in;
+    double *state_out;
+    int t0, t1, job, pad_;
+};
+struct PackTable {
+    std::vector<PackJob> jobs;
+    std::vector<PackSeg> segs;   // beside them
+};
+// The table's entries by level: level 0 holds every job, its first segment
+// where its own call takes several, level l the l-th further segments.  Each
+// level is launched by itself, after the one before.
+struct PackLevel {
+    int first = 0, n = 0;
+    unsigned blocks = 0, spans = 0, flag_blocks = 1;
+};
 struct PackDims {
-    int kind = 0, n_jobs = 0;
-    unsigned total_blocks = 0, total_spans = 0, flag_blocks = 1;
+    int kind = 0, n_jobs = 0, n_entries = 0;
+    std::vector<PackLevel> levels;
 };
 // Validates the jobs like the _device forms and lays out the table; the
 // chunk states and terms of all jobs take work_elems doubles, which
 // pack_bind hands out from `work`.
 vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, size_t n_jobs,
-                       std::vector<PackJob> &tab, size_t *work_elems, PackDims *dims);
-void pack_bind(const PackDims &d, std::vector<PackJob> &tab, double *work);
-// The device image of a pack: the table, then its flags (pack_flags_off bytes
-// in), which start as zeros.
-std::vector<unsigned char> pack_image(const std::vector<PackJob> &tab);
-inline size_t pack_flags_off(size_t n_jobs) { return n_jobs * sizeof(PackJob); }
+                       PackTable &tab, size_t *work_elems, PackDims *dims);
+void pack_bind(const PackDims &d, PackTable &tab, double *work);
+// The device image of a pack: the table, then the jobs' flags, which start as
+// zeros.
+std::vector<unsigned char> pack_image(const PackDims &d, const PackTable &tab);
 // d_image: pack_image on the device.  epoch: positive, another one for every
 // launch over the same flags (a repeated one can only read a clean job as
 // unclean, which runs exactly from first_valid).

@@ -878,14 +878,14 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
         member.push_back(i);
     }
     if (jobs.empty()) return true;
-    std::vector<PackJob> tab;
+    PackTable tab;
     std::vector<unsigned char> image;
     size_t elems = 0;
     PackDims dims;
     vta_status v = pack_layout(ctx, rk, jobs.data(), jobs.size(), tab, &elems, &dims);
     void *d_tab = nullptr, *d_work = nullptr;
     if (v == VTA_OK) {
-        d_tab = s->arena.alloc(pack_image(tab).size());
+        d_tab = s->arena.alloc(pack_image(dims, tab).size());
         d_work = s->arena.alloc(std::max<size_t>(elems, 1) * sizeof(double));
         if (!d_tab || !d_work) {
             for (void *p : {d_tab, d_work})
@@ -894,7 +894,7 @@ bool run_packed(vta_server *s, vta_ctx *ctx, std::vector<std::shared_ptr<Req>> &
             return false;
         }
         pack_bind(dims, tab, static_cast<double *>(d_work));
-        image = pack_image(tab);
+        image = pack_image(dims, tab);
         hipError_t e = hipMemcpyAsync(d_tab, image.data(), image.size(), hipMemcpyHostToDevice,
                                       ctx->stream);
         if (e != hipSuccess) v = fail(VTA_ERR_HIP, "hipMemcpyAsync: %s", hipGetErrorString(e));
