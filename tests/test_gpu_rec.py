@@ -8,6 +8,8 @@ denominator is floored at 1e-3, so a value below 1e-3 must lie within 1e-8 of
 the oracle.  Long series exercise the chunked burn-in path; series with
 interior NaN/Inf exercise the exact path.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -188,6 +190,45 @@ def test_scan_rows_off_the_lines(ctxs, name, n, combos):
     _check(g[-2:], getattr(O, f"{name}_batch")(*f, [combos, combos + 1]), name)
     nan_mask_equal(g[:some], part)
     assert max_rel_err(g[:some], part.astype(np.float64), floor=1e-3) <= 2e-6
+
+
+@pytest.mark.parametrize("n,combos", [(120_032, 560), (700_032, 100)])
+@pytest.mark.parametrize("name", ["ema", "rsi", "adx", "smma", "wilders"])
+def test_same_bits_wherever_the_rows_lie(name, n, combos):
+    """256 MiB of rows and more, on the 128-byte lines (stored tile by tile) and
+    four bytes off them (by whole lines, of which a chunk computes the part that
+    lies in the next): the same bits.  The averages' terms cancel by fours and
+    leave outputs far below them, so the order of f64 sums shows in the f32
+    rows.  RSI and ADX of 700,032 bars run in segments."""
+    require_gpu()
+    ctx, L, P = vta.HipContext(0), vta.lib(), ctypes.c_void_p
+    h, lo, c = _hlc(n, 47)
+    if name not in ("rsi", "adx"):
+        c = np.random.Generator(np.random.PCG64(48)).normal(size=n).astype(np.float32)
+        c += 1e3 * np.tile(np.float32([1, -1, -1, 1]), n // 4)
+    p0 = 15_000 if name not in ("rsi", "adx") else 2
+    ps = np.arange(p0, p0 + combos, dtype=np.int32)
+    d = [ctx.to_device(v) for v in (c, h, lo, ps, ps - 1)]
+    x, hi, low, per, warm = (P(b.ptr) for b in d)
+    out = ctx.alloc(combos * n * 4 + 128)
+    assert combos * n * 4 >= 256 << 20 and out.ptr % 128 == 0
+    got, mp = [], int(ps[-1])
+    for off in (0, 4):
+        o = P(out.ptr + off)
+        call = {"ema": lambda: L.vta_ema_batch_device(ctx.handle, x, per, None, n, 0, combos, o),
+                "rsi": lambda: L.vta_rsi_batch_device(ctx.handle, x, per, mp, n, 0, combos, o),
+                "adx": lambda: L.vta_adx_batch_device(ctx.handle, hi, low, x, per, mp, n, 0,
+                                                      combos, o),
+                "smma": lambda: L.vta_smma_batch_device(ctx.handle, x, per, warm, 0, n, combos, o),
+                "wilders": lambda: L.vta_wilders_batch_device(ctx.handle, x, per, None, warm, n, 0,
+                                                              combos, o)}
+        assert call[name]() == 0
+        ctx.synchronize()
+        got.append(out.copy_to_host(np.uint32)[off // 4:off // 4 + combos * n])
+    bad = np.flatnonzero(got[0] != got[1])
+    assert bad.size == 0, (bad.size, bad[:8] % n, bad[:8] // n)
+    for b in (*d, out):
+        b.free()
 
 
 def test_wilders_seeded_matches_replay(monkeypatch):

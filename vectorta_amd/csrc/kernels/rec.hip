@@ -1303,10 +1303,11 @@ __device__ __forceinline__ void scan_chain(const batch_view &a, const scan_sum &
 // (sum up to bar sw, then beta): the segment's incoming state, the spans, then
 // the chunks, in a cooperative block each wave a share of the chunks before
 // the block as one affine map (lds: 64 (M + 1) doubles per wave; every wave of
-// the block calls it).
-template <int M>
+// the block calls it).  NEXT: and in `next` those at the start of the chunk
+// after it (if there is one), by the operations of that chunk's own fold.
+template <int M, bool NEXT>
 __device__ __forceinline__ void scan_start(const batch_view &a, const scan_sum &q, int S, int i0,
-                                           int c, double *s, double *lds) {
+                                           int c, double *s, double *next, double *lds) {
     const size_t cp = (size_t)a.groups * 64, step = (size_t)S * cp;
     const double *b = a.carry + (size_t)i0 * cp + c;
     const bool idle = wave_idle(a), zero = a.state_in == nullptr;
@@ -1320,9 +1321,40 @@ __device__ __forceinline__ void scan_start(const batch_view &a, const scan_sum &
                       nullptr);
         j = n * a.span;
     }
+    double after[M];                                 // NEXT: the states after the spans
+    if (NEXT)
+#pragma unroll
+        for (int i = 0; i < M; ++i) after[i] = s[i];
+    // onto `after`, where chunk k opens a span: the span before it
+    auto span_before = [&](int k) {
+        const int n = k / a.span - 1;
+        scan_chain<M>(a, q, a.chunk * a.span, b + (size_t)a.nch * step, step, cp, n, n + 1,
+                      zero && n == 0, after, nullptr);
+    };
     if (!a.coop) {
-        if (!idle)
-            scan_chain<M>(a, q, a.chunk, b, step, cp, j, a.k, zero && j == 0, s, nullptr);
+        if (idle) return;
+        const bool more = NEXT && a.k + 1 < a.nch;
+        double bk[M];                                // (loaded ahead of the chain)
+        if (more)
+#pragma unroll
+            for (int i = 0; i < M; ++i) bk[i] = b[(size_t)a.k * step + i * cp];
+        scan_chain<M>(a, q, a.chunk, b, step, cp, j, a.k, zero && j == 0, s, nullptr);
+        if (more) {
+            if (a.span && (a.k + 1) % a.span == 0) {
+                span_before(a.k + 1);
+#pragma unroll
+                for (int i = 0; i < M; ++i) next[i] = after[i];
+            } else {
+                // the step of scan_chain over chunk k
+                const int r = q.sw - a.t0, jm = r < 0 ? -1 : r / a.chunk;
+                const int jl = q.last < a.t0 ? -1 : (q.last - a.t0) / a.chunk;
+                double g = scan_pow(q.beta, a.chunk);
+                if (a.k <= jl && !(zero && a.k == 0 && jl == 0) && a.k <= jm)
+                    g = a.k == jm ? q.kap * scan_pow(q.beta, a.chunk - 1 - r % a.chunk) : 1.0;
+#pragma unroll
+                for (int i = 0; i < M; ++i) next[i] = fma(g, s[i], bk[i]);
+            }
+        }
         return;
     }
     const int lane = threadIdx.x & 63, w = a.k - a.kb;
@@ -1361,6 +1393,40 @@ __device__ __forceinline__ void scan_start(const batch_view &a, const scan_sum &
             for (int i = 0; i < M; ++i) s[i] = fma(g, s[i], v[i][u]);
         }
     __syncthreads();
+    if constexpr (NEXT) {
+        // from the next wave; the last wave's is the first of the next block,
+        // which the block folds as that one does
+#pragma unroll
+        for (int i = 0; i < M; ++i) lds[((w + REC_WPB - 1) % REC_WPB) * 64 * (M + 1) + lane + 64 * i] = s[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < M; ++i) next[i] = lds[w * 64 * (M + 1) + lane + 64 * i];
+        __syncthreads();
+        const int kb = a.kb + REC_WPB;
+        if (kb >= a.nch) return;
+        const int j0 = a.span ? kb / a.span * a.span : 0, all = kb - j0;
+        if (a.span && j0 == kb) span_before(kb);
+        double m[M], gg = 1.0;
+#pragma unroll
+        for (int i = 0; i < M; ++i) m[i] = 0.0;
+        scan_chain<M>(a, q, a.chunk, b, step, cp, j0 + all * w / REC_WPB,
+                      j0 + all * (w + 1) / REC_WPB, false, m, &gg);
+        to[0] = gg;
+#pragma unroll
+        for (int i = 0; i < M; ++i) to[64 * (i + 1)] = m[i];
+        __syncthreads();
+        if (w == REC_WPB - 1) {
+#pragma unroll
+            for (int i = 0; i < M; ++i) next[i] = after[i];
+#pragma unroll
+            for (int v = 0; v < REC_WPB; ++v) {
+                const double *from = lds + v * 64 * (M + 1) + lane;
+#pragma unroll
+                for (int i = 0; i < M; ++i) next[i] = fma(from[0], next[i], from[64 * (i + 1)]);
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // Pass 1: the chunk's states from zero, for G groups [a.group, a.group + G) per
@@ -1483,10 +1549,13 @@ __device__ __forceinline__ float scan_dx(double diff, double all) {
 //
 // RAG (rows that do not all start on a 128-byte line): a wave keeps its last
 // two tiles of 32 bars and stores whole lines only, those that start in its
-// chunk; for the last of them it runs one tile into the next chunk.  Stored
+// chunk; for the last of them it runs one tile into the next chunk, from that
+// chunk's own start state, so that the rows' bits are those of tiles.  Stored
 // tile by tile, each line of such rows is written in two parts some
 // microseconds apart, more of them open at once than the L2 holds: 1,250 EMA x
-// 180,001 bars 466 us, 266 with whole lines (180,000 bars: 220).
+// 180,001 bars 466 us, 255 with whole lines (180,000 bars: 221).  The next
+// chunk's start takes 3% where a wave folds alone, 6% where the block does; its
+// running state would do, but for the last bits.
 template <class E, bool ODD, bool EMIT, bool RAG = false>
 __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
     constexpr bool EMA = __is_same(E, EmaEng), RSI = __is_same(E, RsiEng),
@@ -1505,10 +1574,11 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
     if (!wave_idle(a)) scan_touch<E>(a, c0, c1, keep);
     const scan_lane q = scan_params<E>(a, c, c < a.nlanes);
     double s[N], dxs = 0.0;                          // dxs: ADX's second stage
-    scan_start<N>(a, scan_sum{q.beta, q.kap, q.sw, wave_max(q.sw)}, S, 0, c, s, rec_lds);
+    double sn[N], dxn = 0.0;                         // the next chunk's (RAG)
+    scan_start<N, RAG>(a, scan_sum{q.beta, q.kap, q.sw, wave_max(q.sw)}, S, 0, c, s, sn, rec_lds);
     const int last = wave_max(ADX ? max(q.sw2, q.first) : q.sw);
     if (ADX && EMIT)
-        scan_start<1>(a, scan_sum{q.beta, 1.0, q.sw2, last}, S, S - 1, c, &dxs, rec_lds);
+        scan_start<1, RAG>(a, scan_sum{q.beta, 1.0, q.sw2, last}, S, S - 1, c, &dxs, &dxn, rec_lds);
     if (wave_idle(a) || (!EMIT && a.k + 1 >= a.nch)) return;
     const int nrow = min(64, a.nlanes - a.group * 64);
     float *row0 = out + (size_t)(a.group * 64 + (lane >> 3)) * a.T + 4 * (lane & 7);
@@ -1550,6 +1620,11 @@ __device__ __forceinline__ void scan_output(const batch_view &a, float *out) {
     };
     int tb = c0;
     for (; tb < (RAG && !end ? c1 + 32 : c1); tb += 32) {
+        if (RAG && tb == c1) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) s[i] = sn[i];
+            dxs = dxn;
+        }
         if (tb > last) {
 #pragma unroll
             for (int b = 0; b < 32; b += 4) {

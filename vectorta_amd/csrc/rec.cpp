@@ -305,10 +305,10 @@ vta_status prepare_launch(vta_ctx *ctx, Ind k, const rec_args_host &a, size_t t0
 //   300 EMA x 50,001 bars (60 MB)      39.9 / 49.2
 //   600 EMA x 50,001 (120 MB)          58.1 / 64.2
 //   1,200 ADX x 30,001 (144 MB)         136 /  157
-//   400 RSI x 180,001 (288 MB)          194 /  156
-//   400 ADX x 180,001 (288 MB)          267 /  258
-//   700 EMA x 180,004 (504 MB)          257 /  167
-//   1,250 EMA x 180,001 (900 MB)        466 /  266
+//   400 RSI x 180,001 (288 MB)          194 /  160
+//   400 ADX x 180,001 (288 MB)          267 /  270
+//   700 EMA x 180,004 (504 MB)          257 /  165
+//   1,250 EMA x 180,001 (900 MB)        466 /  255
 constexpr unsigned kRagLds = 64 * 64 * sizeof(float);
 constexpr size_t kRagBytes = 256u << 20;
 bool ragged_rows(const rec_args_host &a) {
