@@ -106,6 +106,70 @@ def test_graph_replays_match_eager():
         b.free()
 
 
+@pytest.mark.parametrize("kind", ["ema", "rsi", "adx"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_replays_recover_from_a_non_finite_bar(kind, packed):
+    """A replay over data with a non-finite bar runs the exact lanes; the next
+    one over finite data in the same buffers is the scan again, bit for bit
+    the eager call's."""
+    require_gpu()
+    T, fv = 30_000, 4
+    _, hi, lo, c = datagen.ohlc_from_close(datagen.gbm_close(T, 0.01, seed=43),
+                                           np.random.Generator(np.random.PCG64(43)))
+    for a in (hi, lo, c):
+        a[:fv] = np.nan
+    bad = c.copy()
+    bad[9_000] = np.nan
+    periods = np.arange(2, 42, dtype=np.int32)
+    ctx = vta.HipContext(0)
+    L, h, C = lib(), ctx.handle, int(periods.size)
+    d = {"c": ctx.to_device(c), "h": ctx.to_device(hi), "l": ctx.to_device(lo),
+         "p": ctx.to_device(periods)}
+    outs = [ctx.alloc(C * T * 4) for _ in range(2)]
+    job = {"close": d["c"], "high": d["h"], "low": d["l"], "periods": d["p"], "series_len": T,
+           "first_valid": fv, "n_combos": C, "max_period": 41}
+    if kind != "adx":
+        del job["high"], job["low"]
+    packs = [vta.RecPack(ctx, kind, [dict(job, out=o)]) for o in outs]
+
+    def launch(i):
+        if packed:
+            return packs[i].launch()
+        o = P(outs[i].ptr)
+        if kind == "ema":
+            check(L.vta_ema_batch_device(h, P(d["c"].ptr), P(d["p"].ptr), None, T, fv, C, o))
+        elif kind == "rsi":
+            check(L.vta_rsi_batch_device(h, P(d["c"].ptr), P(d["p"].ptr), 41, T, fv, C, o))
+        else:
+            check(L.vta_adx_batch_device(h, P(d["h"].ptr), P(d["l"].ptr), P(d["c"].ptr),
+                                         P(d["p"].ptr), 41, T, fv, C, o))
+
+    def rows(i):
+        ctx.synchronize()
+        return outs[i].copy_to_host(np.uint32)
+
+    ref = {}
+    for name, x in (("bad", bad), ("clean", c)):
+        check(L.vta_memcpy_htod(h, P(d["c"].ptr), x.ctypes.data_as(P), x.nbytes))
+        launch(0)
+        ref[name] = rows(0)
+    assert not np.array_equal(ref["bad"], ref["clean"])
+    ctx.begin_capture()
+    launch(1)
+    g = ctx.end_capture()
+    for rep, name in enumerate(("clean", "bad", "clean", "clean", "bad", "bad", "clean")):
+        x = bad if name == "bad" else c
+        check(L.vta_memcpy_htod(h, P(d["c"].ptr), x.ctypes.data_as(P), x.nbytes))
+        g.launch()
+        assert np.array_equal(rows(1), ref[name]), (rep, name)
+        if rep % 3 == 1:                      # eager work between replays
+            launch(0)
+            assert np.array_equal(rows(0), ref[name]), ("eager", rep, name)
+    g.destroy()
+    for pk in packs:
+        pk.close()
+
+
 def test_capture_state_errors():
     require_gpu()
     ctx = vta.HipContext(0)

@@ -36,9 +36,7 @@ struct rec_args {
     const float *l;          // low  (ATR, ADX)
     const int32_t *periods;  // batch: per combo; many-series: [0] only
     const int32_t *fvs;      // many-series: per series
-    const int32_t *clean;    // many-series: per series; batch: [0] a non-finite bar was
-                             // met, [1] an odd one (the word equals clean_epoch); NULL:
-                             // not clean
+    const int32_t *clean;    // many-series: per series; batch: scan_flags; NULL: not clean
     const int32_t *fvs2;     // fused kernel: per-series first_valid of (high, low, close)
     float *out0;
     float *out1;
@@ -60,10 +58,22 @@ struct rec_args {
     int t0, t1;              // batch scan: the bars of this launch
     int tstride;
     int scan;                // batch: 0 burn-in / exact lanes, else the scan (ADX: stage 1 or 2)
-    int clean_epoch;         // batch: the word scan_prepare stores in clean[0], [1]
+    int epoch;               // batch: of the call, 0: counted on the device (scan_flags)
     int rag;                 // batch scan: whole lines of rows that start anywhere (scan_output)
-    int pad_;
+    int last;                // batch: the call's last output pass
 };
+
+// Words of a one-series batch's flags, and of a pack's after its jobs'.  A flag
+// is set where it holds the call's epoch, so that no word needs clearing.  The
+// host counts the epochs of calls that it launches (from 1).  Those of a
+// captured call, whose arguments are the same at every replay, are counted on
+// the device, with flags of their own (0.3 us more on an 18 us call): the
+// launches before the output pass take SF_LAST + 1; scan_states (scan_prepare
+// where there is none) leaves it in SF_EPOCH, where the output pass reads it,
+// and the call's last output pass copies it to SF_LAST: no launch reads a word
+// that it writes.  (A repeated epoch can only read a clean series as unclean,
+// which then runs exactly from first_valid.)
+enum scan_flags { SF_BAD, SF_ODD, SF_EPOCH, SF_LAST };
 
 #define REC_NAN __builtin_bit_cast(double, 0x7ff8000000000000ull)
 
@@ -859,6 +869,7 @@ struct batch_view {
     double *state_out;
     int T, nlanes, chunk, nch, groups, span, fv, t0, t1, tstride, scan, group;
     int kb, k;               // the block's first chunk, this wave's
+    int32_t epoch;           // see scan_flags
     bool clean, odd, coop, rag;
 };
 
@@ -887,7 +898,9 @@ __device__ __forceinline__ bool wave_idle(const batch_view &v) {
     return v.k >= v.nch || v.group >= v.groups;
 }
 
-// The view of a wave of a direct launch: the blocks of a group in order.
+// The view of a wave of a direct launch (OUT: the output pass): the blocks of a
+// group in order.
+template <bool OUT>
 __device__ __forceinline__ batch_view view_of(const rec_args &a) {
     batch_view v;
     v.x = a.x; v.h = a.h; v.l = a.l;
@@ -909,8 +922,13 @@ __device__ __forceinline__ batch_view view_of(const rec_args &a) {
     v.tstride = a.tstride;
     v.scan = a.scan;
     block_chunk(v, blockIdx.x);
-    v.clean = a.clean != nullptr && a.clean[0] != a.clean_epoch;
-    v.odd = a.clean != nullptr && a.clean[1] == a.clean_epoch;
+    v.clean = v.odd = false;
+    v.epoch = 0;
+    if (a.clean) {
+        v.epoch = a.epoch ? a.epoch : OUT ? a.clean[SF_EPOCH] : a.clean[SF_LAST] + 1;
+        v.clean = a.clean[SF_BAD] != v.epoch;
+        v.odd = a.clean[SF_ODD] == v.epoch;
+    }
     v.rag = a.rag != 0;
     return v;
 }
@@ -1869,12 +1887,12 @@ struct rec_seg {
 struct rec_pack_args {
     const rec_job *jobs;
     const rec_seg *segs;
-    const int32_t *flags;    // per job: [2 j] a non-finite bar, [2 j + 1] an odd one was met
-                             // (the word equals epoch)
+    int32_t *flags;          // per job: SF_BAD and SF_ODD
+    int32_t *call;           // SF_EPOCH and SF_LAST
     int n_jobs;
     int scan;
-    int epoch;
-    int pad_;
+    int epoch;               // as in rec_args
+    int last;
 };
 
 // The last job whose first block (span) is <= flat; jobs are in order.
@@ -1890,7 +1908,7 @@ __device__ __forceinline__ int pack_find(const rec_pack_args &p, int flat, bool 
 
 // (SEG: a pack with segments.  In others entry j is all of job j: what segments
 // need beyond that took 2 of the 71 us of 40 RSI series)
-template <bool SEG>
+template <bool SEG, bool OUT>
 __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     const rec_job &jb = p.jobs[j];
     batch_view v;
@@ -1913,19 +1931,20 @@ __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     v.tstride = jb.tstride;
     v.scan = v.nch > 1 || v.t0 > 0 ? p.scan : 0;     // one chunk: exact lanes
     const int f = SEG ? __builtin_amdgcn_readfirstlane(p.segs[j].job) : j;
-    v.clean = p.flags[2 * f] != p.epoch;
-    v.odd = p.flags[2 * f + 1] == p.epoch;
+    v.epoch = p.epoch ? p.epoch : OUT ? p.call[0] : p.call[1] + 1;
+    v.clean = p.flags[2 * f] != v.epoch;
+    v.odd = p.flags[2 * f + 1] == v.epoch;
     v.rag = false;
     v.group = v.kb = v.k = 0;
     v.coop = false;
     return v;
 }
 
-template <bool SEG>
+template <bool SEG, bool OUT>
 __device__ __forceinline__ batch_view pack_block(const rec_pack_args &p, float **out) {
     const int flat = blockIdx.x;
     const int j = pack_find(p, flat, false);
-    batch_view v = pack_view<SEG>(p, j);
+    batch_view v = pack_view<SEG, OUT>(p, j);
     block_chunk(v, flat - __builtin_amdgcn_readfirstlane(p.jobs[j].block0));
     *out = p.jobs[j].out;
     return v;
@@ -1936,34 +1955,47 @@ template <class E, bool SEG>
 __device__ __forceinline__ void packed_spans(const rec_pack_args &p) {
     const int flat = blockIdx.x;
     const int j = pack_find(p, flat, true);
-    batch_view v = pack_view<SEG>(p, j);
+    batch_view v = pack_view<SEG, false>(p, j);
     span_pass<E>(v, flat - __builtin_amdgcn_readfirstlane(p.jobs[j].span0));
+}
+
+// The word that scan_flags asks of scan_states and of a call's last output pass
+// (at their ends: a uniform load after a store goes through the vector cache).
+__device__ __forceinline__ void leave_epoch(const batch_view &v, const int32_t *word) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *const_cast<int32_t *>(word) = v.epoch;
 }
 
 #define REC_BATCH(NAME, ENG, NIN)                                                            \
     extern "C" __global__ __launch_bounds__(256) void NAME##_scan_states(rec_args a) {       \
-        scan_pass1<ENG>(view_of(a));                                                         \
+        const batch_view v = view_of<false>(a);                                              \
+        scan_pass1<ENG>(v);                                                                  \
+        if (!a.epoch) leave_epoch(v, a.clean + SF_EPOCH);                                    \
     }                                                                                        \
     extern "C" __global__ __launch_bounds__(64) void NAME##_scan_spans(rec_args a) {         \
-        batch_view v = view_of(a);                                                           \
+        batch_view v = view_of<false>(a);                                                    \
         span_pass<ENG>(v, blockIdx.x);                                                       \
     }                                                                                        \
     extern "C" __global__ __launch_bounds__(256) void NAME##_batch_f32(rec_args a) {         \
-        batch_pass<ENG, NIN>(view_of(a), a.out0);                                            \
+        const batch_view v = view_of<true>(a);                                               \
+        batch_pass<ENG, NIN>(v, a.out0);                                                     \
+        if (!a.epoch && a.last && a.clean) leave_epoch(v, a.clean + SF_LAST);                \
     }
 #define REC_PACKED_(NAME, ENG, NIN, SEG, X)                                                  \
     extern "C" __global__ __launch_bounds__(256) void NAME##_packed_states##X(               \
         rec_pack_args p) {                                                                   \
         float *out;                                                                          \
-        scan_pass1<ENG>(pack_block<SEG>(p, &out));                                          \
+        const batch_view v = pack_block<SEG, false>(p, &out);                                \
+        scan_pass1<ENG>(v);                                                                  \
+        if (!p.epoch) leave_epoch(v, p.call);                                                \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_spans##X(rec_pack_args p) { \
+    extern "C" __global__ __launch_bounds__(64) void NAME##_packed_spans##X(rec_pack_args p) {\
         packed_spans<ENG, SEG>(p);                                                           \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32##X(rec_pack_args p) { \
+    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32##X(rec_pack_args p) {\
         float *out;                                                                          \
-        const batch_view v = pack_block<SEG>(p, &out);                                      \
+        const batch_view v = pack_block<SEG, true>(p, &out);                                 \
         batch_pass<ENG, NIN>(v, out);                                                        \
+        if (!p.epoch && p.last) leave_epoch(v, p.call + 1);                                  \
     }
 #define REC_PACKED(NAME, ENG, NIN)                                                           \
     REC_PACKED_(NAME, ENG, NIN, false, )                                                     \
@@ -1982,15 +2014,15 @@ REC_PACKED(adx, AdxEng, 3)
 REC_PACKED(smma, SmmaEng, 1)
 REC_PACKED(wilders, WildersEng, 1)
 extern "C" __global__ __launch_bounds__(256) void adx_scan_stage2(rec_args a) {
-    scan_pass2(view_of(a));
+    scan_pass2(view_of<false>(a));
 }
 extern "C" __global__ __launch_bounds__(256) void adx_packed_stage2(rec_pack_args p) {
     float *out;
-    scan_pass2(pack_block<false>(p, &out));
+    scan_pass2(pack_block<false, false>(p, &out));
 }
 extern "C" __global__ __launch_bounds__(256) void adx_packed_stage2_seg(rec_pack_args p) {
     float *out;
-    scan_pass2(pack_block<true>(p, &out));
+    scan_pass2(pack_block<true, false>(p, &out));
 }
 
 // The per-bar terms of one series at bar t (kind: 0 the close, 1 RSI, 2 ATR,
@@ -2032,16 +2064,15 @@ __device__ __forceinline__ scan_bar scan_bar_terms(const float *x, const float *
 
 // The one launch before a device-resident one-series batch: the terms of bars
 // [t0, t1) (t1 up to a whole 64-bar block past the series; none when terms is
-// NULL), meta[2] = epoch when a bar at or after first_valid is not finite and
-// meta[3] = epoch when one is odd, so the batch reads its flags as meta ==
-// epoch and the words need no clearing (each call brings a new epoch); and,
+// NULL), the flags of a bar at or after first_valid that is not finite or is
+// odd, and the call's epoch (scan_flags); and,
 // with warms, vta_check_warms' check of the reference's warm indices against
 // first_valid + period - 1 (a mismatch stores 1 in *err).  Grid: enough threads
 // for the bars checked or formed from bar `from` on, and for n.
 extern "C" __global__ __launch_bounds__(256) void scan_prepare(
     const float *__restrict__ x, const float *__restrict__ h, const float *__restrict__ l, int T,
     int first_valid, int kind, int nterms, int from, int t0, int t1, int tstride,
-    double *__restrict__ terms, int epoch, int32_t *__restrict__ meta,
+    double *__restrict__ terms, int call_epoch, int32_t *__restrict__ flags,
     const int32_t *__restrict__ periods, const int32_t *__restrict__ warms, int n,
     int32_t *__restrict__ err) {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -2050,16 +2081,20 @@ extern "C" __global__ __launch_bounds__(256) void scan_prepare(
     const scan_bar r = scan_bar_terms(x, h, l, T, first_valid, kind, t, f);
     if (terms && t >= t0 && t < t1)
         for (int q = 0; q < nterms; ++q) terms[scan_term_at(nterms, q, tstride, t - t0)] = f[q];
-    if (r.bad) meta[2] = epoch;
-    if (r.odd) meta[3] = epoch;
+    const bool alone = !call_epoch && !terms && i == 0;   // (no pass before the output's)
+    if (r.bad || r.odd || alone) {
+        const int32_t epoch = call_epoch ? call_epoch : flags[SF_LAST] + 1;
+        if (r.bad) flags[SF_BAD] = epoch;
+        if (r.odd) flags[SF_ODD] = epoch;
+        if (alone) flags[SF_EPOCH] = epoch;
+    }
     if (warms && i < n && (long long)warms[i] != (long long)first_valid + periods[i] - 1)
         err[0] = 1;
 }
 
 // The same for every job of a pack: grid (blocks, jobs).
-extern "C" __global__ __launch_bounds__(256) void packed_prepare(const rec_job *jobs,
-                                                                 int32_t *flags, int kind,
-                                                                 int nterms, int epoch) {
+extern "C" __global__ __launch_bounds__(256) void packed_prepare(
+    const rec_job *jobs, int32_t *flags, int kind, int nterms, int call_epoch, int32_t *call) {
     const rec_job &jb = jobs[blockIdx.y];
     const int end = jb.nch > 1 ? jb.tstride : jb.T;  // a one-chunk job has no terms
     bool bad = false, odd = false;
@@ -2072,16 +2107,18 @@ extern "C" __global__ __launch_bounds__(256) void packed_prepare(const rec_job *
         bad = bad || r.bad;
         odd = odd || r.odd;
     }
-    if (bad) flags[2 * blockIdx.y] = epoch;
-    if (odd) flags[2 * blockIdx.y + 1] = epoch;
+    if (bad || odd) {
+        const int32_t epoch = call_epoch ? call_epoch : call[1] + 1;
+        if (bad) flags[2 * blockIdx.y] = epoch;
+        if (odd) flags[2 * blockIdx.y + 1] = epoch;
+    }
 }
 
 // The same for the entries of a level of a pack with segments: grid (blocks,
 // entries).
-extern "C" __global__ __launch_bounds__(256) void packed_prepare_seg(const rec_job *jobs,
-                                                                     const rec_seg *segs,
-                                                                     int32_t *flags, int kind,
-                                                                     int nterms, int epoch) {
+extern "C" __global__ __launch_bounds__(256) void packed_prepare_seg(
+    const rec_job *jobs, const rec_seg *segs, int32_t *flags, int kind, int nterms, int call_epoch,
+    int32_t *call) {
     const rec_job &jb = jobs[blockIdx.y];
     const int t0 = segs[blockIdx.y].t0, job = segs[blockIdx.y].job;
     const bool scan = jb.nch > 1 || t0 > 0;
@@ -2096,8 +2133,11 @@ extern "C" __global__ __launch_bounds__(256) void packed_prepare_seg(const rec_j
         bad = bad || r.bad;
         odd = odd || r.odd;
     }
-    if (bad) flags[2 * job] = epoch;
-    if (odd) flags[2 * job + 1] = epoch;
+    if (bad || odd) {
+        const int32_t epoch = call_epoch ? call_epoch : call[1] + 1;
+        if (bad) flags[2 * job] = epoch;
+        if (odd) flags[2 * job + 1] = epoch;
+    }
 }
 
 // True range of one series (tr_from_hlc_f32 in the reference): 0 before

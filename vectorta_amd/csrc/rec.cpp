@@ -43,9 +43,9 @@ struct rec_args_host {
     int t0, t1;
     int tstride;
     int scan;
-    int clean_epoch;
+    int epoch;
     int rag;
-    int pad_;
+    int last;
 };
 static_assert(sizeof(rec_args_host) == 192, "rec_args layout");
 
@@ -288,14 +288,14 @@ vta_status prepare_launch(vta_ctx *ctx, Ind k, const rec_args_host &a, size_t t0
                           bool terms, const int32_t *d_warms) {
     hipFunction_t prep;
     VTA_TRY(get_function(ctx, "rec", "scan_prepare", &prep));
-    int32_t *meta = static_cast<int32_t *>(ctx->scratch);
     const size_t from = t0;
     size_t end = terms ? t1 : 0;
     if (t0 == 0) end = std::max({end, (size_t)a.T, d_warms ? (size_t)a.nlanes : 0});
     return launch(ctx, prep, dim3((unsigned)((end - from + 255) / 256)), dim3(256), 0, a.x, a.h,
                   a.l, a.T, a.fv, scan_kind(k), (int)scan_terms(k), (int)from, (int)t0, (int)t1,
-                  a.tstride, terms ? ctx->terms : static_cast<double *>(nullptr), a.clean_epoch,
-                  meta, a.periods, d_warms, a.nlanes, meta + kArgErrorWord);
+                  a.tstride, terms ? ctx->terms : static_cast<double *>(nullptr), a.epoch, a.clean,
+                  a.periods, d_warms, a.nlanes,
+                  static_cast<int32_t *>(ctx->scratch) + kArgErrorWord);
 }
 
 // Rows that do not all start on a 128-byte line: from kRagBytes of rows on,
@@ -360,6 +360,7 @@ vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
             }
         }
         a.scan = 1;
+        a.last = t1 == T;
         VTA_TRY(launch(ctx, fb, grid, block, a.rag ? kWpb * kRagLds : batch_lds_bytes(k), a));
     }
     return VTA_OK;
@@ -410,13 +411,13 @@ vta_status batch_launch(vta_ctx *ctx, Ind k, const float *d_x, const float *d_h,
     const bool plain = plain_batch(ctx, k);
     const size_t chunk = clean && !plain ? scan_chunk(ctx, k, T, C) : 0;
     if (clean) {
-        // context scratch words [2] and [3]: the flags of this call, which
-        // hold its epoch where a bar is not finite (odd); an epoch repeated
-        // after 2^31 calls can only read a clean series as unclean, which
-        // runs exactly (and correctly) from first_valid
-        if (++ctx->prep_epoch > INT32_MAX || ctx->prep_epoch == 0) ctx->prep_epoch = 1;
-        a.clean_epoch = (int)ctx->prep_epoch;
-        a.clean = static_cast<int32_t *>(ctx->scratch) + 2;
+        // the context's words of scan_flags, of launches and of captured ones
+        const bool cap = capturing(ctx);
+        a.clean = static_cast<int32_t *>(ctx->scratch) + (cap ? 8 : 4);
+        if (!cap) {
+            if (++ctx->prep_epoch > INT32_MAX) ctx->prep_epoch = 1;
+            a.epoch = (int)ctx->prep_epoch;
+        }
         if (d_warms) ctx->arg_check_pending = true;
     }
     if (chunk) {
@@ -431,6 +432,7 @@ vta_status batch_launch(vta_ctx *ctx, Ind k, const float *d_x, const float *d_h,
                   : pick_chunk_batch(k, max_p, T, (size_t)a.groups, clean);
     a.nch = (int)((T + a.chunk - 1) / a.chunk);
     a.t1 = (int)T;
+    a.last = 1;
     record_batch(ctx, k, a.nch > 1);
     return launch_rec(ctx, batch_kernel(k), a, (unsigned)batch_blocks(a.groups, a.nch), 1, 64 * kWpb,
                       batch_lds_bytes(k));
@@ -1097,13 +1099,14 @@ namespace {
 struct rec_pack_args_host {
     const void *jobs;
     const void *segs;
-    const int32_t *flags;
+    int32_t *flags;
+    int32_t *call;
     int n_jobs;
     int scan;
     int epoch;
-    int pad_;
+    int last;
 };
-static_assert(sizeof(rec_pack_args_host) == 40, "rec_pack_args layout");
+static_assert(sizeof(rec_pack_args_host) == 48, "rec_pack_args layout");
 
 const char *packed_kernel(Ind k, int pass, bool seg) {   // 0 states, 1 spans, 2 output
 #define VTA_PACKED(n)                                                                     \
@@ -1242,11 +1245,17 @@ size_t pack_flags_off(const PackDims &d) {
 }
 
 std::vector<unsigned char> pack_image(const PackDims &d, const PackTable &tab) {
-    std::vector<unsigned char> v(pack_flags_off(d) + (size_t)d.n_jobs * 2 * sizeof(int32_t), 0);
+    std::vector<unsigned char> v(pack_flags_off(d) + ((size_t)d.n_jobs * 4 + 2) * sizeof(int32_t), 0);
     memcpy(v.data(), tab.jobs.data(), pack_segs_off(d));
     if (d.levels.size() > 1)
         memcpy(v.data() + pack_segs_off(d), tab.segs.data(), pack_flags_off(d) - pack_segs_off(d));
     return v;
+}
+
+bool capturing(vta_ctx *ctx) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &st) == hipSuccess &&
+           st == hipStreamCaptureStatusActive;
 }
 
 vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch) {
@@ -1263,18 +1272,20 @@ vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch
     const PackJob *jobs = reinterpret_cast<const PackJob *>(image);
     const PackSeg *segs = reinterpret_cast<const PackSeg *>(image + pack_segs_off(d));
     int32_t *flags = reinterpret_cast<int32_t *>(static_cast<char *>(d_image) + pack_flags_off(d));
+    int32_t *call = flags + 4 * (size_t)d.n_jobs;
+    if (!epoch) flags += 2 * (size_t)d.n_jobs;
     // all terms first: a job's flags are of its whole series
     for (const PackLevel &lv : d.levels) {
         const dim3 grid(lv.flag_blocks, (unsigned)lv.n), block(256);
         const void *j = jobs + lv.first, *s = segs + lv.first;
         VTA_TRY(seg ? launch(ctx, prep, grid, block, 0, j, s, flags, scan_kind(k),
-                             (int)scan_terms(k), epoch)
+                             (int)scan_terms(k), epoch, call)
                     : launch(ctx, prep, grid, block, 0, j, flags, scan_kind(k),
-                             (int)scan_terms(k), epoch));
+                             (int)scan_terms(k), epoch, call));
     }
     const dim3 block(64 * kWpb);
     for (const PackLevel &lv : d.levels) {
-        rec_pack_args_host a{jobs + lv.first, segs + lv.first, flags, lv.n, 1, epoch, 0};
+        rec_pack_args_host a{jobs + lv.first, segs + lv.first, flags, call, lv.n, 1, epoch, 0};
         VTA_TRY(launch(ctx, fs, dim3(lv.blocks), block, 0, a));
         if (lv.spans)
             VTA_TRY(launch(ctx, ff, dim3(lv.spans, (unsigned)scan_terms(k)), dim3(64), 0, a));
@@ -1284,6 +1295,7 @@ vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch
             if (lv.spans) VTA_TRY(launch(ctx, ff, dim3(lv.spans), dim3(64), 0, a));
             a.scan = 1;
         }
+        a.last = &lv == &d.levels.back();
         VTA_TRY(launch(ctx, fb, dim3(lv.blocks), block, batch_lds_bytes(k), a));
     }
     return VTA_OK;
@@ -1325,7 +1337,8 @@ vta_status vta_rec_pack_launch(vta_ctx *ctx, const vta_rec_pack *pk) {
     if (pk->device != ctx->device)
         return fail(VTA_ERR_DEVICE_MISMATCH, "pack built on device %d, context on %d", pk->device,
                     ctx->device);
-    return pack_launch(ctx, pk->dims, pk->image.p, (int)(pk->epoch++ % INT32_MAX) + 1);
+    return pack_launch(ctx, pk->dims, pk->image.p,
+                       capturing(ctx) ? 0 : (int)(pk->epoch++ % INT32_MAX) + 1);
 }
 
 vta_status vta_rec_pack_destroy(vta_rec_pack *pk) {

@@ -45,7 +45,7 @@ struct vta_ctx {
     // an enqueue-only call with device-side argument checks (warm indices) has
     // run since the last vta_ctx_synchronize, which then reads the error word
     bool arg_check_pending = false;
-    // epoch of the last device-resident one-series batch (scan_prepare)
+    // epoch of the last one-series batch launched (scan_flags, kernels/rec.hip)
     uint32_t prep_epoch = 0;
 };
 
@@ -287,13 +287,15 @@ struct PackDims {
 vta_status pack_layout(const vta_ctx *ctx, int kind, const vta_rec_job *jobs, size_t n_jobs,
                        PackTable &tab, size_t *work_elems, PackDims *dims);
 void pack_bind(const PackDims &d, PackTable &tab, double *work);
-// The device image of a pack: the table, then the jobs' flags, which start as
-// zeros.
+// The device image of a pack: the table, then, as zeros, the jobs' flags of
+// launches and of captured launches and the words of the latter's epoch
+// (scan_flags, kernels/rec.hip).
 std::vector<unsigned char> pack_image(const PackDims &d, const PackTable &tab);
-// d_image: pack_image on the device.  epoch: positive, another one for every
-// launch over the same flags (a repeated one can only read a clean job as
-// unclean, which runs exactly from first_valid).
+// d_image: pack_image on the device.
+// epoch: positive, another one for every launch over the same image; 0 for one
+// that is captured.
 vta_status pack_launch(vta_ctx *ctx, const PackDims &d, void *d_image, int epoch);
+bool capturing(vta_ctx *ctx);
 
 // One-series BB batches (rolling.cpp): bb_job of rolling.hip, and a packed
 // table's launches (the tile-form jobs come first in it).
