@@ -302,6 +302,22 @@ def test_warm_index_mismatch_reported_at_synchronize(ops):
     assert np.isnan(d_o.copy_to_host(np.float32)).all()
 
 
+def test_more_combos_than_sixteen_per_workgroup_reach(ops):
+    """1,100,000 combos: more rows of workgroups than the grid's y takes (65,536)
+    at the 16 combos per workgroup of a long SMA batch."""
+    op, T, C = ops["sma"], 64, 1_100_000
+    x = datagen.gbm_close(T, 0.01, seed=210)
+    ps = (np.arange(C) % 40 + 1).astype(np.int32)
+    d_o = op.ctx.alloc(C * T * 4)
+    op.sma_batch_device(op.ctx.to_device(x), op.ctx.to_device(ps), T, C, 0, 40, d_o)
+    op.synchronize()
+    got = d_o.copy_to_host(np.uint32).reshape(C, T)
+    d_o.free()
+    want = op.sma_batch_dev(x, (1, 40, 1)).to_host().view(np.uint32)
+    assert np.array_equal(got[:C // 40 * 40].reshape(-1, 40, T),
+                          np.broadcast_to(want, (C // 40, 40, T)))
+
+
 def _ref_data(n, lead, fa, fb):
     d = np.full(n, np.nan)
     i = np.arange(lead, n, dtype=np.float64)

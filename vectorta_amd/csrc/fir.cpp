@@ -46,8 +46,9 @@ enum Fir { FIR_SMA = 0, FIR_WMA = 1, FIR_SWMA = 2 };
 // knob, else VTA_FIR_GROUP, 1..256).
 // The tile's prefixes are formed once per workgroup: 64 combos share them where
 // there are two arrays, 16 where there is one (SMA; the shorter groups' rows
-// then lie closer together), and a launch of few tiles takes fewer, down to
-// one, for at least kBatchBlocks workgroups.  Whole calls in us at 16 / 32 / 64:
+// then lie closer together; up to 64 where the grid's y has no room), and a
+// launch of few tiles takes fewer, down to one, for at least kBatchBlocks
+// workgroups.  Whole calls in us at 16 / 32 / 64:
 //   1,250 WMA x 200,000 bars     261 / 218 / 212
 //   1,250 SWMA x 200,000         313 / 260 / 238
 //   1,250 SMA x 200,000          198 / 208 / 209
@@ -63,8 +64,10 @@ unsigned fir_group(const vta_ctx *ctx, Fir k, size_t tiles, size_t C) {
         long v = atol(e);
         if (v >= 1 && v <= 256) return (unsigned)v;
     }
-    return (unsigned)std::min<size_t>(k == FIR_SMA ? 16 : 64,
-                                      std::max<size_t>(1, C * tiles / kBatchBlocks));
+    const size_t rows = (size_t)ctx->props.maxGridSize[1];   // (of workgroups)
+    const size_t most = k == FIR_SMA ? std::min<size_t>(64, std::max<size_t>(16, (C + rows - 1) / rows))
+                                     : 64;
+    return (unsigned)std::min(most, std::max<size_t>(1, C * tiles / kBatchBlocks));
 }
 
 // Grids: SMA sma.rs:705-755 (expand_grid_sma), WMA wma_wrapper.rs:324-350
