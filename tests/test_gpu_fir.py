@@ -302,6 +302,31 @@ def test_warm_index_mismatch_reported_at_synchronize(ops):
     assert np.isnan(d_o.copy_to_host(np.float32)).all()
 
 
+@pytest.mark.parametrize("T", [1, 2_047, 2_048, 2_049, 2_100_001, 5_000_003])
+def test_first_non_finite_bar_wherever_it_lies(ops, T):
+    """The device form's search (2,048 bars per block, at most 1,024 blocks, which
+    then go round) against the host form's own, bit for bit: at the edges of its
+    blocks, threads and rounds, before first_valid, and nowhere."""
+    op, p = ops["sma"], min(3, T)
+    x = datagen.gbm_close(T, 0.001, seed=211)
+    fv = 5 if T > 8 else 0
+    x[:fv] = np.nan
+    d_x, d_p, d_o = op.ctx.to_device(x), op.ctx.to_device(np.int32([p])), op.ctx.alloc(T * 4)
+    spots = {None, fv + p, 255, 256, 2_047, 2_048, 2_303, 4_095, 2_097_151, 2_097_152, 2_099_000,
+             4_194_304, T - 2, T - 1}
+    for bad in [b for b in spots if b is None or fv + p <= b < T]:
+        y = x.copy()
+        if bad is not None:
+            y[bad] = np.inf
+            y[-1] = np.nan
+        check(vta.lib().vta_memcpy_htod(op.ctx.handle, ctypes.c_void_p(d_x.ptr),
+                                    y.ctypes.data_as(ctypes.c_void_p), y.nbytes))
+        op.sma_batch_device(d_x, d_p, T, 1, fv, p, d_o)
+        op.synchronize()
+        want = op.sma_batch_dev(y, (p, p, 0)).to_host()[0]
+        assert np.array_equal(d_o.copy_to_host(np.uint32), want.view(np.uint32)), (T, bad)
+
+
 def test_more_combos_than_sixteen_per_workgroup_reach(ops):
     """1,100,000 combos: more rows of workgroups than the grid's y takes (65,536)
     at the 16 combos per workgroup of a long SMA batch."""

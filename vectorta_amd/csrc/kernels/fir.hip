@@ -43,7 +43,7 @@ struct fir_args {
     const float *x;           // batch: [T]; many-series: [T][N] time-major
     const int32_t *periods;   // batch: per combo
     const int32_t *fvp;       // batch: first_valid on the device, or null (fv)
-    const int32_t *zparts;    // batch: nparts (<= 64) candidates, the least of which is the
+    const int32_t *zparts;    // batch: nparts candidates, the least of which is the
                               // first non-finite bar (T if none)
     const int32_t *fvs;       // many-series: per series first_valid
     const int32_t *zs;        // many-series: per series first non-finite bar, or null
@@ -88,7 +88,9 @@ extern "C" __global__ __launch_bounds__(256) void fir_batch_f32(fir_args a) {
     const int c0 = blockIdx.y * a.group;
     const int nc = min(a.group, a.nlanes - c0);
     const int fv = a.fvp ? a.fvp[0] : a.fv;
-    int z = lane < a.nparts ? a.zparts[lane] : T;
+    int z = T;
+#pragma unroll 4
+    for (int i = lane; i < a.nparts; i += 64) z = min(z, a.zparts[i]);
     for (int o = 32; o > 0; o >>= 1) z = min(z, __shfl_xor(z, o));
     z = __builtin_amdgcn_readfirstlane(z);
     int pg = 1, pmin = 1;                        // (each wave looks at all of them)
@@ -467,15 +469,24 @@ extern "C" __global__ __launch_bounds__(64) void fir_ms1p_swma_f32(fir_args a) {
 
 // Single series: every block's first bar at or after first_valid (*fvp, or fv)
 // whose value is not finite, T if it sees none; the batch kernel takes the
-// least of the up to 64 of them, so no word has to be set beforehand.
+// least of them, so no word has to be set beforehand.
 extern "C" __global__ __launch_bounds__(256) void series_nonfinite_parts(
     const float *__restrict__ x, int T, const int32_t *__restrict__ fvp, int fv,
     int32_t *__restrict__ parts) {
     __shared__ int least[4];
     const int from = fvp ? fvp[0] : fv;
     int z = T;
-    for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < T; t += (long)gridDim.x * 256)
-        if (t >= from && !vta_isfinite(x[t])) z = min(z, (int)t);
+    // eight bars at a time, 256 apart, their loads all made before any is looked at
+    for (long t0 = (long)blockIdx.x * 2048 + threadIdx.x; t0 < T; t0 += (long)gridDim.x * 2048) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = x[min(t0 + 256 * u, (long)T - 1)];
+#pragma unroll
+        for (int u = 7; u >= 0; --u) {
+            const long t = t0 + 256 * u;
+            if (t >= from && t < T && !vta_isfinite(v[u])) z = min(z, (int)t);
+        }
+    }
     for (int o = 32; o > 0; o >>= 1) z = min(z, __shfl_xor(z, o));
     if ((threadIdx.x & 63) == 0) least[threadIdx.x >> 6] = z;
     __syncthreads();
