@@ -223,8 +223,8 @@ vta_status plan_enqueue(vta_double_alma_plan *p) {
     VTA_TRY(launch(ctx, f, dim3((unsigned)((p->T + kRowTile - 1) / kRowTile), (unsigned)p->nrows, 1),
                    dim3(256), 0, a));
     VTA_TRY(get_function(ctx, "cross", wide ? "cross_pairs_f64_wide" : "cross_pairs_f64", &f));
-    VTA_TRY(launch(ctx, f, dim3(8u * (unsigned)((p->nseg + 7) / 8 * p->ntiles), 1, 1), dim3(64), 0,
-                   a));
+    const int groups = p->nseg >= 8 ? (p->nseg + 7) / 8 * 8 : p->nseg;
+    VTA_TRY(launch(ctx, f, dim3((unsigned)groups * (unsigned)p->ntiles, 1, 1), dim3(64), 0, a));
     const size_t npairs = (size_t)p->nfast * p->nslow;
     VTA_TRY(get_function(ctx, "cross", "cross_reduce", &f));
     return launch(ctx, f, dim3((unsigned)((npairs + 63) / 64), 1, 1), dim3(256), 0, a);

@@ -32,8 +32,10 @@
 // stride 34 doubles: the 8 rows read at one bar fall on distinct banks) and
 // each value read feeds two pairs.  Each segment reads the position
 // before it from the rows, so the segments are independent; cross_reduce sums
-// them in segment order.  All tiles of a segment run on one XCD (dispatch is
-// round-robin over 8), whose L2 then serves the segment's rows to every tile.
+// them in segment order.  From eight segments on all tiles of a segment run on
+// one XCD (dispatch is round-robin over 8), whose L2 then serves the segment's
+// rows to every tile; fewer are spread over all (1,457,500 pairs x 3,000 bars, two
+// segments: 682 us, 2,304 on two XCDs).
 //
 // Bound: VALU issue (88% of the issue slots): 2.5 instructions per pair and bar
 // (subtract, shift, half a minimum), 0.4 for the words' sums and 0.5 for the
@@ -189,7 +191,8 @@ __device__ __forceinline__ double cross_pos(int at) { return at == 0 ? 1.0 : (at
 // r (r + 1) / 2: the sum of t + 1 over [0, r)
 __device__ __forceinline__ long long tri(int r) { return ((long long)r * ((long long)r + 1)) >> 1; }
 
-// grid.x = 8 x ceil(nseg / 8) x ntiles, block = one wave.  WIDE: the rows take
+// grid.x = 8 x ceil(nseg / 8) x ntiles (nseg x ntiles below eight segments),
+// block = one wave.  WIDE: the rows take
 // 4 GiB or more, so a lane's row offsets need 64 bits (else a scalar base and
 // 32-bit lane offsets, which keep 24 registers and the address arithmetic
 // out of the word loop).
@@ -198,8 +201,9 @@ __device__ __forceinline__ void cross_pairs(const cross_args &a) {
     __shared__ __align__(16) double lr[(CR_F + CR_S) * CR_LD];   // fast rows, then slow
     __shared__ double lx[CR_CH];                 // the word's prices
     const int lane = threadIdx.x;
-    const int in = blockIdx.x >> 3;
-    const int seg = (in / a.ntiles) * 8 + (blockIdx.x & 7);
+    const bool by8 = a.nseg >= 8;                // (fewer would leave XCDs idle)
+    const int in = by8 ? blockIdx.x >> 3 : blockIdx.x;
+    const int seg = by8 ? (in / a.ntiles) * 8 + (blockIdx.x & 7) : in / a.ntiles;
     if (seg >= a.nseg) return;
     const int tile = in % a.ntiles;
     const int f0 = tile / a.ntiles_s * CR_F, s0 = tile % a.ntiles_s * CR_S;
