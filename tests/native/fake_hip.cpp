@@ -30,6 +30,7 @@ void fake_hip_wait_for_waiter() {
     std::unique_lock<std::mutex> lk(g_mu);
     g_cv.wait(lk, [] { return g_waiting > 0; });
 }
+void fake_hip_memory(size_t bytes) { g_total = bytes; }
 size_t fake_hip_launches() {
     std::lock_guard<std::mutex> lk(g_mu);
     return g_launches;

@@ -1,6 +1,6 @@
 // Admission of the request server under a full memory budget, without a device
 // (fake_hip.cpp).  One scenario per run, named by argv[1]; exit status 0 when
-// it holds.  Built with AddressSanitizer by tests/test_server_admission.py.
+// it holds.  Built with AddressSanitizer by tests/test_host_memory.py.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>

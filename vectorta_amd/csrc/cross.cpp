@@ -136,13 +136,21 @@ vta_status plan_build(vta_ctx *ctx, const float *prices, size_t len,
         const long v = atol(e);
         if (v >= 1) waves = (size_t)v;
     }
-    size_t nseg = (waves + ntiles - 1) / ntiles;
+    const size_t least = (len + kSegMax - 1) / kSegMax;
+    size_t nseg = (waves + ntiles - 1) / ntiles, seg_len;
     nseg = std::min((nseg + 7) & ~(size_t)7, std::max<size_t>(1, len / kSegMin));
-    nseg = std::max(nseg, (len + kSegMax - 1) / kSegMax);
-    size_t seg_len = (len + nseg - 1) / nseg;
-    seg_len = (seg_len + kWord - 1) / kWord * kWord;
-    nseg = (len + seg_len - 1) / seg_len;
-    VTA_TRY(check_fits(rows_bytes + nseg * npairs * 28 + npairs * 40 + len * 4));
+    nseg = std::max(nseg, least);
+    // (fewer where the partials of a grid of 10^9 pairs would not fit)
+    for (;; nseg = std::max(nseg / 2, least)) {
+        seg_len = (len + nseg - 1) / nseg;
+        seg_len = (seg_len + kWord - 1) / kWord * kWord;
+        nseg = (len + seg_len - 1) / seg_len;
+        const vta_status fits =
+            check_fits(rows_bytes + nseg * npairs * 28 + npairs * 40 + len * 4);
+        if (fits == VTA_OK) break;
+        if (nseg <= least) return fits;
+    }
+    clear_error();
 
     auto *plan = new vta_double_alma_plan();
     plan->ctx = ctx;
