@@ -532,3 +532,36 @@ def test_window_forms_signed_zeros(ops, monkeypatch):
                 g = _with_form(mad.ctx, form, lambda: mad.medium_ad_many_series_one_param_time_major_dev(
                     x, cols, rows, p).to_host())
                 _exact(g, ref, f"mad zeros form {form} period {p} chunk {chunk}")
+
+
+def test_bb_batch_device_of_the_longest_series():
+    """2^31 - 1 bars, the most an int32 length takes, in one combo (8.6 GB of
+    prices, 25.8 GB of bands): the first and last bars equal, bit for bit, those
+    of a short call over them (each window is summed by itself)."""
+    require_gpu()
+    ctx, L, P = vta.HipContext(0), vta.lib(), ctypes.c_void_p
+    T, n, p = 2**31 - 1, 6_000, 20
+    block = datagen.gbm_close(1 << 24, 0.0001, seed=99)
+    d_x = ctx.alloc(T * 4)
+    for t in range(0, T, block.size):
+        m = min(block.size, T - t)
+        check(L.vta_memcpy_htod(ctx.handle, P(d_x.ptr + 4 * t), block.ctypes.data_as(P), 4 * m))
+    d_p, d_d = ctx.to_device(np.int32([p])), ctx.to_device(np.float64([2.0]))
+    outs = [ctx.alloc(T * 4) for _ in range(3)]
+
+    def run(x, length, out):
+        check(L.vta_bollinger_bands_batch_device(ctx.handle, P(x), length, 0, length, P(d_p.ptr),
+                                                 P(d_d.ptr), P(d_d.ptr), 1, p,
+                                                 *(P(o) for o in out)))
+        ctx.synchronize()
+
+    run(d_x.ptr, T, [o.ptr for o in outs])
+    short = [ctx.alloc(n * 4) for _ in range(3)]
+    for t in (0, T - n):
+        run(d_x.ptr + 4 * t, n, [o.ptr for o in short])
+        for o, s in zip(outs, short):
+            got = np.empty(n, np.uint32)
+            check(L.vta_memcpy_dtoh(ctx.handle, got.ctypes.data_as(P), P(o.ptr + 4 * t), 4 * n))
+            assert np.array_equal(got[p - 1:], s.copy_to_host(np.uint32)[p - 1:]), t
+    for b in (d_x, d_p, d_d, *outs, *short):
+        b.free()
