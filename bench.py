@@ -329,7 +329,7 @@ def bench_rolling(steps, warmup, ev):
     res = {"workload": "bb20_pnr100p70_mad64_many_series_1024x50000"}
     from vectorta_amd import autotune as at
     # PNR window 100 and MAD window 64 run the register-window kernels (window
-    # rounded up to 16 slots); the LDS sorted-window form is timed beside them
+    # rounded up to 4 slots, MAD 2); the LDS sorted-window form is timed beside them
     for name, fn, nout, kern, lds_kern in (
             ("bb", lambda: plan.launch_bb(20, 2.0, 2.0), 3, "bb_ms1p_f32", None),
             ("pnr", lambda: plan.launch_pnr(100, 70.0), 1, "pnr_ms1p_reg100", "pnr_ms1p_f32"),

@@ -231,24 +231,28 @@ def test_same_bits_wherever_the_rows_lie(name, n, combos):
         b.free()
 
 
-def test_wilders_seeded_matches_replay(monkeypatch):
-    """Wilders batches of up to 4,096 combos start each exact lane from a
-    per-combo seed at its last warm-up bar; larger ones replay the warm-up
-    from first_valid.  Both are the same arithmetic, so with one chunk length
-    the 4,096 rows of a seeded batch equal bit for bit those of a 4,097-combo
-    batch over the same periods, and a sample of rows matches the oracle."""
+def test_wilders_long_warm_ups_scan_and_exact_lanes(monkeypatch):
+    """Wilders with warm-ups of up to sixteen 256-bar chunks (periods to 4,096 on a
+    late first_valid): the chunked scan, whose sums start from zero chunk by
+    chunk, against the same call on exact lanes (each from first_valid, the seed
+    summed in groups of four as the oracle's) and a sample of rows of both
+    against the oracle."""
     require_gpu()
     monkeypatch.setenv("VTA_SCAN_CHUNK", "256")
     _, _, c = _hlc(9_000, 37, lead=700)
     op = vta.CudaWilders(0)
-    seeded = op.wilders_batch_dev(c, (1, 4_096, 1)).to_host()
-    replay = op.wilders_batch_dev(c, (1, 4_097, 1)).to_host()
-    assert seeded.shape == (4_096, 9_000) and replay.shape == (4_097, 9_000)
-    assert np.array_equal(seeded.view(np.uint32), replay[:4_096].view(np.uint32))
-    rows = [0, 1, 2, 3, 4, 13, 255, 256, 1_000, 4_095]
+    scan = op.wilders_batch_dev(c, (1, 4_097, 1)).to_host()
+    monkeypatch.setenv("VTA_REC_NO_SCAN", "1")
+    exact = op.wilders_batch_dev(c, (1, 4_097, 1)).to_host()
+    assert scan.shape == exact.shape == (4_097, 9_000)
+    rows = [0, 1, 2, 3, 4, 13, 255, 256, 257, 1_000, 4_095, 4_096]
     ref = np.stack([O.wilders(c.astype(np.float64), r + 1) for r in rows])
-    nan_mask_equal(seeded[rows], ref)
-    assert max_rel_err(seeded[rows], ref, floor=0.0) <= 1e-5
+    for g in (scan, exact):
+        nan_mask_equal(g[rows], ref)
+        assert max_rel_err(g[rows], ref, floor=0.0) <= 1e-5
+    nan_mask_equal(scan, exact)
+    # both round f64 averages within 1e-9 of each other (a burnt-in lane 2.1e-9)
+    assert max_rel_err(scan, exact.astype(np.float64)) <= 2.0**-23 + 5e-9
 
 
 @pytest.mark.parametrize("n,period", [(3_000, (1, 60, 11)), (300_000, (14, 250, 59))])

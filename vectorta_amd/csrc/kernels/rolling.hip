@@ -35,7 +35,6 @@ struct roll_args {
     const float *x;
     const int32_t *p_len;    // batch: per combo
     const double *p_a;       // batch: PNR percentage per combo
-    const double *p_b;
     const int32_t *fvs;      // many-series: per series; batch: [0]
     const int32_t *poison;   // BB: first non-finite bar >= first_valid, per series;
                              // null means none known (one chunk)

@@ -20,7 +20,6 @@ struct roll_args_host {
     const float *x;
     const int32_t *p_len;
     const double *p_a;
-    const double *p_b;
     const int32_t *fvs;
     const int32_t *poison;
     float *out0;
@@ -35,7 +34,7 @@ struct roll_args_host {
     int p1;
     int pad_;
 };
-static_assert(sizeof(roll_args_host) == 112, "roll_args layout");
+static_assert(sizeof(roll_args_host) == 104, "roll_args layout");
 
 enum RInd { R_BB = 0, R_PNR = 1, R_MAD = 2 };
 
@@ -47,7 +46,8 @@ enum RInd { R_BB = 0, R_PNR = 1, R_MAD = 2 };
 // these kernels are bound by the latency of each lane's LDS shift chain, so a
 // second round costs a whole chunk's time); at least 4x the
 // window so the per-chunk rebuild stays a small fraction, at most 4096 bars
-// (BB re-anchors its f64 running sums at every chunk start).  `chunked`
+// (BB re-anchors its f64 running sums at every chunk start; its one-series
+// batches have chunks only for periods above 2,048, see bb_job_of).  `chunked`
 // false: one chunk.
 int roll_chunk(const vta_ctx *ctx, size_t T, size_t lanes, size_t max_w, bool chunked,
                size_t smem, size_t bb_waves = 8192) {
@@ -284,15 +284,14 @@ vta_status batch_dev(vta_ctx *ctx, RInd k, const float *x, size_t len,
         pa[i] = cs[i].a;
         pb[i] = cs[i].b;
     }
-    int32_t meta[2] = {(int32_t)fv, first_nonfinite(x, len, fv, 1)};
-    DevBuf dx, dl, da, db, dm, o[3];
+    DevBuf dx, dl, da, db, o[3];
     VTA_TRY(upload(ctx, dx, x, len * sizeof(float)));
     VTA_TRY(upload(ctx, dl, pl.data(), C * sizeof(int32_t)));
     VTA_TRY(upload(ctx, da, pa.data(), C * sizeof(double)));
-    VTA_TRY(upload(ctx, db, pb.data(), C * sizeof(double)));
-    VTA_TRY(upload(ctx, dm, meta, sizeof(meta)));
     for (int i = 0; i < nout; ++i) VTA_TRY(o[i].alloc(n_out));
+    DevBuf dm;
     if (k == R_BB) {
+        VTA_TRY(upload(ctx, db, pb.data(), C * sizeof(double)));
         vta_bb_job q{};
         q.d_prices = dx.as<float>();
         q.d_periods = dl.as<int32_t>();
@@ -302,25 +301,24 @@ vta_status batch_dev(vta_ctx *ctx, RInd k, const float *x, size_t len,
         q.d_middle = o[1].as<float>();
         q.d_lower = o[2].as<float>();
         q.series_len = (int32_t)len;
-        q.first_valid = meta[0];
-        q.first_nonfinite = meta[1];
+        q.first_valid = (int32_t)fv;
+        q.first_nonfinite = first_nonfinite(x, len, fv, 1);
         q.n_combos = (int32_t)C;
         q.max_period = (int32_t)mx;
         VTA_TRY(bb_batch_launch(ctx, q));
+    } else {
+        const int32_t fv32 = (int32_t)fv;
+        VTA_TRY(upload(ctx, dm, &fv32, sizeof fv32));
+        roll_args_host a{};
+        a.x = dx.as<float>();
+        a.p_len = dl.as<int32_t>();
+        a.p_a = da.as<double>();
+        a.fvs = dm.as<int32_t>();
+        a.out0 = o[0].as<float>();
+        a.T = (int)len;
+        a.nlanes = (int)C;
+        VTA_TRY(roll_launch(ctx, k, true, a, mx, true));
     }
-    roll_args_host a{};
-    a.x = dx.as<float>();
-    a.p_len = dl.as<int32_t>();
-    a.p_a = da.as<double>();
-    a.p_b = db.as<double>();
-    a.fvs = dm.as<int32_t>();
-    a.poison = dm.as<int32_t>() + 1;
-    a.out0 = o[0].as<float>();
-    a.out1 = o[1].as<float>();
-    a.out2 = o[2].as<float>();
-    a.T = (int)len;
-    a.nlanes = (int)C;
-    if (k != R_BB) VTA_TRY(roll_launch(ctx, k, true, a, mx, true));
     VTA_HIP(hipStreamSynchronize(ctx->stream));
     for (int i = 0; i < nout; ++i) {
         out[i].ptr = static_cast<float *>(o[i].release());
