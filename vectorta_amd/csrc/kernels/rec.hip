@@ -59,8 +59,8 @@ struct rec_args {
     int tstride;
     int scan;                // batch: 0 burn-in / exact lanes, else the scan (ADX: stage 1 or 2)
     int epoch;               // batch: of the call, 0: counted on the device (scan_flags)
-    int rag;                 // batch scan: whole lines of rows that start anywhere (scan_output)
     int last;                // batch: the call's last output pass
+    int pad_;
 };
 
 // Words of a one-series batch's flags, and of a pack's after its jobs'.  A flag
@@ -870,7 +870,7 @@ struct batch_view {
     int T, nlanes, chunk, nch, groups, span, fv, t0, t1, tstride, scan, group;
     int kb, k;               // the block's first chunk, this wave's
     int32_t epoch;           // see scan_flags
-    bool clean, odd, coop, rag;
+    bool clean, odd, coop;
 };
 
 // A block is REC_WPB waves: with that many combo groups, one chunk of as many
@@ -929,7 +929,6 @@ __device__ __forceinline__ batch_view view_of(const rec_args &a) {
         v.clean = a.clean[SF_BAD] != v.epoch;
         v.odd = a.clean[SF_ODD] == v.epoch;
     }
-    v.rag = a.rag != 0;
     return v;
 }
 
@@ -1565,8 +1564,9 @@ __device__ __forceinline__ float scan_dx(double diff, double all) {
 // stage from zero for its scan.  Blocks of 32 bars past every sum run the
 // plain updates, eight terms at a time; the others select per bar.
 //
-// RAG (rows that do not all start on a 128-byte line): a wave keeps its last
-// two tiles of 32 bars and stores whole lines only, those that start in its
+// RAG (rows that do not all start on a 128-byte line; kernels of their own,
+// *_batch_lines_f32, or short calls would fetch the longer code): a wave keeps its
+// last two tiles of 32 bars and stores whole lines only, those that start in its
 // chunk; for the last of them it runs one tile into the next chunk, from that
 // chunk's own start state, so that the rows' bits are those of tiles.  Stored
 // tile by tile, each line of such rows is written in two parts some
@@ -1830,7 +1830,7 @@ __device__ __forceinline__ void scan_pass2(const batch_view &a) {
     if (a.odd) scan_output<AdxEng, true, false>(a, nullptr);
     else scan_output<AdxEng, false, false>(a, nullptr);
 }
-template <class E, int NIN>
+template <class E, int NIN, bool RAG>
 __device__ __forceinline__ void batch_pass(batch_view a, float *out) {
     if (a.scan == 0) {
         if (!wave_idle(a)) drive_batch<E, NIN>(a, out);
@@ -1839,12 +1839,9 @@ __device__ __forceinline__ void batch_pass(batch_view a, float *out) {
         a.chunk = a.T;
         drive_batch<E, NIN>(a, out);
     } else if (__is_same(E, AdxEng) && a.odd) {
-        if (a.rag) scan_output<E, true, true, true>(a, out);
-        else scan_output<E, true, true>(a, out);
-    } else if (a.rag) {
-        scan_output<E, false, true, true>(a, out);
+        scan_output<E, true, true, RAG>(a, out);
     } else {
-        scan_output<E, false, true>(a, out);
+        scan_output<E, false, true, RAG>(a, out);
     }
 }
 template <class E>
@@ -1934,7 +1931,6 @@ __device__ __forceinline__ batch_view pack_view(const rec_pack_args &p, int j) {
     v.epoch = p.epoch ? p.epoch : OUT ? p.call[0] : p.call[1] + 1;
     v.clean = p.flags[2 * f] != v.epoch;
     v.odd = p.flags[2 * f + 1] == v.epoch;
-    v.rag = false;
     v.group = v.kb = v.k = 0;
     v.coop = false;
     return v;
@@ -1965,6 +1961,17 @@ __device__ __forceinline__ void leave_epoch(const batch_view &v, const int32_t *
     if (blockIdx.x == 0 && threadIdx.x == 0) *const_cast<int32_t *>(word) = v.epoch;
 }
 
+// Waves per SIMD of the direct output passes, what their LDS allows: scheduled
+// for more they take longer (33 RSI x 10,007 bars 18.2 us, 17.8 so; 1,250 ADX x
+// 200,000 457 and 452).  Packed, it is the other way round (27 ADX jobs 43.5 us,
+// 44.2 so).
+#define REC_WPE __attribute__((amdgpu_waves_per_eu(4, 4)))
+#define REC_OUTPUT(KERNEL, ENG, NIN, RAG)                                                    \
+    extern "C" __global__ __launch_bounds__(256) REC_WPE void KERNEL(rec_args a) {           \
+        const batch_view v = view_of<true>(a);                                               \
+        batch_pass<ENG, NIN, RAG>(v, a.out0);                                                \
+        if (!a.epoch && a.last && a.clean) leave_epoch(v, a.clean + SF_LAST);                \
+    }
 #define REC_BATCH(NAME, ENG, NIN)                                                            \
     extern "C" __global__ __launch_bounds__(256) void NAME##_scan_states(rec_args a) {       \
         const batch_view v = view_of<false>(a);                                              \
@@ -1975,11 +1982,8 @@ __device__ __forceinline__ void leave_epoch(const batch_view &v, const int32_t *
         batch_view v = view_of<false>(a);                                                    \
         span_pass<ENG>(v, blockIdx.x);                                                       \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_batch_f32(rec_args a) {         \
-        const batch_view v = view_of<true>(a);                                               \
-        batch_pass<ENG, NIN>(v, a.out0);                                                     \
-        if (!a.epoch && a.last && a.clean) leave_epoch(v, a.clean + SF_LAST);                \
-    }
+    REC_OUTPUT(NAME##_batch_f32, ENG, NIN, false)                                            \
+    REC_OUTPUT(NAME##_batch_lines_f32, ENG, NIN, true)
 #define REC_PACKED_(NAME, ENG, NIN, SEG, X)                                                  \
     extern "C" __global__ __launch_bounds__(256) void NAME##_packed_states##X(               \
         rec_pack_args p) {                                                                   \
@@ -1991,10 +1995,10 @@ __device__ __forceinline__ void leave_epoch(const batch_view &v, const int32_t *
     extern "C" __global__ __launch_bounds__(64) void NAME##_packed_spans##X(rec_pack_args p) {\
         packed_spans<ENG, SEG>(p);                                                           \
     }                                                                                        \
-    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32##X(rec_pack_args p) {\
+    extern "C" __global__ __launch_bounds__(256) void NAME##_packed_f32##X(rec_pack_args p) { \
         float *out;                                                                          \
         const batch_view v = pack_block<SEG, true>(p, &out);                                 \
-        batch_pass<ENG, NIN>(v, out);                                                        \
+        batch_pass<ENG, NIN, false>(v, out);                                                 \
         if (!p.epoch && p.last) leave_epoch(v, p.call + 1);                                  \
     }
 #define REC_PACKED(NAME, ENG, NIN)                                                           \

@@ -44,8 +44,8 @@ struct rec_args_host {
     int tstride;
     int scan;
     int epoch;
-    int rag;
     int last;
+    int pad_;
 };
 static_assert(sizeof(rec_args_host) == 192, "rec_args layout");
 
@@ -62,11 +62,16 @@ enum Ind {
 // Indicators computed from (high, low, close).
 bool hlc(Ind k) { return k == IND_ATR || k == IND_ADX; }
 
-const char *batch_kernel(Ind k) {
-    static const char *n[] = {"ema_batch_f32",  "rsi_batch_f32",     "atr_batch_f32",
-                              "adx_batch_f32",  "smma_batch_f32",    "wilders_batch_f32",
-                              "atr_tr_batch_f32"};
-    return n[k];
+// (lines: rows stored by whole lines, see ragged_rows)
+const char *batch_kernel(Ind k, bool lines = false) {
+    static const char *n[][2] = {{"ema_batch_f32", "ema_batch_lines_f32"},
+                                 {"rsi_batch_f32", "rsi_batch_lines_f32"},
+                                 {"atr_batch_f32", "atr_batch_lines_f32"},
+                                 {"adx_batch_f32", "adx_batch_lines_f32"},
+                                 {"smma_batch_f32", "smma_batch_lines_f32"},
+                                 {"wilders_batch_f32", "wilders_batch_lines_f32"},
+                                 {"atr_tr_batch_f32", "atr_tr_batch_lines_f32"}};
+    return n[k][lines];
 }
 const char *ms_kernel(Ind k) {
     static const char *n[] = {"ema_ms1p_f32",  "rsi_ms1p_f32",  "atr_ms1p_f32",
@@ -323,7 +328,6 @@ vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
     hipFunction_t fs, ff, fb, f2 = nullptr;
     VTA_TRY(get_function(ctx, "rec", states_kernel(k), &fs));
     VTA_TRY(get_function(ctx, "rec", spans_kernel(k), &ff));
-    VTA_TRY(get_function(ctx, "rec", batch_kernel(k), &fb));
     if (k == IND_ADX) VTA_TRY(get_function(ctx, "rec", "adx_scan_stage2", &f2));
     const size_t row = S * a.groups * 64;
     double *handed[2] = {static_cast<double *>(ctx->carry), nullptr};
@@ -331,7 +335,8 @@ vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
     a.carry = seg < T ? handed[1] + row : handed[0];
     a.terms = ctx->terms;
     a.chunk = (int)chunk;
-    a.rag = ragged_rows(a);
+    const bool rag = ragged_rows(a);
+    VTA_TRY(get_function(ctx, "rec", batch_kernel(k, rag), &fb));
     for (size_t t0 = 0, n = 0; t0 < T; t0 += seg, ++n) {
         const size_t t1 = std::min(T, t0 + seg);
         const size_t nch = (t1 - t0 + chunk - 1) / chunk;
@@ -361,7 +366,7 @@ vta_status scan_launch(vta_ctx *ctx, Ind k, rec_args_host a, size_t chunk,
         }
         a.scan = 1;
         a.last = t1 == T;
-        VTA_TRY(launch(ctx, fb, grid, block, a.rag ? kWpb * kRagLds : batch_lds_bytes(k), a));
+        VTA_TRY(launch(ctx, fb, grid, block, rag ? kWpb * kRagLds : batch_lds_bytes(k), a));
     }
     return VTA_OK;
 }

@@ -401,6 +401,13 @@ vta_status vta_ctx_preload(vta_ctx *ctx) {
         {"rec", "wilders_scan_spans"},
         {"rec", "atr_tr_scan_spans"},
         {"rec", "atr_tr_batch_f32"},
+        {"rec", "ema_batch_lines_f32"},
+        {"rec", "rsi_batch_lines_f32"},
+        {"rec", "atr_batch_lines_f32"},
+        {"rec", "adx_batch_lines_f32"},
+        {"rec", "smma_batch_lines_f32"},
+        {"rec", "wilders_batch_lines_f32"},
+        {"rec", "atr_tr_batch_lines_f32"},
         {"rec", "tr_from_hlc_f32"},
         {"rec", "smma_batch_f32"},
         {"rec", "wilders_batch_f32"},
