@@ -440,13 +440,16 @@ vta_status vta_atr_batch_device_with_tr(vta_ctx *ctx, const float *d_tr, const i
 /* No counterpart in the reference, whose wrappers run one series per call.
  * Many one-series batches of one recurrence indicator -- series of uneven
  * lengths, each with its own period table -- in one launch per scan pass
- * through a device job table (offsets of every job's blocks and combos).
+ * through a device job table (offsets of every job's blocks and spans), and one
+ * per pass and segment where a job's own call runs in segments (EMA, ATR, SMMA
+ * and Wilders above 1,048,576 bars, RSI half, ADX a third of that).
  * Each job's outputs are bit-identical to its own vta_<ind>_batch_device call
  * on a context with the same tuning (same chunking, same kernels), except
- * where that call would skip the scan for a grid of more than ~260k combos
- * (the pack then runs the job exactly in one chunk: within the parity bound).
+ * where that call would skip the scan for a grid of more than ~600k (ADX),
+ * 1.2M (RSI) or 2.4M combos (the pack then runs the job exactly in one chunk:
+ * within the parity bound).
  * vta_rec_pack_create validates the jobs like the _device forms, uploads the
- * table and allocates the pack's own chunk-carry buffer and flags (so
+ * table and allocates the pack's own buffer of terms, chunk states and flags (so
  * launches allocate nothing); vta_rec_pack_launch is enqueue-only (graph-
  * capturable).  Job pointers are device pointers that must stay valid while
  * the pack is used; a launch overwrites every job's output. */

@@ -284,7 +284,7 @@ __device__ __forceinline__ void bb_tile_body(const bb_job &a, int local) {
     __shared__ int p_s[BB_COMBOS];
     const int tid = threadIdx.x;
     const int T = a.T, hist = a.hist, n = hist + BB_BT;
-    const int tiles = (int)(((unsigned)T + BB_BT - 1) / BB_BT);   // (T may be 2^31 - 1)
+    const int tiles = T / BB_BT + (T % BB_BT != 0);         // (T may be 2^31 - 1)
     const int t0 = local % tiles * BB_BT, cg = local / tiles * a.chunk;
     const int nc = min(a.chunk, a.nlanes - cg);
     bb_pair *w16 = reinterpret_cast<bb_pair *>(bb_lds);     // [n]: bars j - 15 .. j

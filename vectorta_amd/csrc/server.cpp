@@ -11,8 +11,9 @@
 // when admission needs room.  A request's outputs and series are placed in the
 // device memory as it is admitted: the budget counts bytes, and with results
 // of all sizes between the free ones a request that it holds may still find no
-// block long enough, and then waits for one like for the budget.  The kernels are the library's public entry
-// points, so a result is bit-identical whether the request runs alone or in
+// block long enough, and then waits for one like for the budget.  The kernels
+// are the library's public entry points, so a result is bit-identical whether
+// the request runs alone or in
 // a mix.
 #include <algorithm>
 #include <chrono>
