@@ -132,10 +132,10 @@ def test_word_and_tile_edges_bit_exact(cx, bars, lead, fast, slow):
     _check(got, ref, f"{bars} bars")
 
 
-@pytest.mark.parametrize("bars", [700, 3_000, 8_191, 8_192, 9_300])
+@pytest.mark.parametrize("bars", [100, 190, 511, 512, 700, 8_191, 9_300])
 def test_segments_below_and_from_eight_on_bit_exact(cx, bars):
-    """One, two and seven segments, whose tiles go to all XCDs, eight and nine,
-    each segment on one XCD; 3 x 2 tiles."""
+    """One, two and seven segments of at least 64 bars, whose tiles go to all XCDs,
+    eight and more, each segment on one XCD; 3 x 2 tiles."""
     x = datagen.gbm_close(bars, 0.015, seed=bars)
     f = vta.AlmaBatchRange(period=(5, 44, 1), **_ONE)
     s = vta.AlmaBatchRange(period=(50, 80, 1), **_ONE)

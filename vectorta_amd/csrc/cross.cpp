@@ -49,11 +49,19 @@ constexpr size_t kWord = 32;              // bars per word of the walk (CR_CH)
 // Waves of the pair walk (16 x 16 pairs x one time segment each).  Tiles of
 // short periods trade more often and walk longer, so small units balance the
 // device: 58,300 pairs x 200k bars took 2.46 / 2.31 / 2.21 / 2.20 ms (the
-// whole call) at 4,096 / 8,192 / 16,384 / 32,768 waves.  Segments are at least
-// 1,024 bars (the partials of a segment are read again) and a multiple of 8
-// in number (one XCD takes every 8th).
+// whole call) at 4,096 / 8,192 / 16,384 / 32,768 waves.  Segments are a multiple
+// of 8 in number (one XCD takes every 8th) and at least 1,024 bars, since the
+// partials of a segment are read again, but where that leaves fewer than those
+// waves a walk is a serial chain, and segments go down to 64 bars (the whole
+// call in us at 1,024 / 256 / 128 / 64, and with 2,048 bars, a pair per lane and
+// a branch per bar before):
+//   58,300 pairs x 300 bars      67 / 67 / 57 / 51 (53)
+//   58,300 x 700                 99 / 68 / 59 / 54 (90)
+//   58,300 x 3,000              161 / 87 / 93 / 90 (318)
+//   496 x 3,000                 139 / 50 / 42 / 37 (350)
+//   58,300 x 10,000             209 / 161 / 163 / 167 (378)
 constexpr size_t kCrossWaves = 16384;
-constexpr size_t kSegMin = 1024;
+constexpr size_t kSegMin = 1024, kSegShort = 64;
 constexpr size_t kSegMax = (size_t)1 << 18;   // CrossRun::s2
 
 // f64 batch weights in the oracle's order (alma.rs:1426-1436), not normalised.
@@ -137,9 +145,9 @@ vta_status plan_build(vta_ctx *ctx, const float *prices, size_t len,
         if (v >= 1) waves = (size_t)v;
     }
     const size_t least = (len + kSegMax - 1) / kSegMax;
-    size_t nseg = (waves + ntiles - 1) / ntiles, seg_len;
-    nseg = std::min((nseg + 7) & ~(size_t)7, std::max<size_t>(1, len / kSegMin));
-    nseg = std::max(nseg, least);
+    const size_t want = (waves + ntiles - 1) / ntiles;
+    size_t nseg = std::min((want + 7) & ~(size_t)7, len / kSegMin), seg_len;
+    nseg = std::max({nseg, std::min(want, std::max<size_t>(1, len / kSegShort)), least});
     // (fewer where the partials of a grid of 10^9 pairs would not fit)
     for (;; nseg = std::max(nseg / 2, least)) {
         seg_len = (len + nseg - 1) / nseg;

@@ -34,8 +34,8 @@
 // before it from the rows, so the segments are independent; cross_reduce sums
 // them in segment order.  From eight segments on all tiles of a segment run on
 // one XCD (dispatch is round-robin over 8), whose L2 then serves the segment's
-// rows to every tile; fewer are spread over all (1,457,500 pairs x 3,000 bars, two
-// segments: 682 us, 2,304 on two XCDs).
+// rows to every tile; fewer are spread over all (1,457,500 pairs x 3,000 bars in
+// two segments: 682 us, 2,304 on two XCDs).
 //
 // Bound: VALU issue (88% of the issue slots): 2.5 instructions per pair and bar
 // (subtract, shift, half a minimum), 0.4 for the words' sums and 0.5 for the
